@@ -556,8 +556,8 @@ hipError_t batch_capture_any(hdog_ctx* ctx, BatchState* B) {
 }
 
 // ---- autotuner of the run-time launch shapes ---------------------------------------
-// Candidate row-segment counts of the two row walkers, 1..4; counts that give the same
-// segmentation as a smaller one are skipped.
+// Candidate launch shapes of the two row walkers, 1..4 halves of the built-in segment count
+// (walk_segments); shapes that equal an earlier candidate's are timed once.
 constexpr int kMaxSegments = 4;
 
 // median of three event-timed runs of f (after one untimed run)
@@ -599,64 +599,43 @@ int autotune_t(hdog_ctx* ctx, hipStream_t s, const hdog_params* p, const uint16_
   const float nz = powf(ctx->sigma[0], p->gamma * 2) * powf(ctx->sigma[1], p->gamma);
   const int wb_gauss = 2 * std::max(ctx->r[0], ctx->r[2]) + 1;
   struct Stage {
-    int wb, *best;
+    int wb;
+    i64 strips;  // waves per segment, all planes
+    int* best;
     float* ms;
     bool dog;
-  } stages[2] = {{21, best_norm, ms_norm, false}, {wb_gauss, best_gauss, ms_gauss, true}};
+  } stages[2] = {{21, (i64)((W + 127) / 128) * D, best_norm, ms_norm, false},
+                 {wb_gauss, (i64)((W + 63) / 64) * D, best_gauss, ms_gauss, true}};
   for (const Stage& st : stages) {
-    // the built-in segment count stays unless another one is faster by more than 3 %: a
+    // the built-in shape (choice 2) stays unless another one is faster by more than 3 %: a
     // choice within the timing noise would change nothing but the launch shape
-    int def_nys, def_rows;
-    walk_segments(H, st.wb, &def_nys, &def_rows);
-    float def_ms = 1e30f;
-    int cand_want[kMaxSegments], ncand = 0;
-    float cand_ms[kMaxSegments];
-    int seen[kMaxSegments + 1] = {0};
-    int nseen = 0;
+    float ms[kMaxSegments + 1];
+    int nys[kMaxSegments + 1];
     for (int want = 1; want <= kMaxSegments; ++want) {
-      int nys, rows;
-      walk_segments(H, st.wb, &nys, &rows, want);
-      bool dup = false;
-      for (int k = 0; k < nseen; ++k) dup |= seen[k] == nys;
-      if (dup) continue;
-      seen[nseen++] = nys;
-      float ms = 0.0f;
+      int rows;
+      walk_segments(H, st.wb, st.strips, &nys[want], &rows, want);
+      ms[want] = -1.0f;
+      for (int k = 1; k < want; ++k)
+        if (nys[k] == nys[want]) ms[want] = ms[k];  // the same shape
+      if (ms[want] >= 0.0f) continue;
       if (st.dog)
         HIPCHK(time_median(s, [&] {
           return launch_dog<TN, TD>(norm, dog, tmp1, tmp2,
                                     (const float*)ctx->weights.p, ctx->r, nz, W, H, D, s, want);
-        }, &ms));
+        }, &ms[want]));
       else
         HIPCHK(time_median(s, [&] {
           return launch_normalize<TN>(img, norm, tmp1, tmp2, p->min_intensity, W, H,
                                       D, p->radius_xy, p->radius_z, s, nullptr, nullptr, want);
-        }, &ms));
-      cand_want[ncand] = want;
-      cand_ms[ncand++] = ms;
-      if (nys == def_nys) def_ms = ms;
+        }, &ms[want]));
     }
-    *st.best = 0;
-    *st.ms = def_ms;
-    for (int k = 0; k < ncand; ++k) {
-      int nys, rows;
-      walk_segments(H, st.wb, &nys, &rows, cand_want[k]);
-      if (nys == def_nys) {
-        if (*st.best == 0) *st.best = cand_want[k];  // the default's own entry
-      } else if (cand_ms[k] < 0.97f * def_ms && cand_ms[k] < *st.ms) {
-        *st.ms = cand_ms[k];
-        *st.best = cand_want[k];
+    *st.best = 2;
+    *st.ms = ms[2];
+    for (int want = 1; want <= kMaxSegments; ++want)
+      if (nys[want] != nys[2] && ms[want] < 0.97f * ms[2] && ms[want] < *st.ms) {
+        *st.ms = ms[want];
+        *st.best = want;
       }
-    }
-    // the default is among the candidates (1 or 2 segments); otherwise the fastest
-    if (*st.best == 0) {
-      *st.best = cand_want[0];
-      *st.ms = cand_ms[0];
-      for (int k = 1; k < ncand; ++k)
-        if (cand_ms[k] < *st.ms) {
-          *st.ms = cand_ms[k];
-          *st.best = cand_want[k];
-        }
-    }
     if (!st.dog)  // the DoG stage is timed on the normalized stack
       HIPCHK(launch_normalize<TN>(img, norm, tmp1, tmp2, p->min_intensity, W, H, D,
                                   p->radius_xy, p->radius_z, s, nullptr, nullptr, *st.best));

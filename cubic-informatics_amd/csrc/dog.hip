@@ -171,20 +171,22 @@ __global__ __launch_bounds__(NT) void k_gauss_walk(const float2* __restrict__ sr
                                                    float2* __restrict__ dst, TS* __restrict__ dog,
                                                    const float* __restrict__ w1,
                                                    const float* __restrict__ w2, float nz, int W,
-                                                   int L, i64 sa, i64 so, int nxb) {
+                                                   int L, i64 sa, i64 so, unsigned nxb,
+                                                   unsigned no, int len) {
   constexpr int R = R1 > R2 ? R1 : R2;
   constexpr int WB = 2 * R + 1;
   constexpr int PF = WB % 3 == 0 ? 3 : WB % 5 == 0 ? 5 : WB % 7 == 0 ? 7 : 1;
-  const int x = (blockIdx.x % nxb) * NT + threadIdx.x;
+  const LineAt la = line_at_block(nxb, no, len, L);
+  const int x = la.x, b0 = la.c0, b1 = la.c1;
   if (x >= W) return;
-  const i64 base = (i64)(blockIdx.x / nxb) * so + x;
+  const i64 base = (i64)la.other * so + x;
   // zero padding in the load itself: position p is read through a buffer descriptor of
   // the wave's 64 columns at p (a uniform base), whose record count is 0 outside the
   // line, so those loads return zeros and no value is tested (or waited for) when it
   // enters the ring
   const int lane = (int)(threadIdx.x & 63);
   const int xw = __builtin_amdgcn_readfirstlane(x - lane);  // the wave's first column
-  const i64 bw = (i64)(blockIdx.x / nxb) * so + xw;
+  const i64 bw = (i64)la.other * so + xw;
   const int nrec = min(64, W - xw) * (int)sizeof(float2);
   auto at = [&](int p) -> float2 {
     const float2* line = src + bw + (i64)p * sa;
@@ -193,17 +195,17 @@ __global__ __launch_bounds__(NT) void k_gauss_walk(const float2* __restrict__ sr
     return __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(
                                           r, lane * (int)sizeof(float2), 0, 0));
   };
-  float2 ring[WB];  // position p lives in ring[(p + R) % WB]
+  float2 ring[WB];  // position p lives in ring[(p - b0 + R) % WB]
 #pragma unroll
-  for (int q = 0; q < WB; ++q) ring[q] = at(q - R);
-  float2 pf[PF];  // the refill of step c (position c + R + 1) waits in slot c % PF
+  for (int q = 0; q < WB; ++q) ring[q] = at(b0 + q - R);
+  float2 pf[PF];  // the refill of step c (position c + R + 1) waits in slot (c - b0) % PF
 #pragma unroll
-  for (int j = 0; j < PF; ++j) pf[j] = at(R + 1 + j);
-  for (int c0 = 0;; c0 += WB) {
+  for (int j = 0; j < PF; ++j) pf[j] = at(b0 + R + 1 + j);
+  for (int c0 = b0;; c0 += WB) {
 #pragma unroll
     for (int q = 0; q < WB; ++q) {
       const int c = c0 + q;
-      if (c >= L) return;
+      if (c >= b1) return;
       float s1 = 0.0f, s2 = 0.0f;
 #pragma unroll
       for (int j = -R1; j <= R1; ++j) s1 = fmaf(w1[R1 - j], ring[(q + j + R) % WB].x, s1);
@@ -374,7 +376,7 @@ bool gauss_xy(const TS* src, float2* dst, const float* w1, const float* w2, int 
   if (r1 == A && r2 == B) {                                                                  \
     const int nxs = (W + 63) / 64;                                                           \
     int nys, rows;                                                                           \
-    walk_segments(H, 2 * (A > B ? A : B) + 1, &nys, &rows, segments);                        \
+    walk_segments(H, 2 * (A > B ? A : B) + 1, (i64)nxs * D, &nys, &rows, segments);          \
     const i64 nblk = (i64)nxs * D * nys;                                                     \
     hipLaunchKernelGGL((k_gauss_xy_walk<A, B, TS>), dim3((unsigned)nblk), dim3(64), 0, s,    \
                        src, dst, w1, w2, W, H, nxs, nys, rows);                              \
@@ -392,10 +394,9 @@ hipError_t gauss_line(const float2* src, float2* dst, TS* dog, const float* w1, 
                       hipStream_t s) {
 #define X(A, B)                                                                              \
   if (r1 == A && r2 == B) {                                                                  \
-    const int nxb = (W + NT - 1) / NT;                                                       \
-    const i64 nblk = (i64)nxb * n_other;                                                     \
-    hipLaunchKernelGGL((k_gauss_walk<A, B, LAST, TS>), dim3((unsigned)nblk), dim3(NT), 0, s, \
-                       src, dst, dog, w1, w2, nz, W, L, sa, so, nxb);                        \
+    const LineGrid g = line_grid(W, L, n_other, 2 * (A > B ? A : B));                        \
+    hipLaunchKernelGGL((k_gauss_walk<A, B, LAST, TS>), dim3(g.blocks), dim3(NT), 0, s, src,  \
+                       dst, dog, w1, w2, nz, W, L, sa, so, g.nxb, g.no, g.len);              \
     return hipGetLastError();                                                                \
   }
   HDOG_GAUSS_PAIRS(X)

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
 #include <hip/hip_bf16.h>
+#include <algorithm>
 #include <cstdint>
 #include <string>
 
@@ -172,23 +173,100 @@ inline void mark(const char* name, hipStream_t s) {
   }
 }
 
+// ---- how long walks are split -------------------------------------------------------
+// A walker (one wave or work-group per strip, walking an axis) may be split along its axis;
+// every later segment starts with the positions of context its window needs.  Its time goes
+// with (x + t) * (steps per segment), x its waves per SIMD: t is what a launch loses to waves
+// that run alone (latency) and to its last, part-empty round.  The splits below take the
+// segment count with the least such time; t is fitted to sweeps of 1 .. 16 segments on
+// stacks from 24 x 96 x 112 to 256 x 1080 x 1280.
+
+// Row segments of a row walker (one wave per strip and segment; `strips`: waves per segment
+// over all planes; segment length: a multiple of the ring period wb, context wb - 1 rows).
+// t = 1.3 gives both walkers' sweeps within 10 %: norm_xy, 32 x 2160 x 2560: 914 us with two
+// segments, 543 with eight, 528 with sixteen; 128 x 256 x 256: 165 us with one, 54 with seven,
+// 60 with thirteen; gauss_xy there 102, 46 and 51 us with one, five and ten; on a full tile
+// 2 to 4 segments are within 2 %.  A tuned launch shape `want` (1 .. 4) takes want / 2 of the
+// built-in count.
+inline void walk_segments(int H, int wb, i64 strips, int* nys, int* rows, int want = 0) {
+  auto shape = [&](int n, int* k, int* r) {
+    const int per = (H + n - 1) / n;
+    *r = (per + wb - 1) / wb * wb;
+    *k = (H + *r - 1) / *r;
+  };
+  const int most = (H + wb - 1) / wb;
+  int best = 1;
+  double best_cost = 0.0;
+  for (int n = 1; n <= most && n <= 64; ++n) {
+    int k, r;
+    shape(n, &k, &r);
+    const double cost = ((double)strips * k / 1024.0 + 1.3) * (std::min(r, H) + wb - 1);
+    if (n == 1 || cost < best_cost) {
+      best_cost = cost;
+      best = n;
+    }
+  }
+  const int n = want > 0 ? std::max(1, std::min(most, (best * want + 1) / 2)) : best;
+  shape(n, nys, rows);
+}
+
+// Segments of a line of L positions, each reading `halo` positions more than it writes.
+// The column walkers (one thread per line) stream: two waves per SIMD already saturate the
+// memory, fewer leave it idle (box_z_norm, 128 x 256 x 256, one wave per SIMD: 39 us whole,
+// 29 in two segments; 64 x 512 x 512, four waves per SIMD: 47 us whole, 51 in two).  So the
+// load of a launch counts as at least `alone`.  groups: launch units per segment, on `slots`
+// of the chip at a time, in whole rounds when `whole` (long work-groups, one per CU).
+inline void line_segments(int L, i64 groups, double slots, double alone, bool whole, int halo,
+                          int* nseg, int* len) {
+  int best = 1;
+  double best_cost = 0.0;
+  for (int n = 1; n <= 32 && n <= L; ++n) {
+    const int l = (L + n - 1) / n;
+    double x = (double)groups * ((L + l - 1) / l) / slots;
+    if (whole) x = (double)(i64)(x + 0.9999);
+    const double cost = (x > alone ? x : alone) * (l + halo);
+    if (n == 1 || cost < best_cost) {
+      best_cost = cost;
+      best = n;
+    }
+  }
+  *len = (L + best - 1) / best;
+  *nseg = (L + *len - 1) / *len;
+}
+
+// Grid of a column walker with work-groups of 256 lines: x blocks, then the n_other lines
+// of the remaining axis, then the segments.
+struct LineGrid {
+  unsigned blocks, nxb, no;
+  int len;
+};
+inline LineGrid line_grid(int W, int L, i64 n_other, int halo) {
+  LineGrid g;
+  g.nxb = (unsigned)((W + 255) / 256);
+  g.no = (unsigned)n_other;
+  int nseg;
+  line_segments(L, (i64)g.nxb * n_other * 4, 1024.0, 2.0, false, halo, &nseg, &g.len);
+  g.blocks = (unsigned)((i64)g.nxb * n_other * nseg);
+  return g;
+}
+struct LineAt {
+  int x, other, c0, c1;  // outputs c0 .. c1-1 of the line (x, other)
+};
+__device__ __forceinline__ LineAt line_at_block(unsigned nxb, unsigned no, int len, int L) {
+  LineAt a;
+  const unsigned r = blockIdx.x / nxb;
+  a.x = (int)(blockIdx.x - r * nxb) * 256 + (int)threadIdx.x;
+  a.other = (int)(r % no);
+  a.c0 = (int)(r / no) * len;
+  a.c1 = min(L, a.c0 + len);
+  return a;
+}
+
 // Work-group b of n runs on XCD b % 8 (the dispatcher deals work-groups to the 8 XCDs in
 // turn, each XCD with its own L2).  Returns the logical tile for b such that every XCD
 // walks one contiguous range of tiles in order: tiles that share cache lines (halo rows,
 // 128-byte lines split between narrow tiles) then meet in the same L2.  A bijection of
 // [0, n) for any n.
-// Row walkers (one wave per plane strip) split tall planes into row segments, each
-// starting with the 2R rows of context its window needs: a C1 plane strip as one wave left
-// the last round of waves part-empty (2.5 and 1.4 rounds of resident waves for the two
-// walkers).  `want` segments (a tuned launch shape), or by default two for planes of at
-// least 16 ring periods; segment length: a multiple of the ring period wb.
-inline void walk_segments(int H, int wb, int* nys, int* rows, int want = 0) {
-  const int n = want > 0 ? want : (H >= 16 * wb ? 2 : 1);
-  const int per = (H + n - 1) / n;
-  *rows = (per + wb - 1) / wb * wb;
-  *nys = (H + *rows - 1) / *rows;
-}
-
 __device__ __forceinline__ unsigned xcd_tile(unsigned b, unsigned n) {
   constexpr unsigned X = 8;
   const unsigned q = n / X, r = n % X, j = b % X;

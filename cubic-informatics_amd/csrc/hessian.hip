@@ -361,7 +361,7 @@ __global__ __launch_bounds__(NT, 5) void k_hessian(const TD* __restrict__ dog, T
 constexpr int kRecTY = 4;                     // output rows per lane
 constexpr int kRecTilesY = HDOG_REC_TILES_Y;  // Hessian tiles per work-group, along y
 constexpr int kRecWaves = kRecTilesY * kHessTY / kRecTY;  // waves per work-group
-constexpr int kRecNZ = 4;                     // Hessian tiles per work-group, along z
+constexpr int kRecNZ = 4;  // most Hessian tiles per work-group along z (records_walk_tiles)
 static_assert(kHessTX == 64 && kHessTY % kRecTY == 0, "one wave spans a tile row");
 
 // v of lane i - 1 (lane 0 keeps old) and of lane i + 1 (lane 63 keeps old); one DPP move
@@ -381,7 +381,7 @@ __device__ __forceinline__ float swap_pairs(float v) {
 
 template <typename TD, typename TS, bool BAND>
 __global__ __launch_bounds__(64 * kRecWaves) void k_hessian_rec(
-    const TD* __restrict__ dog, int W, int H, int D, int nbx, int nby, int nbyg,
+    const TD* __restrict__ dog, int W, int H, int D, int nbx, int nby, int nbyg, int nz,
     float* __restrict__ cand,
     uint32_t* __restrict__ cand_cnt, float band) {
   constexpr int TY = kRecTY, NR = TY + 4, NH = TY + 2;  // dog rows, first-difference rows
@@ -396,7 +396,7 @@ __global__ __launch_bounds__(64 * kRecWaves) void k_hessian_rec(
   const int tt = wy0 / kHessTY, ty0 = wy0 % kHessTY;  // the wave's tile, its row in the tile
   const int by = byg * kRecTilesY + tt;  // past nby: every row is below the plane
   const int x0 = bx * 64, x = x0 + lane, y = by * kHessTY + ty0;
-  const int z0 = gz * kRecNZ * kHessTZ, z1 = min(z0 + kRecNZ * kHessTZ, D);
+  const int z0 = gz * nz * kHessTZ, z1 = min(z0 + nz * kHessTZ, D);
   constexpr uint32_t SZ = sizeof(TD);
   // byte offsets in a row: a negative column wraps past the record count
   const uint32_t vo = (uint32_t)x * SZ;
@@ -447,7 +447,7 @@ __global__ __launch_bounds__(64 * kRecWaves) void k_hessian_rec(
     const int z = s - 2;
     if (z >= z0 && z < z1) {
       const int tz = (z - z0) / kHessTZ;  // Hessian tile of the slice within the walk
-      const unsigned tile = (unsigned)(((gz * kRecNZ + tz) * nby + by) * nbx + bx);
+      const unsigned tile = (unsigned)(((gz * nz + tz) * nby + by) * nbx + bx);
       const uint32_t lz = (uint32_t)(z - (z0 + tz * kHessTZ));
       const __amdgpu_buffer_rsrc_t rr =
           buf_rsrc(cand + (size_t)tile * kCandTile * 7, (uint32_t)kCandTile * 7u * 4u);
@@ -562,9 +562,27 @@ __global__ __launch_bounds__(64 * kRecWaves) void k_hessian_rec(
   if (threadIdx.x < kRecTilesY * kRecNZ) {
     const int ct = (int)threadIdx.x / kRecNZ, cz = (int)threadIdx.x % kRecNZ;
     const int cby = byg * kRecTilesY + ct;
-    if (cby < nby && z0 + cz * kHessTZ < D)
-      cand_cnt[(((unsigned)gz * kRecNZ + cz) * nby + cby) * nbx + bx] = s_cnt[ct][cz];
+    if (cz < nz && cby < nby && z0 + cz * kHessTZ < D)
+      cand_cnt[(((unsigned)gz * nz + cz) * nby + cby) * nbx + bx] = s_cnt[ct][cz];
   }
+}
+
+// Hessian tiles that a records-only work-group walks along z: each walk reads four slices
+// beyond its own, so long walks are better once the chip is full (`columns` work-groups of
+// four waves per layer of walks).  Least (waves per SIMD + t) * (slices per walk), t = 2.3
+// fitted to nz = 1, 2, 4: 64 x 512 x 512: 52, 61, 93 us; 211 x 512 x 1536: 435, 408, 471 us.
+int records_walk_tiles(i64 columns, int nbz) {
+  int best = 1;
+  double best_cost = 0.0;
+  for (int nz = 1; nz <= kRecNZ && nz <= nbz; ++nz) {
+    const double x = (double)columns * ((nbz + nz - 1) / nz) / 256.0;
+    const double cost = (x + 2.3) * (kHessTZ * nz + 4);
+    if (nz == 1 || cost < best_cost) {
+      best_cost = cost;
+      best = nz;
+    }
+  }
+  return best;
 }
 
 }  // namespace
@@ -580,10 +598,11 @@ hipError_t launch_hessian(const TD* dog, TH* hess, uint8_t* pd, int W, int H, in
   constexpr bool reduced = !std::is_same<TD, float>::value || !std::is_same<TH, float>::value;
   if (!hess && !pd && cand && cand_cnt) {  // records only
     const int nbyg = (nby + kRecTilesY - 1) / kRecTilesY;
-    const i64 ngroups = (i64)nbx * nbyg * ((nbz + kRecNZ - 1) / kRecNZ);
+    const int nz = records_walk_tiles((i64)nbx * nbyg, nbz);
+    const i64 ngroups = (i64)nbx * nbyg * ((nbz + nz - 1) / nz);
     hipLaunchKernelGGL((k_hessian_rec<TD, TH, reduced>), dim3((unsigned)ngroups),
-                       dim3(64 * kRecWaves), 0, s, dog, W, H, D, nbx, nby, nbyg, cand, cand_cnt,
-                       band);
+                       dim3(64 * kRecWaves), 0, s, dog, W, H, D, nbx, nby, nbyg, nz, cand,
+                       cand_cnt, band);
   } else {
     hipLaunchKernelGGL((k_hessian<TD, TH, reduced>), dim3((unsigned)nblk), dim3(NT), 0, s, dog,
                        hess, pd, W, H, D, nbx, nby, cand, cand_cnt, band);

@@ -305,13 +305,17 @@ __global__ __launch_bounds__(NT) void k_box_line(const float2* __restrict__ src,
 template <int R, bool FROM_U16>
 __global__ __launch_bounds__(NT) void k_minmax_walk(const void* __restrict__ src,
                                                     uint32_t* __restrict__ dst, int W, int L,
-                                                    i64 sa, i64 so, int nxb) {
+                                                    i64 sa, i64 so, unsigned nxb, unsigned no,
+                                                    int len) {
   constexpr int WB = 2 * R + 1;
-  const int x = (blockIdx.x % nxb) * NT + threadIdx.x;
+  const LineAt la = line_at_block(nxb, no, len, L);
+  const int x = la.x;
   if (x >= W) return;
-  const i64 base = (i64)(blockIdx.x / nxb) * so + x;
+  const i64 base = (i64)la.other * so + x;
+  const int s0 = la.c0;
+  const int n = la.c1 - s0;  // outputs of the segment; below, positions count from s0
   auto load = [&](int k) -> uint32_t {
-    const i64 idx = base + (i64)clampi(k - R, 0, L - 1) * sa;
+    const i64 idx = base + (i64)clampi(s0 + k - R, 0, L - 1) * sa;
     return FROM_U16 ? pack(((const uint16_t*)src)[idx]) : ((const uint32_t*)src)[idx];
   };
   uint32_t S[WB], cur[WB];
@@ -320,7 +324,7 @@ __global__ __launch_bounds__(NT) void k_minmax_walk(const void* __restrict__ src
   S[WB - 1] = cur[WB - 1];
 #pragma unroll
   for (int j = WB - 2; j >= 0; --j) S[j] = pkmin(cur[j], S[j + 1]);
-  const int nb = (L + WB - 1) / WB;
+  const int nb = (n + WB - 1) / WB;
   for (int b = 1; b <= nb; ++b) {
 #pragma unroll
     for (int j = 0; j < WB; ++j) cur[j] = load(b * WB + j);
@@ -329,10 +333,10 @@ __global__ __launch_bounds__(NT) void k_minmax_walk(const void* __restrict__ src
 #pragma unroll
     for (int j = 0; j < WB; ++j) {
       if (j > 0) {
-        if (c0 + j < L) st_nt(dst + base + (i64)(c0 + j) * sa, pkmin(S[j], p));
+        if (c0 + j < n) st_nt(dst + base + (i64)(s0 + c0 + j) * sa, pkmin(S[j], p));
         p = pkmin(p, cur[j]);
-      } else if (c0 < L) {
-        st_nt(dst + base + (i64)c0 * sa, S[0]);
+      } else if (c0 < n) {
+        st_nt(dst + base + (i64)(s0 + c0) * sa, S[0]);
       }
     }
     S[WB - 1] = cur[WB - 1];
@@ -360,7 +364,8 @@ __global__ __launch_bounds__(NT) void k_minmax_walk(const void* __restrict__ src
 template <int RZ, int RY, int PF>
 __global__ __launch_bounds__(1024) void k_minmax_zy_walk(const uint16_t* __restrict__ img,
                                                         uint32_t* __restrict__ dst, int W, int H,
-                                                        int D, int nyt) {
+                                                        int D, unsigned nyt, unsigned nxt,
+                                                        int zlen) {
   constexpr int TY = 32, KR = 2, NWV = TY / KR;  // rows per tile, rows per thread, waves
   constexpr int SR = TY + 2 * RY;                 // staged rows per slice
   constexpr int NLD = (SR + NWV - 1) / NWV;       // row loads per lane and slice
@@ -372,7 +377,9 @@ __global__ __launch_bounds__(1024) void k_minmax_zy_walk(const uint16_t* __restr
   static_assert(RY >= 2, "shared window middle");
   __shared__ uint32_t S[2][SRP * 64];
   const unsigned t = xcd_tile(blockIdx.x, gridDim.x);
-  const int yt = (int)(t % (unsigned)nyt), xt = (int)(t / (unsigned)nyt);
+  const int yt = (int)(t % nyt), xt = (int)(t / nyt % nxt);
+  // outputs z0 .. z1-1 of one of the segments of the volume; below, k and c count from z0
+  const int z0 = (int)(t / nyt / nxt) * zlen, z1 = min(D, z0 + zlen);
   const int lane = (int)(threadIdx.x & 63);
   const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));  // wave-uniform
   const int x = xt * 64 + lane, y0 = yt * TY;
@@ -389,7 +396,7 @@ __global__ __launch_bounds__(1024) void k_minmax_zy_walk(const uint16_t* __restr
   uint32_t q[PF][NLD];  // raw values of slice k wait in slot k % PF
   auto fetch = [&](int k, int slot) {
     const __amdgpu_buffer_rsrc_t r =
-        buf_rsrc(img + (size_t)clampi(k - RZ, 0, D - 1) * WH, (uint32_t)(WH * 2));
+        buf_rsrc(img + (size_t)clampi(z0 + k - RZ, 0, D - 1) * WH, (uint32_t)(WH * 2));
 #pragma unroll
     for (int j = 0; j < NLD; ++j)
       q[slot][j] = __builtin_amdgcn_raw_buffer_load_b16(r, (int)(off[j] * 2u), 0, 0);
@@ -427,7 +434,7 @@ __global__ __launch_bounds__(1024) void k_minmax_zy_walk(const uint16_t* __restr
     ro[i] = x < W && y0 + ty + i < H ? ((uint32_t)(y0 + ty + i) * (uint32_t)W + (uint32_t)x) * 4u
                                      : 0xFFFFFFF0u;
   auto put = [&](int c, const uint32_t v[KR]) {
-    const __amdgpu_buffer_rsrc_t r = buf_rsrc(dst + (size_t)c * WH, (uint32_t)(WH * 4));
+    const __amdgpu_buffer_rsrc_t r = buf_rsrc(dst + (size_t)(z0 + c) * WH, (uint32_t)(WH * 4));
 #pragma unroll
     for (int i = 0; i < KR; ++i)  // streaming (nontemporal) stores
       __builtin_amdgcn_raw_buffer_store_b32(v[i], r, (int)ro[i], 0, kCachePolicyNT);
@@ -461,9 +468,9 @@ __global__ __launch_bounds__(1024) void k_minmax_zy_walk(const uint16_t* __restr
     for (int i = 0; i < KR; ++i) v[i] = zs[i][0];
     put(0, v);
   }
-  // output c leaves when slice k = c + 2RZ has arrived; the last is c = D - 1.  The walk's
+  // output c leaves when slice k = c + 2RZ has arrived; the last is z1 - 1.  The walk's
   // end leaves the kernel (uniform over the work-group: every wave has the same k).
-  const int kend = D + 2 * RZ;
+  const int kend = z1 - z0 + 2 * RZ;
   for (int k0 = WB;; k0 += WB) {
 #pragma unroll
     for (int j = 0; j < WB; ++j) {
@@ -501,20 +508,22 @@ template <int R, bool NORM, typename TS>
 __global__ __launch_bounds__(NT) void k_box_walk(const float2* __restrict__ src,
                                                  float2* __restrict__ dst, TS* __restrict__ norm,
                                                  const uint16_t* __restrict__ img, float min_int,
-                                                 int W, int L, i64 sa, i64 so, int nxb, float k) {
+                                                 int W, int L, i64 sa, i64 so, unsigned nxb,
+                                                 unsigned no, int len, float k) {
   constexpr int WB = 2 * R + 1;
   constexpr int PF = WB % 3 == 0 ? 3 : WB % 5 == 0 ? 5 : WB % 7 == 0 ? 7 : 1;
-  const int x = (blockIdx.x % nxb) * NT + threadIdx.x;
+  const LineAt la = line_at_block(nxb, no, len, L);
+  const int x = la.x, s0 = la.c0, s1 = la.c1;
   if (x >= W) return;
-  const i64 base = (i64)(blockIdx.x / nxb) * so + x;
+  const i64 base = (i64)la.other * so + x;
   auto at = [&](int p) { return src[base + (i64)clampi(p, 0, L - 1) * sa]; };
-  float2 ring[WB];  // position p lives in ring[(p + R) % WB]
+  float2 ring[WB];  // position p lives in ring[(p - s0 + R) % WB]
 #pragma unroll
-  for (int q = 0; q < WB; ++q) ring[q] = at(q - R);
-  float2 pf[PF];  // the refill of step c (position c + R + 1) waits in slot c % PF
+  for (int q = 0; q < WB; ++q) ring[q] = at(s0 + q - R);
+  float2 pf[PF];  // the refill of step c (position c + R + 1) waits in slot (c - s0) % PF
 #pragma unroll
-  for (int j = 0; j < PF; ++j) pf[j] = at(R + 1 + j);
-  for (int c0 = 0;; c0 += WB) {
+  for (int j = 0; j < PF; ++j) pf[j] = at(s0 + R + 1 + j);
+  for (int c0 = s0;; c0 += WB) {
     // with the normalization fused, the raw intensities of this block's WB outputs are
     // loaded up front: loading each one at its output made every output wait for all
     // outstanding loads, the ring refills included
@@ -527,7 +536,7 @@ __global__ __launch_bounds__(NT) void k_box_walk(const float2* __restrict__ src,
 #pragma unroll
     for (int q = 0; q < WB; ++q) {
       const int c = c0 + q;
-      if (c >= L) return;
+      if (c >= s1) return;
       float ve = 0.0f, vd = 0.0f;
 #pragma unroll
       for (int j = 0; j <= 2 * R; ++j) {  // position c - R + j -> ring[(q + j) % WB]
@@ -759,14 +768,13 @@ hipError_t dispatch_xw(int XW, F&& f) {
 template <int R>
 hipError_t minmax_walk(const void* src, bool from_u16, uint32_t* dst, int W, int L, i64 sa, i64 so,
                        i64 n_other, hipStream_t s) {
-  const int nxb = (W + NT - 1) / NT;
-  const i64 nblk = (i64)nxb * n_other;
+  const LineGrid g = line_grid(W, L, n_other, 2 * R);
   if (from_u16)
-    hipLaunchKernelGGL((k_minmax_walk<R, true>), dim3((unsigned)nblk), dim3(NT), 0, s, src, dst, W,
-                       L, sa, so, nxb);
+    hipLaunchKernelGGL((k_minmax_walk<R, true>), dim3(g.blocks), dim3(NT), 0, s, src, dst, W, L, sa,
+                       so, g.nxb, g.no, g.len);
   else
-    hipLaunchKernelGGL((k_minmax_walk<R, false>), dim3((unsigned)nblk), dim3(NT), 0, s, src, dst,
-                       W, L, sa, so, nxb);
+    hipLaunchKernelGGL((k_minmax_walk<R, false>), dim3(g.blocks), dim3(NT), 0, s, src, dst, W, L,
+                       sa, so, g.nxb, g.no, g.len);
   return hipGetLastError();
 }
 
@@ -800,10 +808,9 @@ template <int R, bool NORM, typename TS>
 hipError_t box_line_fast(const float2* src, float2* dst, TS* norm, const uint16_t* img,
                          float min_int, int W, int L, i64 sa, i64 so, i64 n_other, float k,
                          hipStream_t s) {
-  const int nxb = (W + NT - 1) / NT;
-  const i64 nblk = (i64)nxb * n_other;
-  hipLaunchKernelGGL((k_box_walk<R, NORM, TS>), dim3((unsigned)nblk), dim3(NT), 0, s, src, dst,
-                     norm, img, min_int, W, L, sa, so, nxb, k);
+  const LineGrid g = line_grid(W, L, n_other, 2 * R);
+  hipLaunchKernelGGL((k_box_walk<R, NORM, TS>), dim3(g.blocks), dim3(NT), 0, s, src, dst, norm, img,
+                     min_int, W, L, sa, so, g.nxb, g.no, g.len, k);
   return hipGetLastError();
 }
 
@@ -866,9 +873,14 @@ hipError_t launch_normalize(const uint16_t* img, TS* norm, void* tmp1, void* tmp
   if (rxy == 10 && rz == 10 && WH * 4 < 0xFFFFFFF0ll) {
     // min/max along y and z in one z walk over 64 x 32 tiles (slices addressed by buffer
     // descriptors with 32-bit byte offsets)
-    const int nxt = (W + 63) / 64, nyt = (H + 31) / 32;
-    hipLaunchKernelGGL((k_minmax_zy_walk<10, 10, HDOG_ZY_PF>), dim3((unsigned)((i64)nxt * nyt)),
-                       dim3(1024), 0, s, img, p2, W, H, D, nyt);
+    const unsigned nxt = (W + 63) / 64, nyt = (H + 31) / 32;
+    int nzs, zlen;
+    // one 1024-thread work-group per CU: whole rounds of 256 (128 x 256 x 256, 32 work-groups
+    // per segment: 93 us whole, 30 in eight segments, 43 in twelve)
+    line_segments(D, (i64)nxt * nyt, 256.0, 1.0, true, 24, &nzs, &zlen);
+    hipLaunchKernelGGL((k_minmax_zy_walk<10, 10, HDOG_ZY_PF>),
+                       dim3((unsigned)((i64)nxt * nyt * nzs)), dim3(1024), 0, s, img, p2, W, H, D,
+                       nyt, nxt, zlen);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     mark("normalize/minmax_zy", s);
   } else {
@@ -884,7 +896,7 @@ hipError_t launch_normalize(const uint16_t* img, TS* norm, void* tmp1, void* tmp
     constexpr int CW = 128;
     const int nxs = (W + CW - 1) / CW;
     int nys, rows;
-    walk_segments(H, 21, &nys, &rows, segments);
+    walk_segments(H, 21, (i64)nxs * D, &nys, &rows, segments);
     const i64 nblk = (i64)nxs * D * nys;
     hipLaunchKernelGGL((k_norm_xy_walk<10>), dim3((unsigned)nblk), dim3(64), 0, s, p2,
                        (float4*)tmp1, W, H, nxs, nys, rows, 1.0f / 21.0f);
