@@ -131,31 +131,24 @@ void release(Buf& b) {
 // One fixed scratch array per GPU, sized for volumes of at most kNoAllocVoxels voxels once
 // padded to whole Hessian tiles (2^23: a 128 x 256 x 256 stack exactly).  Its layout per
 // call, every part 256-byte aligned: candidate positions and record labels (4 bytes per
-// padded voxel each), per-tile counts, the candidate bit mask (one word per tile row), and
-// the root and region-spanning bitmaps.  The array's name is only a host-side stand-in;
+// padded voxel each), per-tile counts and the candidate bit mask (one word per tile row).
+// The array's name is only a host-side stand-in;
 // kernels get the address hipGetSymbolAddress returns on each device (noalloc_addr).
 constexpr i64 kNoAllocVoxels = (i64)1 << 23;
 constexpr size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 struct NoAllocLayout {
-  size_t cand, lab, cnt, fg, roots, multi, total;
-  i64 ntiles, root_words;
+  size_t cand, lab, cnt, fg, total;
 };
-constexpr NoAllocLayout noalloc_layout(i64 ntiles, i64 N) {
+constexpr NoAllocLayout noalloc_layout(i64 ntiles) {
   NoAllocLayout L{};
-  const i64 nb = (N + kRootBlock - 1) / kRootBlock;
-  L.ntiles = ntiles;
-  L.root_words = nb * (kRootBlock / 64);
   L.cand = 0;
   L.lab = L.cand + align256((size_t)ntiles * kCandTile * 4);
   L.cnt = L.lab + align256((size_t)ntiles * kCandTile * 4);
   L.fg = L.cnt + align256((size_t)ntiles * 4);
-  L.roots = L.fg + align256((size_t)ntiles * kHessTY * kHessTZ * 8);
-  L.multi = L.roots + align256((size_t)L.root_words * 8);
-  L.total = L.multi + align256((size_t)L.root_words * 8);
+  L.total = L.fg + align256((size_t)ntiles * kHessTY * kHessTZ * 8);
   return L;
 }
-constexpr size_t kNoAllocScratchBytes =
-    noalloc_layout(kNoAllocVoxels / kCandTile, kNoAllocVoxels).total;
+constexpr size_t kNoAllocScratchBytes = noalloc_layout(kNoAllocVoxels / kCandTile).total;
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 constexpr int kMaxDevices = 64;
 void* g_noalloc_addr[kMaxDevices] = {};
@@ -839,21 +832,17 @@ int hdog_ccl3d(hdog_ctx* ctx, void* stream, const uint8_t* d_pd, uint32_t* d_lab
   // the mask's candidate positions in the record layout, then the whole path's labeling
   // of candidates with the label volume written in full
   const hipStream_t s = (hipStream_t)stream;
-  const i64 N = (i64)width * height * depth, ntiles = hessian_tiles(width, height, depth);
-  const i64 nb = (N + kRootBlock - 1) / kRootBlock;
+  const i64 ntiles = hessian_tiles(width, height, depth);
   HIPCHK(ensure(ctx->cand, (size_t)ntiles * kCandTile * 4));
   HIPCHK(ensure(ctx->cand_cnt, (size_t)ntiles * 4));
   HIPCHK(ensure(ctx->cand_lab, (size_t)ntiles * kCandTile * 4));
   HIPCHK(ensure(ctx->fgbits, (size_t)fg_words(width, height, depth) * 8));
-  HIPCHK(ensure(ctx->rmask, (size_t)nb * (kRootBlock / 8)));
-  HIPCHK(ensure(ctx->rmulti, (size_t)nb * (kRootBlock / 8)));
   HIPCHK(launch_mask_records(d_pd, (float*)ctx->cand.p, (uint32_t*)ctx->cand_cnt.p, width, height,
                              depth, s));
   HIPCHK(launch_ccl_candidates((const float*)ctx->cand.p, (const uint32_t*)ctx->cand_cnt.p, ntiles,
                                (unsigned long long*)ctx->fgbits.p, d_labels,
-                               (uint32_t*)ctx->cand_lab.p, (unsigned long long*)ctx->rmask.p,
-                               (unsigned long long*)ctx->rmulti.p, nb * (kRootBlock / 64), true,
-                               width, height, depth, s, 1));
+                               (uint32_t*)ctx->cand_lab.p, nullptr, nullptr, 0, true, width, height,
+                               depth, s, 1));
   return HDOG_OK;
 }
 
@@ -863,7 +852,7 @@ int hdog_ccl3d_noalloc(hdog_ctx* ctx, void* stream, const uint8_t* d_pd, uint32_
   int rc = check_shape(ctx, width, height, depth);
   if (rc) return rc;
   if (!d_pd || !d_labels) return fail(ctx, HDOG_ERR_ARG, "NULL device pointer");
-  const i64 N = (i64)width * height * depth, ntiles = hessian_tiles(width, height, depth);
+  const i64 ntiles = hessian_tiles(width, height, depth);
   if (ntiles * kCandTile > kNoAllocVoxels)
     return fail(ctx, HDOG_ERR_ARG,
                 "hdog_ccl3d_noalloc: %d x %d x %d pads to %lld voxels of Hessian tiles, more "
@@ -872,17 +861,15 @@ int hdog_ccl3d_noalloc(hdog_ctx* ctx, void* stream, const uint8_t* d_pd, uint32_
   HIPCHK(hipSetDevice(ctx->device));
   unsigned char* base = (unsigned char*)noalloc_addr(ctx->device);
   if (!base) return fail(ctx, HDOG_ERR_STATE, "no scratch address for device %d", ctx->device);
-  const NoAllocLayout L = noalloc_layout(ntiles, N);
+  const NoAllocLayout L = noalloc_layout(ntiles);
   const hipStream_t s = (hipStream_t)stream;
   // every part is written before it is read: the counts and positions by the mask pass, the
-  // mask rows and record labels by the tile-local labeling, the bitmaps and the label
-  // volume cleared by fill kernels inside launch_ccl_candidates
+  // mask rows and record labels by the tile-local labeling
   HIPCHK(launch_mask_records(d_pd, (float*)(base + L.cand), (uint32_t*)(base + L.cnt), width,
                              height, depth, s));
   HIPCHK(launch_ccl_candidates((const float*)(base + L.cand), (const uint32_t*)(base + L.cnt),
                                ntiles, (unsigned long long*)(base + L.fg), d_labels,
-                               (uint32_t*)(base + L.lab), (unsigned long long*)(base + L.roots),
-                               (unsigned long long*)(base + L.multi), L.root_words, true, width,
+                               (uint32_t*)(base + L.lab), nullptr, nullptr, 0, true, width,
                                height, depth, s, 1));
   return HDOG_OK;
 }

@@ -177,7 +177,8 @@ static_assert(fwd_order(2) == 0 && fwd_order(5) == 3 && fwd_order(6) == 5 && fwd
 //             the global union-find on P;
 //   kernel C: every record's root (the component minimum), root bits for the region
 //             numbering, the roots of regions that reach beyond one region-pass
-//             work-group, and with `dense` the final label written back into P.
+//             work-group;
+//   and, where the full label volume is wanted, a pass that writes it in place of P.
 // 256 threads and 16-bit LDS parents (17 KB of LDS per tile): eight tiles share a CU.
 constexpr int RTX = kHessTX, RTY = kHessTY, RTZ = kHessTZ, RTV = RTX * RTY * RTZ, NTR = 256;
 constexpr int RROWS = RTY * RTZ;  // mask words per tile
@@ -250,11 +251,21 @@ __global__ __launch_bounds__(NTR) void k_cand_local(const float* __restrict__ ca
                                                    const uint32_t* __restrict__ cand_cnt,
                                                    unsigned long long* __restrict__ fgbits,
                                                    uint32_t* __restrict__ P,
-                                                   uint32_t* __restrict__ rlab, int W, int H,
-                                                   int D, int nbx, int nby, int links,
-                                                   int rec_words) {
+                                                   uint32_t* __restrict__ rlab,
+                                                   unsigned long long* __restrict__ roots,
+                                                   unsigned long long* __restrict__ multi,
+                                                   i64 root_words, int W, int H, int D, int nbx,
+                                                   int nby, int links, int rec_words) {
   const unsigned tile = xcd_tile(blockIdx.x, gridDim.x);
   const uint32_t n = cand_cnt[tile];
+  // this work-group's share of the root and region-spanning bitmaps, cleared for kernel C
+  // (a tile's voxels have RTV / 64 words; the tiles' voxels cover the volume's)
+  if (roots) {
+    static_assert(NTR >= 2 * (RTV / 64), "one word per thread, both bitmaps");
+    const i64 w = (i64)tile * (RTV / 64) + (threadIdx.x & (RTV / 64 - 1));
+    if (threadIdx.x < 2 * (RTV / 64) && w < root_words)
+      (threadIdx.x < RTV / 64 ? roots : multi)[w] = 0ull;
+  }
   __shared__ unsigned long long bits[RROWS];  // the tile's mask rows (word = ly + RTY lz)
   // parents, valid at candidate positions; linked by 32-bit compare-and-swap on the word
   // holding two of them, so the array starts on a 4-byte boundary
@@ -324,7 +335,7 @@ __global__ __launch_bounds__(NTR) void k_cand_local(const float* __restrict__ ca
   };
   // P is read at tile-local roots (the find chains) and at candidates another tile's
   // forward neighbours reach (the bottom face and the x / y faces of the clipped tile);
-  // interior entries stay unwritten (kernel C writes every entry when `dense`)
+  // interior entries stay unwritten (a full label volume is written afterwards)
   R.each(rec, n, [&](uint32_t i, uint32_t v) {
     const uint32_t r = lds16_find(lab, v);
     const uint32_t label = global(r);
@@ -479,13 +490,14 @@ __global__ __launch_bounds__(NTR) void k_cand_merge(const float* __restrict__ ca
   }
 }
 
+// roots NULL (a label volume alone is wanted): no bits.
 __global__ __launch_bounds__(NTR) void k_cand_flatten(const float* __restrict__ cand,
                                                      const uint32_t* __restrict__ cand_cnt,
                                                      uint32_t* P, uint32_t* __restrict__ rlab,
                                                      unsigned long long* __restrict__ roots,
                                                      unsigned long long* __restrict__ multi,
-                                                     int dense, int W, int H, int D, int nbx,
-                                                     int nby, int rec_words) {
+                                                     int W, int H, int D, int nbx, int nby,
+                                                     int rec_words) {
   const unsigned tile = blockIdx.x;
   const uint32_t n = cand_cnt[tile];
   if (n == 0) return;
@@ -509,7 +521,7 @@ __global__ __launch_bounds__(NTR) void k_cand_flatten(const float* __restrict__ 
     // written a root
     const uint32_t r = find_root_flat(P, l);
     rl[i] = r;
-    if (dense && ld_parent(P, idx) != r) st_parent(P, idx, r);
+    if (!roots) return;
     if (r == idx) {
       atomicOr(roots + (r >> 6), 1ull << (r & 63));
     } else if (l == idx) {
@@ -532,38 +544,115 @@ __global__ __launch_bounds__(NTR) void k_cand_flatten(const float* __restrict__ 
     one(i, __float_as_uint(rec[i]), rl[i]);
 }
 
-// Candidate positions of a byte mask, in the record layout of the Hessian pass (per
-// Hessian tile a count and the tile positions, one reservation per wave and tile row, in
-// lane order): the labeling of a given mask then runs the same kernels as the whole path.
-// Voxel 0 is background whatever its mask value (its label is 0).
+// The full label volume, in place of the parent array: the tile's labels are laid out in LDS
+// and leave as whole rows, zeros included, 16 bytes per lane where the rows are aligned
+// (vec), so the volume is written once.  A kernel of its own, since the flatten still reads
+// other tiles' entries.  Bound by its 4 bytes per voxel: 102 us for 96 x 1080 x 1280 (5.2
+// TB/s), the flatten 41; clearing the volume first (74 us) and storing each label where it
+// belongs from the flatten (132 us) took 206.
+__global__ __launch_bounds__(NTR) void k_label_rows(const float* __restrict__ cand,
+                                                   const uint32_t* __restrict__ cand_cnt,
+                                                   const uint32_t* __restrict__ rlab,
+                                                   uint32_t* __restrict__ P, int W, int H, int D,
+                                                   int nbx, int nby, int rec_words, int vec) {
+  const unsigned tile = xcd_tile(blockIdx.x, gridDim.x);
+  const uint32_t n = cand_cnt[tile];
+  const CandTile T = cand_tile(tile, W, H, D, nbx, nby);
+  const uint32_t Wu = (uint32_t)W, WH = Wu * (uint32_t)H;
+  __shared__ __align__(16) uint32_t lv[RTV];
+#pragma unroll
+  for (int k = 0; k < RTV / (4 * NTR); ++k)
+    *reinterpret_cast<uint4*>(lv + 4 * (threadIdx.x + k * NTR)) = make_uint4(0u, 0u, 0u, 0u);
+  __syncthreads();
+  const float* rec = cand + (size_t)tile * kCandTile * rec_words;
+  const uint32_t* rl = rlab + (size_t)tile * kCandTile;
+  for (uint32_t i = threadIdx.x; i < n; i += NTR) lv[__float_as_uint(rec[i])] = rl[i];
+  __syncthreads();
+  uint32_t* base = P + (size_t)T.z0 * WH + (size_t)T.y0 * Wu + T.x0;
+  if (vec) {  // width and volume aligned: a quad lies in the row or outside it
+    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+    for (int e = (int)threadIdx.x; e < RTV / 4; e += NTR) {
+      const int lx = e % (RTX / 4) * 4, row = e / (RTX / 4), ly = row % RTY, lz = row / RTY;
+      if (lx < T.ex && ly < T.ey && lz < T.ez)
+        __builtin_nontemporal_store(*reinterpret_cast<const u4*>(lv + 4 * e),
+                                    reinterpret_cast<u4*>(base + (size_t)lz * WH + (size_t)ly * Wu + lx));
+    }
+  } else {
+    for (int e = (int)threadIdx.x; e < RTV; e += NTR) {
+      const int lx = e % RTX, row = e / RTX, ly = row % RTY, lz = row / RTY;
+      if (lx < T.ex && ly < T.ey && lz < T.ez)
+        __builtin_nontemporal_store(lv[e], base + (size_t)lz * WH + (size_t)ly * Wu + lx);
+    }
+  }
+}
+
+// Candidate positions of a byte mask, in the record layout of the Hessian pass (per Hessian
+// tile a count and the tile positions): the labeling of a given mask then runs the same
+// kernels as the whole path.  Voxel 0 is background whatever its mask value (its label is 0).
+// A lane takes four bytes, a wave four rows at a time, all its loads in flight and one
+// reservation per wave; within four rows the records are in row order.  With a byte per lane,
+// a row at a time and a reservation per row, the wave spent its time on the reservations'
+// round trips and on issue: 182 us for 96 x 1080 x 1280, 62 us now (132 MB read).
 __global__ __launch_bounds__(256) void k_mask_records(const uint8_t* __restrict__ pd,
                                                       float* __restrict__ pos,
                                                       uint32_t* __restrict__ cand_cnt, int W,
                                                       int H, int D, int nbx, int nby) {
-  const unsigned tile = blockIdx.x;
+  constexpr int NG = RROWS / 4 / 4;  // groups of four rows per wave
+  const unsigned tile = xcd_tile(blockIdx.x, gridDim.x);
   const CandTile T = cand_tile(tile, W, H, D, nbx, nby);
   __shared__ uint32_t s_cnt;
   if (threadIdx.x == 0) s_cnt = 0;
   __syncthreads();
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const uint32_t WH = (uint32_t)W * (uint32_t)H;
-  float* out = pos + (size_t)tile * kCandTile;
-  for (int row = wave; row < RROWS; row += 4) {  // uniform over the wave
-    const int ly = row % RTY, lz = row / RTY;
-    bool on = false;
-    if (lane < T.ex && ly < T.ey && lz < T.ez) {
-      const uint32_t idx = (uint32_t)(T.z0 + lz) * WH + (uint32_t)(T.y0 + ly) * (uint32_t)W +
-                           (uint32_t)(T.x0 + lane);
-      on = idx != 0 && pd[idx] != 0;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint32_t WH = (uint32_t)W * (uint32_t)H, N = WH * (uint32_t)D;
+  const int lx = (lane & 15) * 4;
+  uint32_t m[NG], at[NG];
+  const bool some = N >= 4u;  // uniform; rows start at any byte, so the quads may too
+#pragma unroll
+  for (int g = 0; g < NG; ++g) {
+    const int row = 4 * (wave * NG + g) + (lane >> 4), ly = row % RTY, lz = row / RTY;
+    const bool in = lx < T.ex && ly < T.ey && lz < T.ez;
+    at[g] = in ? (uint32_t)(T.z0 + lz) * WH + (uint32_t)(T.y0 + ly) * (uint32_t)W +
+                     (uint32_t)(T.x0 + lx)
+               : N;
+    m[g] = 0u;
+    if (some) __builtin_memcpy(&m[g], pd + (at[g] <= N - 4u ? at[g] : 0u), 4);
+  }
+#pragma unroll
+  for (int g = 0; g < NG; ++g) {
+    if (!some || at[g] > N - 4u) {  // outside the tile, or the volume's last bytes
+      m[g] = 0u;
+      for (uint32_t k = at[g]; k < N; ++k) m[g] |= (uint32_t)pd[k] << (8 * (k - at[g]));
     }
-    const unsigned long long bal = __ballot(on);
-    if (!bal) continue;
-    uint32_t base = 0;
-    if (lane == 0) base = atomicAdd(&s_cnt, (uint32_t)__popcll(bal));
-    base = __builtin_amdgcn_readfirstlane(base);  // lane 0 (the whole wave is here)
-    if (on)
-      out[base + (uint32_t)__popcll(bal & ((1ull << lane) - 1ull))] =
-          __uint_as_float((uint32_t)(lane + RTX * (ly + RTY * lz)));
+    if (T.ex - lx < 4) m[g] &= T.ex > lx ? 0xFFFFFFFFu >> (8 * (4 - (T.ex - lx))) : 0u;
+    if (at[g] == 0u) m[g] &= 0xFFFFFF00u;
+  }
+  // per group: bit 8 k + 7 set for a non-zero byte k, then each lane's count (0 .. 4) by bits
+  unsigned long long b0[NG], b1[NG], b2[NG];
+  uint32_t total = 0;  // uniform over the wave
+#pragma unroll
+  for (int g = 0; g < NG; ++g) {
+    m[g] = (((m[g] & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | m[g]) & 0x80808080u;
+    const uint32_t c = (uint32_t)__popc(m[g]);
+    b0[g] = __ballot(c & 1u);
+    b1[g] = __ballot(c & 2u);
+    b2[g] = __ballot(c & 4u);
+    total += (uint32_t)(__popcll(b0[g]) + 2 * __popcll(b1[g]) + 4 * __popcll(b2[g]));
+  }
+  uint32_t base = 0;
+  if (total && lane == 0) base = atomicAdd(&s_cnt, total);
+  base = __builtin_amdgcn_readfirstlane(base);
+  float* out = pos + (size_t)tile * kCandTile;
+  const unsigned long long below = (1ull << lane) - 1ull;
+#pragma unroll
+  for (int g = 0; g < NG; ++g) {
+    uint32_t slot = base + (uint32_t)(__popcll(b0[g] & below) + 2 * __popcll(b1[g] & below) +
+                                      4 * __popcll(b2[g] & below));
+    const uint32_t v = (uint32_t)(lx + RTX * (4 * (wave * NG + g) + (lane >> 4)));
+    for (uint32_t t = m[g]; t; t &= t - 1u)
+      out[slot++] = __uint_as_float(v + ((uint32_t)__builtin_ctz(t) >> 3));
+    base += (uint32_t)(__popcll(b0[g]) + 2 * __popcll(b1[g]) + 4 * __popcll(b2[g]));
   }
   __syncthreads();
   if (threadIdx.x == 0) cand_cnt[tile] = s_cnt;
@@ -609,14 +698,11 @@ hipError_t launch_ccl_candidates(const float* cand, const uint32_t* cand_cnt, i6
                                  int rec_words) {
   const int nbx = (W + RTX - 1) / RTX, nby = (H + RTY - 1) / RTY;
   hipError_t e;
-  if (dense) {  // background of the materialized label volume
-    if ((e = launch_fill_u32(P, (i64)W * H * D, 0u, s)) != hipSuccess) return e;
-  }
   // the 13 forward offsets with one carry per axis are the positive offsets only for
   // width, height >= 2; otherwise every link goes through the generic merge
   const int generic = (W < 2 || H < 2) ? 1 : 0;
   hipLaunchKernelGGL(k_cand_local, dim3((unsigned)ntiles), dim3(NTR), 0, s, cand, cand_cnt, fgbits,
-                     P, rlab, W, H, D, nbx, nby, 1 - generic, rec_words);
+                     P, rlab, roots, multi, root_words, W, H, D, nbx, nby, 1 - generic, rec_words);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark("ccl/cand_local", s);
   hipLaunchKernelGGL(k_cand_merge, dim3((unsigned)ntiles), dim3(NTR), 0, s, cand, cand_cnt,
@@ -624,11 +710,16 @@ hipError_t launch_ccl_candidates(const float* cand, const uint32_t* cand_cnt, i6
                      positive_offsets(W, H), rec_words);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark("ccl/cand_merge", s);
-  if ((e = launch_fill_u64((u64*)roots, root_words, 0ull, s)) != hipSuccess) return e;
-  if ((e = launch_fill_u64((u64*)multi, root_words, 0ull, s)) != hipSuccess) return e;
   hipLaunchKernelGGL(k_cand_flatten, dim3((unsigned)ntiles), dim3(NTR), 0, s, cand, cand_cnt, P,
-                     rlab, roots, multi, dense ? 1 : 0, W, H, D, nbx, nby, rec_words);
+                     rlab, roots, multi, W, H, D, nbx, nby, rec_words);
+  if ((e = hipGetLastError()) != hipSuccess) return e;
   mark("ccl/cand_flatten", s);
+  if (dense) {
+    const int vec = W % 4 == 0 && (uintptr_t)P % 16 == 0;
+    hipLaunchKernelGGL(k_label_rows, dim3((unsigned)ntiles), dim3(NTR), 0, s, cand, cand_cnt,
+                       (const uint32_t*)rlab, P, W, H, D, nbx, nby, rec_words, vec);
+    mark("ccl/label_rows", s);
+  }
   return hipGetLastError();
 }
 

@@ -368,15 +368,14 @@ hipError_t launch_region_finalize(const RegionAcc* acc, i64 R, int is_ave, Regio
 hipError_t launch_tile_reserve(const uint32_t* d_R, i64 acc_cap, i64 arena_cap, u64* running,
                                TileOut* t, hipStream_t s);
 hipError_t launch_fill_u64(u64* p, i64 n, u64 value, hipStream_t s);
-hipError_t launch_fill_u32(uint32_t* p, i64 n, uint32_t value, hipStream_t s);
 // Labeling of the candidates the Hessian pass recorded (cand / cand_cnt, see
 // launch_hessian): fgbits (fg_words() words) receives the candidate bit mask; P is a
 // volume-sized parent array written and read at candidate voxels only; rlab (slot-aligned
 // with the records) receives each record's label, the component's minimum linear index;
 // roots (root_words 64-bit words, cleared here) receives the root bit of every component,
 // in linear order, and multi (same size, cleared here) the root bit of every component
-// with voxels outside the kAccGY x kAccGZ tile group of its root.  dense: P becomes the
-// full label volume (0 for the background).
+// with voxels outside the kAccGY x kAccGZ tile group of its root (both NULL: not wanted).
+// dense: P becomes the full label volume (0 for the background).
 // rec_words: 32-bit words per record slot block (7: the Hessian pass's records; 1: the
 // positions of launch_mask_records).
 hipError_t launch_ccl_candidates(const float* cand, const uint32_t* cand_cnt, i64 ntiles,

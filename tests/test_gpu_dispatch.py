@@ -52,3 +52,19 @@ def test_records_walks_give_the_materialized_regions(hd, shape):
     b = hd.download_regions()
     for k in ("label", "count", "size16", "isum", "imax", "centroid", "norm"):
         np.testing.assert_array_equal(a[k], b[k], err_msg=k)
+
+
+# a mask's bytes are read in fours from any address, its labels written in quads or words:
+# every remainder of the width, fewer than four voxels, a mask that starts at an odd byte
+@pytest.mark.parametrize("shape", [(1, 1, 1), (1, 1, 3), (2, 1, 2), (5, 9, 61), (5, 9, 62),
+                                   (17, 10, 63), (17, 9, 64), (3, 8, 129)])
+@pytest.mark.parametrize("skip", [0, 1, 3])
+def test_labels_of_any_mask_address(hd, shape, skip):
+    import torch
+    n = int(np.prod(shape))
+    mask = (np.random.default_rng(n).random(n) < 0.4).astype(np.uint8) * 255
+    store = torch.zeros(n + 8, dtype=torch.uint8, device=hd.device)
+    store[skip:skip + n] = torch.from_numpy(mask).to(hd.device)
+    pd = store[skip:skip + n].view(shape)
+    store[skip + n:] = 1  # what follows the mask is not read as part of it
+    np.testing.assert_array_equal(hd.CCL(pd).cpu().numpy(), oracle.ccl3d(mask.reshape(shape)))
