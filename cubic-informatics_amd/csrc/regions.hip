@@ -271,22 +271,6 @@ struct LdsTable {
     double ns, h[6];
   };
 
-  __device__ void add(RegionAcc* acc, uint32_t r, uint32_t x, uint32_t y, uint32_t z,
-                      const float* hv, float nv, uint32_t iv, int is_ave, bool has_img,
-                      bool owned = false) {
-    Part q;
-    q.cnt = 1u;
-    q.dx = x - ox;
-    q.dy = y - oy;
-    q.dz = z - oz;
-    q.isum = q.imax = iv;
-    q.nkey = is_ave ? 0u : fkey(nv);
-    q.ns = is_ave ? (double)nv : 0.0;
-#pragma unroll
-    for (int k = 0; k < 6; ++k) q.h[k] = (double)hv[k];
-    add_part(acc, r, q, is_ave, has_img, owned);
-  }
-
   __device__ void add_part(RegionAcc* acc, uint32_t r, const Part& q, int is_ave, bool has_img,
                            bool owned) {
     uint32_t slot = (r * 2654435761u) >> (32 - __builtin_ctz(S));
@@ -351,12 +335,92 @@ struct LdsTable {
   }
 };
 
-// Region sums from the materialized Hessian (the per-stage interface).  A work-group takes
-// a brick of 64 x BY x BZ voxels (one row of 64 x per wave and z step); all loads of the
-// brick are issued up front, then every candidate voxel folds itself into the table
-// (128 slots: at most 128 separate 26-connected regions fit in a 64 x 4 x 4 brick).
-constexpr int BY = 4, BZ = 4;
+// v of lane i + 1 (lane 63 keeps its own) and of lane i - 1 (lane 0 keeps its own); one
+// DPP move each.  The whole wave must be active.
+__device__ __forceinline__ uint32_t lane_next(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x130, 0xf, 0xf, false);
+}
+__device__ __forceinline__ uint32_t lane_prev(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x138, 0xf, 0xf, false);
+}
 
+// Adds one voxel per lane (those with ok) to the table; the whole wave calls it together.
+// hv: the six elements, nv: the normalized value, iv: the raw intensity.
+template <int S>
+__device__ __forceinline__ void fold_wave(LdsTable<S>& tab, RegionAcc* acc, uint32_t cap, bool ok,
+                                          bool owned, uint32_t r, uint32_t x, uint32_t y,
+                                          uint32_t z, const float* hv, float nv, uint32_t iv,
+                                          int is_ave, bool has_img) {
+  const int lane = (int)(threadIdx.x & 63);
+  // Consecutive records are mostly x-neighbours in one row of one region.  Runs of
+  // lanes with the same region are cut into groups of at most four; the first lane of
+  // a group adds the group's sums, so the table sees one set of atomics per group.
+  // (the shifts run in every lane, outside any condition: a lane whose source lane is
+  // inactive would get its own value back)
+  const uint32_t r_prev = lane_prev(r);
+  const uint32_t ok_prev = lane_prev(ok ? 1u : 0u);
+  const bool run_head = (lane == 0) | !ok | (ok_prev == 0u) | (r_prev != r);
+  const unsigned long long heads = __ballot(run_head);
+  const unsigned long long upto = lane == 63 ? ~0ull : (2ull << lane) - 1ull;
+  const int start = 63 - __builtin_clzll(heads & upto);  // first lane of the run
+  const unsigned long long later = heads & ~upto;
+  const int next = later ? __builtin_ctzll(later) : 64;  // first lane of the next run
+  const int last = min(next - 1, lane + 3);  // last lane of a group that starts here
+  typename LdsTable<S>::Part g;
+  g.cnt = 1u;
+  g.dx = x - tab.ox;
+  g.dy = y - tab.oy;
+  g.dz = z - tab.oz;
+  g.isum = g.imax = iv;
+  g.nkey = is_ave ? 0u : fkey(nv);
+  g.ns = is_ave ? (double)nv : 0.0;
+#pragma unroll
+  for (int k = 0; k < 6; ++k) g.h[k] = (double)hv[k];
+  // the values of lanes +1, +2, +3 arrive by one-lane shifts; those past `last` are
+  // left out (a shift keeps lane 63's own value, which is never inside its group)
+  uint32_t sdx = g.dx, sdy = g.dy, sdz = g.dz, siv = iv, snk = g.nkey;
+  float snv = nv, sh[6];
+#pragma unroll
+  for (int k = 0; k < 6; ++k) sh[k] = hv[k];
+#pragma unroll
+  for (int o = 1; o <= 3; ++o) {
+    sdx = lane_next(sdx);
+    sdy = lane_next(sdy);
+    sdz = lane_next(sdz);
+    siv = lane_next(siv);
+    if (is_ave)
+      snv = __uint_as_float(lane_next(__float_as_uint(snv)));
+    else
+      snk = lane_next(snk);
+#pragma unroll
+    for (int k = 0; k < 6; ++k) sh[k] = __uint_as_float(lane_next(__float_as_uint(sh[k])));
+    if (lane + o <= last) {
+      g.cnt += 1u;
+      g.dx += sdx;
+      g.dy += sdy;
+      g.dz += sdz;
+      g.isum += siv;
+      g.imax = max(g.imax, siv);
+      if (is_ave)
+        g.ns += (double)snv;
+      else
+        g.nkey = max(g.nkey, snk);
+#pragma unroll
+      for (int k = 0; k < 6; ++k) g.h[k] += (double)sh[k];
+    }
+  }
+  const bool head = ((lane - start) & 3) == 0;
+  if (ok && head && r < cap) tab.add_part(acc, r, g, is_ave, has_img, owned);
+}
+
+// Region sums from the materialized Hessian (the per-stage interface).  A work-group takes
+// one 64 x 8 x 16 tile: it reads the tile's labels (a row of 64 per wave, eight rows in
+// flight), lists the positions of the labelled voxels in LDS, row by row in lane order, and
+// then folds the list with full waves, as the record form below does.  Bound by its gathers:
+// the label again (from L2), region id, six elements, normalized and raw intensity of the
+// labelled voxels.  Voxel by voxel without the list, on 64 x 4 x 4 bricks, a wave of 64
+// voxels folded about four, with one set of table atomics each and three bricks' global
+// atomics per region: 783 us for 48 x 1080 x 1280 with 6 % labelled, 296 us with the list.
 template <typename TH, typename TN>
 __global__ __launch_bounds__(NT) void k_accum(const uint32_t* __restrict__ L,
                                               const uint32_t* __restrict__ rid,
@@ -365,40 +429,62 @@ __global__ __launch_bounds__(NT) void k_accum(const uint32_t* __restrict__ L,
                                               const uint16_t* __restrict__ img, RegionAcc* acc,
                                               uint32_t cap, int W, int H, int D, i64 N, int nbx,
                                               int nby, int is_ave) {
+  constexpr int ROWS = kHessTY * kHessTZ, NWV = NT / 64, PF = 8;  // rows, waves, loads in flight
+  static_assert(ROWS % (NWV * PF) == 0 && kCandTile <= 65536, "whole batches of rows");
   __shared__ LdsTable<128> tab;
+  __shared__ uint16_t list[kCandTile];
+  __shared__ uint32_t n_list;
   unsigned b = xcd_tile(blockIdx.x, gridDim.x);
-  const int bx = b % nbx; b /= nbx;
-  const int by = b % nby; b /= nby;
-  const int x = bx * 64 + (threadIdx.x & 63);
-  const int y = by * BY + (threadIdx.x >> 6);
-  const int zb = (int)b * BZ;
-  tab.init((uint32_t)(bx * 64), (uint32_t)(by * BY), (uint32_t)zb);
+  const int x0 = (int)(b % (unsigned)nbx) * kHessTX; b /= (unsigned)nbx;
+  const int y0 = (int)(b % (unsigned)nby) * kHessTY; b /= (unsigned)nby;
+  const int z0 = (int)b * kHessTZ;
+  const int lane = (int)(threadIdx.x & 63);
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const i64 WH = (i64)W * H;
   const bool has_img = img != nullptr;
-  uint32_t l[BZ], r[BZ];
+  if (threadIdx.x == 0) n_list = 0u;
+  tab.init((uint32_t)x0, (uint32_t)y0, (uint32_t)z0);
+  __syncthreads();
+  for (int r0 = wave; r0 < ROWS; r0 += NWV * PF) {
+    uint32_t l[PF];
 #pragma unroll
-  for (int zz = 0; zz < BZ; ++zz) {
-    const int z = zb + zz;
-    l[zz] = (x < W && y < H && z < D) ? L[(i64)z * WH + (i64)y * W + x] : 0u;
+    for (int j = 0; j < PF; ++j) {
+      const int row = r0 + NWV * j, y = y0 + row % kHessTY, z = z0 + row / kHessTY;
+      l[j] = (x0 + lane < W && y < H && z < D) ? L[(i64)z * WH + (i64)y * W + x0 + lane] : 0u;
+    }
+#pragma unroll
+    for (int j = 0; j < PF; ++j) {
+      const unsigned long long on = __ballot(l[j] != 0u);
+      if (!on) continue;  // uniform over the wave
+      uint32_t base = 0;
+      if (lane == 0) base = atomicAdd(&n_list, (uint32_t)__popcll(on));
+      base = __builtin_amdgcn_readfirstlane(base);
+      if (l[j] != 0u)
+        list[base + (uint32_t)__popcll(on & ((1ull << lane) - 1ull))] =
+            (uint16_t)(lane + kHessTX * (r0 + NWV * j));
+    }
   }
-  float hv[BZ][6], nv[BZ];
-  uint32_t iv[BZ];
+  __syncthreads();
+  const uint32_t n = n_list;
+  if (n == 0u) return;  // uniform over the work-group
+  for (uint32_t k0 = threadIdx.x - lane; k0 < n; k0 += NT) {
+    const bool ok = k0 + lane < n;
+    uint32_t r = 0u, x = 0u, y = 0u, z = 0u, iv = 0u;
+    float hv[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f}, nv = 0.0f;
+    if (ok) {
+      const uint32_t v = list[k0 + lane];
+      x = (uint32_t)x0 + v % kHessTX;
+      y = (uint32_t)y0 + v / kHessTX % kHessTY;
+      z = (uint32_t)z0 + v / (kHessTX * kHessTY);
+      const i64 i = (i64)z * WH + (i64)y * W + x;
 #pragma unroll
-  for (int zz = 0; zz < BZ; ++zz) {
-    const i64 i = (i64)(zb + zz) * WH + (i64)y * W + x;
-    const bool on = l[zz] != 0u;
-    r[zz] = on ? rid[l[zz]] : 0u;
-#pragma unroll
-    for (int k = 0; k < 6; ++k) hv[zz][k] = on ? ld(hess, (i64)k * N + i) : 0.0f;
-    nv[zz] = on ? ld(norm, i) : 0.0f;
-    iv[zz] = (on && has_img) ? (uint32_t)img[i] : 0u;
+      for (int k = 0; k < 6; ++k) hv[k] = ld(hess, (i64)k * N + i);
+      nv = ld(norm, i);
+      iv = has_img ? (uint32_t)img[i] : 0u;
+      r = rid[L[i]];
+    }
+    fold_wave(tab, acc, cap, ok, false, r, x, y, z, hv, nv, iv, is_ave, has_img);
   }
-  __syncthreads();  // table initialised
-#pragma unroll
-  for (int zz = 0; zz < BZ; ++zz)
-    if (l[zz] && r[zz] < cap)
-      tab.add(acc, r[zz], (uint32_t)x, (uint32_t)y, (uint32_t)(zb + zz), hv[zz], nv[zz], iv[zz],
-              is_ave, has_img);
   __syncthreads();
   tab.flush(acc, is_ave, has_img);
 }
@@ -410,15 +496,6 @@ __global__ __launch_bounds__(NT) void k_accum(const uint32_t* __restrict__ L,
 static_assert(kAccGY * kAccGZ * kCandTile < (1 << 16) && kHessTX <= 256 &&
                   kAccGY * kHessTY <= 256 && kAccGZ * kHessTZ <= 256,
               "packed table sums: count below 2^16, offsets below 256");
-// v of lane i + 1 (lane 63 keeps its own) and of lane i - 1 (lane 0 keeps its own); one
-// DPP move each.  The whole wave must be active.
-__device__ __forceinline__ uint32_t lane_next(uint32_t v) {
-  return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x130, 0xf, 0xf, false);
-}
-__device__ __forceinline__ uint32_t lane_prev(uint32_t v) {
-  return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x138, 0xf, 0xf, false);
-}
-
 template <typename TN>
 __global__ __launch_bounds__(NT) void k_accum_cand(const float* __restrict__ cand,
                                                    const uint32_t* __restrict__ cand_cnt,
@@ -483,65 +560,7 @@ __global__ __launch_bounds__(NT) void k_accum_cand(const float* __restrict__ can
         nv = ld(norm, (i64)idx);
         iv = has_img ? (uint32_t)img[idx] : 0u;
       }
-      // Consecutive records are mostly x-neighbours in one row of one region.  Runs of
-      // lanes with the same region are cut into groups of at most four; the first lane of
-      // a group adds the group's sums, so the table sees one set of atomics per group.
-      // (the shifts run in every lane, outside any condition: a lane whose source lane is
-      // inactive would get its own value back)
-      const uint32_t r_prev = lane_prev(r);
-      const uint32_t ok_prev = lane_prev(ok ? 1u : 0u);
-      const bool run_head = (lane == 0) | !ok | (ok_prev == 0u) | (r_prev != r);
-      const unsigned long long heads = __ballot(run_head);
-      const unsigned long long upto = lane == 63 ? ~0ull : (2ull << lane) - 1ull;
-      const int start = 63 - __builtin_clzll(heads & upto);  // first lane of the run
-      const unsigned long long later = heads & ~upto;
-      const int next = later ? __builtin_ctzll(later) : 64;  // first lane of the next run
-      const int last = min(next - 1, lane + 3);  // last lane of a group that starts here
-      typename LdsTable<256>::Part g;
-      g.cnt = 1u;
-      g.dx = x - tab.ox;
-      g.dy = y - tab.oy;
-      g.dz = z - tab.oz;
-      g.isum = g.imax = iv;
-      g.nkey = is_ave ? 0u : fkey(nv);
-      g.ns = is_ave ? (double)nv : 0.0;
-#pragma unroll
-      for (int k = 0; k < 6; ++k) g.h[k] = (double)hv[k];
-      // the values of lanes +1, +2, +3 arrive by one-lane shifts; those past `last` are
-      // left out (a shift keeps lane 63's own value, which is never inside its group)
-      uint32_t sdx = g.dx, sdy = g.dy, sdz = g.dz, siv = iv, snk = g.nkey;
-      float snv = nv, sh[6];
-#pragma unroll
-      for (int k = 0; k < 6; ++k) sh[k] = hv[k];
-#pragma unroll
-      for (int o = 1; o <= 3; ++o) {
-        sdx = lane_next(sdx);
-        sdy = lane_next(sdy);
-        sdz = lane_next(sdz);
-        siv = lane_next(siv);
-        if (is_ave)
-          snv = __uint_as_float(lane_next(__float_as_uint(snv)));
-        else
-          snk = lane_next(snk);
-#pragma unroll
-        for (int k = 0; k < 6; ++k) sh[k] = __uint_as_float(lane_next(__float_as_uint(sh[k])));
-        if (lane + o <= last) {
-          g.cnt += 1u;
-          g.dx += sdx;
-          g.dy += sdy;
-          g.dz += sdz;
-          g.isum += siv;
-          g.imax = max(g.imax, siv);
-          if (is_ave)
-            g.ns += (double)snv;
-          else
-            g.nkey = max(g.nkey, snk);
-#pragma unroll
-          for (int k = 0; k < 6; ++k) g.h[k] += (double)sh[k];
-        }
-      }
-      const bool head = ((lane - start) & 3) == 0;
-      if (ok && head && r < cap) tab.add_part(acc, r, g, is_ave, has_img, owned);
+      fold_wave(tab, acc, cap, ok, owned, r, x, y, z, hv, nv, iv, is_ave, has_img);
     }
   }
   __syncthreads();
@@ -650,10 +669,6 @@ __global__ __launch_bounds__(NT) void k_fill_u64(u64* p, i64 n, u64 v) {
   for (i64 i = (i64)blockIdx.x * NT + threadIdx.x; i < n; i += (i64)gridDim.x * NT) p[i] = v;
 }
 
-__global__ __launch_bounds__(NT) void k_fill_u32(uint32_t* p, i64 n, uint32_t v) {
-  for (i64 i = (i64)blockIdx.x * NT + threadIdx.x; i < n; i += (i64)gridDim.x * NT) p[i] = v;
-}
-
 // roots per 4096-voxel block from the root bit mask (one wave per block, a word per lane)
 __global__ __launch_bounds__(NT) void k_mask_counts(const unsigned long long* __restrict__ masks,
                                                     i64 nb, uint32_t* __restrict__ cnt) {
@@ -706,8 +721,8 @@ template <typename TH, typename TN>
 hipError_t launch_region_accum(const uint32_t* labels, const uint32_t* rid, const TH* hess,
                                const TN* norm, const uint16_t* img, RegionAcc* acc, i64 cap,
                                int W, int H, int D, int is_ave, hipStream_t s) {
-  const int nbx = (W + 63) / 64, nby = (H + BY - 1) / BY, nbz = (D + BZ - 1) / BZ;
-  const i64 nblk = (i64)nbx * nby * nbz;
+  const int nbx = (W + kHessTX - 1) / kHessTX, nby = (H + kHessTY - 1) / kHessTY;
+  const i64 nblk = hessian_tiles(W, H, D);
   const i64 N = (i64)W * H * D;
   hipLaunchKernelGGL((k_accum<TH, TN>), dim3((unsigned)nblk), dim3(NT), 0, s, labels, rid, hess,
                      norm, img, acc, (uint32_t)std::min<i64>(cap, 0xFFFFFFFFll), W, H, D, N, nbx,
@@ -762,12 +777,6 @@ hipError_t launch_region_finalize(const RegionAcc* acc, i64 R, int is_ave, Regio
 hipError_t launch_tile_reserve(const uint32_t* d_R, i64 acc_cap, i64 arena_cap, u64* running,
                                TileOut* t, hipStream_t s) {
   hipLaunchKernelGGL(k_tile_reserve, dim3(1), dim3(64), 0, s, d_R, acc_cap, arena_cap, running, t);
-  return hipGetLastError();
-}
-
-hipError_t launch_fill_u32(uint32_t* p, i64 n, uint32_t value, hipStream_t s) {
-  const i64 nb = std::max<i64>(1, std::min<i64>((n + NT - 1) / NT, 1 << 16));
-  hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)nb), dim3(NT), 0, s, p, n, value);
   return hipGetLastError();
 }
 

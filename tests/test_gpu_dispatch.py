@@ -41,10 +41,8 @@ def test_split_walks_bitexact(hd, shape):
 # Hessian tiles per records-only work-group: one to four, with a short last walk
 @pytest.mark.parametrize("shape", [(70, 40, 70), (33, 640, 700), (49, 1500, 1600)])
 def test_records_walks_give_the_materialized_regions(hd, shape):
-    import torch
-    vol = synth.make_volume("c0", shape=shape, n_blobs=shape[0] * shape[1] * shape[2] // 20000,
-                            seed=11)
-    img = torch.from_numpy(vol).to(hd.device)
+    blobs = synth.blob_table(shape, shape[0] * shape[1] * shape[2] // 20000, 11)
+    img = hd.synth_volume(shape, blobs, 11, 200.0, 200.0, 20.0)
     p = hd.make_params(shape, 10, 10, 0, 2.0, 2.0, 3.2, 3.2, 4.0)
     hd.run_device(img, p)
     a = hd.download_regions()
@@ -52,6 +50,43 @@ def test_records_walks_give_the_materialized_regions(hd, shape):
     b = hd.download_regions()
     for k in ("label", "count", "size16", "isum", "imax", "centroid", "norm"):
         np.testing.assert_array_equal(a[k], b[k], err_msg=k)
+
+
+# given labels: tiles of one region, of a region per voxel (more than a tile's table holds),
+# of none, regions across tiles, ragged edges; with and without the raw stack, max and sum
+@pytest.mark.parametrize("shape,kind", [((17, 9, 65), "solid"), ((16, 8, 64), "points"),
+                                        ((33, 41, 130), "random"), ((20, 16, 64), "empty")])
+@pytest.mark.parametrize("ave", [False, True])
+def test_features_of_given_labels(hd, shape, kind, ave):
+    rng = np.random.default_rng(7)
+    pd = np.zeros(shape, np.uint8)
+    if kind == "solid":
+        pd[:] = 1
+    elif kind == "points":
+        pd[::2, ::2, ::2] = 1
+    elif kind == "random":
+        pd[:] = rng.random(shape) < 0.07
+    hess = (rng.standard_normal((6,) + shape) * 0.01).astype(np.float32)
+    norm = rng.standard_normal(shape).astype(np.float32)
+    img = noise(shape, 8)
+    labels = hd.CCL(pd)
+    np.testing.assert_array_equal(labels.cpu().numpy(), oracle.ccl3d(pd))
+    o = oracle.regions(labels.cpu().numpy(), hess, norm, img, ave)
+    g = hd.RegionalFeatures(labels, hess, norm, img, ave)
+    for k in ("label", "count", "size16", "isum", "imax"):
+        np.testing.assert_array_equal(g[k][1:], o[k][1:], err_msg=k)
+    np.testing.assert_array_equal(g["centroid"][1:], o["centroid"][1:])
+    # sums: FP64 in another order, rounded once to FP32
+    n = o["count"][1:, None].astype(np.float64)
+    mag = np.abs(hess).max() * n
+    assert np.all(np.abs(g["hsum"][1:].astype(np.float64) - o["hsum"][1:]) <=
+                  1.2e-7 * np.abs(o["hsum"][1:]) + 1e-12 * mag)
+    d = np.abs(g["norm"][1:].astype(np.float64) - o["norm"][1:])
+    assert np.all(d <= (1.2e-7 * np.abs(o["norm"][1:]) + 1e-12 * n[:, 0] * np.abs(norm).max()
+                        if ave else 0.0))
+    bare = hd.RegionalFeatures(labels, hess, norm, None, ave)
+    np.testing.assert_array_equal(bare["count"], g["count"])
+    assert not bare["isum"].any() and not bare["imax"].any()
 
 
 # a mask's bytes are read in fours from any address, its labels written in quads or words:
