@@ -338,7 +338,7 @@ int run_stages(hdog_ctx* ctx, hipStream_t s, const hdog_params* p, const uint16_
                               p->radius_z, s, nullptr, nullptr,
                               tuned_norm(ctx, W, H, D, p->precision)));
   const float nz = powf(ctx->sigma[0], p->gamma * 2) * powf(ctx->sigma[1], p->gamma);
-  HIPCHK(launch_dog<TN, TD>(norm, dog, tmp1, tmp2, (const float*)ctx->weights.p, ctx->r, nz, W,
+  HIPCHK(launch_dog<TN, TD>(norm, dog, tmp1, (const float*)ctx->weights.p, ctx->r, nz, W,
                             H, D, s, tuned_gauss(ctx, W, H, D, p->precision)));
   // the Hessian pass also leaves compact candidate records and the candidate bit mask;
   // labeling and the region pass work from those, not from the mask and element volumes
@@ -468,7 +468,7 @@ hipError_t batch_tile(hdog_ctx* ctx, BatchState* B, BatchLane& L, int t, hipStre
                                 tuned_norm(ctx, W, H, D, p->precision))) != hipSuccess)
     return e;
   const float nz = powf(ctx->sigma[0], p->gamma * 2) * powf(ctx->sigma[1], p->gamma);
-  if ((e = launch_dog<TN, TD>(norm, dog, L.tmp1, L.tmp2, (const float*)B->weights.p, ctx->r, nz, W,
+  if ((e = launch_dog<TN, TD>(norm, dog, L.tmp1, (const float*)B->weights.p, ctx->r, nz, W,
                               H, D, s, tuned_gauss(ctx, W, H, D, p->precision))) != hipSuccess)
     return e;
   const i64 ntiles = hessian_tiles(W, H, D);
@@ -590,15 +590,16 @@ int autotune_t(hdog_ctx* ctx, hipStream_t s, const hdog_params* p, const uint16_
   TN* norm = (TN*)ctx->norm.p;
   TD* dog = (TD*)ctx->dog.p;
   const float nz = powf(ctx->sigma[0], p->gamma * 2) * powf(ctx->sigma[1], p->gamma);
-  const int wb_gauss = 2 * std::max(ctx->r[0], ctx->r[2]) + 1;
+  int gauss_waves, gauss_wb, gauss_halo;
+  gauss_walk_shape(ctx->r[0], ctx->r[2], &gauss_waves, &gauss_wb, &gauss_halo);
   struct Stage {
-    int wb;
+    int wb, halo;
     i64 strips;  // waves per segment, all planes
     int* best;
     float* ms;
     bool dog;
-  } stages[2] = {{21, (i64)((W + 127) / 128) * D, best_norm, ms_norm, false},
-                 {wb_gauss, (i64)((W + 63) / 64) * D, best_gauss, ms_gauss, true}};
+  } stages[2] = {{21, 20, (i64)((W + 127) / 128) * D, best_norm, ms_norm, false},
+                 {gauss_wb, gauss_halo, (i64)((W + 63) / 64) * D * gauss_waves, best_gauss, ms_gauss, true}};
   for (const Stage& st : stages) {
     // the built-in shape (choice 2) stays unless another one is faster by more than 3 %: a
     // choice within the timing noise would change nothing but the launch shape
@@ -606,14 +607,14 @@ int autotune_t(hdog_ctx* ctx, hipStream_t s, const hdog_params* p, const uint16_
     int nys[kMaxSegments + 1];
     for (int want = 1; want <= kMaxSegments; ++want) {
       int rows;
-      walk_segments(H, st.wb, st.strips, &nys[want], &rows, want);
+      walk_segments(H, st.wb, st.strips, &nys[want], &rows, want, st.halo);
       ms[want] = -1.0f;
       for (int k = 1; k < want; ++k)
         if (nys[k] == nys[want]) ms[want] = ms[k];  // the same shape
       if (ms[want] >= 0.0f) continue;
       if (st.dog)
         HIPCHK(time_median(s, [&] {
-          return launch_dog<TN, TD>(norm, dog, tmp1, tmp2,
+          return launch_dog<TN, TD>(norm, dog, tmp1,
                                     (const float*)ctx->weights.p, ctx->r, nz, W, H, D, s, want);
         }, &ms[want]));
       else
@@ -803,9 +804,8 @@ int hdog_dog3d(hdog_ctx* ctx, void* stream, const float* d_norm, float* d_dog, i
   HIPCHK(hipSetDevice(ctx->device));
   const i64 N = (i64)width * height * depth;
   HIPCHK(ensure(ctx->tmp1, (size_t)N * 8));
-  HIPCHK(ensure(ctx->tmp2, (size_t)N * 8));
   const float nz = powf(ctx->sigma[0], gamma * 2) * powf(ctx->sigma[1], gamma);
-  HIPCHK(launch_dog<float, float>(d_norm, d_dog, ctx->tmp1.p, ctx->tmp2.p, (const float*)ctx->weights.p,
+  HIPCHK(launch_dog<float, float>(d_norm, d_dog, ctx->tmp1.p, (const float*)ctx->weights.p,
                            ctx->r, nz, width, height, depth, (hipStream_t)stream));
   return HDOG_OK;
 }

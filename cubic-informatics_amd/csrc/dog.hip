@@ -10,10 +10,10 @@
 // intermediate volumes of the reference become one interleaved stream.  Intermediates
 // stay FP32 whatever the storage type of norm / dog.
 //
-// Radius pairs (r1, r2) that occur in practice have compile-time kernels with the weights
-// in scalar registers: the x pass makes 4 outputs per thread from 128-bit LDS reads, the
-// y / z passes are column walkers (one thread per line, a register ring, every input
-// read once, no LDS).  Other radii use the generic LDS-tile loops.
+// Radius pairs (r1, r2) that occur in practice have compile-time kernels: the x and y passes
+// fused in a row walker, the z pass (and the differentiable form's separate passes) as column
+// walkers (one thread per line, a register ring, every input read once, no LDS).  Other radii
+// have walkers with LDS rings that form eight outputs at a time.
 #include "hdog_internal.hpp"
 
 namespace hdog {
@@ -21,76 +21,320 @@ namespace {
 
 constexpr int NT = 256;
 
-// ------------------------------------------------------------------- generic radii
-template <int ROWS, typename TS>
-__global__ __launch_bounds__(NT) void k_gauss_x(const TS* __restrict__ src, float2* __restrict__ dst,
-                                                const float* __restrict__ w1,
-                                                const float* __restrict__ w2, int r1, int r2,
-                                                int W, i64 nrows, int C, int nct) {
-  extern __shared__ float smf[];
-  const int R = max(r1, r2);
-  const int span = C + 2 * R;
-  const unsigned tile = xcd_tile(blockIdx.x, gridDim.x);
-  const int ct = tile % nct;
-  const i64 row0 = (i64)(tile / nct) * ROWS;
-  const int c0 = ct * C;
-  stage_tile<8, NT, float>(
-      ROWS * span,
-      [&](int e) -> float {
-        const int row = e / span, p = e % span;
-        const i64 grow = row0 + row;
-        const int x = c0 - R + p;
-        return (grow < nrows && x >= 0 && x < W) ? ld(src, grow * W + x) : 0.0f;
-      },
-      [&](int e, float v) { smf[e] = v; });
-  __syncthreads();
-  for (int e = threadIdx.x; e < ROWS * C; e += NT) {
-    const int row = e / C, i = e % C, x = c0 + i;
-    const i64 grow = row0 + row;
-    if (x >= W || grow >= nrows) continue;
-    const float* t = smf + row * span + i + R;
-    float s1 = 0.0f, s2 = 0.0f;
-    for (int j = -r1; j <= r1; ++j) s1 = fmaf(w1[r1 - j], t[j], s1);
-    for (int j = -r2; j <= r2; ++j) s2 = fmaf(w2[r2 - j], t[j], s2);
-    dst[grow * W + x] = make_float2(s1, s2);
+// ------------------------------------------------------------------- any radii
+// Sums of eight consecutive outputs of one Gaussian of radius r: every input is read once and
+// meets its outputs' accumulators in turn, so each output is the chain over ascending inputs,
+// and no tap outside the window is formed (a zero weight would still turn an infinite or NaN
+// input into NaN).  next() gives inputs c - r, c - r + 1, ... c + 7 + r.  The weights are
+// symmetric (both halves are set from one value); the lanes of `wv` hold them, w[j] in lane j
+// or, for more than 64 (WIDE), w[r + j], and a tap's weight is read from there into a scalar
+// register, an operand of its FMAs; loaded from memory, every four inputs waited for their
+// weights, and with them for all LDS reads.
+constexpr int GK = 8;
+constexpr int kLaneRadius = 31;  // 2r + 1 weights fit a wave's lanes
+template <bool WIDE>
+__device__ __forceinline__ float gauss_lanes(const float* w, int r) {
+  const int l = (int)(threadIdx.x & 63);
+  return WIDE ? w[r + min(l, r)] : w[min(l, 2 * r)];
+}
+template <bool WIDE>
+__device__ __forceinline__ float gauss_tap(float wv, int t, int r) {  // weight of tap t
+  const int l = WIDE ? abs(t - r) : t;
+  return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(wv), l));
+}
+template <bool WIDE, int R, typename F>
+__device__ __forceinline__ void gauss8_short(F&& next, float wv, float (&acc)[GK]) {
+  float v[2 * R + GK];
+#pragma unroll
+  for (int i = 0; i < 2 * R + GK; ++i) v[i] = next();
+#pragma unroll
+  for (int i = 0; i < 2 * R + GK; ++i)
+#pragma unroll
+    for (int o = 0; o < GK; ++o)
+      if (i - o >= 0 && i - o <= 2 * R) acc[o] = fmaf(gauss_tap<WIDE>(wv, i - o, R), v[i], acc[o]);
+}
+template <bool WIDE, typename F>
+__device__ __forceinline__ void gauss8(F&& next, float wv, int r, float (&acc)[GK]) {
+#pragma unroll
+  for (int o = 0; o < GK; ++o) acc[o] = 0.0f;
+  if (r < 3) {  // uniform: fewer taps than outputs
+    if (r == 0) gauss8_short<WIDE, 0>(next, wv, acc);
+    if (r == 1) gauss8_short<WIDE, 1>(next, wv, acc);
+    if (r == 2) gauss8_short<WIDE, 2>(next, wv, acc);
+    return;
+  }
+  // inputs 0 .. 6 start the outputs, 7 .. 2r meet all eight, 2r + 1 .. 2r + 7 end them;
+  // four inputs are always read ahead of their use
+  float h[GK - 1], v[4], e[GK - 1];
+  float t[GK + 3];  // weights of taps i - 7 .. i + 3 at input i
+#pragma unroll
+  for (int i = 0; i < GK - 1; ++i) h[i] = next();
+#pragma unroll
+  for (int q = 0; q < 4; ++q) v[q] = next();
+#pragma unroll
+  for (int i = 0; i < GK - 1; ++i) e[i] = t[i] = gauss_tap<WIDE>(wv, i, r);
+#pragma unroll
+  for (int i = 0; i < GK - 1; ++i)
+#pragma unroll
+    for (int o = 0; o <= i; ++o) acc[o] = fmaf(e[i - o], h[i], acc[o]);
+  int i = GK - 1;
+#pragma unroll 1
+  for (; i + 3 <= 2 * r; i += 4) {
+    float n[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) n[q] = next();
+#pragma unroll
+    for (int q = 0; q < 4; ++q) t[GK - 1 + q] = gauss_tap<WIDE>(wv, i + q, r);
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int o = 0; o < GK; ++o) acc[o] = fmaf(t[GK - 1 + q - o], v[q], acc[o]);
+#pragma unroll
+    for (int q = 0; q < GK - 1; ++q) t[q] = t[q + 4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] = n[q];
+  }
+  // the end: tap 2r + u - o of input 2r + u, whose weight is that of tap o - u
+  auto end = [&](const float* z) {
+#pragma unroll
+    for (int u = 1; u < GK; ++u)
+#pragma unroll
+      for (int o = u; o < GK; ++o) acc[o] = fmaf(e[o - u], z[u - 1], acc[o]);
+  };
+  if (i <= 2 * r) {  // two inputs left before it (2r - 6 is even)
+    float z[GK + 1] = {v[0], v[1], v[2], v[3]};
+#pragma unroll
+    for (int q = 4; q < GK + 1; ++q) z[q] = next();
+#pragma unroll
+    for (int q = 0; q < 2; ++q) t[GK - 1 + q] = gauss_tap<WIDE>(wv, i + q, r);
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+      for (int o = 0; o < GK; ++o) acc[o] = fmaf(t[GK - 1 + q - o], z[q], acc[o]);
+    end(z + 2);
+  } else {
+    float z[GK - 1] = {v[0], v[1], v[2], v[3]};
+#pragma unroll
+    for (int q = 4; q < GK - 1; ++q) z[q] = next();
+    end(z);
   }
 }
 
-template <int XW, bool LAST, typename TS>
-__global__ __launch_bounds__(NT) void k_gauss_line(const float2* __restrict__ src,
-                                                   float2* __restrict__ dst, TS* __restrict__ dog,
-                                                   const float* __restrict__ w1,
-                                                   const float* __restrict__ w2, int r1, int r2,
-                                                   float nz, int W, int L, i64 sa, i64 so, int C,
-                                                   int nxt, int nct) {
-  extern __shared__ float2 smf2[];
-  const int R = max(r1, r2);
-  const int span = C + 2 * R;
-  unsigned b = blockIdx.x;
-  const int xt = b % nxt; b /= nxt;
-  const int ct = b % nct; b /= nct;
-  const i64 base = (i64)b * so;
-  const int x0 = xt * XW, c0 = ct * C;
-  stage_tile<8, NT, float2>(
-      span * XW,
-      [&](int e) -> float2 {
-        const int p = e / XW, x = x0 + e % XW, c = c0 - R + p;
-        return (x < W && c >= 0 && c < L) ? src[base + (i64)c * sa + x] : make_float2(0.0f, 0.0f);
-      },
-      [&](int e, float2 v) { smf2[e] = v; });
+// Moves rows STEP .. STEP + hist - 1 of the two planes to rows 0 .. hist - 1 (whole
+// work-group; a barrier before and after is the caller's).
+template <int NTH, int STEP, int PITCH>
+__device__ __forceinline__ void shift_rows(float* B1, float* B2, int hist) {
+  for (int r0 = 0; r0 < hist; r0 += STEP) {  // source and target of one part are disjoint
+    if (r0) __syncthreads();                 // the part before was read from this target
+    const int n = min(STEP, hist - r0) * PITCH;
+    for (int e = (int)threadIdx.x; e < n; e += NTH) {
+      B1[r0 * PITCH + e] = B1[(r0 + STEP) * PITCH + e];
+      B2[r0 * PITCH + e] = B2[(r0 + STEP) * PITCH + e];
+    }
+  }
+}
+
+// x and y passes of both Gaussians for any radii.  A work-group of NW waves walks the rows of
+// one plane for a strip of 64 columns, eight rows per wave and step:
+//   1. a wave's eight rows x0-RX .. x0+63+RX, loaded a step ahead through row descriptors
+//      (zero outside the plane), enter its LDS lines A;
+//   2. lane (row l % 8, columns 8 (l / 8) ..) forms eight x outputs of each Gaussian, which
+//      enter two LDS planes B below the 2RY rows before them (padded pitches: the lanes of
+//      both accesses fall on different banks);
+//   3. lane l forms eight y outputs of column x0 + l; then the last 2RY rows of B move up.
+// The (G1_x, G2_x) volume between the passes is never stored.  Bound by instruction issue
+// (2 (rx1 + rx2 + ry1 + ry2 + 2) FMAs per voxel): the LDS leaves three waves per SIMD at
+// radius 14, and four waves sharing B keep it at that; one wave with B as a ring of its own
+// left one or two, whose ring arithmetic then cost as much as the FMAs (606 us, below).  One
+// output per thread with a read per tap, in two passes through memory, took 1360 us for
+// 61 x 900 x 1111 at radii 9 / 14; this takes 356 us.
+template <typename TS, int NC, int NW>
+__global__ __launch_bounds__(64 * NW) void k_gauss_xy_run(
+    const TS* __restrict__ src, float2* __restrict__ dst, const float* __restrict__ wx1,
+    const float* __restrict__ wx2, const float* __restrict__ wy1, const float* __restrict__ wy2,
+    int rx1, int rx2, int ry1, int ry2, int W, int H, int nxs, int nys, int rows) {
+  extern __shared__ float sm_xy[];
+  constexpr bool WIDE = NC > 2;
+  constexpr int BP = 65, STEP = GK * NW;  // pitch of B, rows per step
+  const int RX = max(rx1, rx2), RY = max(ry1, ry2), hist = 2 * RY;
+  const int AP = (64 + 2 * RX + 7) / 8 * 8 + 1, NRB = hist + STEP;
+  const int l = (int)(threadIdx.x & 63);
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  float* A = sm_xy + wave * (GK * AP);
+  float* B1 = sm_xy + NW * (GK * AP);
+  float* B2 = B1 + NRB * BP;
+  const unsigned t = xcd_tile(blockIdx.x, gridDim.x);
+  const int y0 = (int)(t % (unsigned)nys) * rows, y1 = min(H, y0 + rows);
+  const unsigned tile = t / (unsigned)nys;
+  const int x0 = (int)(tile % (unsigned)nxs) * 64;
+  const i64 pbase = (i64)(tile / (unsigned)nxs) * H * W;
+  typedef typename StoredBits<TS>::type Bits;
+  Bits q[GK][NC];
+  const uint32_t row_bytes = (uint32_t)W * (uint32_t)sizeof(TS);
+  // column x0 - RX + 64 k + l; left of the row the offset wraps past the record count
+  uint32_t off[NC];
+#pragma unroll
+  for (int k = 0; k < NC; ++k) {
+    const int c = 64 * k + l;
+    off[k] = c < 64 + 2 * RX ? (uint32_t)(x0 - RX + c) * (uint32_t)sizeof(TS) : 0xFFFFFFF0u;
+  }
+  auto fetch = [&](int y) {
+#pragma unroll
+    for (int r = 0; r < GK; ++r) {
+      const bool in = y + r >= 0 && y + r < H;
+      const __amdgpu_buffer_rsrc_t rs =
+          buf_rsrc(src + pbase + (i64)(in ? y + r : 0) * W, in ? row_bytes : 0u);
+#pragma unroll
+      for (int k = 0; k < NC; ++k) q[r][k] = buf_load<TS>(rs, off[k]);
+    }
+  };
+  const float vx1 = gauss_lanes<WIDE>(wx1, rx1), vx2 = gauss_lanes<WIDE>(wx2, rx2),
+              vy1 = gauss_lanes<WIDE>(wy1, ry1), vy2 = gauss_lanes<WIDE>(wy2, ry2);
+  const int xr = l % GK, xg = l / GK;
+  // x outputs of the eight fetched rows into rows `row` .. of B, fetching rows `ahead` ..
+  auto xpass = [&](int row, int ahead) {
+#pragma unroll
+    for (int r = 0; r < GK; ++r)
+#pragma unroll
+      for (int k = 0; k < NC; ++k)
+        if (64 * k + l < 64 + 2 * RX) A[r * AP + 64 * k + l] = from_bits<TS>(q[r][k]);
+    fetch(ahead);
+    wave_lds_sync();
+#pragma unroll 1
+    for (int g = 0; g < 2; ++g) {  // one copy of the sums for both Gaussians
+      const int r = g ? rx2 : rx1;
+      const float* p = A + xr * AP + xg * GK + (RX - r);
+      float acc[GK];
+      gauss8<WIDE>([&] { return *p++; }, g ? vx2 : vx1, r, acc);
+      float* b = (g ? B2 : B1) + (row + xr) * BP + xg * GK;
+#pragma unroll
+      for (int o = 0; o < GK; ++o) b[o] = acc[o];
+    }
+    wave_lds_sync();
+  };
+  // the rows above the segment (the last eight may reach into the first step's rows, which
+  // are written again after the barrier)
+  const int main0 = y0 + RY + GK * wave;
+  if (GK * wave < hist) {
+    fetch(y0 - RY + GK * wave);
+    for (int g = wave; GK * g < hist; g += NW)
+      xpass(GK * g, GK * (g + NW) < hist ? y0 - RY + GK * (g + NW) : main0);
+  } else {
+    fetch(main0);
+  }
   __syncthreads();
-  for (int e = threadIdx.x; e < C * XW; e += NT) {
-    const int i = e / XW, xl = e % XW, c = c0 + i, x = x0 + xl;
-    if (c >= L || x >= W) continue;
-    const float2* t = smf2 + (i + R) * XW + xl;
-    float s1 = 0.0f, s2 = 0.0f;
-    for (int j = -r1; j <= r1; ++j) s1 = fmaf(w1[r1 - j], t[j * XW].x, s1);
-    for (int j = -r2; j <= r2; ++j) s2 = fmaf(w2[r2 - j], t[j * XW].y, s2);
-    const i64 idx = base + (i64)c * sa + x;
-    if (LAST)
-      dog[idx] = cvt<TS>((s1 - s2) * nz);
-    else
-      dst[idx] = make_float2(s1, s2);
+  const bool out = x0 + l < W;
+  float2* dcol = dst + pbase + x0 + l;
+  for (int c0 = y0; c0 < y1; c0 += STEP) {
+    xpass(hist + GK * wave, c0 + STEP + RY + GK * wave);
+    __syncthreads();
+    const int c = c0 + GK * wave;
+    if (c < y1) {
+      float a1[GK], a2[GK];
+#pragma unroll 1
+      for (int g = 0; g < 2; ++g) {
+        const int r = g ? ry2 : ry1;
+        const float* p = (g ? B2 : B1) + (GK * wave + RY - r) * BP + l;
+        float acc[GK];
+        gauss8<WIDE>([&] { const float v = *p; p += BP; return v; }, g ? vy2 : vy1, r, acc);
+#pragma unroll
+        for (int o = 0; o < GK; ++o) {
+          if (g == 0) a1[o] = acc[o];
+          a2[o] = acc[o];
+        }
+      }
+      if (out) {
+#pragma unroll
+        for (int o = 0; o < GK; ++o)
+          if (c + o < y1) st_nt(dcol + (i64)(c + o) * W, make_float2(a1[o], a2[o]));
+      }
+    }
+    if (c0 + STEP >= y1) break;  // uniform
+    __syncthreads();
+    shift_rows<64 * NW, STEP, BP>(B1, B2, hist);
+    __syncthreads();
+  }
+}
+
+// One pass along y (sa = W) or z (sa = W H) for any radii: a work-group of four waves walks a
+// segment of 64 x-adjacent lines, eight positions per wave and step, through two LDS planes of
+// the last 2R + 32 positions (zero outside the line).  Bound by its 12 or 16 bytes per voxel
+// for short windows (61 x 900 x 1111 along z at radii 4 / 7: 377 us with one output per thread
+// and a read per tap, 198 us now).
+template <bool LAST, bool WIDE, typename TS>
+__global__ __launch_bounds__(256) void k_gauss_line_run(const float2* __restrict__ src,
+                                                        float2* __restrict__ dst,
+                                                        TS* __restrict__ dog,
+                                                        const float* __restrict__ w1,
+                                                        const float* __restrict__ w2, int r1,
+                                                        int r2, float nz, int W, int L, i64 sa,
+                                                        i64 so, unsigned nxb, unsigned no,
+                                                        int len) {
+  extern __shared__ float sm_line[];
+  constexpr int NW = 4, STEP = GK * NW;
+  const int R = max(r1, r2), hist = 2 * R;
+  float* B1 = sm_line;
+  float* B2 = B1 + (hist + STEP) * 64;
+  const int l = (int)(threadIdx.x & 63);
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const unsigned t = xcd_tile(blockIdx.x, gridDim.x);
+  const int x0 = (int)(t % nxb) * 64;
+  const i64 base = (i64)(t / nxb % no) * so + x0;
+  const int s0 = (int)(t / nxb / no) * len, s1 = min(L, s0 + len);
+  const uint32_t nrec = (uint32_t)min(64, W - x0) * (uint32_t)sizeof(float2);
+  float2 q[GK];
+  auto fetch = [&](int p) {
+#pragma unroll
+    for (int r = 0; r < GK; ++r) {
+      const bool in = p + r >= 0 && p + r < L;
+      const __amdgpu_buffer_rsrc_t rs =
+          buf_rsrc(src + base + (i64)(in ? p + r : 0) * sa, in ? nrec : 0u);
+      q[r] = __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(
+                                            rs, l * (int)sizeof(float2), 0, 0));
+    }
+  };
+  auto put = [&](int row) {
+#pragma unroll
+    for (int r = 0; r < GK; ++r) {
+      B1[(row + r) * 64 + l] = q[r].x;
+      B2[(row + r) * 64 + l] = q[r].y;
+    }
+  };
+  const float v1 = gauss_lanes<WIDE>(w1, r1), v2 = gauss_lanes<WIDE>(w2, r2);
+  for (int g = wave; GK * g < hist; g += NW) {
+    fetch(s0 - R + GK * g);
+    put(GK * g);
+  }
+  fetch(s0 + R + GK * wave);
+  __syncthreads();
+  const bool out = x0 + l < W;
+  for (int c0 = s0; c0 < s1; c0 += STEP) {
+    put(hist + GK * wave);
+    fetch(c0 + STEP + R + GK * wave);
+    __syncthreads();
+    const int c = c0 + GK * wave;
+    if (c < s1) {
+      float a1[GK], a2[GK];
+      const float* p = B1 + (GK * wave + R - r1) * 64 + l;
+      gauss8<WIDE>([&] { const float v = *p; p += 64; return v; }, v1, r1, a1);
+      p = B2 + (GK * wave + R - r2) * 64 + l;
+      gauss8<WIDE>([&] { const float v = *p; p += 64; return v; }, v2, r2, a2);
+      if (out) {
+#pragma unroll
+        for (int o = 0; o < GK; ++o) {
+          if (c + o >= s1) continue;
+          const i64 idx = base + (i64)(c + o) * sa + l;
+          if (LAST)
+            st_nt(dog + idx, (a1[o] - a2[o]) * nz);
+          else
+            st_nt(dst + idx, make_float2(a1[o], a2[o]));
+        }
+      }
+    }
+    if (c0 + STEP >= s1) break;  // uniform
+    __syncthreads();
+    shift_rows<256, STEP, 64>(B1, B2, hist);
+    __syncthreads();
   }
 }
 
@@ -344,6 +588,14 @@ __global__ __launch_bounds__(64) void k_gauss_xy_walk(const TS* __restrict__ src
 // (2.0 / 3.2, 1.6 / 2.56) and of the reference's example sigmas (4.0 / 6.0, 1.8 / 2.7).
 #define HDOG_GAUSS_PAIRS(X) X(8, 13) X(6, 10) X(4, 6) X(3, 5) X(8, 12) X(4, 5) X(7, 11)
 
+bool has_pair(int r1, int r2) {
+#define X(A, B) if (r1 == A && r2 == B) return true;
+  HDOG_GAUSS_PAIRS(X)
+#undef X
+  return false;
+}
+
+// x pass of a radius pair with a compile-time kernel
 template <typename TS>
 hipError_t gauss_x(const TS* src, float2* dst, const float* w1, const float* w2, int r1, int r2,
                    int W, i64 nrows, hipStream_t s) {
@@ -358,20 +610,43 @@ hipError_t gauss_x(const TS* src, float2* dst, const float* w1, const float* w2,
   }
   HDOG_GAUSS_PAIRS(X)
 #undef X
-  constexpr int ROWS = 4;
-  const int C = 256;
-  const int nct = (W + C - 1) / C;
-  const i64 nblk = ((nrows + ROWS - 1) / ROWS) * nct;
-  const size_t lds = (size_t)ROWS * (C + 2 * std::max(r1, r2)) * 4;
-  hipLaunchKernelGGL((k_gauss_x<ROWS, TS>), dim3((unsigned)nblk), dim3(NT), lds, s, src, dst, w1,
-                     w2, r1, r2, W, nrows, C, nct);
+  return hipErrorInvalidValue;
+}
+
+// Waves per work-group of the walker for any radii: four where their LDS stays within the
+// 64 KB of a launch and the weights fit the lanes (radii up to 28), else two.
+size_t xy_run_lds(int RX, int RY, int nw) {
+  return ((size_t)nw * GK * ((64 + 2 * RX + 7) / 8 * 8 + 1) + 2 * (size_t)(2 * RY + GK * nw) * 65) * 4;
+}
+int xy_run_waves(int RX, int RY) {
+  return xy_run_lds(RX, RY, 4) <= 64 * 1024 && std::max(RX, RY) <= kLaneRadius ? 4 : 2;
+}
+
+// x and y passes of any radii, each axis with its own
+template <typename TS>
+hipError_t gauss_xy_run(const TS* src, float2* dst, const float* wx1, const float* wx2,
+                        const float* wy1, const float* wy2, int rx1, int rx2, int ry1, int ry2,
+                        int W, int H, int D, hipStream_t s, int segments) {
+  const int RX = std::max(rx1, rx2), RY = std::max(ry1, ry2);
+  const int nxs = (W + 63) / 64;
+  const int nw = xy_run_waves(RX, RY);
+  int nys, rows;
+  walk_segments(H, GK * 4, (i64)nxs * D * nw, &nys, &rows, segments, 2 * RY);
+  const dim3 grid((unsigned)((i64)nxs * D * nys));
+  const size_t lds = xy_run_lds(RX, RY, nw);
+  if (nw == 4)
+    hipLaunchKernelGGL((k_gauss_xy_run<TS, 2, 4>), grid, dim3(256), lds, s, src, dst, wx1, wx2, wy1,
+                       wy2, rx1, rx2, ry1, ry2, W, H, nxs, nys, rows);
+  else
+    hipLaunchKernelGGL((k_gauss_xy_run<TS, 3, 2>), grid, dim3(128), lds, s, src, dst, wx1, wx2, wy1,
+                       wy2, rx1, rx2, ry1, ry2, W, H, nxs, nys, rows);
   return hipGetLastError();
 }
 
-// Fused x + y passes for the compile-time radius pairs; false when (r1, r2) has none.
+// Fused x + y passes with the same weights on both axes
 template <typename TS>
-bool gauss_xy(const TS* src, float2* dst, const float* w1, const float* w2, int r1, int r2,
-              int W, int H, int D, hipStream_t s, hipError_t* e, int segments) {
+hipError_t gauss_xy(const TS* src, float2* dst, const float* w1, const float* w2, int r1, int r2,
+                    int W, int H, int D, hipStream_t s, int segments) {
 #define X(A, B)                                                                              \
   if (r1 == A && r2 == B) {                                                                  \
     const int nxs = (W + 63) / 64;                                                           \
@@ -380,12 +655,11 @@ bool gauss_xy(const TS* src, float2* dst, const float* w1, const float* w2, int 
     const i64 nblk = (i64)nxs * D * nys;                                                     \
     hipLaunchKernelGGL((k_gauss_xy_walk<A, B, TS>), dim3((unsigned)nblk), dim3(64), 0, s,    \
                        src, dst, w1, w2, W, H, nxs, nys, rows);                              \
-    *e = hipGetLastError();                                                                  \
-    return true;                                                                             \
+    return hipGetLastError();                                                                \
   }
   HDOG_GAUSS_PAIRS(X)
 #undef X
-  return false;
+  return gauss_xy_run<TS>(src, dst, w1, w2, w1, w2, r1, r2, r1, r2, W, H, D, s, segments);
 }
 
 template <bool LAST, typename TS>
@@ -402,25 +676,32 @@ hipError_t gauss_line(const float2* src, float2* dst, TS* dog, const float* w1, 
   HDOG_GAUSS_PAIRS(X)
 #undef X
   const int R = std::max(r1, r2);
-  int XW = R > 24 ? 32 : 64;
-  int C = 64;
-  if (L < C) C = L;
-  const int nxt = (W + XW - 1) / XW, nct = (L + C - 1) / C;
-  const i64 nblk = (i64)nxt * nct * n_other;
-  const size_t lds = (size_t)(C + 2 * R) * XW * 8;
-  if (XW == 64)
-    hipLaunchKernelGGL((k_gauss_line<64, LAST, TS>), dim3((unsigned)nblk), dim3(NT), lds, s, src,
-                       dst, dog, w1, w2, r1, r2, nz, W, L, sa, so, C, nxt, nct);
+  const i64 nxb = (W + 63) / 64;
+  int nseg, len;
+  line_segments(L, nxb * n_other * 4, 1024.0, 2.0, false, 2 * R, &nseg, &len);
+  const dim3 grid((unsigned)(nxb * n_other * nseg));
+  const size_t lds = 2 * (size_t)(2 * R + 4 * GK) * 64 * 4;
+  if (R <= kLaneRadius)
+    hipLaunchKernelGGL((k_gauss_line_run<LAST, false, TS>), grid, dim3(256), lds, s, src, dst, dog,
+                       w1, w2, r1, r2, nz, W, L, sa, so, (unsigned)nxb, (unsigned)n_other, len);
   else
-    hipLaunchKernelGGL((k_gauss_line<32, LAST, TS>), dim3((unsigned)nblk), dim3(NT), lds, s, src,
-                       dst, dog, w1, w2, r1, r2, nz, W, L, sa, so, C, nxt, nct);
+    hipLaunchKernelGGL((k_gauss_line_run<LAST, true, TS>), grid, dim3(256), lds, s, src, dst, dog,
+                       w1, w2, r1, r2, nz, W, L, sa, so, (unsigned)nxb, (unsigned)n_other, len);
   return hipGetLastError();
 }
 
 }  // namespace
 
+void gauss_walk_shape(int r1, int r2, int* waves, int* period, int* halo) {
+  const int R = std::max(r1, r2);
+  const bool pair = has_pair(r1, r2);
+  *waves = pair ? 1 : xy_run_waves(R, R);
+  *period = pair ? 2 * R + 1 : GK * 4;
+  *halo = 2 * R;
+}
+
 template <typename TN, typename TD>
-hipError_t launch_dog(const TN* norm, TD* dog, void* tmp1, void* tmp2, const float* weights,
+hipError_t launch_dog(const TN* norm, TD* dog, void* tmp1, const float* weights,
                       const int r[4], float normalizer, int W, int H, int D, hipStream_t s,
                       int segments) {
   const i64 WH = (i64)W * H;
@@ -428,24 +709,11 @@ hipError_t launch_dog(const TN* norm, TD* dog, void* tmp1, void* tmp2, const flo
   const float* wz1 = weights + kMaxTaps;
   const float* wxy2 = weights + 2 * kMaxTaps;
   const float* wz2 = weights + 3 * kMaxTaps;
-  hipError_t e = hipSuccess;
-  const float2* gxy = (const float2*)tmp2;
-  if (gauss_xy<TN>(norm, (float2*)tmp1, wxy1, wxy2, r[0], r[2], W, H, D, s, &e, segments)) {
-    if (e != hipSuccess) return e;
-    mark("dog/gauss_xy", s);
-    gxy = (const float2*)tmp1;
-  } else {
-    if ((e = gauss_x<TN>(norm, (float2*)tmp1, wxy1, wxy2, r[0], r[2], W, (i64)H * D, s)) !=
-        hipSuccess)
-      return e;
-    mark("dog/gauss_x", s);
-    if ((e = gauss_line<false, TD>((const float2*)tmp1, (float2*)tmp2, nullptr, wxy1, wxy2, r[0],
-                                   r[2], 0.0f, W, H, W, WH, D, s)) != hipSuccess)
-      return e;
-    mark("dog/gauss_y", s);
-  }
-  e = gauss_line<true, TD>(gxy, nullptr, dog, wz1, wz2, r[1], r[3], normalizer, W, D, WH, W, H,
-                           s);
+  hipError_t e = gauss_xy<TN>(norm, (float2*)tmp1, wxy1, wxy2, r[0], r[2], W, H, D, s, segments);
+  if (e != hipSuccess) return e;
+  mark("dog/gauss_xy", s);
+  e = gauss_line<true, TD>((const float2*)tmp1, nullptr, dog, wz1, wz2, r[1], r[3], normalizer, W,
+                           D, WH, W, H, s);
   mark("dog/gauss_z_dog", s);
   return e;
 }
@@ -459,12 +727,17 @@ hipError_t launch_gauss_pair(const float* src, void* tmp1, void* tmp2, const flo
                              int D, hipStream_t s) {
   const i64 WH = (i64)W * H;
   hipError_t e;
-  if ((e = gauss_x<float>(src, (float2*)tmp1, w[0], w[3], r[0], r[3], W, (i64)H * D, s)) !=
-      hipSuccess)
-    return e;
-  if ((e = gauss_line<false, float>((const float2*)tmp1, (float2*)tmp2, nullptr, w[1], w[4], r[1],
-                                    r[4], 0.0f, W, H, W, WH, D, s)) != hipSuccess)
-    return e;
+  if (has_pair(r[0], r[3]) && has_pair(r[1], r[4])) {
+    if ((e = gauss_x<float>(src, (float2*)tmp1, w[0], w[3], r[0], r[3], W, (i64)H * D, s)) !=
+        hipSuccess)
+      return e;
+    e = gauss_line<false, float>((const float2*)tmp1, (float2*)tmp2, nullptr, w[1], w[4], r[1],
+                                 r[4], 0.0f, W, H, W, WH, D, s);
+  } else {
+    e = gauss_xy_run<float>(src, (float2*)tmp2, w[0], w[3], w[1], w[4], r[0], r[3], r[1], r[4], W,
+                            H, D, s, 0);
+  }
+  if (e != hipSuccess) return e;
   if (dog)
     return gauss_line<true, float>((const float2*)tmp2, nullptr, dog, w[2], w[5], r[2], r[5], nz, W,
                                    D, WH, W, H, s);
@@ -473,8 +746,8 @@ hipError_t launch_gauss_pair(const float* src, void* tmp1, void* tmp2, const flo
 }
 
 #define HDOG_INST_DOG(TN, TD)                                                                \
-  template hipError_t launch_dog<TN, TD>(const TN*, TD*, void*, void*, const float*, const int*, \
-                                         float, int, int, int, hipStream_t, int);
+  template hipError_t launch_dog<TN, TD>(const TN*, TD*, void*, const float*, const int*, float, \
+                                         int, int, int, hipStream_t, int);
 HDOG_INST_DOG(float, float)
 HDOG_INST_DOG(__half, __half)
 HDOG_INST_DOG(__hip_bfloat16, __hip_bfloat16)

@@ -182,13 +182,16 @@ inline void mark(const char* name, hipStream_t s) {
 // stacks from 24 x 96 x 112 to 256 x 1080 x 1280.
 
 // Row segments of a row walker (one wave per strip and segment; `strips`: waves per segment
-// over all planes; segment length: a multiple of the ring period wb, context wb - 1 rows).
+// over all planes; segment length: a multiple of wb rows, context: `halo` rows, the wb - 1 of
+// a register ring of period wb by default).
 // t = 1.3 gives both walkers' sweeps within 10 %: norm_xy, 32 x 2160 x 2560: 914 us with two
 // segments, 543 with eight, 528 with sixteen; 128 x 256 x 256: 165 us with one, 54 with seven,
 // 60 with thirteen; gauss_xy there 102, 46 and 51 us with one, five and ten; on a full tile
 // 2 to 4 segments are within 2 %.  A tuned launch shape `want` (1 .. 4) takes want / 2 of the
 // built-in count.
-inline void walk_segments(int H, int wb, i64 strips, int* nys, int* rows, int want = 0) {
+inline void walk_segments(int H, int wb, i64 strips, int* nys, int* rows, int want = 0,
+                          int halo = -1) {
+  if (halo < 0) halo = wb - 1;
   auto shape = [&](int n, int* k, int* r) {
     const int per = (H + n - 1) / n;
     *r = (per + wb - 1) / wb * wb;
@@ -200,7 +203,7 @@ inline void walk_segments(int H, int wb, i64 strips, int* nys, int* rows, int wa
   for (int n = 1; n <= most && n <= 64; ++n) {
     int k, r;
     shape(n, &k, &r);
-    const double cost = ((double)strips * k / 1024.0 + 1.3) * (std::min(r, H) + wb - 1);
+    const double cost = ((double)strips * k / 1024.0 + 1.3) * (std::min(r, H) + halo);
     if (n == 1 || cost < best_cost) {
       best_cost = cost;
       best = n;
@@ -303,12 +306,14 @@ hipError_t launch_normalize(const uint16_t* img, TS* norm, void* tmp1, void* tmp
 // y and z passes.
 hipError_t launch_box_pair(const float2* src, float2* dst, int W, int L, i64 sa, i64 so,
                            i64 n_other, int r, hipStream_t s);
-// DoG stage; weights: device array [4][kMaxTaps] (xy1, z1, xy2, z2); tmp1/tmp2 >= 8*N bytes;
+// DoG stage; weights: device array [4][kMaxTaps] (xy1, z1, xy2, z2); tmp1 >= 8*N bytes;
 // segments as for launch_normalize
 template <typename TN, typename TD>
-hipError_t launch_dog(const TN* norm, TD* dog, void* tmp1, void* tmp2, const float* weights,
-                      const int r[4], float normalizer, int W, int H, int D, hipStream_t s,
+hipError_t launch_dog(const TN* norm, TD* dog, void* tmp1, const float* weights, const int r[4], float normalizer, int W, int H, int D, hipStream_t s,
                       int segments = 0);
+// how the xy walker of a radius pair splits a plane: waves per 64-column strip and the
+// arguments of walk_segments
+void gauss_walk_shape(int r1, int r2, int* waves, int* period, int* halo);
 hipError_t launch_gauss_pair(const float* src, void* tmp1, void* tmp2, const float* const w[6],
                              const int r[6], float nz, float* dog, float2* pair_out, int W, int H,
                              int D, hipStream_t s);

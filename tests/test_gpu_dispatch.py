@@ -103,3 +103,24 @@ def test_labels_of_any_mask_address(hd, shape, skip):
     pd = store[skip:skip + n].view(shape)
     store[skip + n:] = 1  # what follows the mask is not read as part of it
     np.testing.assert_array_equal(hd.CCL(pd).cpu().numpy(), oracle.ccl3d(mask.reshape(shape)))
+
+
+# Gaussian radii without a compile-time kernel: fewer taps than outputs per step, windows wider
+# than the volume, the largest radius, a small radius that exceeds the large one along z; and
+# NaN and infinities, which reach exactly the outputs whose windows hold them
+@pytest.mark.parametrize("shape,s,trunc", [((9, 17, 70), (0.2, 0.2, 0.4, 0.3), 2.0),
+                                           ((11, 23, 65), (1.0, 0.4, 1.4, 0.9), 2.0),
+                                           ((20, 61, 129), (2.2, 1.1, 3.6, 1.8), 4.0),
+                                           ((33, 70, 64), (1.4, 2.6, 2.3, 1.5), 3.0),
+                                           ((7, 200, 90), (5.0, 1.0, 10.0, 3.3), 4.0),
+                                           ((90, 5, 3), (1.5, 9.9, 8.2, 9.0), 4.0)])
+@pytest.mark.parametrize("finite", [True, False])
+def test_dog_of_any_radii(hd, shape, s, trunc, finite):
+    rng = np.random.default_rng(21)
+    norm = (rng.standard_normal(shape) * 0.3).astype(np.float32)
+    if not finite:
+        for v in (np.nan, np.inf, -np.inf):
+            norm[tuple(int(rng.integers(n)) for n in shape)] = v
+    hd.initGaussian3DKernel(*s, truncate=trunc)
+    ref, _ = oracle.dog3d(norm, *s, truncate=trunc, gamma=1.0)
+    np.testing.assert_array_equal(hd.DoG3DFilter(norm).cpu().numpy(), ref)
