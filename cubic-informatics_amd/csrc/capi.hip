@@ -590,16 +590,13 @@ int autotune_t(hdog_ctx* ctx, hipStream_t s, const hdog_params* p, const uint16_
   TN* norm = (TN*)ctx->norm.p;
   TD* dog = (TD*)ctx->dog.p;
   const float nz = powf(ctx->sigma[0], p->gamma * 2) * powf(ctx->sigma[1], p->gamma);
-  int gauss_waves, gauss_wb, gauss_halo;
-  gauss_walk_shape(ctx->r[0], ctx->r[2], &gauss_waves, &gauss_wb, &gauss_halo);
   struct Stage {
-    int wb, halo;
-    i64 strips;  // waves per segment, all planes
+    WalkShape shape;
     int* best;
     float* ms;
     bool dog;
-  } stages[2] = {{21, 20, (i64)((W + 127) / 128) * D, best_norm, ms_norm, false},
-                 {gauss_wb, gauss_halo, (i64)((W + 63) / 64) * D * gauss_waves, best_gauss, ms_gauss, true}};
+  } stages[2] = {{norm_walk_shape(p->radius_xy, W, D), best_norm, ms_norm, false},
+                 {gauss_walk_shape(ctx->r[0], ctx->r[2], W, D), best_gauss, ms_gauss, true}};
   for (const Stage& st : stages) {
     // the built-in shape (choice 2) stays unless another one is faster by more than 3 %: a
     // choice within the timing noise would change nothing but the launch shape
@@ -607,7 +604,7 @@ int autotune_t(hdog_ctx* ctx, hipStream_t s, const hdog_params* p, const uint16_
     int nys[kMaxSegments + 1];
     for (int want = 1; want <= kMaxSegments; ++want) {
       int rows;
-      walk_segments(H, st.wb, st.strips, &nys[want], &rows, want, st.halo);
+      walk_segments(H, st.shape, &nys[want], &rows, want);
       ms[want] = -1.0f;
       for (int k = 1; k < want; ++k)
         if (nys[k] == nys[want]) ms[want] = ms[k];  // the same shape

@@ -120,20 +120,6 @@ __device__ __forceinline__ void gauss8(F&& next, float wv, int r, float (&acc)[G
   }
 }
 
-// Moves rows STEP .. STEP + hist - 1 of the two planes to rows 0 .. hist - 1 (whole
-// work-group; a barrier before and after is the caller's).
-template <int NTH, int STEP, int PITCH>
-__device__ __forceinline__ void shift_rows(float* B1, float* B2, int hist) {
-  for (int r0 = 0; r0 < hist; r0 += STEP) {  // source and target of one part are disjoint
-    if (r0) __syncthreads();                 // the part before was read from this target
-    const int n = min(STEP, hist - r0) * PITCH;
-    for (int e = (int)threadIdx.x; e < n; e += NTH) {
-      B1[r0 * PITCH + e] = B1[(r0 + STEP) * PITCH + e];
-      B2[r0 * PITCH + e] = B2[(r0 + STEP) * PITCH + e];
-    }
-  }
-}
-
 // x and y passes of both Gaussians for any radii.  A work-group of NW waves walks the rows of
 // one plane for a strip of 64 columns, eight rows per wave and step:
 //   1. a wave's eight rows x0-RX .. x0+63+RX, loaded a step ahead through row descriptors
@@ -251,7 +237,8 @@ __global__ __launch_bounds__(64 * NW) void k_gauss_xy_run(
     }
     if (c0 + STEP >= y1) break;  // uniform
     __syncthreads();
-    shift_rows<64 * NW, STEP, BP>(B1, B2, hist);
+    shift_rows<64 * NW, STEP, BP>(B1, hist);
+    shift_rows<64 * NW, STEP, BP>(B2, hist);
     __syncthreads();
   }
 }
@@ -333,7 +320,8 @@ __global__ __launch_bounds__(256) void k_gauss_line_run(const float2* __restrict
     }
     if (c0 + STEP >= s1) break;  // uniform
     __syncthreads();
-    shift_rows<256, STEP, 64>(B1, B2, hist);
+    shift_rows<256, STEP, 64>(B1, hist);
+    shift_rows<256, STEP, 64>(B2, hist);
     __syncthreads();
   }
 }
@@ -595,6 +583,19 @@ bool has_pair(int r1, int r2) {
   return false;
 }
 
+// Waves per work-group of the walker for any radii: four where their LDS stays within the
+// 64 KB of a launch and the weights fit the lanes (radii up to 28), else two.
+size_t xy_run_lds(int RX, int RY, int nw) {
+  return ((size_t)nw * GK * ((64 + 2 * RX + 7) / 8 * 8 + 1) + 2 * (size_t)(2 * RY + GK * nw) * 65) * 4;
+}
+int xy_run_waves(int RX, int RY) {
+  return xy_run_lds(RX, RY, 4) <= 64 * 1024 && std::max(RX, RY) <= kLaneRadius ? 4 : 2;
+}
+
+WalkShape xy_run_shape(int RX, int RY, int W, int D) {
+  return {(i64)((W + 63) / 64) * D * xy_run_waves(RX, RY), GK * 4, 2 * RY};
+}
+
 // x pass of a radius pair with a compile-time kernel
 template <typename TS>
 hipError_t gauss_x(const TS* src, float2* dst, const float* w1, const float* w2, int r1, int r2,
@@ -613,15 +614,6 @@ hipError_t gauss_x(const TS* src, float2* dst, const float* w1, const float* w2,
   return hipErrorInvalidValue;
 }
 
-// Waves per work-group of the walker for any radii: four where their LDS stays within the
-// 64 KB of a launch and the weights fit the lanes (radii up to 28), else two.
-size_t xy_run_lds(int RX, int RY, int nw) {
-  return ((size_t)nw * GK * ((64 + 2 * RX + 7) / 8 * 8 + 1) + 2 * (size_t)(2 * RY + GK * nw) * 65) * 4;
-}
-int xy_run_waves(int RX, int RY) {
-  return xy_run_lds(RX, RY, 4) <= 64 * 1024 && std::max(RX, RY) <= kLaneRadius ? 4 : 2;
-}
-
 // x and y passes of any radii, each axis with its own
 template <typename TS>
 hipError_t gauss_xy_run(const TS* src, float2* dst, const float* wx1, const float* wx2,
@@ -631,7 +623,7 @@ hipError_t gauss_xy_run(const TS* src, float2* dst, const float* wx1, const floa
   const int nxs = (W + 63) / 64;
   const int nw = xy_run_waves(RX, RY);
   int nys, rows;
-  walk_segments(H, GK * 4, (i64)nxs * D * nw, &nys, &rows, segments, 2 * RY);
+  walk_segments(H, xy_run_shape(RX, RY, W, D), &nys, &rows, segments);
   const dim3 grid((unsigned)((i64)nxs * D * nys));
   const size_t lds = xy_run_lds(RX, RY, nw);
   if (nw == 4)
@@ -651,7 +643,7 @@ hipError_t gauss_xy(const TS* src, float2* dst, const float* w1, const float* w2
   if (r1 == A && r2 == B) {                                                                  \
     const int nxs = (W + 63) / 64;                                                           \
     int nys, rows;                                                                           \
-    walk_segments(H, 2 * (A > B ? A : B) + 1, (i64)nxs * D, &nys, &rows, segments);          \
+    walk_segments(H, gauss_walk_shape(A, B, W, D), &nys, &rows, segments);                   \
     const i64 nblk = (i64)nxs * D * nys;                                                     \
     hipLaunchKernelGGL((k_gauss_xy_walk<A, B, TS>), dim3((unsigned)nblk), dim3(64), 0, s,    \
                        src, dst, w1, w2, W, H, nxs, nys, rows);                              \
@@ -692,12 +684,10 @@ hipError_t gauss_line(const float2* src, float2* dst, TS* dog, const float* w1, 
 
 }  // namespace
 
-void gauss_walk_shape(int r1, int r2, int* waves, int* period, int* halo) {
+WalkShape gauss_walk_shape(int r1, int r2, int W, int D) {
   const int R = std::max(r1, r2);
-  const bool pair = has_pair(r1, r2);
-  *waves = pair ? 1 : xy_run_waves(R, R);
-  *period = pair ? 2 * R + 1 : GK * 4;
-  *halo = 2 * R;
+  if (!has_pair(r1, r2)) return xy_run_shape(R, R, W, D);
+  return {(i64)((W + 63) / 64) * D, 2 * R + 1, 2 * R};
 }
 
 template <typename TN, typename TD>

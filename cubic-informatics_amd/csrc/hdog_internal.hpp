@@ -145,6 +145,17 @@ __device__ __forceinline__ void stage_tile(int n, LD&& ldf, ST&& stf) {
   }
 }
 
+// Moves rows STEP .. STEP + hist - 1 of an LDS plane to rows 0 .. hist - 1 (whole work-group;
+// a barrier before and after is the caller's): the history of a walk of STEP rows per step.
+template <int NTH, int STEP, int PITCH, typename T>
+__device__ __forceinline__ void shift_rows(T* B, int hist) {
+  for (int r0 = 0; r0 < hist; r0 += STEP) {  // source and target of one part are disjoint
+    if (r0) __syncthreads();                 // the part before was read from this target
+    const int n = min(STEP, hist - r0) * PITCH;
+    for (int e = (int)threadIdx.x; e < n; e += NTH) B[r0 * PITCH + e] = B[(r0 + STEP) * PITCH + e];
+  }
+}
+
 // ---- per-region accumulator (one 128-byte line per region) -----------------------
 struct alignas(128) RegionAcc {
   unsigned long long sx, sy, sz, isum;
@@ -181,17 +192,18 @@ inline void mark(const char* name, hipStream_t s) {
 // segment count with the least such time; t is fitted to sweeps of 1 .. 16 segments on
 // stacks from 24 x 96 x 112 to 256 x 1080 x 1280.
 
-// Row segments of a row walker (one wave per strip and segment; `strips`: waves per segment
-// over all planes; segment length: a multiple of wb rows, context: `halo` rows, the wb - 1 of
-// a register ring of period wb by default).
+// Row segments of a row walker.
 // t = 1.3 gives both walkers' sweeps within 10 %: norm_xy, 32 x 2160 x 2560: 914 us with two
 // segments, 543 with eight, 528 with sixteen; 128 x 256 x 256: 165 us with one, 54 with seven,
 // 60 with thirteen; gauss_xy there 102, 46 and 51 us with one, five and ten; on a full tile
 // 2 to 4 segments are within 2 %.  A tuned launch shape `want` (1 .. 4) takes want / 2 of the
 // built-in count.
-inline void walk_segments(int H, int wb, i64 strips, int* nys, int* rows, int want = 0,
-                          int halo = -1) {
-  if (halo < 0) halo = wb - 1;
+struct WalkShape {
+  i64 strips;        // waves per segment, all planes
+  int period, halo;  // segment length: a multiple of period; rows of context
+};
+inline void walk_segments(int H, const WalkShape& w, int* nys, int* rows, int want = 0) {
+  const int wb = w.period;
   auto shape = [&](int n, int* k, int* r) {
     const int per = (H + n - 1) / n;
     *r = (per + wb - 1) / wb * wb;
@@ -203,7 +215,7 @@ inline void walk_segments(int H, int wb, i64 strips, int* nys, int* rows, int wa
   for (int n = 1; n <= most && n <= 64; ++n) {
     int k, r;
     shape(n, &k, &r);
-    const double cost = ((double)strips * k / 1024.0 + 1.3) * (std::min(r, H) + halo);
+    const double cost = ((double)w.strips * k / 1024.0 + 1.3) * (std::min(r, H) + w.halo);
     if (n == 1 || cost < best_cost) {
       best_cost = cost;
       best = n;
@@ -311,9 +323,9 @@ hipError_t launch_box_pair(const float2* src, float2* dst, int W, int L, i64 sa,
 template <typename TN, typename TD>
 hipError_t launch_dog(const TN* norm, TD* dog, void* tmp1, const float* weights, const int r[4], float normalizer, int W, int H, int D, hipStream_t s,
                       int segments = 0);
-// how the xy walker of a radius pair splits a plane: waves per 64-column strip and the
-// arguments of walk_segments
-void gauss_walk_shape(int r1, int r2, int* waves, int* period, int* halo);
+// how the xy walkers of the two stages split planes of W columns, D of them
+WalkShape norm_walk_shape(int rxy, int W, int D);
+WalkShape gauss_walk_shape(int r1, int r2, int W, int D);
 hipError_t launch_gauss_pair(const float* src, void* tmp1, void* tmp2, const float* const w[6],
                              const int r[6], float nz, float* dog, float2* pair_out, int W, int H,
                              int D, hipStream_t s);

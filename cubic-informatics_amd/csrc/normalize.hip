@@ -19,7 +19,8 @@
 //     with the normalization.
 //   * For the radii in use, the z box pass (and the separate y / z min/max passes) are
 //     column walkers: one thread per line keeps a compile-time-sized register ring, reads
-//     every input once and needs no LDS.  Other radii use the LDS-tile kernels.
+//     every input once and needs no LDS.  Other radii up to kRunRadius have walks with the
+//     radius at run time and their history in LDS, larger ones the LDS-tile kernels.
 #include "hdog_internal.hpp"
 
 namespace hdog {
@@ -125,15 +126,13 @@ __global__ __launch_bounds__(NT) void k_minmax_line(const void* __restrict__ src
 // gives each lane 4 consecutive window minima (the window middle, shared by all four,
 // plus short prefix / suffix runs: about (2r + 12) / 4 packed mins per output); phase 3
 // gives each lane RUN consecutive box sums by sliding (integers: exact in any order).
-// Output: float2 (E_x, D_x) = (sum(min) * k, sum(max) * k).  R > 0 fixes the radius at
-// compile time (r must equal it); R = 0 takes r at run time.
-template <int R, int RUN>
+// Output: float2 (E_x, D_x) = (sum(min) * k, sum(max) * k).  For r above kRunRadius.
+template <int RUN>
 __global__ __launch_bounds__(NT) void k_minmax_x_box(const uint32_t* __restrict__ src,
                                                      float2* __restrict__ dst, int W, i64 nrows,
-                                                     int r_rt, int nct, float k) {
+                                                     int r, int nct, float k) {
   static_assert(RUN == 4, "four outputs per lane");
   constexpr int C = 64 * RUN;
-  const int r = R > 0 ? R : r_rt;
   extern __shared__ __align__(16) uint32_t smem_x[];
   const int spanmax = C + 4 * r + 4;  // a multiple of 4: both rows stay 16-byte aligned
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -154,87 +153,39 @@ __global__ __launch_bounds__(NT) void k_minmax_x_box(const uint32_t* __restrict_
   // middle A[j0+3 .. j0+2r] is shared by all four, plus short prefix / suffix runs
   for (int j0 = lane * 4; live && j0 < nq; j0 += 256) {
     uint32_t o[4];
-    if constexpr (R >= 2) {  // compile-time radius: 16-byte LDS reads, conflict-free
-      constexpr int NV = (2 * R + 4) / 4;
-      uint32_t w[4 * NV];
-#pragma unroll
-      for (int v = 0; v < NV; ++v) {
-        const uint4 q = *reinterpret_cast<const uint4*>(A + j0 + 4 * v);
-        w[4 * v] = q.x; w[4 * v + 1] = q.y; w[4 * v + 2] = q.z; w[4 * v + 3] = q.w;
-      }
-      const uint32_t mid = mid_min<R>(w);
-      const uint32_t l2 = w[2], l1 = pkmin(w[1], l2), l0 = pkmin(w[0], l1);
-      const uint32_t r1 = w[2 * R + 1], r2 = pkmin(r1, w[2 * R + 2]), r3 = pkmin(r2, w[2 * R + 3]);
-      o[0] = pkmin(mid, l0);
-      o[1] = pkmin(pkmin(mid, l1), r1);
-      o[2] = pkmin(pkmin(mid, l2), r2);
-      o[3] = pkmin(mid, r3);
-    } else if (2 * r + 1 >= 4) {
-      uint32_t mid = A[j0 + 3];
-      for (int t = 4; t <= 2 * r; ++t) mid = pkmin(mid, A[j0 + t]);
-      const uint32_t l2 = A[j0 + 2], l1 = pkmin(A[j0 + 1], l2), l0 = pkmin(A[j0], l1);
-      const uint32_t r1 = A[j0 + 2 * r + 1], r2 = pkmin(r1, A[j0 + 2 * r + 2]),
-                     r3 = pkmin(r2, A[j0 + 2 * r + 3]);
-      o[0] = pkmin(mid, l0);
-      o[1] = pkmin(pkmin(mid, l1), r1);
-      o[2] = pkmin(pkmin(mid, l2), r2);
-      o[3] = pkmin(mid, r3);
-    } else {  // r = 1
-#pragma unroll
-      for (int q = 0; q < 4; ++q) o[q] = pkmin(pkmin(A[j0 + q], A[j0 + q + 1]), A[j0 + q + 2]);
-    }
+    uint32_t mid = A[j0 + 3];
+    for (int t = 4; t <= 2 * r; ++t) mid = pkmin(mid, A[j0 + t]);
+    const uint32_t l2 = A[j0 + 2], l1 = pkmin(A[j0 + 1], l2), l0 = pkmin(A[j0], l1);
+    const uint32_t r1 = A[j0 + 2 * r + 1], r2 = pkmin(r1, A[j0 + 2 * r + 2]),
+                   r3 = pkmin(r2, A[j0 + 2 * r + 3]);
+    o[0] = pkmin(mid, l0);
+    o[1] = pkmin(pkmin(mid, l1), r1);
+    o[2] = pkmin(pkmin(mid, l2), r2);
+    o[3] = pkmin(mid, r3);
     *reinterpret_cast<uint4*>(B + j0) = make_uint4(o[0], o[1], o[2], o[3]);
   }
   __syncthreads();
   const int xs = c0 + lane * RUN;
   if (!live || xs >= W) return;
-  const bool interior = c0 - r >= 0 && c0 + C + r <= W;  // no clamping in this tile
   const uint32_t full = (uint32_t)(2 * r + 1) * 65535u;
   float2 out[RUN];
-  if (R > 0 && interior) {
-    // the window minima of x - r .. x + 3 + r are B[4 lane .. 4 lane + 2r + 3] (qa = c0 - r)
-    constexpr int RR = R > 0 ? R : 1;
-    constexpr int NV = (2 * RR + 4 + 3) / 4;
-    uint32_t w[4 * NV];
+  const uint32_t* m = B - qa;  // m[x]: window minimum at x, x in [qa, qb)
+  auto at = [&](int x) { return m[clampi(x, 0, W - 1)]; };
+  uint32_t se = 0, sdn = 0;
+  for (int j = -r; j <= r; ++j) {
+    const uint32_t v = at(xs + j);
+    se += v & 0xFFFFu;
+    sdn += v >> 16;
+  }
 #pragma unroll
-    for (int v = 0; v < NV; ++v) {
-      const uint4 q = *reinterpret_cast<const uint4*>(B + lane * 4 + 4 * v);
-      w[4 * v] = q.x; w[4 * v + 1] = q.y; w[4 * v + 2] = q.z; w[4 * v + 3] = q.w;
+  for (int q = 0; q < RUN; ++q) {
+    if (q > 0) {
+      const int x = xs + q;
+      const uint32_t vin = at(x + r), vout = at(x - r - 1);
+      se += (vin & 0xFFFFu) - (vout & 0xFFFFu);
+      sdn += (vin >> 16) - (vout >> 16);
     }
-    uint32_t se = 0, sdn = 0;  // sum of min, sum of (65535 - max)
-#pragma unroll
-    for (int t = 0; t <= 2 * RR; ++t) {
-      se += w[t] & 0xFFFFu;
-      sdn += w[t] >> 16;
-    }
-#pragma unroll
-    for (int q = 0; q < RUN; ++q) {
-      if (q > 0) {
-        const uint32_t vin = w[2 * RR + q], vout = w[q - 1];
-        se += (vin & 0xFFFFu) - (vout & 0xFFFFu);
-        sdn += (vin >> 16) - (vout >> 16);
-      }
-      out[q] = make_float2((float)se * k, (float)(full - sdn) * k);
-    }
-  } else {
-    const uint32_t* m = B - qa;  // m[x]: window minimum at x, x in [qa, qb)
-    auto at = [&](int x) { return m[clampi(x, 0, W - 1)]; };
-    uint32_t se = 0, sdn = 0;
-    for (int j = -r; j <= r; ++j) {
-      const uint32_t v = at(xs + j);
-      se += v & 0xFFFFu;
-      sdn += v >> 16;
-    }
-#pragma unroll
-    for (int q = 0; q < RUN; ++q) {
-      if (q > 0) {
-        const int x = xs + q;
-        const uint32_t vin = at(x + r), vout = at(x - r - 1);
-        se += (vin & 0xFFFFu) - (vout & 0xFFFFu);
-        sdn += (vin >> 16) - (vout >> 16);
-      }
-      out[q] = make_float2((float)se * k, (float)(full - sdn) * k);
-    }
+    out[q] = make_float2((float)se * k, (float)(full - sdn) * k);
   }
   float2* drow = dst + row * W;
   // 16-byte stores (a wave writes 1 KB in two instructions) where the row start allows
@@ -740,6 +691,435 @@ __global__ __launch_bounds__(64) void k_norm_xy_walk(const uint32_t* __restrict_
   }
 }
 
+// ---- radii without a kernel of their own, up to kRunRadius ---------------------------
+// The same passes with the radius at run time, eight outputs at a time: each input is read
+// once per group of eight, and the taps that all eight share are taken together.  next()
+// gives the inputs c - r, c - r + 1, ... c + 7 + r in order; R > 0 fixes the radius, for
+// windows shorter than the group (r <= 3), R = 0 takes r >= 4 at run time.
+constexpr int OK = 8;
+constexpr int kRunRadius = 24;
+
+// out[o] = packed minimum of inputs o .. o + 2r
+template <int R, typename F>
+__device__ __forceinline__ void min8(F&& next, int r, uint32_t (&out)[OK]) {
+  if constexpr (R > 0) {
+    uint32_t v[2 * R + OK];
+#pragma unroll
+    for (int i = 0; i < 2 * R + OK; ++i) v[i] = next();
+#pragma unroll
+    for (int o = 0; o < OK; ++o) {
+      out[o] = v[o];
+#pragma unroll
+      for (int i = 1; i <= 2 * R; ++i) out[o] = pkmin(out[o], v[o + i]);
+    }
+  } else {
+    uint32_t h[OK - 1], m[4], t;
+#pragma unroll
+    for (int i = 0; i < OK - 1; ++i) h[i] = next();
+    m[0] = next();  // input 7; inputs 7 .. 2r are in every window (2r - 6 of them, odd)
+#pragma unroll
+    for (int q = 1; q < 4; ++q) m[q] = m[0];
+    int i = OK;
+#pragma unroll 1
+    for (; i + 3 <= 2 * r; i += 4)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) m[q] = pkmin(m[q], next());  // four chains (see mid_min)
+    for (; i <= 2 * r; ++i) m[1] = pkmin(m[1], next());
+    const uint32_t mid = pkmin(pkmin(m[0], m[1]), pkmin(m[2], m[3]));
+    uint32_t e[OK - 1];
+#pragma unroll
+    for (int q = 0; q < OK - 1; ++q) e[q] = next();
+    t = mid;
+    out[OK - 1] = mid;
+#pragma unroll
+    for (int o = OK - 2; o >= 0; --o) out[o] = t = pkmin(t, h[o]);  // inputs o .. 2r
+    t = e[0];
+#pragma unroll
+    for (int o = 1; o < OK; ++o) {
+      if (o > 1) t = pkmin(t, e[o - 1]);
+      out[o] = pkmin(out[o], t);
+    }
+  }
+}
+
+// acc[o] = 0 + input o + input o + 1 ... + input o + 2r, in that order
+template <int R, typename F>
+__device__ __forceinline__ void sum8(F&& next, int r, float (&acc)[OK]) {
+#pragma unroll
+  for (int o = 0; o < OK; ++o) acc[o] = 0.0f;
+  if constexpr (R > 0) {
+    float v[2 * R + OK];
+#pragma unroll
+    for (int i = 0; i < 2 * R + OK; ++i) v[i] = next();
+#pragma unroll
+    for (int i = 0; i < 2 * R + OK; ++i)
+#pragma unroll
+      for (int o = 0; o < OK; ++o)
+        if (i - o >= 0 && i - o <= 2 * R) acc[o] += v[i];
+  } else {
+    float h[OK - 1], v[4], e[OK - 1];
+#pragma unroll
+    for (int i = 0; i < OK - 1; ++i) h[i] = next();
+#pragma unroll
+    for (int q = 0; q < 2; ++q) v[q] = next();
+#pragma unroll
+    for (int i = 0; i < OK - 1; ++i)
+#pragma unroll
+      for (int o = 0; o <= i; ++o) acc[o] += h[i];
+    // inputs 7 .. 2r meet all eight (an even number), two always read ahead
+    int i = OK - 1;
+#pragma unroll 1
+    for (; i + 3 <= 2 * r; i += 2) {
+#pragma unroll
+      for (int q = 2; q < 4; ++q) v[q] = next();
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int o = 0; o < OK; ++o) acc[o] += v[q];
+      v[0] = v[2];
+      v[1] = v[3];
+    }
+#pragma unroll
+    for (int q = 0; q < OK - 1; ++q) e[q] = next();
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+      for (int o = 0; o < OK; ++o) acc[o] += v[q];
+#pragma unroll
+    for (int u = 1; u < OK; ++u)
+#pragma unroll
+      for (int o = u; o < OK; ++o) acc[o] += e[u - 1];
+  }
+}
+
+// integer sums over inputs o .. o + 2r of the two 16-bit channels
+template <int R, typename F>
+__device__ __forceinline__ void sum8_u16(F&& next, int r, uint32_t (&lo)[OK], uint32_t (&hi)[OK]) {
+  const us2 l1 = {1, 0}, h1 = {0, 1};
+  auto add = [&](uint32_t v, uint32_t& a, uint32_t& b) {
+    a = __builtin_amdgcn_udot2(__builtin_bit_cast(us2, v), l1, a, false);
+    b = __builtin_amdgcn_udot2(__builtin_bit_cast(us2, v), h1, b, false);
+  };
+  uint32_t a = 0u, b = 0u;
+  if constexpr (R > 0) {
+    uint32_t v[2 * R + OK];
+#pragma unroll
+    for (int i = 0; i < 2 * R + OK; ++i) v[i] = next();
+#pragma unroll
+    for (int i = 0; i <= 2 * R; ++i) add(v[i], a, b);
+    lo[0] = a;
+    hi[0] = b;
+#pragma unroll
+    for (int o = 1; o < OK; ++o) {
+      lo[o] = lo[o - 1] + (v[2 * R + o] & 0xFFFFu) - (v[o - 1] & 0xFFFFu);
+      hi[o] = hi[o - 1] + (v[2 * R + o] >> 16) - (v[o - 1] >> 16);
+    }
+  } else {
+    uint32_t h[OK - 1], e[OK - 1];
+#pragma unroll
+    for (int i = 0; i < OK - 1; ++i) h[i] = next();
+    int i = OK - 1;
+#pragma unroll 1
+    for (; i <= 2 * r; i += 2) {  // 2r - 6 of them, even
+      const uint32_t v0 = next(), v1 = next();
+      add(v0, a, b);
+      add(v1, a, b);
+    }
+#pragma unroll
+    for (int q = 0; q < OK - 1; ++q) e[q] = next();
+#pragma unroll
+    for (int q = 0; q < OK - 1; ++q) add(h[q], a, b);
+    lo[0] = a;
+    hi[0] = b;
+#pragma unroll
+    for (int o = 1; o < OK; ++o) {
+      lo[o] = lo[o - 1] + (e[o - 1] & 0xFFFFu) - (h[o - 1] & 0xFFFFu);
+      hi[o] = hi[o - 1] + (e[o - 1] >> 16) - (h[o - 1] >> 16);
+    }
+  }
+}
+
+// Where a work-group of four waves stands on its lines: 64 x-adjacent lines, eight positions
+// per wave and step of 32.
+struct RunAt {
+  int l, wave, x0, s0, s1;
+  i64 base;
+};
+__device__ __forceinline__ RunAt run_at(int L, i64 so, unsigned nxb, unsigned no, int len) {
+  RunAt a;
+  a.l = (int)(threadIdx.x & 63);
+  a.wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const unsigned t = xcd_tile(blockIdx.x, gridDim.x);
+  a.x0 = (int)(t % nxb) * 64;
+  a.base = (i64)(t / nxb % no) * so;
+  a.s0 = (int)(t / nxb / no) * len;
+  a.s1 = min(L, a.s0 + len);
+  return a;
+}
+
+// Packed min / max along y or z: a work-group walks a segment of 64 lines through an LDS plane
+// of the last 2r + 32 positions (clamped to the line).  Bound by its 6 (from raw) or 8 bytes
+// per voxel: 130 and 180 us for 70 x 1080 x 1280 at radii 4 and 8 (4.5 and 4.3 TB/s); van Herk
+// blocks on LDS tiles of 64 outputs and their halo, a serial chain each, took 533 and 209.
+template <int R, bool FROM_U16>
+__global__ __launch_bounds__(256) void k_minmax_run(const void* __restrict__ src,
+                                                    uint32_t* __restrict__ dst, int W, int L,
+                                                    i64 sa, i64 so, int r, unsigned nxb,
+                                                    unsigned no, int len) {
+  extern __shared__ uint32_t sm_mm[];
+  constexpr int STEP = 4 * OK;
+  const int hist = 2 * r;
+  const RunAt a = run_at(L, so, nxb, no, len);
+  const int xc = min(a.x0 + a.l, W - 1);
+  uint32_t q[OK];
+  auto fetch = [&](int p) {
+#pragma unroll
+    for (int k = 0; k < OK; ++k) {
+      const i64 at = a.base + (i64)clampi(p + k, 0, L - 1) * sa + xc;
+      q[k] = FROM_U16 ? (uint32_t)((const uint16_t*)src)[at] : ((const uint32_t*)src)[at];
+    }
+  };
+  auto put = [&](int row) {
+#pragma unroll
+    for (int k = 0; k < OK; ++k) sm_mm[(row + k) * 64 + a.l] = FROM_U16 ? pack(q[k]) : q[k];
+  };
+  for (int g = a.wave; OK * g < hist; g += 4) {  // (the last may reach into the step's rows)
+    fetch(a.s0 - r + OK * g);
+    put(OK * g);
+  }
+  fetch(a.s0 + r + OK * a.wave);
+  __syncthreads();
+  for (int c0 = a.s0; c0 < a.s1; c0 += STEP) {
+    put(hist + OK * a.wave);
+    fetch(c0 + STEP + r + OK * a.wave);
+    __syncthreads();
+    const int c = c0 + OK * a.wave;
+    if (c < a.s1) {
+      const uint32_t* p = sm_mm + OK * a.wave * 64 + a.l;
+      uint32_t o[OK];
+      min8<R>([&] { const uint32_t v = *p; p += 64; return v; }, r, o);
+      if (a.x0 + a.l < W) {
+#pragma unroll
+        for (int k = 0; k < OK; ++k)
+          if (c + k < a.s1) st_nt(dst + a.base + (i64)(c + k) * sa + a.x0 + a.l, o[k]);
+      }
+    }
+    if (c0 + STEP >= a.s1) break;  // uniform
+    __syncthreads();
+    shift_rows<256, STEP, 64>(sm_mm, hist);
+    __syncthreads();
+  }
+}
+
+// Clamped box mean of (E, D) pairs along y or z, with NORM fused with the normalization; ero
+// and dil (optional) receive E and D.  Bound by its 14 (16) bytes per voxel: 275 us for
+// 70 x 1080 x 1280 at radius 4 (4.9 TB/s), 568 with an LDS tile per 64 outputs.
+template <int R, bool NORM, typename TS>
+__global__ __launch_bounds__(256) void k_box_run(const float2* __restrict__ src,
+                                                 float2* __restrict__ dst, TS* __restrict__ norm,
+                                                 const uint16_t* __restrict__ img,
+                                                 float* __restrict__ ero, float* __restrict__ dil,
+                                                 float min_int, int W, int L, i64 sa, i64 so,
+                                                 int r, unsigned nxb, unsigned no, int len,
+                                                 float k) {
+  extern __shared__ float sm_box[];
+  constexpr int STEP = 4 * OK;
+  const int hist = 2 * r;
+  float* B1 = sm_box;
+  float* B2 = B1 + (hist + STEP) * 64;
+  const RunAt a = run_at(L, so, nxb, no, len);
+  const int xc = min(a.x0 + a.l, W - 1);
+  float2 q[OK];
+  uint16_t iq[OK];
+  auto fetch = [&](int p) {
+#pragma unroll
+    for (int j = 0; j < OK; ++j) q[j] = src[a.base + (i64)clampi(p + j, 0, L - 1) * sa + xc];
+  };
+  auto put = [&](int row) {
+#pragma unroll
+    for (int j = 0; j < OK; ++j) {
+      B1[(row + j) * 64 + a.l] = q[j].x;
+      B2[(row + j) * 64 + a.l] = q[j].y;
+    }
+  };
+  for (int g = a.wave; OK * g < hist; g += 4) {
+    fetch(a.s0 - r + OK * g);
+    put(OK * g);
+  }
+  fetch(a.s0 + r + OK * a.wave);
+  __syncthreads();
+  for (int c0 = a.s0; c0 < a.s1; c0 += STEP) {
+    const int c = c0 + OK * a.wave;
+    put(hist + OK * a.wave);
+    if (NORM) {
+#pragma unroll
+      for (int j = 0; j < OK; ++j) iq[j] = img[a.base + (i64)min(c + j, L - 1) * sa + xc];
+    }
+    fetch(c0 + STEP + r + OK * a.wave);
+    __syncthreads();
+    if (c < a.s1) {
+      float e[OK], d[OK];
+      const float* p = B1 + OK * a.wave * 64 + a.l;
+      sum8<R>([&] { const float v = *p; p += 64; return v; }, r, e);
+      p = B2 + OK * a.wave * 64 + a.l;
+      sum8<R>([&] { const float v = *p; p += 64; return v; }, r, d);
+      if (a.x0 + a.l < W) {
+#pragma unroll
+        for (int j = 0; j < OK; ++j) {
+          if (c + j >= a.s1) continue;
+          const i64 idx = a.base + (i64)(c + j) * sa + a.x0 + a.l;
+          const float ve = e[j] * k, vd = d[j] * k;
+          if (NORM) {
+            const float I = (float)iq[j];
+            st_nt(norm + idx, (I >= min_int) ? (I - ve) / (vd - ve) : 0.0f);
+            if (ero) {  // uniform
+              st_nt(ero + idx, ve);
+              st_nt(dil + idx, vd);
+            }
+          } else {
+            st_nt(dst + idx, make_float2(ve, vd));
+          }
+        }
+      }
+    }
+    if (c0 + STEP >= a.s1) break;  // uniform
+    __syncthreads();
+    shift_rows<256, STEP, 64>(B1, hist);
+    shift_rows<256, STEP, 64>(B2, hist);
+    __syncthreads();
+  }
+}
+
+// min/max along x, box along x and box along y fused (k_norm_xy_walk for other radii): four
+// waves walk the rows of one plane of the y-min/maxed volume for a strip of 64 columns, eight
+// rows per wave and step.
+//   1. a wave's rows, columns x0-2r .. x0+63+2r clamped to the plane, enter its lines A;
+//   2. lane (row l % 8, columns 8 (l / 8) ..) forms the window minima, two groups of eight at
+//      most, which replace the lines; positions outside the plane take the edge's value;
+//   3. the same lane sums them for its eight columns -> two planes B of the last 2r + 32 rows;
+//   4. lane l sums eight rows of column x0 + l along y, in the reference order.
+// (padded pitches: the lanes of every access fall on different banks.)  Near its 12 bytes per
+// voxel at small radii (70 x 1080 x 1280: 314 us at radius 8, 3.7 TB/s), bound by instruction
+// issue above (478 us at 16); the x pass and the y pass it replaces, one output per thread,
+// took 698 us at 8.
+template <int R, int NC>
+__global__ __launch_bounds__(256) void k_norm_xy_run(const uint32_t* __restrict__ src,
+                                                     float2* __restrict__ dst, int W, int H, int r,
+                                                     int nxs, int nys, int rows, float k) {
+  extern __shared__ uint32_t sm_xy[];
+  constexpr int BP = 65, STEP = 4 * OK;
+  const int hist = 2 * r, span = 64 + 4 * r, AP = (span + 7) / 8 * 8 + 9;
+  const int l = (int)(threadIdx.x & 63);
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  uint32_t* A = sm_xy + wave * (OK * AP);
+  float* B1 = reinterpret_cast<float*>(sm_xy + 4 * (OK * AP));
+  float* B2 = B1 + (hist + STEP) * BP;
+  const unsigned t = xcd_tile(blockIdx.x, gridDim.x);
+  const int y0 = (int)(t % (unsigned)nys) * rows, y1 = min(H, y0 + rows);
+  const unsigned tile = t / (unsigned)nys;
+  const int x0 = (int)(tile % (unsigned)nxs) * 64;
+  const i64 pbase = (i64)(tile / (unsigned)nxs) * H * W;
+  int xl[NC];
+#pragma unroll
+  for (int j = 0; j < NC; ++j) xl[j] = clampi(x0 - 2 * r + 64 * j + l, 0, W - 1);
+  uint32_t q[OK][NC];
+  auto fetch = [&](int y) {
+#pragma unroll
+    for (int i = 0; i < OK; ++i) {
+      const uint32_t* row = src + pbase + (i64)clampi(y + i, 0, H - 1) * W;
+#pragma unroll
+      for (int j = 0; j < NC; ++j) q[i][j] = row[xl[j]];
+    }
+  };
+  const bool edge = x0 - r < 0 || x0 + 64 + r > W;  // uniform
+  const int blo = r - x0, bhi = W - 1 - x0 + r;     // minima positions of x = 0 and W - 1
+  const int nm = 64 + 2 * r;                        // minima per row
+  const int xr = l % OK, xg = l / OK;
+  const uint32_t full = (uint32_t)(2 * r + 1) * 65535u;
+  auto xpass = [&](int row, int ahead) {
+#pragma unroll
+    for (int i = 0; i < OK; ++i)
+#pragma unroll
+      for (int j = 0; j < NC; ++j)
+        if (64 * j + l < span) A[i * AP + 64 * j + l] = q[i][j];
+    fetch(ahead);
+    wave_lds_sync();
+    uint32_t* line = A + xr * AP;
+    uint32_t m[2][OK];
+    {
+      const uint32_t* p = line + OK * xg;
+      min8<R>([&] { return *p++; }, r, m[0]);
+    }
+    const bool two = OK * (xg + 8) < nm;
+    if (two) {
+      const uint32_t* p = line + OK * (xg + 8);
+      min8<R>([&] { return *p++; }, r, m[1]);
+    }
+    wave_lds_sync();
+#pragma unroll
+    for (int o = 0; o < OK; ++o) line[OK * xg + o] = m[0][o];
+    if (two) {
+#pragma unroll
+      for (int o = 0; o < OK; ++o) line[OK * (xg + 8) + o] = m[1][o];
+    }
+    wave_lds_sync();
+    if (edge) {  // each lane its row: positions outside the plane take the edge value
+      const uint32_t lo = line[clampi(blo, 0, nm - 1)], hi = line[clampi(bhi, 0, nm - 1)];
+      wave_lds_sync();
+      for (int j = xg; j < nm; j += 8) {
+        if (j < blo) line[j] = lo;
+        if (j > bhi) line[j] = hi;
+      }
+      wave_lds_sync();
+    }
+    uint32_t se[OK], sd[OK];
+    {
+      const uint32_t* p = line + OK * xg;
+      sum8_u16<R>([&] { return *p++; }, r, se, sd);
+    }
+    const int b = (row + xr) * BP + xg * OK;
+#pragma unroll
+    for (int o = 0; o < OK; ++o) {
+      B1[b + o] = (float)se[o] * k;
+      B2[b + o] = (float)(full - sd[o]) * k;
+    }
+    wave_lds_sync();
+  };
+  const int main0 = y0 + r + OK * wave;
+  if (OK * wave < hist) {
+    fetch(y0 - r + OK * wave);
+    for (int g = wave; OK * g < hist; g += 4)
+      xpass(OK * g, OK * (g + 4) < hist ? y0 - r + OK * (g + 4) : main0);
+  } else {
+    fetch(main0);
+  }
+  __syncthreads();
+  const bool out = x0 + l < W;
+  float2* dcol = dst + pbase + x0 + l;
+  for (int c0 = y0; c0 < y1; c0 += STEP) {
+    xpass(hist + OK * wave, c0 + STEP + r + OK * wave);
+    __syncthreads();
+    const int c = c0 + OK * wave;
+    if (c < y1) {
+      float e[OK], d[OK];
+      const float* p = B1 + OK * wave * BP + l;
+      sum8<R>([&] { const float v = *p; p += BP; return v; }, r, e);
+      p = B2 + OK * wave * BP + l;
+      sum8<R>([&] { const float v = *p; p += BP; return v; }, r, d);
+      if (out) {
+#pragma unroll
+        for (int o = 0; o < OK; ++o)
+          if (c + o < y1) st_nt(dcol + (i64)(c + o) * W, make_float2(e[o] * k, d[o] * k));
+      }
+    }
+    if (c0 + STEP >= y1) break;  // uniform
+    __syncthreads();
+    shift_rows<256, STEP, BP>(B1, hist);
+    shift_rows<256, STEP, BP>(B2, hist);
+    __syncthreads();
+  }
+}
+
 template <typename TS>
 __global__ __launch_bounds__(NT) void k_copy_norm(const uint16_t* __restrict__ img,
                                                   TS* __restrict__ norm, float min_int, i64 N) {
@@ -765,6 +1145,28 @@ hipError_t dispatch_xw(int XW, F&& f) {
   return f(std::integral_constant<int, 16>{});
 }
 
+// f with the radius fixed for windows shorter than a group of outputs, else 0
+template <typename F>
+hipError_t dispatch_short(int r, F&& f) {
+  static_assert(OK == 8, "2 * 3 + 1 < 8");
+  switch (r) {
+    case 1: return f(std::integral_constant<int, 1>{});
+    case 2: return f(std::integral_constant<int, 2>{});
+    case 3: return f(std::integral_constant<int, 3>{});
+    default: return f(std::integral_constant<int, 0>{});
+  }
+}
+// grid of a walk over 64-line strips by work-groups of four waves
+LineGrid run_grid(int W, int L, i64 n_other, int halo) {
+  LineGrid g;
+  g.nxb = (unsigned)((W + 63) / 64);
+  g.no = (unsigned)n_other;
+  int nseg;
+  line_segments(L, (i64)g.nxb * n_other * 4, 1024.0, 2.0, false, halo, &nseg, &g.len);
+  g.blocks = (unsigned)((i64)g.nxb * n_other * nseg);
+  return g;
+}
+
 template <int R>
 hipError_t minmax_walk(const void* src, bool from_u16, uint32_t* dst, int W, int L, i64 sa, i64 so,
                        i64 n_other, hipStream_t s) {
@@ -780,13 +1182,22 @@ hipError_t minmax_walk(const void* src, bool from_u16, uint32_t* dst, int W, int
 
 hipError_t minmax_line(const void* src, bool from_u16, uint32_t* dst, int W, int L, i64 sa,
                        i64 so, i64 n_other, int r, hipStream_t s) {
-  switch (r) {  // radii with a column-walker kernel
-    case 1: return minmax_walk<1>(src, from_u16, dst, W, L, sa, so, n_other, s);
-    case 2: return minmax_walk<2>(src, from_u16, dst, W, L, sa, so, n_other, s);
-    case 3: return minmax_walk<3>(src, from_u16, dst, W, L, sa, so, n_other, s);
-    case 5: return minmax_walk<5>(src, from_u16, dst, W, L, sa, so, n_other, s);
-    case 10: return minmax_walk<10>(src, from_u16, dst, W, L, sa, so, n_other, s);
-    default: break;
+  // the configured radius has a walk with its window in registers (70 x 1080 x 1280 along y:
+  // 166 us; the walk of any radius 180 at 8, 182 at 12; at 3 and 5 the two take the same)
+  if (r == 10) return minmax_walk<10>(src, from_u16, dst, W, L, sa, so, n_other, s);
+  if (r <= kRunRadius) {
+    const LineGrid g = run_grid(W, L, n_other, 2 * r);
+    const size_t lds = (size_t)(2 * r + 32) * 64 * 4;
+    return dispatch_short(r, [&](auto rs) {
+      constexpr int R = decltype(rs)::value;
+      if (from_u16)
+        hipLaunchKernelGGL((k_minmax_run<R, true>), dim3(g.blocks), dim3(256), lds, s, src, dst, W,
+                           L, sa, so, r, g.nxb, g.no, g.len);
+      else
+        hipLaunchKernelGGL((k_minmax_run<R, false>), dim3(g.blocks), dim3(256), lds, s, src, dst, W,
+                           L, sa, so, r, g.nxb, g.no, g.len);
+      return hipGetLastError();
+    });
   }
   const LineCfg c = line_cfg(r, L, 4, 2);
   const int nxt = (W + c.XW - 1) / c.XW, nct = (L + c.C - 1) / c.C;
@@ -816,15 +1227,24 @@ hipError_t box_line_fast(const float2* src, float2* dst, TS* norm, const uint16_
 
 template <bool NORM, typename TS>
 hipError_t box_line(const float2* src, float2* dst, TS* norm, const uint16_t* img, float min_int,
-                    int W, int L, i64 sa, i64 so, i64 n_other, int r, hipStream_t s) {
+                    int W, int L, i64 sa, i64 so, i64 n_other, int r, hipStream_t s,
+                    float* ero = nullptr, float* dil = nullptr) {
   const float k = 1.0f / (float)(2 * r + 1);
-  switch (r) {  // radii with a register-window kernel
-    case 1: return box_line_fast<1, NORM, TS>(src, dst, norm, img, min_int, W, L, sa, so, n_other, k, s);
-    case 2: return box_line_fast<2, NORM, TS>(src, dst, norm, img, min_int, W, L, sa, so, n_other, k, s);
-    case 3: return box_line_fast<3, NORM, TS>(src, dst, norm, img, min_int, W, L, sa, so, n_other, k, s);
-    case 5: return box_line_fast<5, NORM, TS>(src, dst, norm, img, min_int, W, L, sa, so, n_other, k, s);
-    case 10: return box_line_fast<10, NORM, TS>(src, dst, norm, img, min_int, W, L, sa, so, n_other, k, s);
-    default: break;
+  const bool ed = NORM && ero && dil;  // only the walk of any radius writes them
+  // (70 x 1080 x 1280, fused with the normalization: 267 us; the walk of any radius 275 at 4,
+  // 277 at 6)
+  if (r == 10 && !ed)
+    return box_line_fast<10, NORM, TS>(src, dst, norm, img, min_int, W, L, sa, so, n_other, k, s);
+  if (r <= kRunRadius) {
+    const LineGrid g = run_grid(W, L, n_other, 2 * r);
+    const size_t lds = 2 * (size_t)(2 * r + 32) * 64 * 4;
+    return dispatch_short(r, [&](auto rs) {
+      constexpr int R = decltype(rs)::value;
+      hipLaunchKernelGGL((k_box_run<R, NORM, TS>), dim3(g.blocks), dim3(256), lds, s, src, dst,
+                         norm, img, ed ? ero : nullptr, ed ? dil : nullptr, min_int, W, L, sa, so,
+                         r, g.nxb, g.no, g.len, k);
+      return hipGetLastError();
+    });
   }
   const LineCfg c = line_cfg(r, L, 8, 1);
   const int nxt = (W + c.XW - 1) / c.XW, nct = (L + c.C - 1) / c.C;
@@ -853,6 +1273,11 @@ __global__ __launch_bounds__(NT) void k_split_ed(const float2* __restrict__ ed,
 hipError_t launch_box_pair(const float2* src, float2* dst, int W, int L, i64 sa, i64 so,
                            i64 n_other, int r, hipStream_t s) {
   return box_line<false, float>(src, dst, nullptr, nullptr, 0.0f, W, L, sa, so, n_other, r, s);
+}
+
+WalkShape norm_walk_shape(int rxy, int W, int D) {
+  if (rxy == 10) return {(i64)((W + 127) / 128) * D, 21, 20};
+  return {(i64)((W + 63) / 64) * D * 4, 32, 2 * rxy};
 }
 
 template <typename TS>
@@ -890,56 +1315,68 @@ hipError_t launch_normalize(const uint16_t* img, TS* norm, void* tmp1, void* tmp
     if ((e = minmax_line(p1, false, p2, W, H, W, WH, D, rxy, s)) != hipSuccess) return e;
     mark("normalize/minmax_y", s);
   }
-  if (rxy == 10 && !(ero && dil)) {
-    // min/max along x, box along x and box along y in one row walker -> (E, D) in tmp1,
-    // then box along z fused with normalization
+  // min/max along x, box along x and box along y in one row walker -> (E, D) in tmp1
+  const float2* exy = (const float2*)tmp1;
+  const float k = 1.0f / (float)(2 * rxy + 1);
+  if (rxy == 10) {
     constexpr int CW = 128;
     const int nxs = (W + CW - 1) / CW;
     int nys, rows;
-    walk_segments(H, 21, (i64)nxs * D, &nys, &rows, segments);
+    walk_segments(H, norm_walk_shape(rxy, W, D), &nys, &rows, segments);
     const i64 nblk = (i64)nxs * D * nys;
     hipLaunchKernelGGL((k_norm_xy_walk<10>), dim3((unsigned)nblk), dim3(64), 0, s, p2,
-                       (float4*)tmp1, W, H, nxs, nys, rows, 1.0f / 21.0f);
+                       (float4*)tmp1, W, H, nxs, nys, rows, k);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     mark("normalize/minmax_x_box_xy", s);
-    e = box_line<true, TS>((const float2*)tmp1, nullptr, norm, img, min_intensity, W, D, WH, W, H,
-                           rz, s);
-    mark("normalize/box_z_norm", s);
-    return e;
-  }
-  // min/max along x fused with the box x pass -> float2 (E, D) in tmp1
-  {
+  } else if (rxy <= kRunRadius) {
+    const int nxs = (W + 63) / 64;
+    int nys, rows;
+    walk_segments(H, norm_walk_shape(rxy, W, D), &nys, &rows, segments);
+    const dim3 grid((unsigned)((i64)nxs * D * nys));
+    const int ap = (64 + 4 * rxy + 7) / 8 * 8 + 9;  // the kernel's line pitch
+    const size_t lds = (size_t)(4 * OK * ap + 2 * (2 * rxy + 32) * 65) * 4;
+    e = dispatch_short(rxy, [&](auto rs) {
+      constexpr int R = decltype(rs)::value;
+      if (rxy <= 16)
+        hipLaunchKernelGGL((k_norm_xy_run<R, 2>), grid, dim3(256), lds, s, p2, (float2*)tmp1, W, H,
+                           rxy, nxs, nys, rows, k);
+      else
+        hipLaunchKernelGGL((k_norm_xy_run<0, 3>), grid, dim3(256), lds, s, p2, (float2*)tmp1, W, H,
+                           rxy, nxs, nys, rows, k);
+      return hipGetLastError();
+    });
+    if (e != hipSuccess) return e;
+    mark("normalize/minmax_x_box_xy", s);
+  } else {
+    // min/max along x fused with the box x pass -> float2 (E, D) in tmp1, then box along y
     constexpr int RUN = 4, C = 64 * RUN, ROWS = NT / 64;
     const int nct = (W + C - 1) / C;
     const i64 nrows = (i64)H * D;
     const i64 nblk = ((nrows + ROWS - 1) / ROWS) * nct;
     const size_t lds = (size_t)ROWS * 2 * (C + 4 * rxy + 4) * 4;
-    const float k = 1.0f / (float)(2 * rxy + 1);
-    if (rxy == 10)
-      hipLaunchKernelGGL((k_minmax_x_box<10, RUN>), dim3((unsigned)nblk), dim3(NT), lds, s, p2,
-                         (float2*)tmp1, W, nrows, rxy, nct, k);
-    else
-      hipLaunchKernelGGL((k_minmax_x_box<0, RUN>), dim3((unsigned)nblk), dim3(NT), lds, s, p2,
-                         (float2*)tmp1, W, nrows, rxy, nct, k);
+    hipLaunchKernelGGL((k_minmax_x_box<RUN>), dim3((unsigned)nblk), dim3(NT), lds, s, p2,
+                       (float2*)tmp1, W, nrows, rxy, nct, k);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     mark("normalize/minmax_x_box_x", s);
+    if ((e = box_line<false, TS>((const float2*)tmp1, (float2*)tmp2, nullptr, nullptr, 0.0f, W, H,
+                                 W, WH, D, rxy, s)) != hipSuccess)
+      return e;
+    mark("normalize/box_y", s);
+    exy = (const float2*)tmp2;
   }
-  // box along y, then along z fused with normalization
-  if ((e = box_line<false, TS>((const float2*)tmp1, (float2*)tmp2, nullptr, nullptr, 0.0f, W, H,
-                               W, WH, D, rxy, s)) != hipSuccess)
-    return e;
-  mark("normalize/box_y", s);
-  if (ero && dil) {  // E and D on request: the same z pass without normalization, then split
-    if ((e = box_line<false, TS>((const float2*)tmp2, (float2*)tmp1, nullptr, nullptr, 0.0f, W, D,
-                                 WH, W, H, rz, s)) != hipSuccess)
+  // box along z fused with the normalization
+  if (ero && dil && rz > kRunRadius) {  // E and D by a z pass of their own, then split
+    float2* ed = exy == (const float2*)tmp1 ? (float2*)tmp2 : (float2*)tmp1;
+    if ((e = box_line<false, TS>(exy, ed, nullptr, nullptr, 0.0f, W, D, WH, W, H, rz, s)) !=
+        hipSuccess)
       return e;
     const i64 nb = std::min<i64>((N + NT - 1) / NT, 1 << 20);
-    hipLaunchKernelGGL(k_split_ed, dim3((unsigned)nb), dim3(NT), 0, s, (const float2*)tmp1, ero,
-                       dil, N);
+    hipLaunchKernelGGL(k_split_ed, dim3((unsigned)nb), dim3(NT), 0, s, (const float2*)ed, ero, dil,
+                       N);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
-  e = box_line<true, TS>((const float2*)tmp2, nullptr, norm, img, min_intensity, W, D, WH, W, H,
-                         rz, s);
+  e = box_line<true, TS>(exy, nullptr, norm, img, min_intensity, W, D, WH, W, H, rz, s,
+                         rz <= kRunRadius ? ero : nullptr, dil);
   mark("normalize/box_z_norm", s);
   return e;
 }

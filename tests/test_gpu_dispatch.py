@@ -124,3 +124,19 @@ def test_dog_of_any_radii(hd, shape, s, trunc, finite):
     hd.initGaussian3DKernel(*s, truncate=trunc)
     ref, _ = oracle.dog3d(norm, *s, truncate=trunc, gamma=1.0)
     np.testing.assert_array_equal(hd.DoG3DFilter(norm).cpu().numpy(), ref)
+
+
+# normalization radii: windows shorter than a group of outputs, those with walks of their own,
+# the walks of any radius on both sides of their column and LDS limits, larger ones; ragged
+# strips, planes narrower and lower than a window; E and D with the same values
+@pytest.mark.parametrize("rxy,rz", [(1, 2), (2, 4), (3, 7), (4, 1), (7, 3), (9, 9), (10, 6),
+                                    (16, 11), (17, 5), (24, 24), (25, 10), (11, 25)])
+@pytest.mark.parametrize("shape", [(3, 7, 5), (34, 41, 70), (9, 75, 193)])
+def test_normalize_of_any_radii(hd, shape, rxy, rz):
+    img = np.random.default_rng(rxy).integers(0, 65536, shape, dtype=np.uint16)
+    want, e, d = oracle.normalize3d(img, 20000, rxy, rz, return_ed=True)
+    np.testing.assert_array_equal(hd.Normalize3DFilter(img, 20000, rxy, rz).cpu().numpy(), want)
+    n, ge, gd = hd.Normalize3DFilterWithBounds(img, 20000, rxy, rz)
+    np.testing.assert_array_equal(n.cpu().numpy(), want)
+    np.testing.assert_array_equal(ge.cpu().numpy(), e)
+    np.testing.assert_array_equal(gd.cpu().numpy(), d)
