@@ -68,7 +68,8 @@ struct hdog_ctx {
   double truncate = 0.0;
   int r[4] = {0, 0, 0, 0};
   i64 R = 0;
-  uint32_t* h_R = nullptr;  // pinned
+  uint32_t* h_R = nullptr;         // page-locked: the region count, written by the device
+  hipEvent_t counted = nullptr;   // recorded after the kernel that writes it
   bool prof = false;        // record an event after every kernel of run_device
   Prof pool;
   bool ev_valid = false;
@@ -218,10 +219,12 @@ int gaussian_weights(float sigma, double truncate, float* w) {
   return lw;
 }
 
+// Accumulators and output arrays for R regions, with room to spare: the next stack of the
+// same shape has about as many.
 int ensure_regions(hdog_ctx* ctx, i64 R) {
-  HIPCHK(ensure(ctx->acc, (size_t)R * sizeof(RegionAcc)));
   if (R > ctx->out_cap) {
-    const i64 cap = std::max<i64>(R, ctx->out_cap * 3 / 2);
+    const i64 cap = std::max<i64>(R + R / 8 + 1024, ctx->out_cap * 3 / 2);
+    ctx->out_cap = 0;  // until every array has grown
     HIPCHK(ensure(ctx->o_label, cap * 4));
     HIPCHK(ensure(ctx->o_size, cap * 2));
     HIPCHK(ensure(ctx->o_vox, cap * 8));
@@ -233,7 +236,12 @@ int ensure_regions(hdog_ctx* ctx, i64 R) {
     HIPCHK(ensure(ctx->o_imax, cap * 2));
     ctx->out_cap = cap;
   }
+  HIPCHK(ensure(ctx->acc, (size_t)ctx->out_cap * sizeof(RegionAcc)));
   return HDOG_OK;
+}
+// regions that both hold now (a batch plan may have taken the accumulators' memory)
+i64 region_capacity(const hdog_ctx* ctx) {
+  return std::min<i64>(ctx->out_cap, (i64)(ctx->acc.bytes / sizeof(RegionAcc)));
 }
 
 // Candidate records of the Hessian pass, when the pipeline produced them.
@@ -256,47 +264,57 @@ int regional_features_t(hdog_ctx* ctx, hipStream_t s, uint32_t* labels, const TH
   const i64 N = (i64)W * H * D;
   HIPCHK(ensure(ctx->rid, (size_t)N * 4));
   const i64 nb = (N + kRootBlock - 1) / kRootBlock;
-  HIPCHK(ensure(ctx->bcnt, (size_t)block_count_words(N) * 4));
+  HIPCHK(ensure(ctx->bcnt, (size_t)count_layout(N).words * 4));
   HIPCHK(ensure(ctx->rmask, (size_t)nb * (kRootBlock / 8)));
   HIPCHK(ensure(ctx->dR, 64));
-  i64 nbo = 0;
   unsigned long long* masks = (unsigned long long*)ctx->rmask.p;
+  uint32_t* counts = (uint32_t*)ctx->bcnt.p;
+  uint32_t* rid = (uint32_t*)ctx->rid.p;
+  uint32_t* dR = (uint32_t*)ctx->dR.p;
   if (cand.rec)
-    HIPCHK(launch_region_count_masks(masks, (uint32_t*)ctx->bcnt.p, (uint32_t*)ctx->dR.p, N, s,
-                                     &nbo));
+    HIPCHK(launch_region_count_masks(masks, counts, N, s));
   else
-    HIPCHK(launch_region_ids(labels, (uint32_t*)ctx->bcnt.p, masks, (uint32_t*)ctx->dR.p, N, s,
-                             &nbo));
-  HIPCHK(hipMemcpyAsync(ctx->h_R, ctx->dR.p, 4, hipMemcpyDeviceToHost, s));
-  HIPCHK(hipStreamSynchronize(s));
-  const i64 R = *ctx->h_R;
-  int rc = ensure_regions(ctx, R);
-  if (rc) return rc;
-  RegionAcc* acc = (RegionAcc*)ctx->acc.p;
-  HIPCHK(launch_region_assign(masks, (const uint32_t*)ctx->bcnt.p, (uint32_t*)ctx->rid.p, acc, R, N,
-                              s));
-  if (cand.rec)
-    HIPCHK(launch_region_accum_cand<TN>(cand.rec, cand.cnt, cand.ntiles, cand.rlab, cand.multi,
-                                        (const uint32_t*)ctx->rid.p, norm, img, acc, R, W, H,
-                                        is_ave, s));
-  else
-    HIPCHK(launch_region_accum<TH, TN>(labels, (const uint32_t*)ctx->rid.p, hess, norm, img, acc, R,
-                                       W, H, D, is_ave, s));
-  const i64 cap = ctx->out_cap;
-  RegionOut o;
-  o.label = (uint32_t*)ctx->o_label.p;
-  o.size = (uint16_t*)ctx->o_size.p;
-  o.voxels = (u64*)ctx->o_vox.p;
-  o.cx = (float*)ctx->o_cen.p;
-  o.cy = o.cx + cap;
-  o.cz = o.cx + 2 * cap;
-  o.st = (float*)ctx->o_eig.p;
-  o.bl = o.st + cap;
-  o.nrm = (float*)ctx->o_nrm.p;
-  o.hess = (float*)ctx->o_hess.p;
-  o.isum = (u64*)ctx->o_isum.p;
-  o.imax = (uint16_t*)ctx->o_imax.p;
-  HIPCHK(launch_region_finalize(acc, R, is_ave, o, cap, s));
+    HIPCHK(launch_region_ids(labels, counts, masks, N, s));
+  // The rest is launched for as many regions as the arrays hold, and the count, which the
+  // first of its kernels writes, read meanwhile; only when they hold too few (the first call,
+  // a stack with more regions) are they grown and the rest run again.
+  i64 R = 0, cap = region_capacity(ctx);
+  for (;;) {
+    RegionAcc* acc = (RegionAcc*)ctx->acc.p;
+    HIPCHK(launch_region_assign(masks, counts, rid, acc, cap, N, dR, ctx->h_R, s));
+    HIPCHK(hipEventRecord(ctx->counted, s));
+    if (cap > 0) {
+      if (cand.rec)
+        HIPCHK(launch_region_accum_cand<TN>(cand.rec, cand.cnt, cand.ntiles, cand.rlab, cand.multi,
+                                            rid, norm, img, acc, cap, W, H, is_ave, s));
+      else
+        HIPCHK(launch_region_accum<TH, TN>(labels, rid, hess, norm, img, acc, cap, W, H, D, is_ave,
+                                           s));
+      const i64 pitch = ctx->out_cap;
+      RegionOut o;
+      o.label = (uint32_t*)ctx->o_label.p;
+      o.size = (uint16_t*)ctx->o_size.p;
+      o.voxels = (u64*)ctx->o_vox.p;
+      o.cx = (float*)ctx->o_cen.p;
+      o.cy = o.cx + pitch;
+      o.cz = o.cx + 2 * pitch;
+      o.st = (float*)ctx->o_eig.p;
+      o.bl = o.st + pitch;
+      o.nrm = (float*)ctx->o_nrm.p;
+      o.hess = (float*)ctx->o_hess.p;
+      o.isum = (u64*)ctx->o_isum.p;
+      o.imax = (uint16_t*)ctx->o_imax.p;
+      // (a 26-connected labeling has at most N / 8 regions)
+      HIPCHK(launch_region_finalize(acc, dR, cap, std::min(cap, N / 8 + 2), is_ave, o, pitch,
+                                    s));
+    }
+    HIPCHK(hipEventSynchronize(ctx->counted));
+    R = *(volatile uint32_t*)ctx->h_R;
+    if (R <= cap) break;
+    const int rc = ensure_regions(ctx, R);
+    if (rc) return rc;
+    cap = region_capacity(ctx);
+  }
   ctx->R = R;
   if (num_regions) *num_regions = R;
   return HDOG_OK;
@@ -349,6 +367,8 @@ int run_stages(hdog_ctx* ctx, hipStream_t s, const hdog_params* p, const uint16_
   HIPCHK(ensure(ctx->fgbits, (size_t)fg_words(W, H, D) * 8));
   HIPCHK(ensure(ctx->rmask, (size_t)nb * (kRootBlock / 8)));
   HIPCHK(ensure(ctx->rmulti, (size_t)nb * (kRootBlock / 8)));
+  const CountLayout cl = count_layout(N);
+  HIPCHK(ensure(ctx->bcnt, (size_t)cl.words * 4));
   cand.rec = (const float*)ctx->cand.p;
   cand.cnt = (const uint32_t*)ctx->cand_cnt.p;
   cand.rlab = (const uint32_t*)ctx->cand_lab.p;
@@ -359,7 +379,8 @@ int run_stages(hdog_ctx* ctx, hipStream_t s, const hdog_params* p, const uint16_
                                (unsigned long long*)ctx->fgbits.p, labels,
                                (uint32_t*)ctx->cand_lab.p, (unsigned long long*)ctx->rmask.p,
                                (unsigned long long*)ctx->rmulti.p, nb * (kRootBlock / 64), dense,
-                               W, H, D, s));
+                               W, H, D, s, 7, (uint32_t*)ctx->bcnt.p + cl.chunks_off,
+                               (int)cl.chunks));
   int rc = regional_features_t<TH, TN>(ctx, s, labels, hess, norm, img, W, H, D, p->is_ave_mode,
                                        num_regions, cand);
   if (rc) return rc;
@@ -475,25 +496,26 @@ hipError_t batch_tile(hdog_ctx* ctx, BatchState* B, BatchLane& L, int t, hipStre
   if ((e = launch_hessian<TD, TH>(dog, hess, nullptr, W, H, D, s, (float*)L.cand.p,
                                   (uint32_t*)L.cand_cnt.p, minor_band(&B->p))) != hipSuccess)
     return e;
-  i64 nbo = 0;
   uint32_t* dR = (uint32_t*)L.dR.p;
+  uint32_t* counts = (uint32_t*)L.bcnt.p;
   unsigned long long* masks = (unsigned long long*)L.rmask.p;
   const i64 nb = (N + kRootBlock - 1) / kRootBlock;
+  const CountLayout cl = count_layout(N);
   if ((e = launch_ccl_candidates((const float*)L.cand.p, (const uint32_t*)L.cand_cnt.p, ntiles,
                                  (unsigned long long*)L.fgbits.p, labels,
                                  (uint32_t*)L.cand_lab.p, masks,
                                  (unsigned long long*)L.rmulti.p, nb * (kRootBlock / 64), false,
-                                 W, H, D, s)) != hipSuccess)
+                                 W, H, D, s, 7, counts + cl.chunks_off, (int)cl.chunks)) !=
+      hipSuccess)
     return e;
-  if ((e = launch_region_count_masks(masks, (uint32_t*)L.bcnt.p, dR, N, s, &nbo)) != hipSuccess)
+  if ((e = launch_region_count_masks(masks, counts, N, s)) != hipSuccess) return e;
+  RegionAcc* acc = (RegionAcc*)L.acc.p;
+  if ((e = launch_region_assign(masks, counts, (uint32_t*)L.rid.p, acc, L.acc_cap, N, dR, nullptr,
+                                s)) != hipSuccess)
     return e;
   TileOut* tout = (TileOut*)B->tout.p + t;
   if ((e = launch_tile_reserve(dR, L.acc_cap, B->arena_cap, (u64*)B->running.p, tout, s)) !=
       hipSuccess)
-    return e;
-  RegionAcc* acc = (RegionAcc*)L.acc.p;
-  if ((e = launch_region_assign(masks, (const uint32_t*)L.bcnt.p, (uint32_t*)L.rid.p, acc,
-                                L.acc_cap, N, s)) != hipSuccess)
     return e;
   if ((e = launch_region_accum_cand<TN>((const float*)L.cand.p, (const uint32_t*)L.cand_cnt.p,
                                         ntiles, (const uint32_t*)L.cand_lab.p,
@@ -515,7 +537,8 @@ hipError_t batch_tile(hdog_ctx* ctx, BatchState* B, BatchLane& L, int t, hipStre
   o.hess = (float*)B->a_hess.p;
   o.isum = (u64*)B->a_isum.p;
   o.imax = (uint16_t*)B->a_imax.p;
-  return launch_region_finalize(acc, L.acc_cap, p->is_ave_mode, o, cap, s, tout);
+  return launch_region_finalize(acc, dR, L.acc_cap, std::min(L.acc_cap, N / 64 + 2),
+                                p->is_ave_mode, o, cap, s, tout);
 }
 
 // Captures on B->cs: the arena counter is cleared, the other branches fork from it through
@@ -653,6 +676,11 @@ int hdog_create(hdog_ctx** out, int device) {
     delete c;
     return HDOG_ERR_HIP;
   }
+  if (hipEventCreateWithFlags(&c->counted, hipEventDisableTiming) != hipSuccess) {
+    (void)hipHostFree(c->h_R);
+    delete c;
+    return HDOG_ERR_HIP;
+  }
   *out = c;
   return HDOG_OK;
 }
@@ -686,6 +714,7 @@ void hdog_destroy(hdog_ctx* ctx) {
   if (ctx->prof)
     for (hipEvent_t& e : ctx->pool.ev) (void)hipEventDestroy(e);
   release(ctx->weights);
+  if (ctx->counted) (void)hipEventDestroy(ctx->counted);
   if (ctx->h_R) (void)hipHostFree(ctx->h_R);
   delete ctx;
 }
@@ -1266,7 +1295,7 @@ int hdog_batch_plan(hdog_ctx* ctx, const hdog_params* p, const hdog_tile* tiles,
     const i64 nb = (b.maxN + kRootBlock - 1) / kRootBlock;
     return {{&m.norm, (size_t)b.maxN * es}, {&m.dog, (size_t)b.maxN * ed},
             {&m.labels, (size_t)b.maxN * 4}, {&m.rid, (size_t)b.maxN * 4},
-            {&m.bcnt, (size_t)block_count_words(b.maxN) * 4},
+            {&m.bcnt, (size_t)count_layout(b.maxN).words * 4},
             {&m.rmask, (size_t)nb * (kRootBlock / 8)}, {&m.rmulti, (size_t)nb * (kRootBlock / 8)},
             {&m.dR, 64}, {&m.acc, (size_t)b.acc_cap * sizeof(RegionAcc)},
             {&m.cand, std::max((size_t)b.maxT * kCandTile * 7 * 4, tmp2_off(b) + (size_t)b.maxN * 8)},

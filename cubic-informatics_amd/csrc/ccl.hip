@@ -254,8 +254,10 @@ __global__ __launch_bounds__(NTR) void k_cand_local(const float* __restrict__ ca
                                                    uint32_t* __restrict__ rlab,
                                                    unsigned long long* __restrict__ roots,
                                                    unsigned long long* __restrict__ multi,
-                                                   i64 root_words, int W, int H, int D, int nbx,
-                                                   int nby, int links, int rec_words) {
+                                                   i64 root_words,
+                                                   uint32_t* __restrict__ chunk_counts, int chunks,
+                                                   int W, int H, int D, int nbx, int nby,
+                                                   int links, int rec_words) {
   const unsigned tile = xcd_tile(blockIdx.x, gridDim.x);
   const uint32_t n = cand_cnt[tile];
   // this work-group's share of the root and region-spanning bitmaps, cleared for kernel C
@@ -266,6 +268,8 @@ __global__ __launch_bounds__(NTR) void k_cand_local(const float* __restrict__ ca
     if (threadIdx.x < 2 * (RTV / 64) && w < root_words)
       (threadIdx.x < RTV / 64 ? roots : multi)[w] = 0ull;
   }
+  if (tile == 0)  // and the region numbering's chunk counts
+    for (int i = (int)threadIdx.x; i < chunks; i += NTR) chunk_counts[i] = 0u;
   __shared__ unsigned long long bits[RROWS];  // the tile's mask rows (word = ly + RTY lz)
   // parents, valid at candidate positions; linked by 32-bit compare-and-swap on the word
   // holding two of them, so the array starts on a 4-byte boundary
@@ -695,14 +699,15 @@ hipError_t launch_ccl_candidates(const float* cand, const uint32_t* cand_cnt, i6
                                  unsigned long long* fgbits, uint32_t* P, uint32_t* rlab,
                                  unsigned long long* roots, unsigned long long* multi,
                                  i64 root_words, bool dense, int W, int H, int D, hipStream_t s,
-                                 int rec_words) {
+                                 int rec_words, uint32_t* chunk_counts, int chunks) {
   const int nbx = (W + RTX - 1) / RTX, nby = (H + RTY - 1) / RTY;
   hipError_t e;
   // the 13 forward offsets with one carry per axis are the positive offsets only for
   // width, height >= 2; otherwise every link goes through the generic merge
   const int generic = (W < 2 || H < 2) ? 1 : 0;
   hipLaunchKernelGGL(k_cand_local, dim3((unsigned)ntiles), dim3(NTR), 0, s, cand, cand_cnt, fgbits,
-                     P, rlab, roots, multi, root_words, W, H, D, nbx, nby, 1 - generic, rec_words);
+                     P, rlab, roots, multi, root_words, chunk_counts, chunks, W, H, D, nbx, nby,
+                     1 - generic, rec_words);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark("ccl/cand_local", s);
   hipLaunchKernelGGL(k_cand_merge, dim3((unsigned)ntiles), dim3(NTR), 0, s, cand, cand_cnt,

@@ -17,12 +17,20 @@ constexpr int kMaxGaussRadius = 40;            // 2r+1 <= 81 taps per axis
 constexpr int kMaxTaps = 2 * kMaxGaussRadius + 1;
 constexpr int kMaxNormRadius = 200;
 constexpr int kRootBlock = 4096;  // voxels per root-numbering block (64 mask words)
-// per-block root counts of a volume of N voxels, followed (at a 64-word boundary) by the
-// scan's chunk sums, one per 4096 blocks
-inline i64 scan_chunk_offset(i64 nb) { return (nb + 63) / 64 * 64; }
-inline i64 block_count_words(i64 N) {
-  const i64 nb = (N + kRootBlock - 1) / kRootBlock;
-  return scan_chunk_offset(nb) + (nb + 4095) / 4096;
+// Root counts of a volume of N voxels: per numbering block, per group of 64 blocks, per chunk
+// of 64 groups (one 32-bit word each, the levels at 64-word boundaries).
+struct CountLayout {
+  i64 nb, groups_off, groups, chunks_off, chunks, words;
+};
+inline CountLayout count_layout(i64 N) {
+  CountLayout c;
+  c.nb = (N + kRootBlock - 1) / kRootBlock;
+  c.groups = (c.nb + 63) / 64;
+  c.chunks = (c.groups + 63) / 64;
+  c.groups_off = (c.nb + 63) / 64 * 64;
+  c.chunks_off = c.groups_off + (c.groups + 63) / 64 * 64;
+  c.words = c.chunks_off + c.chunks;
+  return c;
 }
 // word 3 of a raw buffer descriptor on gfx9-family GPUs (32-bit data format; no swizzle)
 constexpr int kBufferWord3 = 0x00020000;
@@ -339,19 +347,20 @@ template <typename TD, typename TH>
 hipError_t launch_hessian(const TD* dog, TH* hess, uint8_t* pd, int W, int H, int D,
                           hipStream_t s, float* cand = nullptr, uint32_t* cand_cnt = nullptr,
                           float band = kDefaultMinorBand);
-// Exclusive scan of the nb per-block counts in place (block_cnt: block_count_words() words),
-// *d_R = 1 + their total.
-hipError_t launch_scan_counts(uint32_t* block_cnt, i64 nb, uint32_t* d_R, hipStream_t s);
-// Region numbering of a label volume: root counts per block of 4096 voxels and their
-// positions (masks: 64 words per block), then *d_R = 1 + number of roots.
-hipError_t launch_region_ids(const uint32_t* labels, uint32_t* block_cnt,
-                             unsigned long long* masks, uint32_t* d_R, i64 N, hipStream_t s,
-                             i64* nblocks_out);
-// Region ids from the root bits and the scanned block counts: rid at every root, and a
-// cleared accumulator line (with the root) for every id below cap; ids >= cap are skipped
-// (graph-captured batches, where the host never sees the count, rely on that).
-hipError_t launch_region_assign(const unsigned long long* masks, const uint32_t* block_off,
-                                uint32_t* rid, RegionAcc* acc, i64 cap, i64 N, hipStream_t s);
+// Region numbering.  Root counts of a label volume (launch_region_ids, which also writes the
+// root bit mask) or of a root bit mask whose chunk counts the labeling has cleared
+// (launch_region_count_masks), in the layout of count_layout(N).
+hipError_t launch_region_ids(const uint32_t* labels, uint32_t* counts, unsigned long long* masks,
+                             i64 N, hipStream_t s);
+hipError_t launch_region_count_masks(const unsigned long long* masks, uint32_t* counts, i64 N,
+                                     hipStream_t s);
+// Region ids from the root bits and the counts: rid at every root, a cleared accumulator line
+// (with the root) for every id below cap, and the number of regions, 1 + the number of roots,
+// in *d_R and, if given, *h_R (page-locked host memory).  Ids >= cap are skipped: the host may
+// launch this and what follows before it has seen the count.
+hipError_t launch_region_assign(const unsigned long long* masks, const uint32_t* counts,
+                                uint32_t* rid, RegionAcc* acc, i64 cap, i64 N, uint32_t* d_R,
+                                uint32_t* h_R, hipStream_t s);
 template <typename TH, typename TN>
 hipError_t launch_region_accum(const uint32_t* labels, const uint32_t* rid, const TH* hess,
                                const TN* norm, const uint16_t* img, RegionAcc* acc, i64 cap,
@@ -376,10 +385,12 @@ struct TileOut {
   u64 offset, count;
   uint32_t overflow, found;  // found: regions of the stack, also when they did not fit
 };
-// With t == nullptr: region r goes to slot r, r < R.  With t: regions 1..t->count go to
-// slots t->offset + r - 1 (nothing when t->overflow); R then only sizes the grid.
-hipError_t launch_region_finalize(const RegionAcc* acc, i64 R, int is_ave, RegionOut o,
-                                  i64 pitch, hipStream_t s, const TileOut* t = nullptr);
+// With t == nullptr: region r goes to slot r, r < min(*d_R, cap).  With t: regions
+// 1..t->count go to slots t->offset + r - 1 (nothing when t->overflow).  `expect`: sizes the
+// grid.
+hipError_t launch_region_finalize(const RegionAcc* acc, const uint32_t* d_R, i64 cap, i64 expect,
+                                  int is_ave, RegionOut o, i64 pitch, hipStream_t s,
+                                  const TileOut* t = nullptr);
 // t->offset = *running, t->count = *d_R - 1, *running += t->count; overflow (count 0) when
 // *d_R > acc_cap or the arena of arena_cap slots would overflow
 hipError_t launch_tile_reserve(const uint32_t* d_R, i64 acc_cap, i64 arena_cap, u64* running,
@@ -392,22 +403,20 @@ hipError_t launch_fill_u64(u64* p, i64 n, u64 value, hipStream_t s);
 // roots (root_words 64-bit words, cleared here) receives the root bit of every component,
 // in linear order, and multi (same size, cleared here) the root bit of every component
 // with voxels outside the kAccGY x kAccGZ tile group of its root (both NULL: not wanted).
-// dense: P becomes the full label volume (0 for the background).
+// dense: P becomes the full label volume (0 for the background).  chunk_counts (optional,
+// chunks words) is cleared for launch_region_count_masks.
 // rec_words: 32-bit words per record slot block (7: the Hessian pass's records; 1: the
 // positions of launch_mask_records).
 hipError_t launch_ccl_candidates(const float* cand, const uint32_t* cand_cnt, i64 ntiles,
                                  unsigned long long* fgbits, uint32_t* P, uint32_t* rlab,
                                  unsigned long long* roots, unsigned long long* multi,
                                  i64 root_words, bool dense, int W, int H, int D, hipStream_t s,
-                                 int rec_words = 7);
+                                 int rec_words = 7, uint32_t* chunk_counts = nullptr,
+                                 int chunks = 0);
 // The candidate positions of a byte mask (pd != 0, voxel 0 excluded) in the Hessian pass's
 // record layout with one word per slot (pos: hessian_tiles() * kCandTile words).
 hipError_t launch_mask_records(const uint8_t* pd, float* pos, uint32_t* cand_cnt, int W, int H,
                                int D, hipStream_t s);
-// Roots per numbering block from a root bit mask in linear order, then the exclusive scan
-// of the counts; *d_R = 1 + number of roots.
-hipError_t launch_region_count_masks(const unsigned long long* masks, uint32_t* block_cnt,
-                                     uint32_t* d_R, i64 N, hipStream_t s, i64* nblocks_out);
 // differentiable blob response (soft.hip)
 hipError_t launch_soft_loss(const float* hess, const uint8_t* mask, const uint8_t* target, i64 N,
                             double inv_tau, double* sums, hipStream_t s);

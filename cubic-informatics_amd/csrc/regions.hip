@@ -8,8 +8,8 @@
 // sorts of (label, value) pairs and reduce-by-key, about 1 KB of traffic per voxel.
 //
 // MI355X design: the labels already are the component minima, so a region's id is the
-// rank of its root among all roots in linear order -- a block-count / scan / assign
-// pass that preserves the reference's ascending order.  Each work-group folds its voxels
+// rank of its root among all roots in linear order -- root counts at three levels, then an
+// assign pass that preserves the reference's ascending order.  Each work-group folds its voxels
 // into an LDS table of partial sums (packed integer sums, FP64 Hessian and
 // intensity-float sums, ordered-integer max for the float max); each table entry then
 // ends in the region's 128-byte accumulator line, stored when the work-group holds the
@@ -31,24 +31,15 @@ __device__ __forceinline__ int wave_sum_int(int v) {
   return v;  // lane 0 holds the sum
 }
 
-__device__ __forceinline__ int block_sum_int(int v, int* sh) {
-  // wave64 reduction, then across the 4 waves
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (lane == 0) sh[wave] = v;
-  __syncthreads();
-  int t = 0;
-  if (threadIdx.x == 0) t = sh[0] + sh[1] + sh[2] + sh[3];
-  return t;
-}
-
-// Per block of BLK voxels: the number of roots (L[i] == i, i > 0) and their positions as
-// a bitmask (masks[64 b + 4 k + wave] bit lane <-> voxel b*BLK + k*NT + 64 wave + lane,
-// so bit order is linear order).
-__global__ __launch_bounds__(NT) void k_count_roots(const uint32_t* __restrict__ L, i64 N,
-                                                    uint32_t* __restrict__ cnt,
-                                                    unsigned long long* __restrict__ masks) {
-  __shared__ int sh[4];
+// Per block of BLK voxels: the positions of the roots (L[i] == i, i > 0) as a bitmask
+// (masks[64 b + 4 k + wave] bit lane <-> voxel b*BLK + k*NT + 64 wave + lane, so bit order is
+// linear order).  Clears the chunk counts for the counting kernel.
+__global__ __launch_bounds__(NT) void k_root_bits(const uint32_t* __restrict__ L, i64 N,
+                                                  unsigned long long* __restrict__ masks,
+                                                  uint32_t* __restrict__ chunk_counts,
+                                                  int chunks) {
+  if (blockIdx.x == 0)
+    for (int i = (int)threadIdx.x; i < chunks; i += NT) chunk_counts[i] = 0u;
   const i64 base = (i64)blockIdx.x * BLK;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   uint32_t v[ITEMS];
@@ -57,103 +48,93 @@ __global__ __launch_bounds__(NT) void k_count_roots(const uint32_t* __restrict__
     const i64 i = base + (i64)k * NT + threadIdx.x;
     v[k] = i < N ? L[i] : 0u;
   }
-  int c = 0;
 #pragma unroll
   for (int k = 0; k < ITEMS; ++k) {
     const i64 i = base + (i64)k * NT + threadIdx.x;
-    const bool root = i > 0 && i < N && v[k] == (uint32_t)i;
-    const unsigned long long m = __ballot(root);
+    const unsigned long long m = __ballot(i > 0 && i < N && v[k] == (uint32_t)i);
     if (lane == 0) masks[(size_t)blockIdx.x * (BLK / 64) + k * (NT / 64) + wave] = m;
-    c += root ? 1 : 0;
   }
-  const int t = block_sum_int(c, sh);
-  if (threadIdx.x == 0) cnt[blockIdx.x] = (uint32_t)t;
 }
 
-// Exclusive scan of cnt[0..nb) in place, *d_R = 1 + total (totals stay below 2^32 as
-// N < 2^32), in three short kernels: the sums of chunks of 4096 counts (one work-group of
-// 1024 threads, 4 consecutive counts each), the exclusive scan of the <= 256 chunk sums
-// (one work-group), and every chunk's scan from its offset.
-constexpr int SCAN_V = 4, SCAN_CH = 1024 * SCAN_V;
-
-// inclusive scan of x over the 1024 threads of the work-group; *total = the sum
-__device__ __forceinline__ uint32_t block_scan_1024(uint32_t x, uint32_t* wsum,
-                                                    uint32_t* total) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+// Roots per block, per group of 64 blocks (one work-group) and per chunk of 64 groups (added;
+// cleared before) from the root bit mask, whose 512 bytes per block bound it.  A wave takes 16
+// blocks, all their words in flight, and folds the 16 sums together: after the exchange over
+// lane bits 5 .. 2 a lane holds a quarter of one block's count.
+__global__ __launch_bounds__(NT) void k_mask_counts(const unsigned long long* __restrict__ masks,
+                                                    i64 nb, uint32_t* __restrict__ cnt,
+                                                    uint32_t* __restrict__ groups,
+                                                    uint32_t* __restrict__ chunks) {
+  __shared__ uint32_t part[NT / 64];
+  const int lane = (int)(threadIdx.x & 63), wave = (int)(threadIdx.x >> 6);
+  const i64 b0 = (i64)blockIdx.x * 64 + wave * 16;
+  uint32_t v[16];
 #pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const uint32_t y = __shfl_up(x, o, 64);
-    if (lane >= o) x += y;
-  }
-  if (lane == 63) wsum[wave] = x;
-  __syncthreads();
-  if (wave == 0) {
-    uint32_t w = lane < 16 ? wsum[lane] : 0u;
+  for (int j = 0; j < 16; ++j)
+    v[j] = b0 + j < nb ? (uint32_t)__popcll(masks[(b0 + j) * (BLK / 64) + lane]) : 0u;
 #pragma unroll
-    for (int o = 1; o < 16; o <<= 1) {
-      const uint32_t y = __shfl_up(w, o, 64);
-      if (lane >= o) w += y;
+  for (int k = 8; k >= 1; k >>= 1) {  // lane bit 4 k picks the upper half of the blocks
+    const bool up = (lane & (4 * k)) != 0;
+#pragma unroll
+    for (int j = 0; j < k; ++j) {
+      const uint32_t keep = up ? v[j + k] : v[j], give = up ? v[j] : v[j + k];
+      v[j] = keep + __shfl_xor(give, 4 * k, 64);
     }
-    if (lane < 16) wsum[lane] = w;
   }
+  uint32_t t = v[0];
+  t += __shfl_xor(t, 1, 64);
+  t += __shfl_xor(t, 2, 64);
+  const i64 blk = b0 + (lane >> 2);  // bits 5 .. 2 of the lane: its block's bits 3 .. 0
+  if ((lane & 3) == 0 && blk < nb) cnt[blk] = t;
+#pragma unroll
+  for (int o = 4; o < 64; o <<= 1) t += __shfl_xor(t, o, 64);
+  if (lane == 0) part[wave] = t;
   __syncthreads();
-  *total = wsum[15];
-  return x + (wave ? wsum[wave - 1] : 0u);
-}
-
-__global__ __launch_bounds__(1024) void k_chunk_sums(const uint32_t* __restrict__ cnt, i64 nb,
-                                                     uint32_t* __restrict__ csum) {
-  __shared__ uint32_t wsum[16];
-  const i64 i0 = (i64)blockIdx.x * SCAN_CH + (i64)threadIdx.x * SCAN_V;
-  uint32_t v = 0;
-#pragma unroll
-  for (int j = 0; j < SCAN_V; ++j) v += (i0 + j < nb) ? cnt[i0 + j] : 0u;
-  uint32_t total;
-  (void)block_scan_1024(v, wsum, &total);
-  if (threadIdx.x == 0) csum[blockIdx.x] = total;
-}
-
-__global__ __launch_bounds__(1024) void k_chunk_offsets(uint32_t* csum, int nch,
-                                                        uint32_t* d_R) {
-  __shared__ uint32_t wsum[16];
-  const uint32_t v = (int)threadIdx.x < nch ? csum[threadIdx.x] : 0u;
-  uint32_t total;
-  const uint32_t incl = block_scan_1024(v, wsum, &total);
-  if ((int)threadIdx.x < nch) csum[threadIdx.x] = incl - v;
-  if (threadIdx.x == 0) *d_R = 1u + total;
-}
-
-__global__ __launch_bounds__(1024) void k_chunk_scan(uint32_t* cnt, i64 nb,
-                                                     const uint32_t* __restrict__ coff) {
-  __shared__ uint32_t wsum[16];
-  const i64 i0 = (i64)blockIdx.x * SCAN_CH + (i64)threadIdx.x * SCAN_V;
-  uint32_t cur[SCAN_V], sum = 0;
-#pragma unroll
-  for (int j = 0; j < SCAN_V; ++j) {
-    cur[j] = (i0 + j < nb) ? cnt[i0 + j] : 0u;
-    sum += cur[j];
-  }
-  uint32_t total;
-  uint32_t run = coff[blockIdx.x] + block_scan_1024(sum, wsum, &total) - sum;
-#pragma unroll
-  for (int j = 0; j < SCAN_V; ++j) {
-    if (i0 + j < nb) cnt[i0 + j] = run;
-    run += cur[j];
+  if (threadIdx.x == 0) {
+    const uint32_t g = part[0] + part[1] + part[2] + part[3];
+    groups[blockIdx.x] = g;
+    atomicAdd(chunks + blockIdx.x / 64, g);
   }
 }
 
-// rid[root] = 1 + rank of the root in linear order; acc[rid] = zero sums with .root =
-// root (a whole 128-byte line per region, which also clears the accumulator; block 0
-// clears acc[0], the background's).  One wave per block of BLK voxels: lane m takes root
-// mask m of the block, a wave scan of the mask popcounts gives each mask's rank offset,
-// and only the (few) roots are visited.
-__global__ __launch_bounds__(64) void k_assign_ids(const unsigned long long* __restrict__ masks,
-                                                   const uint32_t* __restrict__ off,
-                                                   uint32_t* __restrict__ rid,
-                                                   RegionAcc* __restrict__ acc, i64 cap) {
+// rid[root] = 1 + rank of the root in linear order; acc[rid] = zero sums with .root = root (a
+// whole 128-byte line per region, which also clears the accumulator; acc[0], the background's,
+// is cleared too); *d_R and *h_R = 1 + number of roots.  One wave per block of BLK voxels: its
+// first rank is the sum of the chunks, groups and blocks before it, a few words per lane, so
+// no scan runs before; lane m takes root mask m of the block, a wave scan of the mask
+// popcounts gives each mask's rank, and only the (few) roots are visited: each round takes one
+// root per lane and writes their lines with eight lanes per line.
+__global__ __launch_bounds__(NT) void k_assign_ids(const unsigned long long* __restrict__ masks,
+                                                   const uint32_t* __restrict__ cnt,
+                                                   const uint32_t* __restrict__ groups,
+                                                   const uint32_t* __restrict__ chunks,
+                                                   int n_chunks, i64 nb, uint32_t* __restrict__ rid,
+                                                   RegionAcc* __restrict__ acc, i64 cap,
+                                                   uint32_t* d_R, uint32_t* h_R) {
   static_assert(BLK / 64 == 64, "one mask per lane");
-  const int lane = threadIdx.x;
-  unsigned long long m = masks[(size_t)blockIdx.x * 64 + lane];
+  static_assert(sizeof(RegionAcc) == 128 && offsetof(RegionAcc, root) == 100, "line layout");
+  __shared__ uint2 ent[NT / 64][64];
+  const int lane = (int)(threadIdx.x & 63), wave = (int)(threadIdx.x >> 6);
+  const i64 blk = (i64)blockIdx.x * (NT / 64) + wave;
+  if (blk >= nb) return;  // whole waves
+  if (blk == 0) {
+    uint32_t t = 0u;
+    for (int i = lane; i < n_chunks; i += 64) t += chunks[i];
+    t = 1u + (uint32_t)wave_sum_int((int)t);
+    if (lane == 0) {
+      *d_R = t;
+      if (h_R) *h_R = t;
+      if (cap > 0) acc[0] = RegionAcc{};
+    }
+  }
+  unsigned long long m = masks[blk * (BLK / 64) + lane];
+  const i64 g = blk / 64, c = g / 64;
+  uint32_t before = 0u;
+  for (int i = lane; i < (int)c; i += 64) before += chunks[i];
+  if (lane < (int)(g % 64)) before += groups[c * 64 + lane];
+  if (lane < (int)(blk % 64)) before += cnt[g * 64 + lane];
+  if (!__ballot(m != 0ull)) return;  // uniform over the wave
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) before += __shfl_xor(before, o, 64);
   const uint32_t n = (uint32_t)__popcll(m);
   uint32_t incl = n;
 #pragma unroll
@@ -161,20 +142,28 @@ __global__ __launch_bounds__(64) void k_assign_ids(const unsigned long long* __r
     const uint32_t y = __shfl_up(incl, o, 64);
     if (lane >= o) incl += y;
   }
-  uint32_t r = 1 + off[blockIdx.x] + (incl - n);
-  const i64 base = (i64)blockIdx.x * BLK + 64 * lane;
-  if (blockIdx.x == 0 && lane == 0 && cap > 0) acc[0] = RegionAcc{};
-  while (m) {
-    const int bit = __builtin_ctzll(m);
-    m &= m - 1;
-    const i64 i = base + bit;
-    rid[i] = r;
-    if ((i64)r < cap) {
-      RegionAcc a{};
-      a.root = (uint32_t)i;
-      acc[r] = a;
+  uint32_t r = 1u + before + (incl - n);
+  const i64 base = blk * BLK + 64 * lane;
+  const unsigned long long below = (1ull << lane) - 1ull;
+  while (true) {
+    const unsigned long long on = __ballot(m != 0ull);
+    if (!on) break;
+    if (m) {
+      const uint32_t i = (uint32_t)(base + __builtin_ctzll(m));
+      m &= m - 1;
+      rid[i] = r;
+      ent[wave][__popcll(on & below)] = make_uint2(i, r);
+      ++r;
     }
-    ++r;
+    wave_lds_sync();
+    const int ne = __popcll(on);
+    for (int e = lane >> 3; e < ne; e += 8) {
+      const uint2 v = ent[wave][e];
+      if ((i64)v.y < cap)
+        reinterpret_cast<uint4*>(acc + v.y)[lane & 7] =
+            make_uint4(0u, (lane & 7) == 6 ? v.x : 0u, 0u, 0u);
+    }
+    wave_lds_sync();
   }
 }
 
@@ -598,10 +587,11 @@ __device__ void eigen_features(const float h6[6], float* st, float* bl) {
   *bl = (float)(e2 * e2 / (e0 * e1));
 }
 
-__global__ __launch_bounds__(NT) void k_finalize(const RegionAcc* __restrict__ acc, i64 R,
+__global__ __launch_bounds__(NT) void k_finalize(const RegionAcc* __restrict__ acc,
+                                                 const uint32_t* __restrict__ d_R, i64 cap,
                                                  int is_ave, RegionOut o, i64 pitch,
                                                  const TileOut* __restrict__ tile) {
-  i64 base = 0, first = 0;
+  i64 base = 0, first = 0, R = min((i64)*d_R, cap);
   if (tile) {
     if (tile->overflow) return;
     R = (i64)tile->count + 1;
@@ -669,50 +659,35 @@ __global__ __launch_bounds__(NT) void k_fill_u64(u64* p, i64 n, u64 v) {
   for (i64 i = (i64)blockIdx.x * NT + threadIdx.x; i < n; i += (i64)gridDim.x * NT) p[i] = v;
 }
 
-// roots per 4096-voxel block from the root bit mask (one wave per block, a word per lane)
-__global__ __launch_bounds__(NT) void k_mask_counts(const unsigned long long* __restrict__ masks,
-                                                    i64 nb, uint32_t* __restrict__ cnt) {
-  const i64 blk = (i64)blockIdx.x * (NT / 64) + (threadIdx.x >> 6);
-  if (blk >= nb) return;  // whole waves
-  const int c = __popcll(masks[blk * (kRootBlock / 64) + (threadIdx.x & 63)]);
-  const int t = wave_sum_int(c);
-  if ((threadIdx.x & 63) == 0) cnt[blk] = (uint32_t)t;
-}
-
 }  // namespace
 
-// block_cnt holds block_count_words(N) words: the nb counts, then the chunk sums
-hipError_t launch_scan_counts(uint32_t* block_cnt, i64 nb, uint32_t* d_R, hipStream_t s) {
-  const int nch = (int)((nb + SCAN_CH - 1) / SCAN_CH);
-  if (nch > 1024) return hipErrorInvalidValue;  // N < 2^32: at most 256 chunks
-  uint32_t* csum = block_cnt + scan_chunk_offset(nb);
-  hipLaunchKernelGGL(k_chunk_sums, dim3((unsigned)nch), dim3(1024), 0, s, block_cnt, nb, csum);
-  hipLaunchKernelGGL(k_chunk_offsets, dim3(1), dim3(1024), 0, s, csum, nch, d_R);
-  hipLaunchKernelGGL(k_chunk_scan, dim3((unsigned)nch), dim3(1024), 0, s, block_cnt, nb,
-                     (const uint32_t*)csum);
-  mark("regions/scan", s);
+hipError_t launch_region_count_masks(const unsigned long long* masks, uint32_t* counts, i64 N,
+                                     hipStream_t s) {
+  const CountLayout c = count_layout(N);
+  hipLaunchKernelGGL(k_mask_counts, dim3((unsigned)c.groups), dim3(NT), 0, s, masks, c.nb, counts,
+                     counts + c.groups_off, counts + c.chunks_off);
+  mark("regions/count_root_bits", s);
   return hipGetLastError();
 }
 
-hipError_t launch_region_ids(const uint32_t* labels, uint32_t* block_cnt,
-                             unsigned long long* masks, uint32_t* d_R, i64 N, hipStream_t s,
-                             i64* nblocks_out) {
-  const i64 nb = (N + BLK - 1) / BLK;
-  *nblocks_out = nb;
-  hipLaunchKernelGGL(k_count_roots, dim3((unsigned)nb), dim3(NT), 0, s, labels, N, block_cnt,
-                     masks);
-  hipError_t e = hipGetLastError();
+hipError_t launch_region_ids(const uint32_t* labels, uint32_t* counts, unsigned long long* masks,
+                             i64 N, hipStream_t s) {
+  const CountLayout c = count_layout(N);
+  hipLaunchKernelGGL(k_root_bits, dim3((unsigned)c.nb), dim3(NT), 0, s, labels, N, masks,
+                     counts + c.chunks_off, (int)c.chunks);
+  const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  mark("regions/count_roots", s);
-  return launch_scan_counts(block_cnt, nb, d_R, s);
+  mark("regions/root_bits", s);
+  return launch_region_count_masks(masks, counts, N, s);
 }
 
-hipError_t launch_region_assign(const unsigned long long* masks, const uint32_t* block_off,
-                                uint32_t* rid, RegionAcc* acc, i64 cap, i64 N, hipStream_t s) {
-  mark(nullptr, s);  // the host waited for the region count: start a new interval
-  const i64 nb = (N + BLK - 1) / BLK;
-  hipLaunchKernelGGL(k_assign_ids, dim3((unsigned)nb), dim3(64), 0, s, masks, block_off, rid, acc,
-                     cap);
+hipError_t launch_region_assign(const unsigned long long* masks, const uint32_t* counts,
+                                uint32_t* rid, RegionAcc* acc, i64 cap, i64 N, uint32_t* d_R,
+                                uint32_t* h_R, hipStream_t s) {
+  const CountLayout c = count_layout(N);
+  hipLaunchKernelGGL(k_assign_ids, dim3((unsigned)((c.nb + NT / 64 - 1) / (NT / 64))), dim3(NT), 0,
+                     s, masks, counts, counts + c.groups_off, counts + c.chunks_off, (int)c.chunks,
+                     c.nb, rid, acc, cap, d_R, h_R);
   mark("regions/assign_ids", s);
   return hipGetLastError();
 }
@@ -766,10 +741,12 @@ HDOG_INST_ACCC(__half)
 HDOG_INST_ACCC(__hip_bfloat16)
 #undef HDOG_INST_ACCC
 
-hipError_t launch_region_finalize(const RegionAcc* acc, i64 R, int is_ave, RegionOut o, i64 pitch,
-                                  hipStream_t s, const TileOut* t) {
-  const i64 nb = std::max<i64>(1, std::min<i64>((R + NT - 1) / NT, 1 << 16));
-  hipLaunchKernelGGL(k_finalize, dim3((unsigned)nb), dim3(NT), 0, s, acc, R, is_ave, o, pitch, t);
+hipError_t launch_region_finalize(const RegionAcc* acc, const uint32_t* d_R, i64 cap, i64 expect,
+                                  int is_ave, RegionOut o, i64 pitch, hipStream_t s,
+                                  const TileOut* t) {
+  const i64 nb = std::max<i64>(1, std::min<i64>((expect + NT - 1) / NT, 1 << 16));
+  hipLaunchKernelGGL(k_finalize, dim3((unsigned)nb), dim3(NT), 0, s, acc, d_R, cap, is_ave, o,
+                     pitch, t);
   mark("regions/finalize", s);
   return hipGetLastError();
 }
@@ -778,18 +755,6 @@ hipError_t launch_tile_reserve(const uint32_t* d_R, i64 acc_cap, i64 arena_cap, 
                                TileOut* t, hipStream_t s) {
   hipLaunchKernelGGL(k_tile_reserve, dim3(1), dim3(64), 0, s, d_R, acc_cap, arena_cap, running, t);
   return hipGetLastError();
-}
-
-hipError_t launch_region_count_masks(const unsigned long long* masks, uint32_t* block_cnt,
-                                     uint32_t* d_R, i64 N, hipStream_t s, i64* nblocks_out) {
-  const i64 nb = (N + kRootBlock - 1) / kRootBlock;
-  if (nblocks_out) *nblocks_out = nb;
-  hipLaunchKernelGGL(k_mask_counts, dim3((unsigned)((nb + NT / 64 - 1) / (NT / 64))), dim3(NT), 0,
-                     s, masks, nb, block_cnt);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  mark("regions/count_root_bits", s);
-  return launch_scan_counts(block_cnt, nb, d_R, s);
 }
 
 hipError_t launch_fill_u64(u64* p, i64 n, u64 value, hipStream_t s) {

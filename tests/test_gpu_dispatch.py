@@ -140,3 +140,25 @@ def test_normalize_of_any_radii(hd, shape, rxy, rz):
     np.testing.assert_array_equal(n.cpu().numpy(), want)
     np.testing.assert_array_equal(ge.cpu().numpy(), e)
     np.testing.assert_array_equal(gd.cpu().numpy(), d)
+
+
+# region numbers and counts across blocks, groups and chunks of the root counts, and a stack
+# with more regions than the arrays of the call before hold, then one with fewer
+def test_region_numbering_over_growing_and_shrinking_lists(hd):
+    from hdog import HDoG
+    fresh = HDoG(0)
+    try:
+        for shape, step in (((3, 40, 70), 3), ((40, 300, 1500), 2), ((5, 64, 64), 4)):
+            pd = np.zeros(shape, np.uint8)
+            pd[::step, ::step, 1::step] = 1
+            # (steps of two keep neighbours apart, also where rows wrap)
+            labels = fresh.CCL(pd)
+            hess = np.zeros((6,) + shape, np.float32)
+            g = fresh.RegionalFeatures(labels, hess, np.ones(shape, np.float32), None)
+            at = np.flatnonzero(pd)
+            lab = labels.cpu().numpy().ravel()
+            roots = at[lab[at] == at]
+            np.testing.assert_array_equal(g["label"][1:], roots.astype(np.uint32))
+            np.testing.assert_array_equal(g["count"][1:], np.unique(lab[at], return_counts=True)[1])
+    finally:
+        fresh.close()
