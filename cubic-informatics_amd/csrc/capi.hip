@@ -70,6 +70,7 @@ struct hdog_ctx {
   i64 R = 0;
   uint32_t* h_R = nullptr;         // page-locked: the region count, written by the device
   hipEvent_t counted = nullptr;   // recorded after the kernel that writes it
+  void* stage = nullptr;          // page-locked, kStageBytes: short region lists on their way
   bool prof = false;        // record an event after every kernel of run_device
   Prof pool;
   bool ev_valid = false;
@@ -223,7 +224,8 @@ int gaussian_weights(float sigma, double truncate, float* w) {
 // same shape has about as many.
 int ensure_regions(hdog_ctx* ctx, i64 R) {
   if (R > ctx->out_cap) {
-    const i64 cap = std::max<i64>(R + R / 8 + 1024, ctx->out_cap * 3 / 2);
+    // (a multiple of 64: the arrays' parts stay aligned for wide copies)
+    const i64 cap = (std::max<i64>(R + R / 8 + 1024, ctx->out_cap * 3 / 2) + 63) / 64 * 64;
     ctx->out_cap = 0;  // until every array has grown
     HIPCHK(ensure(ctx->o_label, cap * 4));
     HIPCHK(ensure(ctx->o_size, cap * 2));
@@ -257,6 +259,69 @@ struct CandRecords {
 // in ctx->rmask, each record's label in cand.rlab) and the region sums from the records
 // (labels and hess unused); else from the label volume (final labels, only read) and the
 // materialized Hessian.
+// What the caller's array [p, p + bytes) is: page-locked host memory that the device can write
+// (*view is the device's address of p), pageable memory, or something only the runtime's copies
+// handle.
+enum class HostMem { locked, pageable, other };
+HostMem host_memory(void* p, size_t bytes, void** view) {
+  hipPointerAttribute_t a[2];
+  for (int k = 0; k < 2; ++k) {
+    const hipError_t e = hipPointerGetAttributes(&a[k], (char*)p + (k ? bytes - 1 : 0));
+    if (e != hipSuccess) {  // memory the runtime does not know
+      (void)hipGetLastError();
+      a[k].type = hipMemoryTypeUnregistered;
+      a[k].devicePointer = nullptr;
+    }
+  }
+  if (a[0].type == hipMemoryTypeUnregistered && a[1].type == hipMemoryTypeUnregistered)
+    return HostMem::pageable;
+  if (a[0].type != hipMemoryTypeHost || a[1].type != hipMemoryTypeHost || !a[0].devicePointer ||
+      (char*)a[1].devicePointer != (char*)a[0].devicePointer + (bytes - 1))
+    return HostMem::other;
+  *view = a[0].devicePointer;
+  return HostMem::locked;
+}
+
+// Brings a region list's arrays (device sources) to the caller and waits for them: by one
+// kernel when the device can write all of them, or into a page-locked buffer of the context
+// when they are short, else by one copy each.
+constexpr size_t kStageBytes = 2 << 20;
+int copy_out(hdog_ctx* ctx, const CopyList& want, hipStream_t s) {
+  CopyList l;
+  size_t total = 0;
+  int locked = 0, pageable = 0;
+  for (int k = 0; k < want.n; ++k) {
+    total += (want.bytes[k] + 15) / 16 * 16;
+    void* d = nullptr;
+    const HostMem m = host_memory(want.dst[k], want.bytes[k], &d);
+    locked += m == HostMem::locked;
+    pageable += m == HostMem::pageable;
+    l.add(d, want.src[k], want.bytes[k]);
+  }
+  if (locked == want.n) {
+    HIPCHK(launch_copy_list(l, s));
+    HIPCHK(hipStreamSynchronize(s));
+    return HDOG_OK;
+  }
+  if (locked + pageable == want.n && total <= kStageBytes) {
+    if (!ctx->stage) HIPCHK(hipHostMalloc(&ctx->stage, kStageBytes, hipHostMallocDefault));
+    l.n = 0;
+    size_t at = 0;
+    for (int k = 0; k < want.n; ++k) {
+      l.add((char*)ctx->stage + at, want.src[k], want.bytes[k]);
+      at += (want.bytes[k] + 15) / 16 * 16;
+    }
+    HIPCHK(launch_copy_list(l, s));
+    HIPCHK(hipStreamSynchronize(s));
+    for (int k = 0; k < want.n; ++k) std::memcpy(want.dst[k], l.dst[k], want.bytes[k]);
+    return HDOG_OK;
+  }
+  for (int k = 0; k < want.n; ++k)
+    HIPCHK(hipMemcpyAsync(want.dst[k], want.src[k], want.bytes[k], hipMemcpyDeviceToHost, s));
+  HIPCHK(hipStreamSynchronize(s));
+  return HDOG_OK;
+}
+
 template <typename TH, typename TN>
 int regional_features_t(hdog_ctx* ctx, hipStream_t s, uint32_t* labels, const TH* hess,
                         const TN* norm, const uint16_t* img, int W, int H, int D, int is_ave,
@@ -716,6 +781,7 @@ void hdog_destroy(hdog_ctx* ctx) {
   release(ctx->weights);
   if (ctx->counted) (void)hipEventDestroy(ctx->counted);
   if (ctx->h_R) (void)hipHostFree(ctx->h_R);
+  if (ctx->stage) (void)hipHostFree(ctx->stage);
   delete ctx;
 }
 
@@ -924,28 +990,27 @@ int hdog_regions_download(hdog_ctx* ctx, void* stream, hdog_regions* out) {
   HIPCHK(hipSetDevice(ctx->device));
   hipStream_t s = (hipStream_t)stream;
   const i64 cap = ctx->out_cap;
-  auto cp = [&](void* dst, const void* src, size_t bytes) -> hipError_t {
-    if (!dst || bytes == 0) return hipSuccess;
-    return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
+  CopyList l;
+  auto cp = [&](void* dst, const void* src, size_t bytes) {
+    if (dst && bytes) l.add(dst, src, bytes);
   };
   const float* cen = (const float*)ctx->o_cen.p;
   const float* eig = (const float*)ctx->o_eig.p;
-  HIPCHK(cp(out->label, ctx->o_label.p, R * 4));
-  HIPCHK(cp(out->size, ctx->o_size.p, R * 2));
-  HIPCHK(cp(out->voxels, ctx->o_vox.p, R * 8));
-  HIPCHK(cp(out->centroid_x, cen, R * 4));
-  HIPCHK(cp(out->centroid_y, cen + cap, R * 4));
-  HIPCHK(cp(out->centroid_z, cen + 2 * cap, R * 4));
-  HIPCHK(cp(out->structureness, eig, R * 4));
-  HIPCHK(cp(out->blobness, eig + cap, R * 4));
-  HIPCHK(cp(out->max_normalized, ctx->o_nrm.p, R * 4));
+  cp(out->label, ctx->o_label.p, R * 4);
+  cp(out->size, ctx->o_size.p, R * 2);
+  cp(out->voxels, ctx->o_vox.p, R * 8);
+  cp(out->centroid_x, cen, R * 4);
+  cp(out->centroid_y, cen + cap, R * 4);
+  cp(out->centroid_z, cen + 2 * cap, R * 4);
+  cp(out->structureness, eig, R * 4);
+  cp(out->blobness, eig + cap, R * 4);
+  cp(out->max_normalized, ctx->o_nrm.p, R * 4);
   if (out->hessian)
     for (int k = 0; k < 6; ++k)
-      HIPCHK(cp(out->hessian + k * out->capacity, (const float*)ctx->o_hess.p + k * cap, R * 4));
-  HIPCHK(cp(out->intensity_sum, ctx->o_isum.p, R * 8));
-  HIPCHK(cp(out->intensity_max, ctx->o_imax.p, R * 2));
-  HIPCHK(hipStreamSynchronize(s));
-  return HDOG_OK;
+      cp(out->hessian + k * out->capacity, (const float*)ctx->o_hess.p + k * cap, R * 4);
+  cp(out->intensity_sum, ctx->o_isum.p, R * 8);
+  cp(out->intensity_max, ctx->o_imax.p, R * 2);
+  return copy_out(ctx, l, s);
 }
 
 static int ensure_gauss(hdog_ctx* ctx, const hdog_params* p) {
@@ -1431,31 +1496,29 @@ int hdog_batch_download(hdog_ctx* ctx, void* stream, int tile, hdog_regions* out
   hipStream_t s = (hipStream_t)stream;
   const i64 cap = B->arena_cap;
   // entry 0 (background) is zero, entries 1..n come from arena slots off..off+n-1
-  auto cp = [&](void* dst, const void* src, size_t esz) -> hipError_t {
-    if (!dst) return hipSuccess;
+  CopyList l;
+  auto cp = [&](void* dst, const void* src, size_t esz) {
+    if (!dst) return;
     std::memset(dst, 0, esz);
-    if (n == 0) return hipSuccess;
-    return hipMemcpyAsync((char*)dst + esz, (const char*)src + off * esz, n * esz,
-                          hipMemcpyDeviceToHost, s);
+    if (n) l.add((char*)dst + esz, (const char*)src + off * esz, n * esz);
   };
   const float* cen = (const float*)B->a_cen.p;
   const float* eig = (const float*)B->a_eig.p;
-  HIPCHK(cp(out->label, B->a_label.p, 4));
-  HIPCHK(cp(out->size, B->a_size.p, 2));
-  HIPCHK(cp(out->voxels, B->a_vox.p, 8));
-  HIPCHK(cp(out->centroid_x, cen, 4));
-  HIPCHK(cp(out->centroid_y, cen + cap, 4));
-  HIPCHK(cp(out->centroid_z, cen + 2 * cap, 4));
-  HIPCHK(cp(out->structureness, eig, 4));
-  HIPCHK(cp(out->blobness, eig + cap, 4));
-  HIPCHK(cp(out->max_normalized, B->a_nrm.p, 4));
+  cp(out->label, B->a_label.p, 4);
+  cp(out->size, B->a_size.p, 2);
+  cp(out->voxels, B->a_vox.p, 8);
+  cp(out->centroid_x, cen, 4);
+  cp(out->centroid_y, cen + cap, 4);
+  cp(out->centroid_z, cen + 2 * cap, 4);
+  cp(out->structureness, eig, 4);
+  cp(out->blobness, eig + cap, 4);
+  cp(out->max_normalized, B->a_nrm.p, 4);
   if (out->hessian)
     for (int k = 0; k < 6; ++k)
-      HIPCHK(cp(out->hessian + k * out->capacity, (const float*)B->a_hess.p + k * cap, 4));
-  HIPCHK(cp(out->intensity_sum, B->a_isum.p, 8));
-  HIPCHK(cp(out->intensity_max, B->a_imax.p, 2));
-  HIPCHK(hipStreamSynchronize(s));
-  return HDOG_OK;
+      cp(out->hessian + k * out->capacity, (const float*)B->a_hess.p + k * cap, 4);
+  cp(out->intensity_sum, B->a_isum.p, 8);
+  cp(out->intensity_max, B->a_imax.p, 2);
+  return copy_out(ctx, l, s);
 }
 
 int hdog_host_alloc(hdog_ctx* ctx, size_t bytes, void** p) {

@@ -396,6 +396,20 @@ hipError_t launch_region_finalize(const RegionAcc* acc, const uint32_t* d_R, i64
 hipError_t launch_tile_reserve(const uint32_t* d_R, i64 acc_cap, i64 arena_cap, u64* running,
                                TileOut* t, hipStream_t s);
 hipError_t launch_fill_u64(u64* p, i64 n, u64 value, hipStream_t s);
+// Copies of a region list's arrays in one launch (device memory to page-locked host memory).
+struct CopyList {
+  static constexpr int kMax = 18;
+  const void* src[kMax];
+  void* dst[kMax];
+  u64 bytes[kMax];
+  int n = 0;
+  void add(void* d, const void* s, size_t b) {
+    src[n] = s;
+    dst[n] = d;
+    bytes[n++] = b;
+  }
+};
+hipError_t launch_copy_list(const CopyList& l, hipStream_t s);
 // Labeling of the candidates the Hessian pass recorded (cand / cand_cnt, see
 // launch_hessian): fgbits (fg_words() words) receives the candidate bit mask; P is a
 // volume-sized parent array written and read at candidate voxels only; rlab (slot-aligned

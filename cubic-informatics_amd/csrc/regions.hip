@@ -655,6 +655,41 @@ __global__ void k_tile_reserve(const uint32_t* __restrict__ d_R, i64 acc_cap, i6
   t->found = (uint32_t)(R - 1);
 }
 
+template <typename V>
+__device__ __forceinline__ void copy_as(const void* s, void* d, u64 bytes) {
+  const u64 n = bytes / sizeof(V), step = (u64)gridDim.x * NT;
+  u64 i = (u64)blockIdx.x * NT + threadIdx.x;
+  for (; i + 3 * step < n; i += 4 * step) {
+    V v[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = ((const V*)s)[i + k * step];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) ((V*)d)[i + k * step] = v[k];
+  }
+  for (; i < n; i += step) ((V*)d)[i] = ((const V*)s)[i];
+  if (blockIdx.x == 0 && threadIdx.x < bytes % sizeof(V)) {
+    const u64 t = n * sizeof(V) + threadIdx.x;
+    ((uint8_t*)d)[t] = ((const uint8_t*)s)[t];
+  }
+}
+
+// gridDim.y arrays, each with the widest access its two addresses allow.  One launch in place
+// of one copy per array: the copies of a short list are launches (17 of them 75 us of a
+// 24 x 96 x 112 stack's 214), a long one is bound by the host link either way.
+__global__ __launch_bounds__(NT) void k_copy_list(CopyList l) {
+  const void* s = l.src[blockIdx.y];
+  void* d = l.dst[blockIdx.y];
+  const u64 bytes = l.bytes[blockIdx.y], at = (u64)s | (u64)d;
+  if (at % 16 == 0)
+    copy_as<uint4>(s, d, bytes);
+  else if (at % 4 == 0)
+    copy_as<uint32_t>(s, d, bytes);
+  else if (at % 2 == 0)
+    copy_as<uint16_t>(s, d, bytes);
+  else
+    copy_as<uint8_t>(s, d, bytes);
+}
+
 __global__ __launch_bounds__(NT) void k_fill_u64(u64* p, i64 n, u64 v) {
   for (i64 i = (i64)blockIdx.x * NT + threadIdx.x; i < n; i += (i64)gridDim.x * NT) p[i] = v;
 }
@@ -754,6 +789,15 @@ hipError_t launch_region_finalize(const RegionAcc* acc, const uint32_t* d_R, i64
 hipError_t launch_tile_reserve(const uint32_t* d_R, i64 acc_cap, i64 arena_cap, u64* running,
                                TileOut* t, hipStream_t s) {
   hipLaunchKernelGGL(k_tile_reserve, dim3(1), dim3(64), 0, s, d_R, acc_cap, arena_cap, running, t);
+  return hipGetLastError();
+}
+
+hipError_t launch_copy_list(const CopyList& l, hipStream_t s) {
+  if (l.n == 0) return hipSuccess;
+  u64 most = 0;
+  for (int k = 0; k < l.n; ++k) most = std::max(most, l.bytes[k]);
+  const u64 nb = std::max<u64>(1, std::min<u64>((most + NT * 16 - 1) / (NT * 16), 64));
+  hipLaunchKernelGGL(k_copy_list, dim3((unsigned)nb, (unsigned)l.n), dim3(NT), 0, s, l);
   return hipGetLastError();
 }
 

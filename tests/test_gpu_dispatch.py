@@ -162,3 +162,37 @@ def test_region_numbering_over_growing_and_shrinking_lists(hd):
             np.testing.assert_array_equal(g["count"][1:], np.unique(lab[at], return_counts=True)[1])
     finally:
         fresh.close()
+
+
+# region lists into page-locked memory (one kernel), pageable memory (short ones staged, long
+# ones copied) and a mix of both: the same arrays, nothing written past the count
+@pytest.mark.parametrize("shape,step", [((6, 40, 70), 4), ((40, 300, 1200), 3)])
+def test_region_lists_in_any_host_memory(hd, shape, step):
+    import torch
+    from hdog import _capi as C
+    pd = np.zeros(shape, np.uint8)
+    pd[::step, ::step, 1::step] = 1
+    rng = np.random.default_rng(31)
+    g = hd.RegionalFeatures(hd.CCL(pd), rng.standard_normal((6,) + shape).astype(np.float32),
+                            rng.standard_normal(shape).astype(np.float32), noise(shape, 1))
+    n = len(g["label"])
+    fields = (("label", torch.int32, "label"), ("size", torch.int16, "size16"),
+              ("voxels", torch.int64, "count"), ("centroid_x", torch.float32, "cx"),
+              ("structureness", torch.float32, "structureness"),
+              ("intensity_sum", torch.int64, "isum"), ("intensity_max", torch.int16, "imax"))
+    for kind in ("locked", "mixed", "odd"):
+        reg = C.Regions()
+        reg.capacity = n + 5
+        held = []
+        for k, (field, dt, _) in enumerate(fields):
+            pin = kind != "mixed" or k % 2 == 0
+            size = torch.empty(0, dtype=dt).element_size()
+            skip = 1 if kind == "odd" else 0  # elements past the start: every alignment
+            a = torch.full((n + 5 + skip,), 7, dtype=dt, pin_memory=pin)
+            held.append(a[skip:])
+            setattr(reg, field, a.data_ptr() + skip * size)
+        hd._check(C.hdog_regions_download(hd._h, hd._stream(), C.ctypes.byref(reg)))
+        assert reg.count == n
+        for a, (_, _, key) in zip(held, fields):
+            np.testing.assert_array_equal(a[:n].numpy().view(g[key].dtype), g[key], err_msg=key)
+            assert (a[n:] == 7).all()
