@@ -420,36 +420,47 @@ __global__ __launch_bounds__(NT) void k_gauss_walk(const float2* __restrict__ sr
   const int xw = __builtin_amdgcn_readfirstlane(x - lane);  // the wave's first column
   const i64 bw = (i64)la.other * so + xw;
   const int nrec = min(64, W - xw) * (int)sizeof(float2);
-  auto at = [&](int p) -> float2 {
-    const float2* line = src + bw + (i64)p * sa;
+  auto load = [&](const float2* line, bool in) -> float2 {
     const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<float2*>(line), 0, (p >= 0 && p < L) ? nrec : 0, kBufferWord3);
+        const_cast<float2*>(line), 0, in ? nrec : 0, kBufferWord3);
     return __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(
                                           r, lane * (int)sizeof(float2), 0, 0));
   };
   float2 ring[WB];  // position p lives in ring[(p - b0 + R) % WB]
 #pragma unroll
-  for (int q = 0; q < WB; ++q) ring[q] = at(b0 + q - R);
+  for (int q = 0; q < WB; ++q) {
+    const int p = b0 - R + q;
+    ring[q] = load(src + bw + (i64)p * sa, (unsigned)p < (unsigned)L);
+  }
+  // the refills are read front to back: a pointer and the positions left on the line
+  const float2* line = src + bw + (i64)(b0 + R + 1) * sa;
+  int left = L - (b0 + R + 1);
+  auto refill = [&]() -> float2 {
+    const float2 v = load(line, left > 0);
+    line += sa;
+    --left;
+    return v;
+  };
   float2 pf[PF];  // the refill of step c (position c + R + 1) waits in slot (c - b0) % PF
 #pragma unroll
-  for (int j = 0; j < PF; ++j) pf[j] = at(b0 + R + 1 + j);
-  for (int c0 = b0;; c0 += WB) {
+  for (int j = 0; j < PF; ++j) pf[j] = refill();
+  i64 idx = base + (i64)b0 * sa;
+  for (int n = b1 - b0;; n -= WB) {  // outputs left
 #pragma unroll
     for (int q = 0; q < WB; ++q) {
-      const int c = c0 + q;
-      if (c >= b1) return;
+      if (q >= n) return;
       float s1 = 0.0f, s2 = 0.0f;
 #pragma unroll
       for (int j = -R1; j <= R1; ++j) s1 = fmaf(w1[R1 - j], ring[(q + j + R) % WB].x, s1);
 #pragma unroll
       for (int j = -R2; j <= R2; ++j) s2 = fmaf(w2[R2 - j], ring[(q + j + R) % WB].y, s2);
-      const i64 idx = base + (i64)c * sa;
       if (LAST)
         st_nt(dog + idx, (s1 - s2) * nz);
       else
         st_nt(dst + idx, make_float2(s1, s2));
+      idx += sa;
       ring[q] = pf[q % PF];  // position c + R + 1 replaces position c - R
-      pf[q % PF] = at(c + R + 1 + PF);
+      pf[q % PF] = refill();
     }
   }
 }
