@@ -241,6 +241,10 @@ int ensure_regions(hdog_ctx* ctx, i64 R) {
   HIPCHK(ensure(ctx->acc, (size_t)ctx->out_cap * sizeof(RegionAcc)));
   return HDOG_OK;
 }
+// sxy^2 sz of the narrow Gaussian (launch_region_accum_cand)
+float blob_volume(const hdog_ctx* ctx) {
+  return ctx->sigma[0] * ctx->sigma[0] * ctx->sigma[1];
+}
 // regions that both hold now (a batch plan may have taken the accumulators' memory)
 i64 region_capacity(const hdog_ctx* ctx) {
   return std::min<i64>(ctx->out_cap, (i64)(ctx->acc.bytes / sizeof(RegionAcc)));
@@ -351,7 +355,7 @@ int regional_features_t(hdog_ctx* ctx, hipStream_t s, uint32_t* labels, const TH
     if (cap > 0) {
       if (cand.rec)
         HIPCHK(launch_region_accum_cand<TN>(cand.rec, cand.cnt, cand.ntiles, cand.rlab, cand.multi,
-                                            rid, norm, img, acc, cap, W, H, is_ave, s));
+                                            rid, norm, img, acc, cap, W, H, is_ave, blob_volume(ctx), s));
       else
         HIPCHK(launch_region_accum<TH, TN>(labels, rid, hess, norm, img, acc, cap, W, H, D, is_ave,
                                            s));
@@ -586,7 +590,8 @@ hipError_t batch_tile(hdog_ctx* ctx, BatchState* B, BatchLane& L, int t, hipStre
                                         ntiles, (const uint32_t*)L.cand_lab.p,
                                         (const unsigned long long*)L.rmulti.p,
                                         (const uint32_t*)L.rid.p, norm, T.image,
-                                        acc, L.acc_cap, W, H, p->is_ave_mode, s)) != hipSuccess)
+                                        acc, L.acc_cap, W, H, p->is_ave_mode, blob_volume(ctx),
+                                        s)) != hipSuccess)
     return e;
   const i64 cap = B->arena_cap;
   RegionOut o;

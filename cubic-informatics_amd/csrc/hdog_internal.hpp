@@ -368,12 +368,13 @@ hipError_t launch_region_accum(const uint32_t* labels, const uint32_t* rid, cons
 // Region sums from the candidate records of launch_hessian (ntiles = hessian_tiles()).
 // rlab and multi come from launch_ccl_candidates: each record's root, and the roots of
 // regions reaching beyond one work-group's tiles (all others are summed by one work-group
-// and stored without atomics).
+// and stored without atomics).  blob: sxy^2 sz of the narrow Gaussian, which sets how many
+// regions to expect.
 template <typename TN>
 hipError_t launch_region_accum_cand(const float* cand, const uint32_t* cand_cnt, i64 ntiles,
                                     const uint32_t* rlab, const unsigned long long* multi,
                                     const uint32_t* rid, const TN* norm, const uint16_t* img,
-                                    RegionAcc* acc, i64 cap, int W, int H, int is_ave,
+                                    RegionAcc* acc, i64 cap, int W, int H, int is_ave, float blob,
                                     hipStream_t s);
 struct RegionOut {
   uint32_t* label; uint16_t* size; u64* voxels; float* cx; float* cy; float* cz;

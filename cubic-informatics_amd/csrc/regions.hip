@@ -184,15 +184,15 @@ struct RunSums {
   double h[6], ns;
 };
 
-__device__ __forceinline__ void flush_global(RegionAcc* a, const RunSums& v, int is_ave,
-                                             bool has_img) {
+template <bool AVE>
+__device__ __forceinline__ void flush_global(RegionAcc* a, const RunSums& v, bool has_img) {
   atomicAdd(&a->cnt, v.cnt);
   atomicAdd(&a->sx, v.sx);
   atomicAdd(&a->sy, v.sy);
   atomicAdd(&a->sz, v.sz);
 #pragma unroll
   for (int k = 0; k < 6; ++k) unsafeAtomicAdd(&a->h[k], v.h[k]);
-  if (is_ave)
+  if (AVE)
     unsafeAtomicAdd(&a->nsum, v.ns);
   else
     atomicMax(&a->nmax_key, v.nkey);
@@ -220,25 +220,29 @@ __device__ __forceinline__ void store_final(RegionAcc* a, const RunSums& v) {
 // Per-work-group hash table in LDS keyed by region id (open addressing, LDS atomics, FP64
 // for the Hessian and normalized sums).  Each occupied slot ends as one set of global
 // atomics, so a region pays one set per work-group that touches it instead of one per
-// voxel; a voxel that finds the table full goes straight to the global atomics.  A slot
-// whose region the caller marks `owned` (no other work-group holds any of its voxels) is
-// stored instead, unless some voxel of the work-group found the table full.
+// voxel; a region that finds no slot in kProbes tries goes straight to the global atomics.  A
+// slot whose region the caller marks `owned` (no other work-group holds any of its voxels) is
+// stored instead.  (Slots are never freed, so a region that once found its kProbes slots taken
+// always does: all its voxels are in the table or none.)
 // Coordinates are summed relative to the work-group's origin (ox, oy, oz), with the count
 // and the x and y sums packed in one 64-bit word (count: bits 0-15, x: 16-39, y: 40-63)
 // and the z sums with the raw intensity sums in another (z: bits 0-23, intensity: 24-63):
 // two LDS atomics instead of five.  For the < 2^16 voxels of a work-group whose offsets
 // stay below 256 in x, y and z the fields cannot carry into each other.
-template <int S>
+// AVE: the normalized value's sum in place of its maximum.
+template <int S, bool AVE>
 struct LdsTable {
+  static constexpr int kProbes = S < 32 ? S : 32;
+  static constexpr uint32_t kOwn = 1u << 16;
   uint32_t key[S];
   unsigned long long cxy[S], zis[S];
-  uint32_t im[S], nk[S], own[S];
-  double h[6][S], ns[S];
-  uint32_t spilled, ox, oy, oz;
+  uint32_t im[S];  // maximum raw intensity; kOwn: an owned region
+  typename std::conditional<AVE, double, uint32_t>::type nv[S];  // sum, or maximum key
+  double h[6][S];
+  uint32_t ox, oy, oz;
 
   __device__ void init(uint32_t x0, uint32_t y0, uint32_t z0) {
     if (threadIdx.x == 0) {
-      spilled = 0u;
       ox = x0;
       oy = y0;
       oz = z0;
@@ -246,10 +250,10 @@ struct LdsTable {
     for (int t = threadIdx.x; t < S; t += blockDim.x) {
       key[t] = EMPTY;
       cxy[t] = zis[t] = 0ull;
-      im[t] = nk[t] = own[t] = 0u;
+      im[t] = 0u;
+      nv[t] = 0;
 #pragma unroll
       for (int k = 0; k < 6; ++k) h[k][t] = 0.0;
-      ns[t] = 0.0;
     }
   }
 
@@ -260,11 +264,10 @@ struct LdsTable {
     double ns, h[6];
   };
 
-  __device__ void add_part(RegionAcc* acc, uint32_t r, const Part& q, int is_ave, bool has_img,
-                           bool owned) {
+  __device__ void add_part(RegionAcc* acc, uint32_t r, const Part& q, bool has_img, bool owned) {
     uint32_t slot = (r * 2654435761u) >> (32 - __builtin_ctz(S));
     bool placed = false;
-    for (int probes = 0; probes < S; ++probes) {
+    for (int probes = 0; probes < kProbes; ++probes) {
       // a key, once set, never changes: a plain read finds the region's slot, and only an
       // empty slot needs the compare-and-swap
       uint32_t k0 = __atomic_load_n(&key[slot], __ATOMIC_RELAXED);
@@ -284,24 +287,23 @@ struct LdsTable {
       v.ns = q.ns;
 #pragma unroll
       for (int k = 0; k < 6; ++k) v.h[k] = q.h[k];
-      flush_global(acc + r, v, is_ave, has_img);
-      spilled = 1u;
+      flush_global<AVE>(acc + r, v, has_img);
       return;
     }
-    if (owned) own[slot] = 1u;  // the same value from every voxel of the region
     atomicAdd(&cxy[slot], (unsigned long long)q.cnt | ((unsigned long long)q.dx << 16) |
                               ((unsigned long long)q.dy << 40));
     atomicAdd(&zis[slot], (unsigned long long)q.dz | ((unsigned long long)q.isum << 24));
 #pragma unroll
     for (int k = 0; k < 6; ++k) unsafeAtomicAdd(&h[k][slot], q.h[k]);
-    if (is_ave)
-      unsafeAtomicAdd(&ns[slot], q.ns);
+    if constexpr (AVE)
+      unsafeAtomicAdd(&nv[slot], q.ns);
     else
-      atomicMax(&nk[slot], q.nkey);
-    if (has_img) atomicMax(&im[slot], q.imax);
+      atomicMax(&nv[slot], q.nkey);
+    // (owned is the same for every voxel of a region)
+    atomicMax(&im[slot], q.imax | (owned ? kOwn : 0u));
   }
 
-  __device__ void flush(RegionAcc* acc, int is_ave, bool has_img) {
+  __device__ void flush(RegionAcc* acc, bool has_img) {
     for (int t = threadIdx.x; t < S; t += blockDim.x) {
       const uint32_t rr = key[t];
       if (rr == EMPTY) continue;
@@ -313,13 +315,19 @@ struct LdsTable {
       const unsigned long long q = zis[t];
       v.sz = (q & 0xFFFFFFull) + (unsigned long long)v.cnt * oz;
       v.isum = q >> 24;
-      v.imax = im[t]; v.nkey = nk[t]; v.ns = ns[t];
+      v.imax = im[t] & (kOwn - 1u);
+      v.nkey = 0u;
+      v.ns = 0.0;
+      if constexpr (AVE)
+        v.ns = nv[t];
+      else
+        v.nkey = nv[t];
 #pragma unroll
       for (int k = 0; k < 6; ++k) v.h[k] = h[k][t];
-      if (own[t] && !spilled)
+      if (im[t] & kOwn)
         store_final(acc + rr, v);
       else
-        flush_global(acc + rr, v, is_ave, has_img);
+        flush_global<AVE>(acc + rr, v, has_img);
     }
   }
 };
@@ -335,11 +343,11 @@ __device__ __forceinline__ uint32_t lane_prev(uint32_t v) {
 
 // Adds one voxel per lane (those with ok) to the table; the whole wave calls it together.
 // hv: the six elements, nv: the normalized value, iv: the raw intensity.
-template <int S>
-__device__ __forceinline__ void fold_wave(LdsTable<S>& tab, RegionAcc* acc, uint32_t cap, bool ok,
+template <int S, bool AVE>
+__device__ __forceinline__ void fold_wave(LdsTable<S, AVE>& tab, RegionAcc* acc, uint32_t cap, bool ok,
                                           bool owned, uint32_t r, uint32_t x, uint32_t y,
                                           uint32_t z, const float* hv, float nv, uint32_t iv,
-                                          int is_ave, bool has_img) {
+                                          bool has_img) {
   const int lane = (int)(threadIdx.x & 63);
   // Consecutive records are mostly x-neighbours in one row of one region.  Runs of
   // lanes with the same region are cut into groups of at most four; the first lane of
@@ -355,14 +363,14 @@ __device__ __forceinline__ void fold_wave(LdsTable<S>& tab, RegionAcc* acc, uint
   const unsigned long long later = heads & ~upto;
   const int next = later ? __builtin_ctzll(later) : 64;  // first lane of the next run
   const int last = min(next - 1, lane + 3);  // last lane of a group that starts here
-  typename LdsTable<S>::Part g;
+  typename LdsTable<S, AVE>::Part g;
   g.cnt = 1u;
   g.dx = x - tab.ox;
   g.dy = y - tab.oy;
   g.dz = z - tab.oz;
   g.isum = g.imax = iv;
-  g.nkey = is_ave ? 0u : fkey(nv);
-  g.ns = is_ave ? (double)nv : 0.0;
+  g.nkey = AVE ? 0u : fkey(nv);
+  g.ns = AVE ? (double)nv : 0.0;
 #pragma unroll
   for (int k = 0; k < 6; ++k) g.h[k] = (double)hv[k];
   // the values of lanes +1, +2, +3 arrive by one-lane shifts; those past `last` are
@@ -377,7 +385,7 @@ __device__ __forceinline__ void fold_wave(LdsTable<S>& tab, RegionAcc* acc, uint
     sdy = lane_next(sdy);
     sdz = lane_next(sdz);
     siv = lane_next(siv);
-    if (is_ave)
+    if (AVE)
       snv = __uint_as_float(lane_next(__float_as_uint(snv)));
     else
       snk = lane_next(snk);
@@ -390,7 +398,7 @@ __device__ __forceinline__ void fold_wave(LdsTable<S>& tab, RegionAcc* acc, uint
       g.dz += sdz;
       g.isum += siv;
       g.imax = max(g.imax, siv);
-      if (is_ave)
+      if (AVE)
         g.ns += (double)snv;
       else
         g.nkey = max(g.nkey, snk);
@@ -399,7 +407,7 @@ __device__ __forceinline__ void fold_wave(LdsTable<S>& tab, RegionAcc* acc, uint
     }
   }
   const bool head = ((lane - start) & 3) == 0;
-  if (ok && head && r < cap) tab.add_part(acc, r, g, is_ave, has_img, owned);
+  if (ok && head && r < cap) tab.add_part(acc, r, g, has_img, owned);
 }
 
 // Region sums from the materialized Hessian (the per-stage interface).  A work-group takes
@@ -410,17 +418,17 @@ __device__ __forceinline__ void fold_wave(LdsTable<S>& tab, RegionAcc* acc, uint
 // labelled voxels.  Voxel by voxel without the list, on 64 x 4 x 4 bricks, a wave of 64
 // voxels folded about four, with one set of table atomics each and three bricks' global
 // atomics per region: 783 us for 48 x 1080 x 1280 with 6 % labelled, 296 us with the list.
-template <typename TH, typename TN>
+template <typename TH, typename TN, bool AVE>
 __global__ __launch_bounds__(NT) void k_accum(const uint32_t* __restrict__ L,
                                               const uint32_t* __restrict__ rid,
                                               const TH* __restrict__ hess,
                                               const TN* __restrict__ norm,
                                               const uint16_t* __restrict__ img, RegionAcc* acc,
                                               uint32_t cap, int W, int H, int D, i64 N, int nbx,
-                                              int nby, int is_ave) {
+                                              int nby) {
   constexpr int ROWS = kHessTY * kHessTZ, NWV = NT / 64, PF = 8;  // rows, waves, loads in flight
   static_assert(ROWS % (NWV * PF) == 0 && kCandTile <= 65536, "whole batches of rows");
-  __shared__ LdsTable<128> tab;
+  __shared__ LdsTable<128, AVE> tab;
   __shared__ uint16_t list[kCandTile];
   __shared__ uint32_t n_list;
   unsigned b = xcd_tile(blockIdx.x, gridDim.x);
@@ -472,10 +480,10 @@ __global__ __launch_bounds__(NT) void k_accum(const uint32_t* __restrict__ L,
       iv = has_img ? (uint32_t)img[i] : 0u;
       r = rid[L[i]];
     }
-    fold_wave(tab, acc, cap, ok, false, r, x, y, z, hv, nv, iv, is_ave, has_img);
+    fold_wave(tab, acc, cap, ok, false, r, x, y, z, hv, nv, iv, has_img);
   }
   __syncthreads();
-  tab.flush(acc, is_ave, has_img);
+  tab.flush(acc, has_img);
 }
 
 // Region sums from the candidate records of the Hessian kernel: one work-group per
@@ -485,7 +493,8 @@ __global__ __launch_bounds__(NT) void k_accum(const uint32_t* __restrict__ L,
 static_assert(kAccGY * kAccGZ * kCandTile < (1 << 16) && kHessTX <= 256 &&
                   kAccGY * kHessTY <= 256 && kAccGZ * kHessTZ <= 256,
               "packed table sums: count below 2^16, offsets below 256");
-template <typename TN>
+// S: table slots.
+template <typename TN, bool AVE, int S>
 __global__ __launch_bounds__(NT) void k_accum_cand(const float* __restrict__ cand,
                                                    const uint32_t* __restrict__ cand_cnt,
                                                    const uint32_t* __restrict__ rlab,
@@ -494,8 +503,8 @@ __global__ __launch_bounds__(NT) void k_accum_cand(const float* __restrict__ can
                                                    const TN* __restrict__ norm,
                                                    const uint16_t* __restrict__ img,
                                                    RegionAcc* acc, uint32_t cap, uint32_t W,
-                                                   uint32_t WH, int is_ave, unsigned nbx,
-                                                   unsigned nby, unsigned nbz) {
+                                                   uint32_t WH, unsigned nbx, unsigned nby,
+                                                   unsigned nbz) {
   // work-group p takes the tiles (bx, kAccGY gy + a, kAccGZ gz + b) of the Hessian tiling;
   // a region within them is final here, others pay one set of global atomics
   constexpr int TPW = kAccGY * kAccGZ;
@@ -516,7 +525,7 @@ __global__ __launch_bounds__(NT) void k_accum_cand(const float* __restrict__ can
     any |= n[q];
   }
   if (any == 0) return;  // uniform over the work-group
-  __shared__ LdsTable<256> tab;
+  __shared__ LdsTable<S, AVE> tab;
   tab.init(bx * kHessTX, gy * kAccGY * kHessTY, gz * kAccGZ * kHessTZ);
   const bool has_img = img != nullptr;
   __syncthreads();
@@ -549,11 +558,11 @@ __global__ __launch_bounds__(NT) void k_accum_cand(const float* __restrict__ can
         nv = ld(norm, (i64)idx);
         iv = has_img ? (uint32_t)img[idx] : 0u;
       }
-      fold_wave(tab, acc, cap, ok, owned, r, x, y, z, hv, nv, iv, is_ave, has_img);
+      fold_wave(tab, acc, cap, ok, owned, r, x, y, z, hv, nv, iv, has_img);
     }
   }
   __syncthreads();
-  tab.flush(acc, is_ave, has_img);
+  tab.flush(acc, has_img);
 }
 
 // src/3D/Eigenvalues.cu:32-94 (Eberly's closed form, FP64)
@@ -734,9 +743,15 @@ hipError_t launch_region_accum(const uint32_t* labels, const uint32_t* rid, cons
   const int nbx = (W + kHessTX - 1) / kHessTX, nby = (H + kHessTY - 1) / kHessTY;
   const i64 nblk = hessian_tiles(W, H, D);
   const i64 N = (i64)W * H * D;
-  hipLaunchKernelGGL((k_accum<TH, TN>), dim3((unsigned)nblk), dim3(NT), 0, s, labels, rid, hess,
-                     norm, img, acc, (uint32_t)std::min<i64>(cap, 0xFFFFFFFFll), W, H, D, N, nbx,
-                     nby, is_ave);
+  auto go = [&](auto ave) {
+    hipLaunchKernelGGL((k_accum<TH, TN, decltype(ave)::value>), dim3((unsigned)nblk), dim3(NT), 0, s,
+                       labels, rid, hess, norm, img, acc,
+                       (uint32_t)std::min<i64>(cap, 0xFFFFFFFFll), W, H, D, N, nbx, nby);
+  };
+  if (is_ave)
+    go(std::true_type{});
+  else
+    go(std::false_type{});
   mark("regions/accum", s);
   return hipGetLastError();
 }
@@ -745,16 +760,31 @@ template <typename TN>
 hipError_t launch_region_accum_cand(const float* cand, const uint32_t* cand_cnt, i64 ntiles,
                                     const uint32_t* rlab, const unsigned long long* multi,
                                     const uint32_t* rid, const TN* norm, const uint16_t* img,
-                                    RegionAcc* acc, i64 cap, int W, int H, int is_ave,
+                                    RegionAcc* acc, i64 cap, int W, int H, int is_ave, float blob,
                                     hipStream_t s) {
   const unsigned nbx = (unsigned)((W + kHessTX - 1) / kHessTX),
                  nby = (unsigned)((H + kHessTY - 1) / kHessTY);
   const unsigned nbz = (unsigned)(ntiles / ((i64)nbx * nby));
   const i64 ngroups =
       (i64)nbx * ((nby + kAccGY - 1) / kAccGY) * ((nbz + kAccGZ - 1) / kAccGZ);
-  hipLaunchKernelGGL((k_accum_cand<TN>), dim3((unsigned)ngroups), dim3(NT), 0, s, cand, cand_cnt,
-                     rlab, multi, rid, norm, img, acc, (uint32_t)std::min<i64>(cap, 0xFFFFFFFFll),
-                     (uint32_t)W, (uint32_t)((i64)W * H), is_ave, nbx, nby, nbz);
+  // Noise and blobs give a region per about 70 sxy^2 sz voxels of the narrow Gaussian, so a
+  // work-group's 32768 voxels hold 470 / (sxy^2 sz) regions.  256 slots leave room for twice
+  // the waves: 2111 us for 256 x 2160 x 2560 at 74 regions, 2225 with 512 slots.  Past about
+  // 150 they fill up and regions pay global atomics per voxel: 61 x 900 x 1111 at 270 regions
+  // takes 362 us with 256 slots, 222 with 512.
+  const bool many = blob < 3.2f;
+  auto go = [&](auto ave, auto slots) {
+    hipLaunchKernelGGL((k_accum_cand<TN, decltype(ave)::value, decltype(slots)::value>),
+                       dim3((unsigned)ngroups), dim3(NT), 0, s, cand, cand_cnt, rlab, multi, rid,
+                       norm, img, acc, (uint32_t)std::min<i64>(cap, 0xFFFFFFFFll), (uint32_t)W,
+                       (uint32_t)((i64)W * H), nbx, nby, nbz);
+  };
+  using S256 = std::integral_constant<int, 256>;
+  using S512 = std::integral_constant<int, 512>;
+  if (is_ave)
+    many ? go(std::true_type{}, S512{}) : go(std::true_type{}, S256{});
+  else
+    many ? go(std::false_type{}, S512{}) : go(std::false_type{}, S256{});
   mark("regions/accum_candidates", s);
   return hipGetLastError();
 }
@@ -770,7 +800,8 @@ HDOG_INST_ACC(__hip_bfloat16, __hip_bfloat16)
 #define HDOG_INST_ACCC(TN)                                                                  \
   template hipError_t launch_region_accum_cand<TN>(                                         \
       const float*, const uint32_t*, i64, const uint32_t*, const unsigned long long*,         \
-      const uint32_t*, const TN*, const uint16_t*, RegionAcc*, i64, int, int, int, hipStream_t);
+      const uint32_t*, const TN*, const uint16_t*, RegionAcc*, i64, int, int, int, float,     \
+      hipStream_t);
 HDOG_INST_ACCC(float)
 HDOG_INST_ACCC(__half)
 HDOG_INST_ACCC(__hip_bfloat16)

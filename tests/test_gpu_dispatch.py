@@ -196,3 +196,26 @@ def test_region_lists_in_any_host_memory(hd, shape, step):
         for a, (_, _, key) in zip(held, fields):
             np.testing.assert_array_equal(a[:n].numpy().view(g[key].dtype), g[key], err_msg=key)
             assert (a[n:] == 7).all()
+
+
+# region sums of noise with narrow Gaussians: more regions per work-group than its table holds
+# (512 slots below sxy^2 sz = 3.2, 256 above), maximum and sum, against the materialized path
+@pytest.mark.parametrize("sigmas", [(0.9, 0.7, 1.5, 1.2), (1.6, 1.25, 2.6, 2.0)])
+@pytest.mark.parametrize("ave", [False, True])
+def test_region_sums_beyond_the_table(hd, sigmas, ave):
+    shape = (35, 70, 150)
+    img = hd._dev(noise(shape, 12), __import__("torch").uint16)
+    p = hd.make_params(shape, 3, 3, 0, *sigmas, truncate=3.0, is_ave_mode=ave)
+    bufs = hd.alloc_intermediates(shape)
+    hd.run_device(img, p, bufs)
+    want = hd.RegionalFeatures(bufs["labels"], bufs["hess"], bufs["norm"], img, ave)
+    hd.run_device(img, p)
+    got = hd.download_regions()
+    for k in ("label", "count", "isum", "imax", "centroid"):
+        np.testing.assert_array_equal(got[k], want[k], err_msg=k)
+    # FP64 sums in another order, rounded once to FP32
+    n = want["count"][:, None].astype(np.float64)
+    big = max(float(bufs["hess"].abs().max()), float(bufs["norm"].abs().max()))
+    for k in ("hsum", "norm"):
+        a, b = (x[k].astype(np.float64).reshape(len(n), -1) for x in (got, want))
+        assert np.all(np.abs(a - b) <= 1.2e-7 * np.abs(b) + 1e-12 * n * big), k
