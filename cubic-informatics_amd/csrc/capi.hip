@@ -58,11 +58,11 @@ struct BatchState {
 struct hdog_ctx {
   int device = 0;
   std::string err;
-  Buf tmp1, tmp2, rid, bcnt, rmask, rmulti, dR, acc, weights, blobs, sw, sums, ddog, cand,
+  Buf tmp1, tmp2, rid, bcnt, rmask, rmulti, dR, acc, weights, blobs, sw, sums, ddog, rows, cand,
       cand_cnt, fgbits, cand_lab;
   Buf o_label, o_size, o_vox, o_cen, o_eig, o_nrm, o_hess, o_isum, o_imax;
   i64 out_cap = 0;
-  Buf img, norm, dog, hess, pd, labels;  // substack buffers of hdog_process_substack
+  Buf img, norm, dog, labels;  // substack buffers of hdog_process_substack
   bool gauss_ready = false;
   float sigma[4] = {0, 0, 0, 0};
   double truncate = 0.0;
@@ -760,10 +760,10 @@ int hdog_release_scratch(hdog_ctx* ctx) {
   (void)hipSetDevice(ctx->device);
   for (Buf* b : {&ctx->tmp1, &ctx->tmp2, &ctx->rid, &ctx->bcnt, &ctx->rmask, &ctx->rmulti, &ctx->dR, &ctx->acc,
                  &ctx->blobs, &ctx->cand_lab, &ctx->fgbits,
-                 &ctx->sw, &ctx->sums, &ctx->ddog,
+                 &ctx->sw, &ctx->sums, &ctx->ddog, &ctx->rows,
                  &ctx->o_label, &ctx->o_size, &ctx->o_vox, &ctx->o_cen, &ctx->o_eig, &ctx->o_nrm,
                  &ctx->o_hess, &ctx->o_isum, &ctx->o_imax, &ctx->img, &ctx->norm, &ctx->dog,
-                 &ctx->hess, &ctx->pd, &ctx->labels, &ctx->cand, &ctx->cand_cnt})
+                 &ctx->labels, &ctx->cand, &ctx->cand_cnt})
     release(*b);
   ctx->out_cap = 0;
   ctx->R = 0;
@@ -1188,13 +1188,16 @@ int hdog_soft_forward(hdog_ctx* ctx, void* stream, const float* d_v, const uint8
   const i64 N = (i64)width * height * depth;
   HIPCHK(ensure(ctx->tmp1, (size_t)N * 8));
   HIPCHK(ensure(ctx->tmp2, (size_t)N * 8));
-  HIPCHK(ensure(ctx->hess, (size_t)N * 24));
+  const i64 ntiles = hessian_tiles(width, height, depth);
+  HIPCHK(ensure(ctx->cand, (size_t)ntiles * kCandTile * 7 * 4));
+  HIPCHK(ensure(ctx->cand_cnt, (size_t)ntiles * 4));
   HIPCHK(ensure(ctx->sums, 64 * 8));
   HIPCHK(launch_gauss_pair(d_v, ctx->tmp1.p, ctx->tmp2.p, S.w, S.r, (float)S.s, d_dog, nullptr,
                            width, height, depth, s));
-  HIPCHK(launch_hessian<float, float>(d_dog, (float*)ctx->hess.p, d_mask, width, height, depth, s));
-  HIPCHK(launch_soft_loss((const float*)ctx->hess.p, d_mask, d_target, N, 1.0 / tau,
-                          (double*)ctx->sums.p, s));
+  HIPCHK(launch_hessian_records(d_dog, d_mask, nullptr, width, height, depth, (float*)ctx->cand.p,
+                                (uint32_t*)ctx->cand_cnt.p, s));
+  HIPCHK(launch_soft_loss((const float*)ctx->cand.p, (const uint32_t*)ctx->cand_cnt.p, d_target,
+                          width, height, depth, 1.0 / tau, (double*)ctx->sums.p, s));
   double h[2];
   HIPCHK(hipMemcpyAsync(h, ctx->sums.p, 16, hipMemcpyDeviceToHost, s));
   HIPCHK(hipStreamSynchronize(s));
@@ -1221,25 +1224,30 @@ int hdog_soft_backward(hdog_ctx* ctx, void* stream, const float* d_v, const floa
   const i64 N = (i64)width * height * depth;
   HIPCHK(ensure(ctx->tmp1, (size_t)N * 8));
   HIPCHK(ensure(ctx->tmp2, (size_t)N * 8));
-  HIPCHK(ensure(ctx->hess, (size_t)N * 24));
+  const i64 ntiles = hessian_tiles(width, height, depth);
+  HIPCHK(ensure(ctx->cand, (size_t)ntiles * kCandTile * 7 * 4));
+  HIPCHK(ensure(ctx->cand_cnt, (size_t)ntiles * 4));
   HIPCHK(ensure(ctx->ddog, (size_t)N * 4));
-  HIPCHK(ensure(ctx->pd, (size_t)N));
   HIPCHK(ensure(ctx->sums, 64 * 8));
   double* sums = (double*)ctx->sums.p;
-  float* gh = (float*)ctx->hess.p;
+  float* cand = (float*)ctx->cand.p;
+  uint32_t* cnt = (uint32_t*)ctx->cand_cnt.p;
   float* ddog = (float*)ctx->ddog.p;
+  HIPCHK(ensure(ctx->rows, (size_t)fg_words(width, height, depth) * sizeof(TileRow)));
+  TileRow* rows = (TileRow*)ctx->rows.p;
+  HIPCHK(launch_zero_f64(sums, 8, s));
   // H is recomputed from the checkpointed DoG; the mask from the forward pass is used
-  HIPCHK(launch_hessian<float, float>(d_dog, gh, (uint8_t*)ctx->pd.p, width, height, depth, s));
+  HIPCHK(launch_hessian_records(d_dog, const_cast<uint8_t*>(d_mask), rows, width, height, depth,
+                                cand, cnt, s));
   const double inv_count = count > 0 ? grad_out / (double)count : 0.0;
-  HIPCHK(launch_soft_grad_h(gh, d_mask, d_target, N, 1.0 / tau, inv_count, sums, s));
-  // P_x, P_y, P_z (3N floats) in tmp1, grown to 12 bytes per voxel
-  HIPCHK(ensure(ctx->tmp1, (size_t)N * 12));
-  HIPCHK(launch_hessian_adjoint(gh, (float*)ctx->tmp1.p, ddog, width, height, depth, s));
+  HIPCHK(launch_soft_grad_h(cand, cnt, d_target, width, height, depth, 1.0 / tau, inv_count, sums,
+                            s));
+  // dL/ddog, and <dL/ddog, dog>
+  HIPCHK(launch_hessian_adjoint(cand, rows, d_dog, ddog, width, height, depth, sums + 1, s));
   // dL/dv = s (G1 - G2) dL/ddog
   HIPCHK(launch_gauss_pair(ddog, ctx->tmp1.p, ctx->tmp2.p, S.w, S.r, (float)S.s, d_grad_v, nullptr,
                            width, height, depth, s));
   double h[16];
-  HIPCHK(launch_dot(ddog, d_dog, N, sums + 1, s));  // <dL/ddog, dog>
   for (int a = 0; a < 3; ++a) {
     const float* w[6] = {S.w[0], S.w[1], S.w[2], S.w[3], S.w[4], S.w[5]};
     w[a] = S.dw[a];
@@ -1392,7 +1400,7 @@ int hdog_batch_plan(hdog_ctx* ctx, const hdog_params* p, const hdog_tile* tiles,
       // call's region arrays stay) may hold the memory, e.g. after the tuner ran
       for (Buf* w : {&ctx->tmp1, &ctx->tmp2, &ctx->rid, &ctx->bcnt, &ctx->rmask, &ctx->rmulti,
                      &ctx->dR, &ctx->acc, &ctx->cand_lab, &ctx->fgbits, &ctx->img, &ctx->norm,
-                     &ctx->dog, &ctx->hess, &ctx->pd, &ctx->labels, &ctx->cand, &ctx->cand_cnt})
+                     &ctx->dog, &ctx->labels, &ctx->cand, &ctx->cand_cnt})
         release(*w);
       (void)hipMemGetInfo(&free_b, &total_b);
       if ((double)need > 0.9 * (double)free_b) B->lanes = deal(1);

@@ -433,12 +433,27 @@ hipError_t launch_ccl_candidates(const float* cand, const uint32_t* cand_cnt, i6
 hipError_t launch_mask_records(const uint8_t* pd, float* pos, uint32_t* cand_cnt, int W, int H,
                                int D, hipStream_t s);
 // differentiable blob response (soft.hip)
-hipError_t launch_soft_loss(const float* hess, const uint8_t* mask, const uint8_t* target, i64 N,
-                            double inv_tau, double* sums, hipStream_t s);
-hipError_t launch_soft_grad_h(float* hess, const uint8_t* mask, const uint8_t* target, i64 N,
-                              double inv_tau, double inv_count, double* sums, hipStream_t s);
-hipError_t launch_hessian_adjoint(const float* gh, float* P, float* out, int W, int H, int D,
-                                  hipStream_t s);
+// One 64-voxel row of a Hessian tile (ly + kHessTY lz): its masked voxels, and where in the
+// tile's records theirs start (consecutive, in x order).
+struct TileRow {
+  unsigned long long bits;
+  unsigned long long first;
+};
+// The records of the masked voxels of a DoG volume, voxel 0 included, in the Hessian pass's
+// layout; the mask volume is written, or, with `rows` (one per tile row, written), decides.
+hipError_t launch_hessian_records(const float* dog, uint8_t* mask, TileRow* rows, int W, int H,
+                                  int D, float* cand, uint32_t* cand_cnt, hipStream_t s);
+// sums[0] = loss sum, sums[1] = |M| over the records
+hipError_t launch_soft_loss(const float* cand, const uint32_t* cand_cnt, const uint8_t* target,
+                            int W, int H, int D, double inv_tau, double* sums, hipStream_t s);
+// the records' elements become dL/dH; *sums += dL/dtau
+hipError_t launch_soft_grad_h(float* cand, const uint32_t* cand_cnt, const uint8_t* target, int W,
+                              int H, int D, double inv_tau, double inv_count, double* sums,
+                              hipStream_t s);
+// dL/ddog from those records; *dot += <dL/ddog, dog>
+hipError_t launch_hessian_adjoint(const float* cand, const TileRow* rows, const float* dog,
+                                  float* out, int W, int H, int D, double* dot, hipStream_t s);
+hipError_t launch_zero_f64(double* p, int n, hipStream_t s);
 // Differentiable form, local-contrast normalization of a float volume (clamped min / max
 // and box of radius (rxy, rxy, rz)): norm, the (E, D) pairs and the window argmin / argmax
 // (N each) for the backward pass; scratch 8 N words.
@@ -451,8 +466,8 @@ hipError_t launch_soft_normalize_adjoint(const float* v, const float2* ed, const
                                          const float* gn, float* gv, void* scratch,
                                          float min_int, int W, int H, int D, int rxy, int rz,
                                          hipStream_t s);
+// out[0] += <a, pair.x>, out[1] += <a, pair.y>
 hipError_t launch_dot_pair(const float* a, const float2* pair, i64 N, double* out, hipStream_t s);
-hipError_t launch_dot(const float* a, const float* b, i64 N, double* out, hipStream_t s);
 hipError_t launch_synth(uint16_t* img, float* scratch, int W, int H, int D, u64 seed,
                         double mean0, double mean1, double sd, const double* d_blobs,
                         i64 n_blobs, hipStream_t s);

@@ -379,11 +379,16 @@ __device__ __forceinline__ float swap_pairs(float v) {
   return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xf, 0xf, false));
 }
 
-template <typename TD, typename TS, bool BAND>
+// MODE: kDetect, or for the differentiable form, which keeps voxel 0 as any other,
+// kWriteMask (the mask volume is written too) or kGivenMask (the records of the voxels that
+// the mask volume holds, whatever their minors, and each tile row's bits and first record:
+// the records of a row are consecutive, in lane order).
+constexpr int kDetect = 0, kWriteMask = 1, kGivenMask = 2;
+template <typename TD, typename TS, bool BAND, int MODE>
 __global__ __launch_bounds__(64 * kRecWaves) void k_hessian_rec(
     const TD* __restrict__ dog, int W, int H, int D, int nbx, int nby, int nbyg, int nz,
-    float* __restrict__ cand,
-    uint32_t* __restrict__ cand_cnt, float band) {
+    float* __restrict__ cand, uint32_t* __restrict__ cand_cnt, float band,
+    uint8_t* __restrict__ mask, TileRow* __restrict__ rows) {
   constexpr int TY = kRecTY, NR = TY + 4, NH = TY + 2;  // dog rows, first-difference rows
   __shared__ uint32_t s_cnt[kRecTilesY][kRecNZ];
   if (threadIdx.x < kRecTilesY * kRecNZ) s_cnt[threadIdx.x / kRecNZ][threadIdx.x % kRecNZ] = 0u;
@@ -410,6 +415,7 @@ __global__ __launch_bounds__(64 * kRecWaves) void k_hessian_rec(
   using Bits = typename StoredBits<TD>::type;
   Bits qd[3][NR], qh[3][NH];  // slices in flight: dog rows, halo columns
   float Hx[3][NH], Hy[3][NH], Hz[3][TY], Hxx[3][TY];
+  uint8_t qm[TY];  // kGivenMask: the mask of the next step's outputs
   const uint32_t row_bytes = (uint32_t)W * SZ;
   // CLIP: some of the wave's dog rows lie outside the plane
   auto fetch = [&](int s, auto q_c, auto clip_c) {
@@ -460,7 +466,9 @@ __global__ __launch_bounds__(64 * kRecWaves) void k_hessian_rec(
         const float yz = (Hy[B][r + 1] - Hy[A][r + 1]) * 0.5f;
         const float zz = (Hz[B][r] - Hz[A][r]) * 0.5f;
         bool m;
-        if (BAND) {
+        if (MODE == kGivenMask) {
+          m = qm[r] != 0;
+        } else if (BAND) {
           m = negdef_band(xx, xy, xz, yy, yz, zz, band) != 0;
         } else {  // negdef32's minors, without branches
           const float m2 = xx * yy - xy * xy;
@@ -468,10 +476,13 @@ __global__ __launch_bounds__(64 * kRecWaves) void k_hessian_rec(
               xx * yy * zz + 2 * xy * yz * xz - xx * yz * yz - yy * xz * xz - zz * xy * xy;
           m = (xx < 0.0f) & (m2 > 0.0f) & (m3 < 0.0f);
         }
+        const bool in = (!EDGE || xin) && (!CLIP || y + r < H);
+        if (MODE == kWriteMask && in)
+          mask[(size_t)z * WH + (size_t)(y + r) * (size_t)W + (size_t)x] = m ? 1 : 0;
         // voxel 0 is background whatever its mask (its label is 0): no record (only an
         // EDGE and CLIP wave holds it)
-        const bool is_c = m && (!EDGE || xin) && (!CLIP || y + r < H) &&
-                          (!(EDGE && CLIP) || (x | (y + r) | z) != 0);
+        const bool is_c = m && in &&
+                          (MODE != kDetect || !(EDGE && CLIP) || (x | (y + r) | z) != 0);
         // one LDS reservation per wave and row, consecutive slots in lane order (ds_append
         // would do both in one instruction, but as compiled for this target it adds to the
         // counter at LDS address 0 whatever the address asked for)
@@ -479,6 +490,8 @@ __global__ __launch_bounds__(64 * kRecWaves) void k_hessian_rec(
         uint32_t base = 0;
         if (act && lane == 0) base = atomicAdd(&s_cnt[tt][tz], (uint32_t)__popcll(act));
         base = __builtin_amdgcn_readfirstlane(base);
+        if (MODE == kGivenMask && lane == 0 && by < nby)
+          rows[(size_t)tile * (kHessTY * kHessTZ) + (uint32_t)(ty0 + r) + kHessTY * lz] = {act, base};
         if (is_c) {
           const uint32_t slot = base + __builtin_amdgcn_mbcnt_hi(
                                            (uint32_t)(act >> 32),
@@ -535,6 +548,18 @@ __global__ __launch_bounds__(64 * kRecWaves) void k_hessian_rec(
       }
     }
     fetch(s + 2, std::integral_constant<int, B>(), clip_c);
+    if (MODE == kGivenMask) {
+      const int zm = s - 1;  // the next step's output slice
+      const bool zin = zm >= z0 && zm < z1;
+#pragma unroll
+      for (int r = 0; r < TY; ++r) {
+        const bool rin = zin && (!CLIP || y + r < H);
+        const __amdgpu_buffer_rsrc_t rm =
+            buf_rsrc(mask + (rin ? (size_t)zm * WH + (size_t)(y + r) * (size_t)W : 0),
+                     rin ? (uint32_t)W : 0u);
+        qm[r] = (uint8_t)__builtin_amdgcn_raw_buffer_load_b8(rm, x, 0, 0);
+      }
+    }
   };
   using I0 = std::integral_constant<int, 0>;
   using I1 = std::integral_constant<int, 1>;
@@ -600,14 +625,32 @@ hipError_t launch_hessian(const TD* dog, TH* hess, uint8_t* pd, int W, int H, in
     const int nbyg = (nby + kRecTilesY - 1) / kRecTilesY;
     const int nz = records_walk_tiles((i64)nbx * nbyg, nbz);
     const i64 ngroups = (i64)nbx * nbyg * ((nbz + nz - 1) / nz);
-    hipLaunchKernelGGL((k_hessian_rec<TD, TH, reduced>), dim3((unsigned)ngroups),
+    hipLaunchKernelGGL((k_hessian_rec<TD, TH, reduced, kDetect>), dim3((unsigned)ngroups),
                        dim3(64 * kRecWaves), 0, s, dog, W, H, D, nbx, nby, nbyg, nz, cand,
-                       cand_cnt, band);
+                       cand_cnt, band, (uint8_t*)nullptr, (TileRow*)nullptr);
   } else {
     hipLaunchKernelGGL((k_hessian<TD, TH, reduced>), dim3((unsigned)nblk), dim3(NT), 0, s, dog,
                        hess, pd, W, H, D, nbx, nby, cand, cand_cnt, band);
   }
   mark("hessian/hessian_pd", s);
+  return hipGetLastError();
+}
+
+// The records of the differentiable form: voxel 0 included; the mask volume is written, or,
+// with rows, decides.
+hipError_t launch_hessian_records(const float* dog, uint8_t* mask, TileRow* rows, int W, int H,
+                                  int D, float* cand, uint32_t* cand_cnt, hipStream_t s) {
+  const int nbx = (W + TX - 1) / TX, nby = (H + TY - 1) / TY, nbz = (D + ZC - 1) / ZC;
+  if ((i64)W * H * (i64)sizeof(float) >= 0xFFFFFFF0ll) return hipErrorInvalidValue;
+  const int nbyg = (nby + kRecTilesY - 1) / kRecTilesY;
+  const int nz = records_walk_tiles((i64)nbx * nbyg, nbz);
+  const dim3 grid((unsigned)((i64)nbx * nbyg * ((nbz + nz - 1) / nz)));
+  if (rows)
+    hipLaunchKernelGGL((k_hessian_rec<float, float, false, kGivenMask>), grid, dim3(64 * kRecWaves),
+                       0, s, dog, W, H, D, nbx, nby, nbyg, nz, cand, cand_cnt, 0.0f, mask, rows);
+  else
+    hipLaunchKernelGGL((k_hessian_rec<float, float, false, kWriteMask>), grid, dim3(64 * kRecWaves),
+                       0, s, dog, W, H, D, nbx, nby, nbyg, nz, cand, cand_cnt, 0.0f, mask, rows);
   return hipGetLastError();
 }
 

@@ -73,54 +73,233 @@ __device__ __forceinline__ double softplus(double u) {
   return u > 0 ? u + log1p(exp(-u)) : log1p(exp(u));
 }
 
+// The records of the masked voxels (launch_hessian_records): per Hessian tile a count and
+// the voxels' positions and six elements, so the FP64 work below runs on full waves and
+// touches nothing else.  A pass over the dense volumes and mask instead spent 282 us on the
+// loss and 326 on the gradient at 128 x 512 x 512 with 7 % masked (now 34 and 34).
+struct TileOf {
+  int x0, y0, z0;
+};
+__device__ __forceinline__ TileOf tile_of(unsigned tile, unsigned nbx, unsigned nby) {
+  const unsigned r = tile / nbx;
+  return {(int)(tile - r * nbx) * kHessTX, (int)(r % nby) * kHessTY, (int)(r / nby) * kHessTZ};
+}
+
 // sums[0] += sum over M of softplus(u) - t*u ; sums[1] += |M|
-__global__ __launch_bounds__(NT) void k_soft_loss(const float* __restrict__ hess,
-                                                  const uint8_t* __restrict__ mask,
-                                                  const uint8_t* __restrict__ target, i64 N,
-                                                  double inv_tau, double* sums) {
+__global__ __launch_bounds__(NT) void k_soft_loss(const float* __restrict__ cand,
+                                                  const uint32_t* __restrict__ cand_cnt,
+                                                  const uint8_t* __restrict__ target,
+                                                  unsigned ntiles, unsigned nbx, unsigned nby,
+                                                  int W, int H, double inv_tau, double* sums) {
   double ls = 0.0, cnt = 0.0;
-  for (i64 i = (i64)blockIdx.x * NT + threadIdx.x; i < N; i += (i64)gridDim.x * NT) {
-    if (!mask[i]) continue;
-    const double d = det3(hess[i], hess[N + i], hess[2 * N + i], hess[3 * N + i],
-                          hess[4 * N + i], hess[5 * N + i]);
-    const double u = -d * inv_tau;
-    ls += softplus(u) - (target[i] ? u : 0.0);
-    cnt += 1.0;
+  for (unsigned tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    const uint32_t n = cand_cnt[tile];
+    const float* rec = cand + (size_t)tile * kCandTile * 7;
+    const TileOf T = tile_of(tile, nbx, nby);
+    for (uint32_t i = threadIdx.x; i < n; i += NT) {
+      const uint32_t v = __float_as_uint(rec[i]);
+      const size_t at = ((size_t)(T.z0 + (int)(v / (kHessTX * kHessTY))) * H +
+                         (T.y0 + (int)(v / kHessTX % kHessTY))) * W + T.x0 + (int)(v % kHessTX);
+      float e[6];
+#pragma unroll
+      for (int k = 0; k < 6; ++k) e[k] = rec[(size_t)kCandTile * (1 + k) + i];
+      const double u = -det3(e[0], e[1], e[2], e[3], e[4], e[5]) * inv_tau;
+      ls += softplus(u) - (target[at] ? u : 0.0);
+      cnt += 1.0;
+    }
   }
   double a[2] = {ls, cnt};
   group_add<2>(a, sums);
 }
 
-// hess (6N) is overwritten by dL/dH; sums[0] += dL/dtau contributions
-__global__ __launch_bounds__(NT) void k_soft_grad_h(float* __restrict__ hess,
-                                                    const uint8_t* __restrict__ mask,
-                                                    const uint8_t* __restrict__ target, i64 N,
-                                                    double inv_tau, double inv_count,
-                                                    double* sums) {
+// the records' elements are overwritten by dL/dH; sums[0] += dL/dtau contributions
+__global__ __launch_bounds__(NT) void k_soft_grad_h(float* __restrict__ cand,
+                                                    const uint32_t* __restrict__ cand_cnt,
+                                                    const uint8_t* __restrict__ target,
+                                                    unsigned ntiles, unsigned nbx, unsigned nby,
+                                                    int W, int H, double inv_tau,
+                                                    double inv_count, double* sums) {
   double gt = 0.0;
-  for (i64 i = (i64)blockIdx.x * NT + threadIdx.x; i < N; i += (i64)gridDim.x * NT) {
-    if (!mask[i]) {
-#pragma unroll
-      for (int k = 0; k < 6; ++k) hess[k * N + i] = 0.0f;
-      continue;
+  for (unsigned tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    const uint32_t n = cand_cnt[tile];
+    float* rec = cand + (size_t)tile * kCandTile * 7;
+    const TileOf T = tile_of(tile, nbx, nby);
+    for (uint32_t i = threadIdx.x; i < n; i += NT) {
+      const uint32_t v = __float_as_uint(rec[i]);
+      const size_t at = ((size_t)(T.z0 + (int)(v / (kHessTX * kHessTY))) * H +
+                         (T.y0 + (int)(v / kHessTX % kHessTY))) * W + T.x0 + (int)(v % kHessTX);
+      float* h = rec + kCandTile + i;
+      const double xx = h[0], xy = h[kCandTile], xz = h[2 * kCandTile], yy = h[3 * kCandTile],
+                   yz = h[4 * kCandTile], zz = h[5 * kCandTile];
+      const double d = det3(xx, xy, xz, yy, yz, zz);
+      const double u = -d * inv_tau;
+      const double p = 1.0 / (1.0 + exp(-u));
+      const double gu = (p - (target[at] ? 1.0 : 0.0)) * inv_count;  // dL/du
+      gt += gu * d * inv_tau * inv_tau;                               // du/dtau = det / tau^2
+      const double gd = -gu * inv_tau;                                // dL/ddet
+      h[0] = (float)(gd * (yy * zz - yz * yz));
+      h[kCandTile] = (float)(gd * 2.0 * (xz * yz - zz * xy));
+      h[2 * kCandTile] = (float)(gd * 2.0 * (xy * yz - yy * xz));
+      h[3 * kCandTile] = (float)(gd * (xx * zz - xz * xz));
+      h[4 * kCandTile] = (float)(gd * 2.0 * (xy * xz - xx * yz));
+      h[5 * kCandTile] = (float)(gd * (xx * yy - xy * xy));
     }
-    const double xx = hess[i], xy = hess[N + i], xz = hess[2 * N + i], yy = hess[3 * N + i],
-                 yz = hess[4 * N + i], zz = hess[5 * N + i];
-    const double d = det3(xx, xy, xz, yy, yz, zz);
-    const double u = -d * inv_tau;
-    const double p = 1.0 / (1.0 + exp(-u));
-    const double gu = (p - (target[i] ? 1.0 : 0.0)) * inv_count;  // dL/du
-    gt += gu * d * inv_tau * inv_tau;                               // du/dtau = det / tau^2
-    const double gd = -gu * inv_tau;                                // dL/ddet
-    hess[i] = (float)(gd * (yy * zz - yz * yz));
-    hess[N + i] = (float)(gd * 2.0 * (xz * yz - zz * xy));
-    hess[2 * N + i] = (float)(gd * 2.0 * (xy * yz - yy * xz));
-    hess[3 * N + i] = (float)(gd * (xx * zz - xz * xz));
-    hess[4 * N + i] = (float)(gd * 2.0 * (xy * xz - xx * yz));
-    hess[5 * N + i] = (float)(gd * (xx * yy - xy * xy));
   }
   double a[1] = {gt};
   group_add<1>(a, sums);
+}
+
+// dL/ddog from the records of dL/dH, and *dot += <dL/ddog, dog>:
+//   P_x = g_x Gxx + g_y Gxy + g_z Gxz, P_y = g_y Gyy + g_z Gyz, P_z = g_z Gzz,
+//   dL/ddog = g_x P_x + g_y P_y + g_z P_z,
+// g the zero-padded central difference, P zero outside the volume.  A wave owns kAdjX columns
+// of AR rows and marches over the slices of a segment: its lanes hold the columns and two more
+// on either side, so the differences along x are lane shifts, those along y differences of its
+// own registers, and those along z of the ones it kept.  A row of a slice is laid out straight
+// from the records: its bits (from the two tiles that the 64 lanes touch) say which lanes hold
+// one and which one; a lane without one reads past the end of the buffer, which gives 0 without
+// touching memory.  Nothing dense but the result leaves the chip.  Bound by instruction issue
+// (two row lookups and eight loads per output row).  As dense volumes dL/dH went out and back
+// in two passes: 262 + 132 us at 128 x 512 x 512 with 7 % masked, and 76 for the dot product
+// (229 here; with tiles of 64 x 8 x 8 in LDS, one element at a time, 820).
+constexpr int AR = 4;       // rows of outputs of a wave
+constexpr int kAdjX = 60;   // columns of outputs: lanes 2 .. 61
+constexpr int AI = AR + 4;  // rows of inputs, two beyond either side
+__device__ __forceinline__ float lane_up(float v) {  // the value of lane - 1
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, false));
+}
+__device__ __forceinline__ float lane_down(float v) {  // the value of lane + 1
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xf, 0xf, false));
+}
+__device__ __forceinline__ uint32_t read_lane(uint32_t v, int l) {
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, l);
+}
+__global__ __launch_bounds__(NT, 4) void k_hessian_adjoint(const float* __restrict__ cand,
+                                                           const TileRow* __restrict__ rows,
+                                                           const float* __restrict__ dog,
+                                                           float* __restrict__ out, int nsx,
+                                                           int nsy, int nbx, int nby, int len,
+                                                           int W, int H, int D, double* dot) {
+  constexpr uint32_t kTileWords = (uint32_t)kCandTile * 7u;
+  const int lane = (int)(threadIdx.x & 63);
+  const int strip = __builtin_amdgcn_readfirstlane(
+      (int)blockIdx.x * (NT / 64) + (int)(threadIdx.x >> 6));  // x fastest, then y, then z
+  const int c0 = strip % nsx * kAdjX - 2, y0 = strip / nsx % nsy * AR,
+            z0 = strip / nsx / nsy * len, z1 = min(z0 + len, D);
+  double acc = 0.0;
+  if (z0 < D) {
+    const int col = c0 + lane;
+    const bool colin = col >= 0 && col < W, writes = colin && lane >= 2 && lane < 2 + kAdjX;
+    // the tile of column c0 covers the lanes below `split`, the next one the others
+    const int tl = (c0 + 64) / 64 - 1, sh = (c0 + 64) % 64, split = 64 - sh;
+    const bool right = lane >= split;
+    // lane j < AI looks up row y0 - 2 + j, of the left tile, lane AI + j of the right one
+    const int lt = lane >= AI ? tl + 1 : tl, ly = y0 - 2 + (lane >= AI ? lane - AI : lane);
+    const bool look = lane < 2 * AI && lt >= 0 && lt < nbx && ly >= 0 && ly < H;
+    const i64 rowbase = ((i64)(look ? ly / kHessTY : 0) * nbx + (look ? lt : 0)) *
+                            (kHessTY * kHessTZ) + (look ? ly % kHessTY : 0);
+    auto find = [&](int z) -> TileRow {
+      TileRow r = {0ull, 0ull};
+      if (look && z >= 0 && z < D)
+        r = rows[rowbase + (i64)(z / kHessTZ) * nby * nbx * (kHessTY * kHessTZ) +
+                 z % kHessTZ * kHessTY];
+      return r;
+    };
+    auto half = [](float hi, float lo) { return (hi - lo) * 0.5f; };
+    // [z & 1]: the values of two slices ago until this one's replace them
+    float xz[2][AR] = {}, yz[2][AR + 2] = {}, zz[2][AR] = {}, pz[2][AR] = {};
+    float ax[AR] = {}, ay[AR + 2] = {}, o[AR] = {};
+    TileRow next = find(z0 - 2);
+    auto slice = [&](int z, auto par) {
+      constexpr int q = decltype(par)::value;
+      const TileRow cur = next;
+      next = find(z + 1);
+      const int zo = z - 2;  // the slice that leaves
+      const bool leaves = zo >= z0 && writes;
+      const i64 at = ((i64)zo * H + y0) * W + col;
+      float gxx[AR] = {}, gxy[AR + 2] = {}, gyy[AI] = {}, nxz[AR] = {}, nyz[AR + 2] = {}, nzz[AR] = {};
+      // bits of the lanes' columns and, per side, the slot of the first record among them
+      const unsigned long long own = lane < AI ? cur.bits >> sh : sh ? cur.bits << split : 0ull;
+      const uint32_t first = (uint32_t)cur.first +
+          (lane < AI && sh ? (uint32_t)__popcll(cur.bits << split) : 0u);
+      if (__ballot(own != 0ull)) {
+        const uint32_t olo = (uint32_t)own, ohi = (uint32_t)(own >> 32);
+#pragma unroll
+        for (int j = 0; j < AI; ++j) {
+          const int y = y0 - 2 + j;
+          const int ty = max(y, 0) / kHessTY, tz = max(z, 0) / kHessTZ;
+          const unsigned long long mlo = read_lane(olo, j), mhi = read_lane(ohi, j);
+          const unsigned long long ml = mhi << 32 | mlo;
+          const unsigned long long m = ml | (unsigned long long)read_lane(ohi, AI + j) << 32 |
+                                       read_lane(olo, AI + j);
+          const uint32_t fl = read_lane(first, j);
+          const uint32_t fr = read_lane(first, AI + j) - (uint32_t)__popcll(ml) + kTileWords;
+          // two tiles' records, never used beyond the last tile's (no bits there)
+          const __amdgpu_buffer_rsrc_t r = buf_rsrc(
+              cand + ((i64)tz * nby * nbx + (i64)ty * nbx + tl) * (i64)kTileWords, kTileWords * 8u);
+          const uint32_t rank = __builtin_amdgcn_mbcnt_hi(
+              (uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+          const uint32_t slot = rank + (right ? fr : fl);
+          const int off = (int)((m >> lane) & 1ull ? slot * 4u : 0xF0000000u);
+          auto get = [&](int k) {
+            return __uint_as_float(
+                __builtin_amdgcn_raw_buffer_load_b32(r, off, kCandTile * (1 + k) * 4, 0));
+          };
+          gyy[j] = get(3);
+          if (j >= 1 && j <= AR + 2) {
+            gxy[j - 1] = get(1);
+            nyz[j - 1] = get(4);
+          }
+          if (j >= 2 && j <= AR + 1) {
+            gxx[j - 2] = get(0);
+            nxz[j - 2] = get(2);
+            nzz[j - 2] = get(5);
+          }
+        }
+      }
+      // z - 2 leaves: g_z P_z
+      const bool zin = z >= 1 && z <= D;  // slice z - 1
+#pragma unroll
+      for (int j = 0; j < AR; ++j) {
+        const float p = zin ? half(nzz[j], zz[q][j]) : 0.0f;  // P_z(z - 1)
+        const float v = o[j] + half(p, pz[1 - q][j]);  // P_z(z - 3)
+        if (leaves && y0 + j < H) {
+          out[at + (i64)j * W] = v;
+          acc += (double)v * dog[at + (i64)j * W];
+        }
+        pz[1 - q][j] = p;
+        zz[q][j] = nzz[j];
+      }
+      // z - 1 is completed but for P_z
+#pragma unroll
+      for (int j = 0; j < AR; ++j) {
+        const float p = colin ? ax[j] + half(nxz[j], xz[q][j]) : 0.0f;
+        o[j] = half(lane_down(p), lane_up(p));
+        xz[q][j] = nxz[j];
+      }
+      float py[AR + 2];
+#pragma unroll
+      for (int j = 0; j < AR + 2; ++j) {
+        const int y = y0 - 1 + j;
+        py[j] = y >= 0 && y < H ? ay[j] + half(nyz[j], yz[q][j]) : 0.0f;
+        yz[q][j] = nyz[j];
+      }
+#pragma unroll
+      for (int j = 0; j < AR; ++j) o[j] += half(py[j + 2], py[j]);
+      // z
+#pragma unroll
+      for (int j = 0; j < AR; ++j)
+        ax[j] = half(lane_down(gxx[j]), lane_up(gxx[j])) + half(gxy[j + 2], gxy[j]);
+#pragma unroll
+      for (int j = 0; j < AR + 2; ++j) ay[j] = half(gyy[j + 2], gyy[j]);
+    };
+    for (int z = z0 - 2; z < z1 + 2; z += 2) {
+      slice(z, std::integral_constant<int, 0>());
+      if (z + 1 < z1 + 2) slice(z + 1, std::integral_constant<int, 1>());
+    }
+  }
+  double a[1] = {acc};
+  group_add<1>(a, dot);
 }
 
 // Line kernels run one element per thread on a grid of nxb x-blocks per row (y + H z):
@@ -141,49 +320,6 @@ __device__ __forceinline__ bool pos_of(int W, int H, unsigned nxb, Pos& p) {
 unsigned xblocks(int W) { return (unsigned)((W + NT - 1) / NT); }
 unsigned grid_rows(int W, int H, int D) { return xblocks(W) * (unsigned)H * (unsigned)D; }
 
-// zero-padded central difference of field f along axis `a` at (x, y, z)
-__device__ __forceinline__ float cdiff(const float* f, int x, int y, int z, int a, int W, int H,
-                                       int D, i64 WH) {
-  int xp = x, xm = x, yp = y, ym = y, zp = z, zm = z;
-  bool okp, okm;
-  if (a == 0) { xp = x + 1; xm = x - 1; okp = xp < W; okm = xm >= 0; }
-  else if (a == 1) { yp = y + 1; ym = y - 1; okp = yp < H; okm = ym >= 0; }
-  else { zp = z + 1; zm = z - 1; okp = zp < D; okm = zm >= 0; }
-  const float hi = okp ? f[(i64)zp * WH + (i64)yp * W + xp] : 0.0f;
-  const float lo = okm ? f[(i64)zm * WH + (i64)ym * W + xm] : 0.0f;
-  return (hi - lo) * 0.5f;
-}
-
-__global__ __launch_bounds__(NT) void k_hadj1(const float* __restrict__ g, float* __restrict__ P,
-                                              int W, int H, int D, unsigned nxb) {
-  const i64 WH = (i64)W * H, N = WH * D;
-  Pos q;
-  if (!pos_of(W, H, nxb, q)) return;
-  {
-    const i64 i = q.i;
-    const int x = q.x, y = q.y, z = q.z;
-    const float* gxx = g; const float* gxy = g + N; const float* gxz = g + 2 * N;
-    const float* gyy = g + 3 * N; const float* gyz = g + 4 * N; const float* gzz = g + 5 * N;
-    P[i] = cdiff(gxx, x, y, z, 0, W, H, D, WH) + cdiff(gxy, x, y, z, 1, W, H, D, WH) +
-           cdiff(gxz, x, y, z, 2, W, H, D, WH);
-    P[N + i] = cdiff(gyy, x, y, z, 1, W, H, D, WH) + cdiff(gyz, x, y, z, 2, W, H, D, WH);
-    P[2 * N + i] = cdiff(gzz, x, y, z, 2, W, H, D, WH);
-  }
-}
-
-__global__ __launch_bounds__(NT) void k_hadj2(const float* __restrict__ P, float* __restrict__ out,
-                                              int W, int H, int D, unsigned nxb) {
-  const i64 WH = (i64)W * H, N = WH * D;
-  Pos q;
-  if (!pos_of(W, H, nxb, q)) return;
-  {
-    const i64 i = q.i;
-    const int x = q.x, y = q.y, z = q.z;
-    out[i] = cdiff(P, x, y, z, 0, W, H, D, WH) + cdiff(P + N, x, y, z, 1, W, H, D, WH) +
-             cdiff(P + 2 * N, x, y, z, 2, W, H, D, WH);
-  }
-}
-
 // out[0] += <a, pair.x>, out[1] += <a, pair.y>
 __global__ __launch_bounds__(NT) void k_dot_pair(const float* __restrict__ a,
                                                  const float2* __restrict__ pair, i64 N,
@@ -197,15 +333,6 @@ __global__ __launch_bounds__(NT) void k_dot_pair(const float* __restrict__ a,
   }
   double t[2] = {s0, s1};
   group_add<2>(t, out);
-}
-
-__global__ __launch_bounds__(NT) void k_dot(const float* __restrict__ a,
-                                            const float* __restrict__ b, i64 N, double* out) {
-  double s = 0.0;
-  for (i64 i = (i64)blockIdx.x * NT + threadIdx.x; i < N; i += (i64)gridDim.x * NT)
-    s += (double)a[i] * b[i];
-  double t[1] = {s};
-  group_add<1>(t, out);
 }
 
 __global__ __launch_bounds__(NT) void k_pack_pair(const float* __restrict__ a,
@@ -714,42 +841,51 @@ hipError_t launch_soft_normalize_adjoint(const float* v, const float2* ed, const
   return hipGetLastError();
 }
 
-hipError_t launch_soft_loss(const float* hess, const uint8_t* mask, const uint8_t* target, i64 N,
-                            double inv_tau, double* sums, hipStream_t s) {
+// grid of a pass over tiles that ends in a reduction
+static unsigned grid_tiles(i64 ntiles) { return (unsigned)std::min<i64>(ntiles, kReduceGroups); }
+
+hipError_t launch_soft_loss(const float* cand, const uint32_t* cand_cnt, const uint8_t* target,
+                            int W, int H, int D, double inv_tau, double* sums, hipStream_t s) {
+  const i64 nt = hessian_tiles(W, H, D);
+  const unsigned nbx = (unsigned)((W + kHessTX - 1) / kHessTX),
+                 nby = (unsigned)((H + kHessTY - 1) / kHessTY);
   hipLaunchKernelGGL(k_zero_f64, dim3(1), dim3(64), 0, s, sums, 2);
-  hipLaunchKernelGGL(k_soft_loss, dim3(grid_reduce(N)), dim3(NT), 0, s, hess, mask, target, N,
-                     inv_tau, sums);
+  hipLaunchKernelGGL(k_soft_loss, dim3(grid_tiles(nt)), dim3(NT), 0, s, cand, cand_cnt, target,
+                     (unsigned)nt, nbx, nby, W, H, inv_tau, sums);
   return hipGetLastError();
 }
 
-hipError_t launch_soft_grad_h(float* hess, const uint8_t* mask, const uint8_t* target, i64 N,
-                              double inv_tau, double inv_count, double* sums, hipStream_t s) {
-  hipLaunchKernelGGL(k_zero_f64, dim3(1), dim3(64), 0, s, sums, 1);
-  hipLaunchKernelGGL(k_soft_grad_h, dim3(grid_reduce(N)), dim3(NT), 0, s, hess, mask, target, N,
-                     inv_tau, inv_count, sums);
+hipError_t launch_soft_grad_h(float* cand, const uint32_t* cand_cnt, const uint8_t* target, int W,
+                              int H, int D, double inv_tau, double inv_count, double* sums,
+                              hipStream_t s) {
+  const i64 nt = hessian_tiles(W, H, D);
+  const unsigned nbx = (unsigned)((W + kHessTX - 1) / kHessTX),
+                 nby = (unsigned)((H + kHessTY - 1) / kHessTY);
+  hipLaunchKernelGGL(k_soft_grad_h, dim3(grid_tiles(nt)), dim3(NT), 0, s, cand, cand_cnt, target,
+                     (unsigned)nt, nbx, nby, W, H, inv_tau, inv_count, sums);
   return hipGetLastError();
 }
 
-hipError_t launch_hessian_adjoint(const float* gh, float* P, float* out, int W, int H, int D,
-                                  hipStream_t s) {
-  hipLaunchKernelGGL(k_hadj1, dim3(grid_rows(W, H, D)), dim3(NT), 0, s, gh, P, W, H, D,
-                     xblocks(W));
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_hadj2, dim3(grid_rows(W, H, D)), dim3(NT), 0, s, P, out, W, H, D,
-                     xblocks(W));
+hipError_t launch_hessian_adjoint(const float* cand, const TileRow* rows, const float* dog,
+                                  float* out, int W, int H, int D, double* dot, hipStream_t s) {
+  const int nsx = (W + kAdjX - 1) / kAdjX, nsy = (H + AR - 1) / AR;
+  const i64 groups = ((i64)nsx * nsy + NT / 64 - 1) / (NT / 64);
+  int nseg, len;
+  line_segments(D, groups, 1024.0, 1.0, false, 4, &nseg, &len);
+  const i64 waves = (i64)nsx * nsy * nseg;
+  hipLaunchKernelGGL(k_hessian_adjoint, dim3((unsigned)((waves + NT / 64 - 1) / (NT / 64))),
+                     dim3(NT), 0, s, cand, rows, dog, out, nsx, nsy, (W + kHessTX - 1) / kHessTX,
+                     (H + kHessTY - 1) / kHessTY, len, W, H, D, dot);
+  return hipGetLastError();
+}
+
+hipError_t launch_zero_f64(double* p, int n, hipStream_t s) {
+  hipLaunchKernelGGL(k_zero_f64, dim3(1), dim3(64), 0, s, p, n);
   return hipGetLastError();
 }
 
 hipError_t launch_dot_pair(const float* a, const float2* pair, i64 N, double* out, hipStream_t s) {
-  hipLaunchKernelGGL(k_zero_f64, dim3(1), dim3(64), 0, s, out, 2);
   hipLaunchKernelGGL(k_dot_pair, dim3(grid_reduce(N)), dim3(NT), 0, s, a, pair, N, out);
-  return hipGetLastError();
-}
-
-hipError_t launch_dot(const float* a, const float* b, i64 N, double* out, hipStream_t s) {
-  hipLaunchKernelGGL(k_zero_f64, dim3(1), dim3(64), 0, s, out, 1);
-  hipLaunchKernelGGL(k_dot, dim3(grid_reduce(N)), dim3(NT), 0, s, a, b, N, out);
   return hipGetLastError();
 }
 

@@ -219,3 +219,39 @@ def test_region_sums_beyond_the_table(hd, sigmas, ave):
     for k in ("hsum", "norm"):
         a, b = (x[k].astype(np.float64).reshape(len(n), -1) for x in (got, want))
         assert np.all(np.abs(a - b) <= 1.2e-7 * np.abs(b) + 1e-12 * n * big), k
+
+
+# soft response, gradient of the Hessian step for a given mask: tiles and strips with
+# remainders, volumes smaller than a difference's reach, all voxels (the first one too), some,
+# and one tile's corner only.  FP32 volumes and weights behind FP64 products of three
+# elements: some 1e-5 of the largest gradient; the bound is that of the other gradient tests
+@pytest.mark.parametrize("shape", [(1, 1, 1), (3, 2, 5), (17, 9, 65), (16, 8, 120), (33, 13, 190)])
+@pytest.mark.parametrize("kind", ["all", "some", "corner"])
+def test_soft_gradient_of_given_masks(hd, shape, kind):
+    import types
+
+    import soft_reference as ref
+    import torch
+    from hdog import soft
+    s1, s2, tau = [1.6, 2.0, 2.0], [2.56, 3.2, 3.2], 0.05
+    rad1, rad2 = soft.radii(s1), soft.radii(s2)
+    rng = np.random.default_rng(shape[2])
+    v = torch.from_numpy(rng.standard_normal(shape).astype(np.float32))
+    t = torch.from_numpy((rng.random(shape) < 0.1).astype(np.uint8))
+    m = {"all": np.ones(shape), "some": rng.random(shape) < 0.2, "corner": np.zeros(shape)}[kind]
+    if kind == "corner":
+        m[min(15, shape[0] - 1):18, min(7, shape[1] - 1):9, min(63, shape[2] - 1):66] = 1
+    m = torch.from_numpy(m.astype(np.uint8))
+    vd, td = v.to(hd.device), t.to(hd.device)
+    dog = soft.run_forward(hd, vd, td, s1, s2, tau, rad1, rad2)[2]
+    ctx = types.SimpleNamespace(saved_tensors=(vd, dog, m.to(hd.device), td), hd=hd, s1=s1[::-1],
+                                s2=s2[::-1], r1=list(rad1)[::-1], r2=list(rad2)[::-1], gamma=1.0,
+                                tau=tau, count=int(m.sum()), dev_sigma=torch.device("cpu"))
+    gv, _, _, gtau = soft._SoftFn.backward(ctx, 1.0)[:4]
+    v64 = v.double().requires_grad_()
+    t64 = torch.tensor(tau, dtype=torch.float64, requires_grad=True)
+    ref.forward(v64, torch.tensor(s1, dtype=torch.float64), torch.tensor(s2, dtype=torch.float64),
+                t64, t, rad1, rad2, mask=m.bool())[0].backward()
+    err = float((gv.cpu().double() - v64.grad).abs().max())
+    assert err <= 2e-3 * float(v64.grad.abs().max())
+    assert abs(float(gtau) - float(t64.grad)) <= 2e-3 * abs(float(t64.grad)) + 1e-6
