@@ -1187,13 +1187,11 @@ int hdog_soft_forward(hdog_ctx* ctx, void* stream, const float* d_v, const uint8
   hipStream_t s = (hipStream_t)stream;
   const i64 N = (i64)width * height * depth;
   HIPCHK(ensure(ctx->tmp1, (size_t)N * 8));
-  HIPCHK(ensure(ctx->tmp2, (size_t)N * 8));
   const i64 ntiles = hessian_tiles(width, height, depth);
   HIPCHK(ensure(ctx->cand, (size_t)ntiles * kCandTile * 7 * 4));
   HIPCHK(ensure(ctx->cand_cnt, (size_t)ntiles * 4));
   HIPCHK(ensure(ctx->sums, 64 * 8));
-  HIPCHK(launch_gauss_pair(d_v, ctx->tmp1.p, ctx->tmp2.p, S.w, S.r, (float)S.s, d_dog, nullptr,
-                           width, height, depth, s));
+  HIPCHK(launch_gauss_dog(d_v, ctx->tmp1.p, S.w, S.r, (float)S.s, d_dog, width, height, depth, s));
   HIPCHK(launch_hessian_records(d_dog, d_mask, nullptr, width, height, depth, (float*)ctx->cand.p,
                                 (uint32_t*)ctx->cand_cnt.p, s));
   HIPCHK(launch_soft_loss((const float*)ctx->cand.p, (const uint32_t*)ctx->cand_cnt.p, d_target,
@@ -1223,7 +1221,6 @@ int hdog_soft_backward(hdog_ctx* ctx, void* stream, const float* d_v, const floa
   hipStream_t s = (hipStream_t)stream;
   const i64 N = (i64)width * height * depth;
   HIPCHK(ensure(ctx->tmp1, (size_t)N * 8));
-  HIPCHK(ensure(ctx->tmp2, (size_t)N * 8));
   const i64 ntiles = hessian_tiles(width, height, depth);
   HIPCHK(ensure(ctx->cand, (size_t)ntiles * kCandTile * 7 * 4));
   HIPCHK(ensure(ctx->cand_cnt, (size_t)ntiles * 4));
@@ -1245,16 +1242,15 @@ int hdog_soft_backward(hdog_ctx* ctx, void* stream, const float* d_v, const floa
   // dL/ddog, and <dL/ddog, dog>
   HIPCHK(launch_hessian_adjoint(cand, rows, d_dog, ddog, width, height, depth, sums + 1, s));
   // dL/dv = s (G1 - G2) dL/ddog
-  HIPCHK(launch_gauss_pair(ddog, ctx->tmp1.p, ctx->tmp2.p, S.w, S.r, (float)S.s, d_grad_v, nullptr,
-                           width, height, depth, s));
+  HIPCHK(launch_gauss_dog(ddog, ctx->tmp1.p, S.w, S.r, (float)S.s, d_grad_v, width, height, depth,
+                          s));
   double h[16];
   for (int a = 0; a < 3; ++a) {
     const float* w[6] = {S.w[0], S.w[1], S.w[2], S.w[3], S.w[4], S.w[5]};
     w[a] = S.dw[a];
     w[3 + a] = S.dw[3 + a];
-    HIPCHK(launch_gauss_pair(d_v, ctx->tmp1.p, ctx->tmp2.p, w, S.r, 0.0f, nullptr,
-                             (float2*)ctx->tmp1.p, width, height, depth, s));
-    HIPCHK(launch_dot_pair(ddog, (const float2*)ctx->tmp1.p, N, sums + 2 + 2 * a, s));
+    HIPCHK(launch_gauss_dots(d_v, ctx->tmp1.p, w, S.r, ddog, sums + 2 + 2 * a, width, height,
+                             depth, s));
   }
   HIPCHK(hipMemcpyAsync(h, sums, 8 * 8, hipMemcpyDeviceToHost, s));
   HIPCHK(hipStreamSynchronize(s));

@@ -248,10 +248,11 @@ __global__ __launch_bounds__(64 * NW) void k_gauss_xy_run(
 // the last 2R + 32 positions (zero outside the line).  Bound by its 12 or 16 bytes per voxel
 // for short windows (61 x 900 x 1111 along z at radii 4 / 7: 377 us with one output per thread
 // and a read per tap, 198 us now).
-template <bool LAST, bool WIDE, typename TS>
+template <bool DOT, bool WIDE, typename TS>
 __global__ __launch_bounds__(256) void k_gauss_line_run(const float2* __restrict__ src,
-                                                        float2* __restrict__ dst,
                                                         TS* __restrict__ dog,
+                                                        const float* __restrict__ a,
+                                                        double* __restrict__ dots,
                                                         const float* __restrict__ w1,
                                                         const float* __restrict__ w2, int r1,
                                                         int r2, float nz, int W, int L, i64 sa,
@@ -295,6 +296,7 @@ __global__ __launch_bounds__(256) void k_gauss_line_run(const float2* __restrict
   fetch(s0 + R + GK * wave);
   __syncthreads();
   const bool out = x0 + l < W;
+  double d[2] = {0.0, 0.0};
   for (int c0 = s0; c0 < s1; c0 += STEP) {
     put(hist + GK * wave);
     fetch(c0 + STEP + R + GK * wave);
@@ -311,10 +313,13 @@ __global__ __launch_bounds__(256) void k_gauss_line_run(const float2* __restrict
         for (int o = 0; o < GK; ++o) {
           if (c + o >= s1) continue;
           const i64 idx = base + (i64)(c + o) * sa + l;
-          if (LAST)
+          if (DOT) {
+            const double v = a[idx];
+            d[0] += v * a1[o];
+            d[1] += v * a2[o];
+          } else {
             st_nt(dog + idx, (a1[o] - a2[o]) * nz);
-          else
-            st_nt(dst + idx, make_float2(a1[o], a2[o]));
+          }
         }
       }
     }
@@ -324,83 +329,22 @@ __global__ __launch_bounds__(256) void k_gauss_line_run(const float2* __restrict
     shift_rows<256, STEP, 64>(B2, hist);
     __syncthreads();
   }
+  if (DOT) group_add<256>(d, dots);
 }
 
 // ------------------------------------------------------------- compile-time radii
-// x pass: tile ROWS rows x (64*4) outputs; thread (row, seg) makes 4 consecutive outputs.
-// LDS row position p <-> x = c0 - RP + p with RP = R rounded up to 4 (16-byte aligned
-// window reads).
-template <int R1, int R2, typename TS>
-__global__ __launch_bounds__(NT) void k_gauss_x_r(const TS* __restrict__ src,
-                                                  float2* __restrict__ dst,
-                                                  const float* __restrict__ w1,
-                                                  const float* __restrict__ w2, int W, i64 nrows,
-                                                  int nct) {
-  constexpr int ROWS = 4, RUN = 4, C = NT / ROWS * RUN;
-  constexpr int R = R1 > R2 ? R1 : R2;
-  constexpr int RP = (R + 3) / 4 * 4;
-  constexpr int SPAN = C + 2 * RP;
-  constexpr int NV = (RUN + 2 * RP) / 4;  // float4 reads per window
-  __shared__ __align__(16) float T[ROWS * SPAN];
-  const unsigned tile = xcd_tile(blockIdx.x, gridDim.x);
-  const int ct = tile % nct;
-  const i64 row0 = (i64)(tile / nct) * ROWS;
-  const int c0 = ct * C;
-  stage_tile<8, NT, float>(
-      ROWS * SPAN,
-      [&](int e) -> float {
-        const int row = e / SPAN, p = e % SPAN;
-        const i64 grow = row0 + row;
-        const int x = c0 - RP + p;
-        return (grow < nrows && x >= 0 && x < W) ? ld(src, grow * W + x) : 0.0f;
-      },
-      [&](int e, float v) { T[e] = v; });
-  __syncthreads();
-  const int row = threadIdx.x / (NT / ROWS), seg = threadIdx.x % (NT / ROWS);
-  const i64 grow = row0 + row;
-  const int xs = c0 + seg * RUN;
-  if (grow >= nrows || xs >= W) return;
-  float win[4 * NV];
-  const float4* T4 = reinterpret_cast<const float4*>(T + row * SPAN + seg * RUN);
-#pragma unroll
-  for (int v = 0; v < NV; ++v) {
-    const float4 q = T4[v];
-    win[4 * v] = q.x; win[4 * v + 1] = q.y; win[4 * v + 2] = q.z; win[4 * v + 3] = q.w;
-  }
-  float2 out[RUN];
-#pragma unroll
-  for (int o = 0; o < RUN; ++o) {
-    // window index of x = xs + o + j is o + j + RP
-    float s1 = 0.0f, s2 = 0.0f;
-#pragma unroll
-    for (int j = -R1; j <= R1; ++j) s1 = fmaf(w1[R1 - j], win[o + j + RP], s1);
-#pragma unroll
-    for (int j = -R2; j <= R2; ++j) s2 = fmaf(w2[R2 - j], win[o + j + RP], s2);
-    out[o] = make_float2(s1, s2);
-  }
-  float2* drow = dst + grow * W;
-  // 16-byte stores (a wave writes 1 KB in two instructions) where the row start allows
-  if (xs + RUN <= W && ((grow * W) & 1) == 0) {
-#pragma unroll
-    for (int o = 0; o < RUN; o += 2)
-      *reinterpret_cast<float4*>(drow + xs + o) =
-          make_float4(out[o].x, out[o].y, out[o + 1].x, out[o + 1].y);
-  } else {
-#pragma unroll
-    for (int o = 0; o < RUN; ++o)
-      if (xs + o < W) drow[xs + o] = out[o];
-  }
-}
-
-// y / z pass as a column walker: one thread per line, a register ring of the last 2R+1
+// z pass as a column walker: one thread per line, a register ring of the last 2R+1
 // (G1, G2) pairs (zero outside the line), unrolled by the ring period so every index is
 // static; every input is read once and no LDS is used.  Ring refills are loaded PF steps
 // before they enter the ring (PF divides the ring period: static queue slots), and the
-// walk leaves the kernel at the line's end so no merged control path makes the compiler
-// wait for the whole queue.
-template <int R1, int R2, bool LAST, typename TS>
+// walk ends at the line's end so no merged control path makes the compiler wait for the
+// whole queue.  DOT: the outputs meet the volume `a` in FP64 sums instead of leaving (as a
+// pair volume and a pass of its own over it: 97 + 85 us at 128 x 512 x 512, here 87).
+template <int R1, int R2, bool DOT, typename TS>
 __global__ __launch_bounds__(NT) void k_gauss_walk(const float2* __restrict__ src,
-                                                   float2* __restrict__ dst, TS* __restrict__ dog,
+                                                   TS* __restrict__ dog,
+                                                   const float* __restrict__ a,
+                                                   double* __restrict__ dots,
                                                    const float* __restrict__ w1,
                                                    const float* __restrict__ w2, float nz, int W,
                                                    int L, i64 sa, i64 so, unsigned nxb,
@@ -410,59 +354,80 @@ __global__ __launch_bounds__(NT) void k_gauss_walk(const float2* __restrict__ sr
   constexpr int PF = WB % 3 == 0 ? 3 : WB % 5 == 0 ? 5 : WB % 7 == 0 ? 7 : 1;
   const LineAt la = line_at_block(nxb, no, len, L);
   const int x = la.x, b0 = la.c0, b1 = la.c1;
-  if (x >= W) return;
-  const i64 base = (i64)la.other * so + x;
-  // zero padding in the load itself: position p is read through a buffer descriptor of
-  // the wave's 64 columns at p (a uniform base), whose record count is 0 outside the
-  // line, so those loads return zeros and no value is tested (or waited for) when it
-  // enters the ring
-  const int lane = (int)(threadIdx.x & 63);
-  const int xw = __builtin_amdgcn_readfirstlane(x - lane);  // the wave's first column
-  const i64 bw = (i64)la.other * so + xw;
-  const int nrec = min(64, W - xw) * (int)sizeof(float2);
-  auto load = [&](const float2* line, bool in) -> float2 {
-    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<float2*>(line), 0, in ? nrec : 0, kBufferWord3);
-    return __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(
-                                          r, lane * (int)sizeof(float2), 0, 0));
-  };
-  float2 ring[WB];  // position p lives in ring[(p - b0 + R) % WB]
-#pragma unroll
-  for (int q = 0; q < WB; ++q) {
-    const int p = b0 - R + q;
-    ring[q] = load(src + bw + (i64)p * sa, (unsigned)p < (unsigned)L);
-  }
-  // the refills are read front to back: a pointer and the positions left on the line
-  const float2* line = src + bw + (i64)(b0 + R + 1) * sa;
-  int left = L - (b0 + R + 1);
-  auto refill = [&]() -> float2 {
-    const float2 v = load(line, left > 0);
-    line += sa;
-    --left;
-    return v;
-  };
-  float2 pf[PF];  // the refill of step c (position c + R + 1) waits in slot (c - b0) % PF
-#pragma unroll
-  for (int j = 0; j < PF; ++j) pf[j] = refill();
-  i64 idx = base + (i64)b0 * sa;
-  for (int n = b1 - b0;; n -= WB) {  // outputs left
+  double d[2] = {0.0, 0.0};
+  auto walk = [&] {
+    const i64 base = (i64)la.other * so + x;
+    // zero padding in the load itself: position p is read through a buffer descriptor of
+    // the wave's 64 columns at p (a uniform base), whose record count is 0 outside the
+    // line, so those loads return zeros and no value is tested (or waited for) when it
+    // enters the ring
+    const int lane = (int)(threadIdx.x & 63);
+    const int xw = __builtin_amdgcn_readfirstlane(x - lane);  // the wave's first column
+    const i64 bw = (i64)la.other * so + xw;
+    const int nrec = min(64, W - xw) * (int)sizeof(float2);
+    auto load = [&](const float2* line, bool in) -> float2 {
+      const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<float2*>(line), 0, in ? nrec : 0, kBufferWord3);
+      return __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(
+                                            r, lane * (int)sizeof(float2), 0, 0));
+    };
+    float2 ring[WB];  // position p lives in ring[(p - b0 + R) % WB]
 #pragma unroll
     for (int q = 0; q < WB; ++q) {
-      if (q >= n) return;
-      float s1 = 0.0f, s2 = 0.0f;
-#pragma unroll
-      for (int j = -R1; j <= R1; ++j) s1 = fmaf(w1[R1 - j], ring[(q + j + R) % WB].x, s1);
-#pragma unroll
-      for (int j = -R2; j <= R2; ++j) s2 = fmaf(w2[R2 - j], ring[(q + j + R) % WB].y, s2);
-      if (LAST)
-        st_nt(dog + idx, (s1 - s2) * nz);
-      else
-        st_nt(dst + idx, make_float2(s1, s2));
-      idx += sa;
-      ring[q] = pf[q % PF];  // position c + R + 1 replaces position c - R
-      pf[q % PF] = refill();
+      const int p = b0 - R + q;
+      ring[q] = load(src + bw + (i64)p * sa, (unsigned)p < (unsigned)L);
     }
-  }
+    // the refills are read front to back: a pointer and the positions left on the line
+    const float2* line = src + bw + (i64)(b0 + R + 1) * sa;
+    const float* aline = a + bw + (i64)b0 * sa;
+    int left = L - (b0 + R + 1), aleft = L - b0;
+    auto refill = [&]() -> float2 {
+      const float2 v = load(line, left > 0);
+      line += sa;
+      --left;
+      return v;
+    };
+    auto next_a = [&]() -> float {
+      const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<float*>(aline), 0, aleft > 0 ? nrec / 2 : 0, kBufferWord3);
+      aline += sa;
+      --aleft;
+      return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, lane * 4, 0, 0));
+    };
+    // what step c needs (position c + R + 1, and a at c) waits in slot (c - b0) % PF
+    float2 pf[PF];
+    float pa[PF];
+#pragma unroll
+    for (int j = 0; j < PF; ++j) {
+      pf[j] = refill();
+      if (DOT) pa[j] = next_a();
+    }
+    i64 idx = base + (i64)b0 * sa;
+    for (int n = b1 - b0;; n -= WB) {  // outputs left
+#pragma unroll
+      for (int q = 0; q < WB; ++q) {
+        if (q >= n) return;
+        float s1 = 0.0f, s2 = 0.0f;
+#pragma unroll
+        for (int j = -R1; j <= R1; ++j) s1 = fmaf(w1[R1 - j], ring[(q + j + R) % WB].x, s1);
+#pragma unroll
+        for (int j = -R2; j <= R2; ++j) s2 = fmaf(w2[R2 - j], ring[(q + j + R) % WB].y, s2);
+        if (DOT) {
+          const double v = pa[q % PF];
+          d[0] += v * s1;
+          d[1] += v * s2;
+          pa[q % PF] = next_a();
+        } else {
+          st_nt(dog + idx, (s1 - s2) * nz);
+          idx += sa;
+        }
+        ring[q] = pf[q % PF];  // position c + R + 1 replaces position c - R
+        pf[q % PF] = refill();
+      }
+    }
+  };
+  if (x < W) walk();
+  if (DOT) group_add<NT>(d, dots);
 }
 
 // x and y passes fused: a one-wave work-group walks the rows of one plane for a strip of
@@ -474,11 +439,14 @@ __global__ __launch_bounds__(NT) void k_gauss_walk(const float2* __restrict__ sr
 // use.  The Gaussian weights are symmetric (set pairwise from one value,
 // w[r - i] == w[r + i]), so tap j reads w[r + |j|]: r + 1 distinct values per Gaussian,
 // held in registers for the whole walk.
-template <int R1, int R2, typename TS>
+// AXES: weights of their own along y (wy1, wy2), else those along x.
+template <int R1, int R2, bool AXES, typename TS>
 __global__ __launch_bounds__(64) void k_gauss_xy_walk(const TS* __restrict__ src,
                                                       float2* __restrict__ dst,
                                                       const float* __restrict__ w1,
-                                                      const float* __restrict__ w2, int W, int H,
+                                                      const float* __restrict__ w2,
+                                                      const float* __restrict__ wy1,
+                                                      const float* __restrict__ wy2, int W, int H,
                                                       int nxs, int nys, int rows) {
   constexpr int R = R1 > R2 ? R1 : R2;
   constexpr int WB = 2 * R + 1;
@@ -521,6 +489,17 @@ __global__ __launch_bounds__(64) void k_gauss_xy_walk(const TS* __restrict__ src
   for (int i = 0; i <= R2; ++i) {
     v2[i] = w2[R2 + i];
     asm volatile("" : "+v"(v2[i]));
+  }
+  float u1[R1 + 1], u2[R2 + 1];  // along y
+#pragma unroll
+  for (int i = 0; i <= R1; ++i) {
+    u1[i] = AXES ? wy1[R1 + i] : v1[i];
+    if (AXES) asm volatile("" : "+v"(u1[i]));
+  }
+#pragma unroll
+  for (int i = 0; i <= R2; ++i) {
+    u2[i] = AXES ? wy2[R2 + i] : v2[i];
+    if (AXES) asm volatile("" : "+v"(u2[i]));
   }
   // row y waits in queue slot y % PF (y0 is a multiple of WB, so of PF): every slot index
   // below is a compile-time constant
@@ -574,9 +553,9 @@ __global__ __launch_bounds__(64) void k_gauss_xy_walk(const TS* __restrict__ src
       if (c >= y1) return;
       float s1 = 0.0f, s2 = 0.0f;
 #pragma unroll
-      for (int j = -R1; j <= R1; ++j) s1 = fmaf(v1[j < 0 ? -j : j], ring[(q + j + R) % WB].x, s1);
+      for (int j = -R1; j <= R1; ++j) s1 = fmaf(u1[j < 0 ? -j : j], ring[(q + j + R) % WB].x, s1);
 #pragma unroll
-      for (int j = -R2; j <= R2; ++j) s2 = fmaf(v2[j < 0 ? -j : j], ring[(q + j + R) % WB].y, s2);
+      for (int j = -R2; j <= R2; ++j) s2 = fmaf(u2[j < 0 ? -j : j], ring[(q + j + R) % WB].y, s2);
       if (out) st_nt(dcol + (i64)c * W, make_float2(s1, s2));
       ring[q] = xrow(c + R + 1, (q + R + 1) % PF);  // row c + R + 1 replaces row c - R
     }
@@ -607,24 +586,6 @@ WalkShape xy_run_shape(int RX, int RY, int W, int D) {
   return {(i64)((W + 63) / 64) * D * xy_run_waves(RX, RY), GK * 4, 2 * RY};
 }
 
-// x pass of a radius pair with a compile-time kernel
-template <typename TS>
-hipError_t gauss_x(const TS* src, float2* dst, const float* w1, const float* w2, int r1, int r2,
-                   int W, i64 nrows, hipStream_t s) {
-#define X(A, B)                                                                              \
-  if (r1 == A && r2 == B) {                                                                  \
-    constexpr int C = NT / 4 * 4;                                                            \
-    const int nct = (W + C - 1) / C;                                                         \
-    const i64 nblk = ((nrows + 3) / 4) * nct;                                                \
-    hipLaunchKernelGGL((k_gauss_x_r<A, B, TS>), dim3((unsigned)nblk), dim3(NT), 0, s, src,   \
-                       dst, w1, w2, W, nrows, nct);                                          \
-    return hipGetLastError();                                                                \
-  }
-  HDOG_GAUSS_PAIRS(X)
-#undef X
-  return hipErrorInvalidValue;
-}
-
 // x and y passes of any radii, each axis with its own
 template <typename TS>
 hipError_t gauss_xy_run(const TS* src, float2* dst, const float* wx1, const float* wx2,
@@ -646,34 +607,36 @@ hipError_t gauss_xy_run(const TS* src, float2* dst, const float* wx1, const floa
   return hipGetLastError();
 }
 
-// Fused x + y passes with the same weights on both axes
-template <typename TS>
-hipError_t gauss_xy(const TS* src, float2* dst, const float* w1, const float* w2, int r1, int r2,
-                    int W, int H, int D, hipStream_t s, int segments) {
+// Fused x + y passes of radii r1, r2 on both axes; AXES: with their own weights along y
+template <bool AXES, typename TS>
+hipError_t gauss_xy(const TS* src, float2* dst, const float* w1, const float* w2, const float* wy1,
+                    const float* wy2, int r1, int r2, int W, int H, int D, hipStream_t s,
+                    int segments) {
 #define X(A, B)                                                                              \
   if (r1 == A && r2 == B) {                                                                  \
     const int nxs = (W + 63) / 64;                                                           \
     int nys, rows;                                                                           \
     walk_segments(H, gauss_walk_shape(A, B, W, D), &nys, &rows, segments);                   \
     const i64 nblk = (i64)nxs * D * nys;                                                     \
-    hipLaunchKernelGGL((k_gauss_xy_walk<A, B, TS>), dim3((unsigned)nblk), dim3(64), 0, s,    \
-                       src, dst, w1, w2, W, H, nxs, nys, rows);                              \
+    hipLaunchKernelGGL((k_gauss_xy_walk<A, B, AXES, TS>), dim3((unsigned)nblk), dim3(64), 0, \
+                       s, src, dst, w1, w2, wy1, wy2, W, H, nxs, nys, rows);                 \
     return hipGetLastError();                                                                \
   }
   HDOG_GAUSS_PAIRS(X)
 #undef X
-  return gauss_xy_run<TS>(src, dst, w1, w2, w1, w2, r1, r2, r1, r2, W, H, D, s, segments);
+  return gauss_xy_run<TS>(src, dst, w1, w2, wy1, wy2, r1, r2, r1, r2, W, H, D, s, segments);
 }
 
-template <bool LAST, typename TS>
-hipError_t gauss_line(const float2* src, float2* dst, TS* dog, const float* w1, const float* w2,
-                      int r1, int r2, float nz, int W, int L, i64 sa, i64 so, i64 n_other,
-                      hipStream_t s) {
+// z pass: the difference (dog), or with DOT the sums of both with a
+template <bool DOT, typename TS>
+hipError_t gauss_z(const float2* src, TS* dog, const float* a, double* dots, const float* w1,
+                   const float* w2, int r1, int r2, float nz, int W, int H, int D, hipStream_t s) {
+  const i64 WH = (i64)W * H;
 #define X(A, B)                                                                              \
   if (r1 == A && r2 == B) {                                                                  \
-    const LineGrid g = line_grid(W, L, n_other, 2 * (A > B ? A : B));                        \
-    hipLaunchKernelGGL((k_gauss_walk<A, B, LAST, TS>), dim3(g.blocks), dim3(NT), 0, s, src,  \
-                       dst, dog, w1, w2, nz, W, L, sa, so, g.nxb, g.no, g.len);              \
+    const LineGrid g = line_grid(W, D, H, 2 * (A > B ? A : B));                              \
+    hipLaunchKernelGGL((k_gauss_walk<A, B, DOT, TS>), dim3(g.blocks), dim3(NT), 0, s, src,   \
+                       dog, a, dots, w1, w2, nz, W, D, WH, (i64)W, g.nxb, g.no, g.len);      \
     return hipGetLastError();                                                                \
   }
   HDOG_GAUSS_PAIRS(X)
@@ -681,15 +644,15 @@ hipError_t gauss_line(const float2* src, float2* dst, TS* dog, const float* w1, 
   const int R = std::max(r1, r2);
   const i64 nxb = (W + 63) / 64;
   int nseg, len;
-  line_segments(L, nxb * n_other * 4, 1024.0, 2.0, false, 2 * R, &nseg, &len);
-  const dim3 grid((unsigned)(nxb * n_other * nseg));
+  line_segments(D, nxb * H * 4, 1024.0, 2.0, false, 2 * R, &nseg, &len);
+  const dim3 grid((unsigned)(nxb * H * nseg));
   const size_t lds = 2 * (size_t)(2 * R + 4 * GK) * 64 * 4;
   if (R <= kLaneRadius)
-    hipLaunchKernelGGL((k_gauss_line_run<LAST, false, TS>), grid, dim3(256), lds, s, src, dst, dog,
-                       w1, w2, r1, r2, nz, W, L, sa, so, (unsigned)nxb, (unsigned)n_other, len);
+    hipLaunchKernelGGL((k_gauss_line_run<DOT, false, TS>), grid, dim3(256), lds, s, src, dog, a,
+                       dots, w1, w2, r1, r2, nz, W, D, WH, (i64)W, (unsigned)nxb, (unsigned)H, len);
   else
-    hipLaunchKernelGGL((k_gauss_line_run<LAST, true, TS>), grid, dim3(256), lds, s, src, dst, dog,
-                       w1, w2, r1, r2, nz, W, L, sa, so, (unsigned)nxb, (unsigned)n_other, len);
+    hipLaunchKernelGGL((k_gauss_line_run<DOT, true, TS>), grid, dim3(256), lds, s, src, dog, a,
+                       dots, w1, w2, r1, r2, nz, W, D, WH, (i64)W, (unsigned)nxb, (unsigned)H, len);
   return hipGetLastError();
 }
 
@@ -705,45 +668,46 @@ template <typename TN, typename TD>
 hipError_t launch_dog(const TN* norm, TD* dog, void* tmp1, const float* weights,
                       const int r[4], float normalizer, int W, int H, int D, hipStream_t s,
                       int segments) {
-  const i64 WH = (i64)W * H;
   const float* wxy1 = weights;
   const float* wz1 = weights + kMaxTaps;
   const float* wxy2 = weights + 2 * kMaxTaps;
   const float* wz2 = weights + 3 * kMaxTaps;
-  hipError_t e = gauss_xy<TN>(norm, (float2*)tmp1, wxy1, wxy2, r[0], r[2], W, H, D, s, segments);
+  hipError_t e = gauss_xy<false, TN>(norm, (float2*)tmp1, wxy1, wxy2, wxy1, wxy2, r[0], r[2], W, H,
+                                     D, s, segments);
   if (e != hipSuccess) return e;
   mark("dog/gauss_xy", s);
-  e = gauss_line<true, TD>((const float2*)tmp1, nullptr, dog, wz1, wz2, r[1], r[3], normalizer, W,
-                           D, WH, W, H, s);
+  e = gauss_z<false, TD>((const float2*)tmp1, dog, nullptr, nullptr, wz1, wz2, r[1], r[3],
+                         normalizer, W, H, D, s);
   mark("dog/gauss_z_dog", s);
   return e;
 }
 
-// Separable pair of Gaussians with independent weights per axis (w[0..2] = x, y, z of the
-// first, w[3..5] of the second; radii r[6]).  With dog != nullptr the z pass writes
-// (G1 - G2) * nz; otherwise it writes the (G1, G2) pair to pair_out.  Used by the
-// differentiable form (anisotropic sigmas and their weight derivatives).
-hipError_t launch_gauss_pair(const float* src, void* tmp1, void* tmp2, const float* const w[6],
-                             const int r[6], float nz, float* dog, float2* pair_out, int W, int H,
-                             int D, hipStream_t s) {
-  const i64 WH = (i64)W * H;
-  hipError_t e;
-  if (has_pair(r[0], r[3]) && has_pair(r[1], r[4])) {
-    if ((e = gauss_x<float>(src, (float2*)tmp1, w[0], w[3], r[0], r[3], W, (i64)H * D, s)) !=
-        hipSuccess)
-      return e;
-    e = gauss_line<false, float>((const float2*)tmp1, (float2*)tmp2, nullptr, w[1], w[4], r[1],
-                                 r[4], 0.0f, W, H, W, WH, D, s);
-  } else {
-    e = gauss_xy_run<float>(src, (float2*)tmp2, w[0], w[3], w[1], w[4], r[0], r[3], r[1], r[4], W,
-                            H, D, s, 0);
-  }
+// The differentiable form's pair: weights of their own per axis (anisotropic sigmas and their
+// derivatives).  x and y fused as in the detector (in two passes over the pair volume: 118 +
+// 140 us at radii 8 / 13 and 128 x 512 x 512, here 148).
+static hipError_t gauss_xy_axes(const float* src, void* tmp1, const float* const w[6],
+                                const int r[6], int W, int H, int D, hipStream_t s) {
+  if (r[0] == r[1] && r[3] == r[4])
+    return gauss_xy<true, float>(src, (float2*)tmp1, w[0], w[3], w[1], w[4], r[0], r[3], W, H, D, s,
+                                 0);
+  return gauss_xy_run<float>(src, (float2*)tmp1, w[0], w[3], w[1], w[4], r[0], r[3], r[1], r[4], W,
+                             H, D, s, 0);
+}
+
+hipError_t launch_gauss_dog(const float* src, void* tmp1, const float* const w[6], const int r[6],
+                            float nz, float* dog, int W, int H, int D, hipStream_t s) {
+  const hipError_t e = gauss_xy_axes(src, tmp1, w, r, W, H, D, s);
   if (e != hipSuccess) return e;
-  if (dog)
-    return gauss_line<true, float>((const float2*)tmp2, nullptr, dog, w[2], w[5], r[2], r[5], nz, W,
-                                   D, WH, W, H, s);
-  return gauss_line<false, float>((const float2*)tmp2, pair_out, nullptr, w[2], w[5], r[2], r[5],
-                                  0.0f, W, D, WH, W, H, s);
+  return gauss_z<false, float>((const float2*)tmp1, dog, nullptr, nullptr, w[2], w[5], r[2], r[5],
+                               nz, W, H, D, s);
+}
+
+hipError_t launch_gauss_dots(const float* src, void* tmp1, const float* const w[6], const int r[6],
+                             const float* a, double* out, int W, int H, int D, hipStream_t s) {
+  const hipError_t e = gauss_xy_axes(src, tmp1, w, r, W, H, D, s);
+  if (e != hipSuccess) return e;
+  return gauss_z<true, float>((const float2*)tmp1, nullptr, a, out, w[2], w[5], r[2], r[5], 0.0f, W,
+                              H, D, s);
 }
 
 #define HDOG_INST_DOG(TN, TD)                                                                \

@@ -296,6 +296,28 @@ __device__ __forceinline__ unsigned xcd_tile(unsigned b, unsigned n) {
   return j * q + min(j, r) + b / X;
 }
 
+// Adds the sums of a[k] over a work-group of NT threads to out[k] (K <= 2) with one FP64
+// atomic each: a handful of atomics meet at one address (one per wave over a grid sized for
+// the volume serialized hundreds of thousands of them there).
+constexpr int kReduceGroups = 1024;  // work-groups of a pass that is a reduction only
+template <int NT, int K>
+__device__ __forceinline__ void group_add(double (&a)[K], double* out) {
+  __shared__ double part[NT / 64][K];
+#pragma unroll
+  for (int k = 0; k < K; ++k)
+    for (int o = 32; o > 0; o >>= 1) a[k] += __shfl_down(a[k], o, 64);
+  if ((threadIdx.x & 63) == 0)
+#pragma unroll
+    for (int k = 0; k < K; ++k) part[threadIdx.x >> 6][k] = a[k];
+  __syncthreads();
+  if (threadIdx.x < K) {
+    double t = 0.0;
+#pragma unroll
+    for (int w = 0; w < NT / 64; ++w) t += part[w][threadIdx.x];
+    unsafeAtomicAdd(out + threadIdx.x, t);
+  }
+}
+
 // One zero-padded central difference ((0 + hi) - lo) * 0.5 in the reference's order; the
 // Hessian kernel and the region pass that recomputes the Hessian share it.
 __device__ __forceinline__ float cdiff_half(float hi, float lo) {
@@ -334,9 +356,13 @@ hipError_t launch_dog(const TN* norm, TD* dog, void* tmp1, const float* weights,
 // how the xy walkers of the two stages split planes of W columns, D of them
 WalkShape norm_walk_shape(int rxy, int W, int D);
 WalkShape gauss_walk_shape(int r1, int r2, int W, int D);
-hipError_t launch_gauss_pair(const float* src, void* tmp1, void* tmp2, const float* const w[6],
-                             const int r[6], float nz, float* dog, float2* pair_out, int W, int H,
-                             int D, hipStream_t s);
+// Differentiable form: separable pair of Gaussians, weights w[0..2] = x, y, z of the first and
+// w[3..5] of the second, each symmetric, radii r[6]; tmp1 >= 8*N bytes.  launch_gauss_dog:
+// dog = (G1 - G2) * nz; launch_gauss_dots: out[0] += <a, G1>, out[1] += <a, G2>.
+hipError_t launch_gauss_dog(const float* src, void* tmp1, const float* const w[6], const int r[6],
+                            float nz, float* dog, int W, int H, int D, hipStream_t s);
+hipError_t launch_gauss_dots(const float* src, void* tmp1, const float* const w[6], const int r[6],
+                             const float* a, double* out, int W, int H, int D, hipStream_t s);
 template <typename TD, typename TH>
 // hess and pd may be NULL (not written).  cand / cand_cnt (optional): per Hessian tile
 // (kHessTX x kHessTY x kHessTZ, tiles x-fastest), the number of candidate voxels and their
@@ -466,8 +492,6 @@ hipError_t launch_soft_normalize_adjoint(const float* v, const float2* ed, const
                                          const float* gn, float* gv, void* scratch,
                                          float min_int, int W, int H, int D, int rxy, int rz,
                                          hipStream_t s);
-// out[0] += <a, pair.x>, out[1] += <a, pair.y>
-hipError_t launch_dot_pair(const float* a, const float2* pair, i64 N, double* out, hipStream_t s);
 hipError_t launch_synth(uint16_t* img, float* scratch, int W, int H, int D, u64 seed,
                         double mean0, double mean1, double sd, const double* d_blobs,
                         i64 n_blobs, hipStream_t s);

@@ -37,33 +37,6 @@ namespace {
 
 constexpr int NT = 256;
 
-__device__ __forceinline__ double wave_sum(double v) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-  return v;
-}
-
-// Adds the work-group's sums of a[k] to out[k] (K <= 2) with one FP64 atomic each: the
-// reductions run on a grid of at most kReduceGroups work-groups, so a handful of atomics
-// meet at one address (one atomic per wave over a grid sized for the volume serialized
-// hundreds of thousands of them there).
-constexpr int kReduceGroups = 1024;
-template <int K>
-__device__ __forceinline__ void group_add(double (&a)[K], double* out) {
-  __shared__ double part[NT / 64][K];
-#pragma unroll
-  for (int k = 0; k < K; ++k) a[k] = wave_sum(a[k]);
-  if ((threadIdx.x & 63) == 0)
-#pragma unroll
-    for (int k = 0; k < K; ++k) part[threadIdx.x >> 6][k] = a[k];
-  __syncthreads();
-  if (threadIdx.x < K) {
-    double t = 0.0;
-#pragma unroll
-    for (int w = 0; w < NT / 64; ++w) t += part[w][threadIdx.x];
-    unsafeAtomicAdd(out + threadIdx.x, t);
-  }
-}
-
 __device__ __forceinline__ double det3(double xx, double xy, double xz, double yy, double yz,
                                        double zz) {
   return xx * yy * zz + 2 * xy * yz * xz - xx * yz * yz - yy * xz * xz - zz * xy * xy;
@@ -109,7 +82,7 @@ __global__ __launch_bounds__(NT) void k_soft_loss(const float* __restrict__ cand
     }
   }
   double a[2] = {ls, cnt};
-  group_add<2>(a, sums);
+  group_add<NT>(a, sums);
 }
 
 // the records' elements are overwritten by dL/dH; sums[0] += dL/dtau contributions
@@ -146,7 +119,7 @@ __global__ __launch_bounds__(NT) void k_soft_grad_h(float* __restrict__ cand,
     }
   }
   double a[1] = {gt};
-  group_add<1>(a, sums);
+  group_add<NT>(a, sums);
 }
 
 // dL/ddog from the records of dL/dH, and *dot += <dL/ddog, dog>:
@@ -299,7 +272,7 @@ __global__ __launch_bounds__(NT, 4) void k_hessian_adjoint(const float* __restri
     }
   }
   double a[1] = {acc};
-  group_add<1>(a, dot);
+  group_add<NT>(a, dot);
 }
 
 // Line kernels run one element per thread on a grid of nxb x-blocks per row (y + H z):
@@ -320,21 +293,6 @@ __device__ __forceinline__ bool pos_of(int W, int H, unsigned nxb, Pos& p) {
 unsigned xblocks(int W) { return (unsigned)((W + NT - 1) / NT); }
 unsigned grid_rows(int W, int H, int D) { return xblocks(W) * (unsigned)H * (unsigned)D; }
 
-// out[0] += <a, pair.x>, out[1] += <a, pair.y>
-__global__ __launch_bounds__(NT) void k_dot_pair(const float* __restrict__ a,
-                                                 const float2* __restrict__ pair, i64 N,
-                                                 double* out) {
-  double s0 = 0.0, s1 = 0.0;
-  for (i64 i = (i64)blockIdx.x * NT + threadIdx.x; i < N; i += (i64)gridDim.x * NT) {
-    const double v = a[i];
-    const float2 p = pair[i];
-    s0 += v * p.x;
-    s1 += v * p.y;
-  }
-  double t[2] = {s0, s1};
-  group_add<2>(t, out);
-}
-
 __global__ __launch_bounds__(NT) void k_pack_pair(const float* __restrict__ a,
                                                   const float* __restrict__ b,
                                                   float2* __restrict__ out, i64 N) {
@@ -347,10 +305,6 @@ __global__ void k_zero_f64(double* p, int n) {
 }
 
 unsigned grid_for(i64 N) { return (unsigned)std::min<i64>((N + NT - 1) / NT, 1 << 16); }
-unsigned grid_reduce(i64 N) {
-  return (unsigned)std::max<i64>(1, std::min<i64>((N + NT - 1) / NT, kReduceGroups));
-}
-
 struct Line {  // the line through a voxel along one axis
   i64 base, stride;
   int c, L;
@@ -881,11 +835,6 @@ hipError_t launch_hessian_adjoint(const float* cand, const TileRow* rows, const 
 
 hipError_t launch_zero_f64(double* p, int n, hipStream_t s) {
   hipLaunchKernelGGL(k_zero_f64, dim3(1), dim3(64), 0, s, p, n);
-  return hipGetLastError();
-}
-
-hipError_t launch_dot_pair(const float* a, const float2* pair, i64 N, double* out, hipStream_t s) {
-  hipLaunchKernelGGL(k_dot_pair, dim3(grid_reduce(N)), dim3(NT), 0, s, a, pair, N, out);
   return hipGetLastError();
 }
 

@@ -255,3 +255,32 @@ def test_soft_gradient_of_given_masks(hd, shape, kind):
     err = float((gv.cpu().double() - v64.grad).abs().max())
     assert err <= 2e-3 * float(v64.grad.abs().max())
     assert abs(float(gtau) - float(t64.grad)) <= 2e-3 * abs(float(t64.grad)) + 1e-6
+
+
+# soft response, sigma gradients through each pair of passes: one compiled radius pair along x
+# and y, two, none, more weights than lanes along z.  Bound of the other gradient tests, on the
+# scale of the largest (FP32 volumes of unit size: some 1e-6 of it)
+@pytest.mark.parametrize("s1,s2", [([1.6, 2.0, 2.0], [2.56, 3.2, 3.2]),
+                                   ([2.0, 1.6, 2.0], [3.2, 2.56, 3.2]),
+                                   ([1.1, 2.3, 0.9], [1.9, 3.1, 1.7]),
+                                   ([8.0, 1.0, 1.2], [9.0, 1.6, 1.5])])
+def test_soft_sigma_gradients_of_any_radii(hd, s1, s2):
+    import soft_reference as ref
+    import torch
+    from hdog import soft
+    shape = (19, 21, 70)
+    rad1, rad2 = soft.radii(s1), soft.radii(s2)
+    rng = np.random.default_rng(5)
+    v = torch.from_numpy(rng.standard_normal(shape).astype(np.float32))
+    t = torch.from_numpy((rng.random(shape) < 0.1).astype(np.uint8))
+    a, b = (torch.tensor(s, dtype=torch.float64, requires_grad=True) for s in (s1, s2))
+    tau = torch.tensor(0.05, dtype=torch.float64)
+    vd, td = v.to(hd.device), t.to(hd.device)
+    mask = soft.run_forward(hd, vd, td, s1, s2, 0.05, rad1, rad2)[3].cpu()
+    soft.soft_loss(hd, vd, td, a, b, tau, rad1, rad2).backward()
+    got = torch.cat([a.grad, b.grad])
+    a2, b2 = (torch.tensor(s, dtype=torch.float64, requires_grad=True) for s in (s1, s2))
+    ref.forward(v.double(), a2, b2, tau, t, rad1, rad2, mask=mask.bool())[0].backward()
+    want = torch.cat([a2.grad, b2.grad])
+    assert int(mask.sum()) > 100
+    assert float((got - want).abs().max()) <= 2e-3 * float(want.abs().max())
