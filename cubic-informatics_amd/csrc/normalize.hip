@@ -21,7 +21,7 @@
 //     column walkers: one thread per line keeps a compile-time-sized register ring, reads
 //     every input once and needs no LDS.  Other radii up to kRunRadius have walks with the
 //     radius at run time and their history in LDS, larger ones the LDS-tile kernels.
-#include "hdog_internal.hpp"
+#include "run8.hpp"
 
 namespace hdog {
 namespace {
@@ -692,12 +692,7 @@ __global__ __launch_bounds__(64) void k_norm_xy_walk(const uint32_t* __restrict_
 }
 
 // ---- radii without a kernel of their own, up to kRunRadius ---------------------------
-// The same passes with the radius at run time, eight outputs at a time: each input is read
-// once per group of eight, and the taps that all eight share are taken together.  next()
-// gives the inputs c - r, c - r + 1, ... c + 7 + r in order; R > 0 fixes the radius, for
-// windows shorter than the group (r <= 3), R = 0 takes r >= 4 at run time.
-constexpr int OK = 8;
-constexpr int kRunRadius = 24;
+// The same passes with the radius at run time, eight outputs at a time (run8.hpp).
 
 // out[o] = packed minimum of inputs o .. o + 2r
 template <int R, typename F>
@@ -739,56 +734,6 @@ __device__ __forceinline__ void min8(F&& next, int r, uint32_t (&out)[OK]) {
       if (o > 1) t = pkmin(t, e[o - 1]);
       out[o] = pkmin(out[o], t);
     }
-  }
-}
-
-// acc[o] = 0 + input o + input o + 1 ... + input o + 2r, in that order
-template <int R, typename F>
-__device__ __forceinline__ void sum8(F&& next, int r, float (&acc)[OK]) {
-#pragma unroll
-  for (int o = 0; o < OK; ++o) acc[o] = 0.0f;
-  if constexpr (R > 0) {
-    float v[2 * R + OK];
-#pragma unroll
-    for (int i = 0; i < 2 * R + OK; ++i) v[i] = next();
-#pragma unroll
-    for (int i = 0; i < 2 * R + OK; ++i)
-#pragma unroll
-      for (int o = 0; o < OK; ++o)
-        if (i - o >= 0 && i - o <= 2 * R) acc[o] += v[i];
-  } else {
-    float h[OK - 1], v[4], e[OK - 1];
-#pragma unroll
-    for (int i = 0; i < OK - 1; ++i) h[i] = next();
-#pragma unroll
-    for (int q = 0; q < 2; ++q) v[q] = next();
-#pragma unroll
-    for (int i = 0; i < OK - 1; ++i)
-#pragma unroll
-      for (int o = 0; o <= i; ++o) acc[o] += h[i];
-    // inputs 7 .. 2r meet all eight (an even number), two always read ahead
-    int i = OK - 1;
-#pragma unroll 1
-    for (; i + 3 <= 2 * r; i += 2) {
-#pragma unroll
-      for (int q = 2; q < 4; ++q) v[q] = next();
-#pragma unroll
-      for (int q = 0; q < 2; ++q)
-#pragma unroll
-        for (int o = 0; o < OK; ++o) acc[o] += v[q];
-      v[0] = v[2];
-      v[1] = v[3];
-    }
-#pragma unroll
-    for (int q = 0; q < OK - 1; ++q) e[q] = next();
-#pragma unroll
-    for (int q = 0; q < 2; ++q)
-#pragma unroll
-      for (int o = 0; o < OK; ++o) acc[o] += v[q];
-#pragma unroll
-    for (int u = 1; u < OK; ++u)
-#pragma unroll
-      for (int o = u; o < OK; ++o) acc[o] += e[u - 1];
   }
 }
 
@@ -837,24 +782,6 @@ __device__ __forceinline__ void sum8_u16(F&& next, int r, uint32_t (&lo)[OK], ui
       hi[o] = hi[o - 1] + (e[o - 1] >> 16) - (h[o - 1] >> 16);
     }
   }
-}
-
-// Where a work-group of four waves stands on its lines: 64 x-adjacent lines, eight positions
-// per wave and step of 32.
-struct RunAt {
-  int l, wave, x0, s0, s1;
-  i64 base;
-};
-__device__ __forceinline__ RunAt run_at(int L, i64 so, unsigned nxb, unsigned no, int len) {
-  RunAt a;
-  a.l = (int)(threadIdx.x & 63);
-  a.wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const unsigned t = xcd_tile(blockIdx.x, gridDim.x);
-  a.x0 = (int)(t % nxb) * 64;
-  a.base = (i64)(t / nxb % no) * so;
-  a.s0 = (int)(t / nxb / no) * len;
-  a.s1 = min(L, a.s0 + len);
-  return a;
 }
 
 // Packed min / max along y or z: a work-group walks a segment of 64 lines through an LDS plane
@@ -1143,28 +1070,6 @@ hipError_t dispatch_xw(int XW, F&& f) {
   if (XW == 64) return f(std::integral_constant<int, 64>{});
   if (XW == 32) return f(std::integral_constant<int, 32>{});
   return f(std::integral_constant<int, 16>{});
-}
-
-// f with the radius fixed for windows shorter than a group of outputs, else 0
-template <typename F>
-hipError_t dispatch_short(int r, F&& f) {
-  static_assert(OK == 8, "2 * 3 + 1 < 8");
-  switch (r) {
-    case 1: return f(std::integral_constant<int, 1>{});
-    case 2: return f(std::integral_constant<int, 2>{});
-    case 3: return f(std::integral_constant<int, 3>{});
-    default: return f(std::integral_constant<int, 0>{});
-  }
-}
-// grid of a walk over 64-line strips by work-groups of four waves
-LineGrid run_grid(int W, int L, i64 n_other, int halo) {
-  LineGrid g;
-  g.nxb = (unsigned)((W + 63) / 64);
-  g.no = (unsigned)n_other;
-  int nseg;
-  line_segments(L, (i64)g.nxb * n_other * 4, 1024.0, 2.0, false, halo, &nseg, &g.len);
-  g.blocks = (unsigned)((i64)g.nxb * n_other * nseg);
-  return g;
 }
 
 template <int R>

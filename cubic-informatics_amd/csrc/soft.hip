@@ -30,7 +30,7 @@
 // (the lowest linear index among equal minima), likewise for the max.  The argmin / argmax
 // of the 3-D window are found by three separable passes over (value, index) pairs, which
 // is exact because the order "smaller value, then smaller index" is total.
-#include "hdog_internal.hpp"
+#include "run8.hpp"
 
 namespace hdog {
 namespace {
@@ -318,6 +318,444 @@ __device__ __forceinline__ Line line_at(const Pos& p, int axis, int W, int H, in
   return l;
 }
 
+// ---- radii up to kArgRadius: eight outputs at a time (run8.hpp) ------------------------
+// Window extremes with their positions.  A value travels as a 32-bit key that orders as the
+// floats do (-0 taken as +0, as == takes them), one for the minimum, kx = kn + 1 for the
+// maximum: a NaN, which no window picks, is the largest kn and the smallest kx.  Windows are
+// joined front to back and the earlier one wins a tie, so with x, then y, then z a window's
+// extreme is the one of the lowest linear index.  Its position travels as its taps (0 .. 2r)
+// along the axes so far, eight bits each.
+struct Arg {
+  uint32_t kn, kx, cn, cx;  // keys, taps
+};
+__device__ __forceinline__ uint32_t order_key(float v) {
+  const uint32_t b = __float_as_uint(v + 0.0f);
+  const uint32_t k = b ^ ((uint32_t)((int)b >> 31) | 0x80000000u);
+  return v != v ? 0xFFFFFFFFu : k;
+}
+__device__ __forceinline__ float key_value(uint32_t k) {
+  return __uint_as_float(k & 0x80000000u ? k ^ 0x80000000u : ~k);
+}
+__device__ __forceinline__ Arg arg_join(const Arg& a, const Arg& b) {  // b comes after a
+  Arg o;
+  o.cn = b.kn < a.kn ? b.cn : a.cn;
+  o.kn = min(a.kn, b.kn);
+  o.cx = b.kx > a.kx ? b.cx : a.cx;
+  o.kx = max(a.kx, b.kx);
+  return o;
+}
+// out[o] = extremes of inputs o .. o + 2r; next(i) gives input i, i = 0, 1, ... 2r + 7
+template <int R, typename F>
+__device__ __forceinline__ void arg8(F&& next, int r, Arg (&out)[OK]) {
+  if constexpr (R > 0) {
+    Arg v[2 * R + OK];
+#pragma unroll
+    for (int i = 0; i < 2 * R + OK; ++i) v[i] = next(i);
+#pragma unroll
+    for (int o = 0; o < OK; ++o) {
+      out[o] = v[o];
+#pragma unroll
+      for (int i = 1; i <= 2 * R; ++i) out[o] = arg_join(out[o], v[o + i]);
+    }
+  } else {
+    Arg h[OK - 1];
+#pragma unroll
+    for (int i = 0; i < OK - 1; ++i) h[i] = next(i);
+    // inputs 7 .. 2r are in every window (an even number, 2r - 6), two always read ahead
+    Arg mid = next(OK - 1), v = next(OK);
+#pragma unroll 1
+    for (int i = OK + 1; i < 2 * r; i += 2) {
+      const Arg n0 = next(i), n1 = next(i + 1);
+      mid = arg_join(arg_join(mid, v), n0);
+      v = n1;
+    }
+    mid = arg_join(mid, v);
+    Arg e[OK - 1];
+#pragma unroll
+    for (int q = 0; q < OK - 1; ++q) e[q] = next(2 * r + 1 + q);
+    Arg t = mid;
+    out[OK - 1] = mid;
+#pragma unroll
+    for (int o = OK - 2; o >= 0; --o) out[o] = t = arg_join(h[o], t);  // inputs o .. 2r
+    t = e[0];
+#pragma unroll
+    for (int o = 1; o < OK; ++o) {
+      if (o > 1) t = arg_join(t, e[o - 1]);
+      out[o] = arg_join(out[o], t);
+    }
+  }
+}
+
+constexpr int kArgRadius = 23;  // the work-group's LDS below stays within 64 KB
+constexpr int kStep = 4 * OK;   // positions per step of a work-group
+constexpr int arg_line_pitch(int r) { return (64 + 2 * r + 7) / 8 * 8 + 1; }
+constexpr size_t arg_xy_lds(int r) {
+  return (size_t)4 * OK * arg_line_pitch(r) * 4 + (size_t)(2 * r + kStep) * (65 * 8 + 66 * 2);
+}
+static_assert(arg_xy_lds(kArgRadius) <= 64 * 1024, "LDS of a launch");
+
+// First and second pass (x, y) of the window extremes: four waves walk the rows of one plane
+// for a strip of 64 columns, eight rows per wave and step.
+//   1. a wave's rows (clamped to the plane, loaded a step ahead) enter its LDS lines as keys;
+//   2. lane (row l % 8, columns 8 (l / 8) ..) forms eight x windows -> three LDS planes of the
+//      last 2r + 32 rows: both keys, and both taps;
+//   3. lane l forms eight y windows of column x0 + l, which leave as keys and taps.
+// 4 bytes in and 12 out per voxel and nothing between the passes: 153 us at 128 x 512 x 512,
+// radius 10 (a kernel per axis, 16 bytes per voxel and side between them, a tap each along x
+// and van Herk blocks along y: 383 + 281).
+template <int R>
+__global__ __launch_bounds__(256) void k_soft_arg_xy(const float* __restrict__ v,
+                                                     uint32_t* __restrict__ pkn,
+                                                     uint32_t* __restrict__ pkx,
+                                                     uint32_t* __restrict__ ptap, int W, int H,
+                                                     int r, int nxs, int nys, int rows) {
+  extern __shared__ uint32_t sm_arg[];
+  constexpr int BP = 65, TP = 66;
+  const int hist = 2 * r, span = 64 + 2 * r, AP = arg_line_pitch(r);
+  const int l = (int)(threadIdx.x & 63);
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  uint32_t* A = sm_arg + wave * (OK * AP);
+  uint32_t* Bn = sm_arg + 4 * (OK * AP);
+  uint32_t* Bx = Bn + (hist + kStep) * BP;
+  uint16_t* Bt = reinterpret_cast<uint16_t*>(Bx + (hist + kStep) * BP);
+  const unsigned t = xcd_tile(blockIdx.x, gridDim.x);
+  const int y0 = (int)(t % (unsigned)nys) * rows, y1 = min(H, y0 + rows);
+  const unsigned tile = t / (unsigned)nys;
+  const int x0 = (int)(tile % (unsigned)nxs) * 64;
+  const i64 pbase = (i64)(tile / (unsigned)nxs) * H * W;
+  int xl[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) xl[j] = clampi(x0 - r + 64 * j + l, 0, W - 1);
+  float q[OK][2];
+  auto fetch = [&](int y) {
+#pragma unroll
+    for (int i = 0; i < OK; ++i) {
+      const float* row = v + pbase + (i64)clampi(y + i, 0, H - 1) * W;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) q[i][j] = row[xl[j]];
+    }
+  };
+  const int xr = l % OK, xg = l / OK;
+  auto xpass = [&](int row, int ahead) {
+#pragma unroll
+    for (int i = 0; i < OK; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        if (64 * j + l < span) A[i * AP + 64 * j + l] = order_key(q[i][j]);
+    fetch(ahead);
+    wave_lds_sync();
+    const uint32_t* p = A + xr * AP + OK * xg;
+    Arg o[OK];
+    arg8<R>([&](int i) -> Arg {
+      const uint32_t k = *p++;
+      return {k, k + 1u, (uint32_t)i, (uint32_t)i};
+    }, r, o);
+    const int at = row + xr;
+#pragma unroll
+    for (int k = 0; k < OK; ++k) {
+      Bn[at * BP + OK * xg + k] = o[k].kn;
+      Bx[at * BP + OK * xg + k] = o[k].kx;
+      Bt[at * TP + OK * xg + k] = (uint16_t)((o[k].cn - k) | (o[k].cx - k) << 8);
+    }
+    wave_lds_sync();
+  };
+  // the rows above the segment (the last eight may reach into the first step's rows, which
+  // are written again after the barrier)
+  const int main0 = y0 + r + OK * wave;
+  if (OK * wave < hist) {
+    fetch(y0 - r + OK * wave);
+    for (int g = wave; OK * g < hist; g += 4)
+      xpass(OK * g, OK * (g + 4) < hist ? y0 - r + OK * (g + 4) : main0);
+  } else {
+    fetch(main0);
+  }
+  __syncthreads();
+  const bool out = x0 + l < W;
+  for (int c0 = y0; c0 < y1; c0 += kStep) {
+    xpass(hist + OK * wave, c0 + kStep + r + OK * wave);
+    __syncthreads();
+    const int c = c0 + OK * wave;
+    if (c < y1) {
+      const uint32_t* pn = Bn + OK * wave * BP + l;
+      const uint32_t* px = Bx + OK * wave * BP + l;
+      const uint16_t* pt = Bt + OK * wave * TP + l;
+      Arg o[OK];
+      arg8<R>([&](int i) -> Arg {
+        const uint32_t tp = *pt;
+        const Arg a = {*pn, *px, (tp & 0xFFu) | (uint32_t)i << 8, tp >> 8 | (uint32_t)i << 8};
+        pn += BP;
+        px += BP;
+        pt += TP;
+        return a;
+      }, r, o);
+      if (out) {
+#pragma unroll
+        for (int k = 0; k < OK; ++k)
+          if (c + k < y1) {
+            const i64 at = pbase + (i64)(c + k) * W + x0 + l;
+            st_nt(pkn + at, o[k].kn);
+            st_nt(pkx + at, o[k].kx);
+            st_nt(ptap + at, (o[k].cn - (k << 8)) | (o[k].cx - (k << 8)) << 16);
+          }
+      }
+    }
+    if (c0 + kStep >= y1) break;  // uniform
+    __syncthreads();
+    shift_rows<256, kStep, BP>(Bn, hist);
+    shift_rows<256, kStep, BP>(Bx, hist);
+    shift_rows<256, kStep, TP>(Bt, hist);
+    __syncthreads();
+  }
+}
+
+// Third pass (z): the extremes leave as (min, max) pairs and linear indices (none: an index of
+// all ones).  Bound by its 28 bytes per voxel: 207 us at 128 x 512 x 512 (van Herk blocks over
+// 16 bytes per voxel, two copies and a pass that paired the values: 226 + 107 + 94).
+template <int R>
+__global__ __launch_bounds__(256) void k_soft_arg_z(const uint32_t* __restrict__ pkn,
+                                                    const uint32_t* __restrict__ pkx,
+                                                    const uint32_t* __restrict__ ptap,
+                                                    float2* __restrict__ pair,
+                                                    uint32_t* __restrict__ amn,
+                                                    uint32_t* __restrict__ amx, int W, int H,
+                                                    int D, int rxy, int r, unsigned nxb,
+                                                    unsigned no, int len) {
+  extern __shared__ uint32_t sm_argz[];
+  const int hist = 2 * r;
+  const i64 sa = (i64)W * H;
+  uint32_t* Bn = sm_argz;
+  uint32_t* Bx = Bn + (hist + kStep) * 64;
+  uint32_t* Bt = Bx + (hist + kStep) * 64;
+  const RunAt a = run_at(D, W, nxb, no, len);
+  const int x = a.x0 + a.l, y = (int)(a.base / W), xc = min(x, W - 1);
+  uint32_t qn[OK], qx[OK], qt[OK];
+  auto fetch = [&](int p) {
+#pragma unroll
+    for (int k = 0; k < OK; ++k) {
+      const i64 at = a.base + (i64)clampi(p + k, 0, D - 1) * sa + xc;
+      qn[k] = pkn[at];
+      qx[k] = pkx[at];
+      qt[k] = ptap[at];
+    }
+  };
+  auto put = [&](int row) {
+#pragma unroll
+    for (int k = 0; k < OK; ++k) {
+      Bn[(row + k) * 64 + a.l] = qn[k];
+      Bx[(row + k) * 64 + a.l] = qx[k];
+      Bt[(row + k) * 64 + a.l] = qt[k];
+    }
+  };
+  for (int g = a.wave; OK * g < hist; g += 4) {  // (the last may reach into the step's rows)
+    fetch(a.s0 - r + OK * g);
+    put(OK * g);
+  }
+  fetch(a.s0 + r + OK * a.wave);
+  __syncthreads();
+  for (int c0 = a.s0; c0 < a.s1; c0 += kStep) {
+    put(hist + OK * a.wave);
+    fetch(c0 + kStep + r + OK * a.wave);
+    __syncthreads();
+    const int c = c0 + OK * a.wave;
+    if (c < a.s1) {
+      const uint32_t* p = Bn + OK * a.wave * 64 + a.l;
+      const int plane = (hist + kStep) * 64;
+      Arg o[OK];
+      arg8<R>([&](int i) -> Arg {
+        const uint32_t tp = p[2 * plane];
+        const Arg b = {p[0], p[plane], (tp & 0xFFFFu) | (uint32_t)i << 16,
+                       tp >> 16 | (uint32_t)i << 16};
+        p += 64;
+        return b;
+      }, r, o);
+      if (x < W) {
+#pragma unroll
+        for (int k = 0; k < OK; ++k) {
+          const int z = c + k;
+          if (z >= a.s1) continue;
+          auto index = [&](uint32_t tap) -> uint32_t {
+            const int jx = clampi(x - rxy + (int)(tap & 0xFFu), 0, W - 1),
+                      jy = clampi(y - rxy + (int)(tap >> 8 & 0xFFu), 0, H - 1),
+                      jz = clampi(z - r + (int)(tap >> 16) - k, 0, D - 1);
+            return ((uint32_t)jz * (uint32_t)H + (uint32_t)jy) * (uint32_t)W + (uint32_t)jx;
+          };
+          const i64 at = a.base + (i64)z * sa + x;
+          const bool none = o[k].kn == 0xFFFFFFFFu;  // NaN only: then kx is 0
+          st_nt(pair + at, make_float2(none ? INFINITY : key_value(o[k].kn),
+                                       none ? -INFINITY : key_value(o[k].kx - 1u)));
+          st_nt(amn + at, none ? 0xFFFFFFFFu : index(o[k].cn));
+          st_nt(amx + at, none ? 0xFFFFFFFFu : index(o[k].cx));
+        }
+      }
+    }
+    if (c0 + kStep >= a.s1) break;  // uniform
+    __syncthreads();
+    shift_rows<256, kStep, 64>(Bn, hist);
+    shift_rows<256, kStep, 64>(Bx, hist);
+    shift_rows<256, kStep, 64>(Bt, hist);
+    __syncthreads();
+  }
+}
+
+// Clamped box means of the pairs along x and y, sums in window order: as k_soft_arg_xy, with
+// the two channels one after the other through the wave's lines.  128 us at 128 x 512 x 512,
+// radius 10 (a pass each, 8 bytes per voxel out and back between them: 156 + 185).
+template <int R>
+__global__ __launch_bounds__(256) void k_soft_box_xy(const float2* __restrict__ src,
+                                                     float2* __restrict__ dst, int W, int H, int r,
+                                                     int nxs, int nys, int rows, float k) {
+  extern __shared__ float sm_bxy[];
+  constexpr int BP = 65;
+  const int hist = 2 * r, span = 64 + 2 * r, AP = arg_line_pitch(r);
+  const int l = (int)(threadIdx.x & 63);
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  float* A = sm_bxy + wave * (OK * AP);
+  float* B1 = sm_bxy + 4 * (OK * AP);
+  float* B2 = B1 + (hist + kStep) * BP;
+  const unsigned t = xcd_tile(blockIdx.x, gridDim.x);
+  const int y0 = (int)(t % (unsigned)nys) * rows, y1 = min(H, y0 + rows);
+  const unsigned tile = t / (unsigned)nys;
+  const int x0 = (int)(tile % (unsigned)nxs) * 64;
+  const i64 pbase = (i64)(tile / (unsigned)nxs) * H * W;
+  int xl[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) xl[j] = clampi(x0 - r + 64 * j + l, 0, W - 1);
+  float2 q[OK][2];
+  auto fetch = [&](int y) {
+#pragma unroll
+    for (int i = 0; i < OK; ++i) {
+      const float2* row = src + pbase + (i64)clampi(y + i, 0, H - 1) * W;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) q[i][j] = row[xl[j]];
+    }
+  };
+  const int xr = l % OK, xg = l / OK;
+  auto xsum = [&](float* b) {
+    wave_lds_sync();
+    const float* p = A + xr * AP + OK * xg;
+    float o[OK];
+    sum8<R>([&] { return *p++; }, r, o);
+#pragma unroll
+    for (int i = 0; i < OK; ++i) b[i] = o[i] * k;
+    wave_lds_sync();
+  };
+  auto xpass = [&](int row, int ahead) {
+    const int b = (row + xr) * BP + OK * xg;
+#pragma unroll
+    for (int i = 0; i < OK; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        if (64 * j + l < span) A[i * AP + 64 * j + l] = q[i][j].x;
+    xsum(B1 + b);
+#pragma unroll
+    for (int i = 0; i < OK; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        if (64 * j + l < span) A[i * AP + 64 * j + l] = q[i][j].y;
+    fetch(ahead);
+    xsum(B2 + b);
+  };
+  const int main0 = y0 + r + OK * wave;
+  if (OK * wave < hist) {
+    fetch(y0 - r + OK * wave);
+    for (int g = wave; OK * g < hist; g += 4)
+      xpass(OK * g, OK * (g + 4) < hist ? y0 - r + OK * (g + 4) : main0);
+  } else {
+    fetch(main0);
+  }
+  __syncthreads();
+  const bool out = x0 + l < W;
+  float2* dcol = dst + pbase + x0 + l;
+  for (int c0 = y0; c0 < y1; c0 += kStep) {
+    xpass(hist + OK * wave, c0 + kStep + r + OK * wave);
+    __syncthreads();
+    const int c = c0 + OK * wave;
+    if (c < y1) {
+      float e[OK], d[OK];
+      const float* p = B1 + OK * wave * BP + l;
+      sum8<R>([&] { const float u = *p; p += BP; return u; }, r, e);
+      p = B2 + OK * wave * BP + l;
+      sum8<R>([&] { const float u = *p; p += BP; return u; }, r, d);
+      if (out) {
+#pragma unroll
+        for (int o = 0; o < OK; ++o)
+          if (c + o < y1) st_nt(dcol + (i64)(c + o) * W, make_float2(e[o] * k, d[o] * k));
+      }
+    }
+    if (c0 + kStep >= y1) break;  // uniform
+    __syncthreads();
+    shift_rows<256, kStep, BP>(B1, hist);
+    shift_rows<256, kStep, BP>(B2, hist);
+    __syncthreads();
+  }
+}
+
+// Clamped box means along z -> (E, D), and the normalization.  Bound by its 24 bytes per
+// voxel: 164 us at 128 x 512 x 512 (in two passes, 104 + 109).
+template <int R>
+__global__ __launch_bounds__(256) void k_soft_box_norm(const float2* __restrict__ src,
+                                                       const float* __restrict__ v,
+                                                       float2* __restrict__ ed,
+                                                       float* __restrict__ norm, float min_int,
+                                                       int W, int D, i64 sa, int r, unsigned nxb,
+                                                       unsigned no, int len, float k) {
+  extern __shared__ float sm_bz[];
+  const int hist = 2 * r;
+  float* B1 = sm_bz;
+  float* B2 = B1 + (hist + kStep) * 64;
+  const RunAt a = run_at(D, W, nxb, no, len);
+  const int xc = min(a.x0 + a.l, W - 1);
+  float2 q[OK];
+  float vq[OK];
+  auto fetch = [&](int p) {
+#pragma unroll
+    for (int j = 0; j < OK; ++j) q[j] = src[a.base + (i64)clampi(p + j, 0, D - 1) * sa + xc];
+  };
+  auto put = [&](int row) {
+#pragma unroll
+    for (int j = 0; j < OK; ++j) {
+      B1[(row + j) * 64 + a.l] = q[j].x;
+      B2[(row + j) * 64 + a.l] = q[j].y;
+    }
+  };
+  for (int g = a.wave; OK * g < hist; g += 4) {
+    fetch(a.s0 - r + OK * g);
+    put(OK * g);
+  }
+  fetch(a.s0 + r + OK * a.wave);
+  __syncthreads();
+  for (int c0 = a.s0; c0 < a.s1; c0 += kStep) {
+    const int c = c0 + OK * a.wave;
+    put(hist + OK * a.wave);
+#pragma unroll
+    for (int j = 0; j < OK; ++j) vq[j] = v[a.base + (i64)min(c + j, D - 1) * sa + xc];
+    fetch(c0 + kStep + r + OK * a.wave);
+    __syncthreads();
+    if (c < a.s1) {
+      float e[OK], d[OK];
+      const float* p = B1 + OK * a.wave * 64 + a.l;
+      sum8<R>([&] { const float u = *p; p += 64; return u; }, r, e);
+      p = B2 + OK * a.wave * 64 + a.l;
+      sum8<R>([&] { const float u = *p; p += 64; return u; }, r, d);
+      if (a.x0 + a.l < W) {
+#pragma unroll
+        for (int j = 0; j < OK; ++j) {
+          if (c + j >= a.s1) continue;
+          const i64 idx = a.base + (i64)(c + j) * sa + a.x0 + a.l;
+          const float ve = e[j] * k, vd = d[j] * k;
+          st_nt(ed + idx, make_float2(ve, vd));
+          st_nt(norm + idx, vq[j] >= min_int ? (vq[j] - ve) / (vd - ve) : 0.0f);
+        }
+      }
+    }
+    if (c0 + kStep >= a.s1) break;  // uniform
+    __syncthreads();
+    shift_rows<256, kStep, 64>(B1, hist);
+    shift_rows<256, kStep, 64>(B2, hist);
+    __syncthreads();
+  }
+}
+
 // one separable pass of the windowed (value, index) minimum and maximum, clamp-to-edge;
 // first pass: indices are the voxels' own (imn == NULL)
 __global__ __launch_bounds__(NT) void k_soft_argminmax(const float* __restrict__ vmn,
@@ -440,93 +878,7 @@ __global__ __launch_bounds__(NT) void k_soft_box_adj_x(const float2* __restrict_
   out[base + p] = make_float2(se * k, sd * k);
 }
 
-// The same pass along y or z (second and third passes, indices given) as a column walker
-// for radius R: one thread per line (x-consecutive threads), van Herk blocks of 2R+1 over
-// the clamp-extended line g[k] = f[clamp(k - R)] held in place in registers (slot j keeps
-// the previous block's suffix extreme until the current block's j-th element takes it; a
-// running prefix extreme covers the current block), so every element is read once instead
-// of 2R+1 times.  Output c leaves when g[c + 2R] has arrived.  (value, index) pairs under
-// "smaller value, then smaller index" (min) and "larger value, then smaller index" (max)
-// form total orders, so the blocks give the window extremes exactly.
-struct Ext {
-  float vn, vx;       // min value, max value
-  uint32_t jn, jx;    // their indices
-};
-// (by value: a select between two elements' fields must not become a select between
-// their addresses, which keeps the register arrays in scratch memory)
-__device__ __forceinline__ Ext ext_join(Ext a, Ext b) {
-  const float an = a.vn, bn = b.vn, ax = a.vx, bx = b.vx;
-  const uint32_t ajn = a.jn, bjn = b.jn, ajx = a.jx, bjx = b.jx;
-  const bool mn = an < bn || (an == bn && ajn < bjn);
-  const bool mx = ax > bx || (ax == bx && ajx < bjx);
-  Ext o;
-  o.vn = mn ? an : bn;
-  o.jn = mn ? ajn : bjn;
-  o.vx = mx ? ax : bx;
-  o.jx = mx ? ajx : bjx;
-  return o;
-}
-template <int R>
-__global__ __launch_bounds__(NT) void k_soft_argminmax_walk(
-    const float* __restrict__ vmn, const uint32_t* __restrict__ imn,
-    const float* __restrict__ vmx, const uint32_t* __restrict__ imx, float* __restrict__ omn,
-    uint32_t* __restrict__ oimn, float* __restrict__ omx, uint32_t* __restrict__ oimx, int W,
-    int L, i64 sa, i64 so, unsigned nxb) {
-  constexpr int WB = 2 * R + 1;
-  constexpr int PF = WB % 3 == 0 ? 3 : 1;  // loads queued PF steps ahead (static slots)
-  const int x = (int)(blockIdx.x % nxb) * NT + (int)threadIdx.x;
-  if (x >= W) return;
-  const i64 base = (i64)(blockIdx.x / nxb) * so + x;
-  auto load = [&](int k) -> Ext {
-    const i64 p = base + (i64)clampi(k - R, 0, L - 1) * sa;
-    Ext e;
-    e.vn = vmn[p];
-    e.jn = imn[p];
-    e.vx = vmx[p];
-    e.jx = imx[p];
-    return e;
-  };
-  auto put = [&](int c, const Ext& e) {
-    const i64 p = base + (i64)c * sa;
-    omn[p] = e.vn;
-    oimn[p] = e.jn;
-    omx[p] = e.vx;
-    oimx[p] = e.jx;
-  };
-  Ext slot[WB], q[PF], P;
-#pragma unroll
-  for (int k = 0; k < PF; ++k) q[k] = load(k);
-  // block 0 (k = 0 .. WB-1) fills the slots; its suffix extreme S[0] is output 0
-#pragma unroll
-  for (int j = 0; j < WB; ++j) {
-    slot[j] = q[j % PF];
-    q[j % PF] = load(j + PF);
-  }
-#pragma unroll
-  for (int j = WB - 2; j >= 0; --j) slot[j] = ext_join(slot[j], slot[j + 1]);
-  put(0, slot[0]);
-  const int kend = L + 2 * R;
-  for (int k0 = WB;; k0 += WB) {
-#pragma unroll
-    for (int j = 0; j < WB; ++j) {
-      const int k = k0 + j;
-      if (k >= kend) return;
-      const Ext v = q[j % PF];  // (k0 + j) % PF == j % PF
-      q[j % PF] = load(k + PF);
-      P = j == 0 ? v : ext_join(P, v);
-      if (j < WB - 1) {
-        put(k - 2 * R, ext_join(slot[j + 1], P));
-        slot[j] = v;
-      } else {
-        slot[j] = v;
-#pragma unroll
-        for (int t = WB - 2; t >= 0; --t) slot[t] = ext_join(slot[t], slot[t + 1]);
-        put(k - 2 * R, slot[0]);
-      }
-    }
-  }
-}
-
+// ---- any radius ------------------------------------------------------------------------
 // clamped box mean of the (E, D) pair along one axis (FP32 sums in window order)
 __global__ __launch_bounds__(NT) void k_soft_box(const float2* __restrict__ in,
                                                  float2* __restrict__ out, int W, int H, int D,
@@ -699,11 +1051,52 @@ __global__ __launch_bounds__(NT) void k_soft_route(const float2* __restrict__ g,
 }  // namespace
 
 // norm, and for the backward pass ed (E, D pairs) and arg (argmin N, then argmax N);
-// scratch: 4 N words + 4 N words
+// scratch: 8 N words (radii up to kArgRadius: 5 N)
 hipError_t launch_soft_normalize(const float* v, float* norm, float2* ed, uint32_t* arg,
                                  void* scratch, float min_int, int W, int H, int D, int rxy,
                                  int rz, hipStream_t s) {
-  const i64 N = (i64)W * H * D;
+  const i64 N = (i64)W * H * D, WH = (i64)W * H;
+  if (rxy <= kArgRadius && rz <= kArgRadius) {
+    uint32_t* pk = (uint32_t*)scratch;       // keys and taps, 3 N words
+    float2* pair = (float2*)(pk + 3 * N);    // 2 N words
+    float2* exy = (float2*)scratch;          // in the place of the keys
+    const int nxs = (W + 63) / 64;
+    int nys, rows;
+    walk_segments(H, WalkShape{(i64)nxs * D * 4, kStep, 2 * rxy}, &nys, &rows);
+    const dim3 grid((unsigned)((i64)nxs * D * nys));
+    const LineGrid g = run_grid(W, D, H, 2 * rz);
+    const float kxy = 1.0f / (float)(2 * rxy + 1), kz = 1.0f / (float)(2 * rz + 1);
+    const size_t zrows = (size_t)(2 * rz + kStep) * 64 * 4;
+    hipError_t e = dispatch_short(rxy, [&](auto rs) {
+      constexpr int R = decltype(rs)::value;
+      hipLaunchKernelGGL((k_soft_arg_xy<R>), grid, dim3(256), arg_xy_lds(rxy), s, v, pk, pk + N,
+                         pk + 2 * N, W, H, rxy, nxs, nys, rows);
+      return hipGetLastError();
+    });
+    if (e != hipSuccess) return e;
+    e = dispatch_short(rz, [&](auto rs) {
+      constexpr int R = decltype(rs)::value;
+      hipLaunchKernelGGL((k_soft_arg_z<R>), dim3(g.blocks), dim3(256), 3 * zrows, s, pk, pk + N,
+                         pk + 2 * N, pair, arg, arg + N, W, H, D, rxy, rz, g.nxb, g.no, g.len);
+      return hipGetLastError();
+    });
+    if (e != hipSuccess) return e;
+    e = dispatch_short(rxy, [&](auto rs) {
+      constexpr int R = decltype(rs)::value;
+      const size_t lds =
+          ((size_t)4 * OK * arg_line_pitch(rxy) + 2 * (size_t)(2 * rxy + kStep) * 65) * 4;
+      hipLaunchKernelGGL((k_soft_box_xy<R>), grid, dim3(256), lds, s, pair, exy, W, H, rxy, nxs,
+                         nys, rows, kxy);
+      return hipGetLastError();
+    });
+    if (e != hipSuccess) return e;
+    return dispatch_short(rz, [&](auto rs) {
+      constexpr int R = decltype(rs)::value;
+      hipLaunchKernelGGL((k_soft_box_norm<R>), dim3(g.blocks), dim3(256), 2 * zrows, s, exy, v, ed,
+                         norm, min_int, W, D, WH, rz, g.nxb, g.no, g.len, kz);
+      return hipGetLastError();
+    });
+  }
   float* a = (float*)scratch;  // ping-pong (value, index) min / max planes
   float* fmn[2] = {a, a + 4 * N};
   const unsigned g = grid_for(N);
@@ -715,15 +1108,7 @@ hipError_t launch_soft_normalize(const float* v, float* norm, float2* ed, uint32
     const float* vmx = axis ? src + 2 * N : v;
     const uint32_t* imn = axis ? (const uint32_t*)(src + N) : nullptr;
     const uint32_t* imx = axis ? (const uint32_t*)(src + 3 * N) : nullptr;
-    if (axis > 0 && rad[axis] == 10) {  // y or z: column walker
-      const i64 WH = (i64)W * H;
-      const int L = axis == 1 ? H : D;
-      const i64 sa = axis == 1 ? W : WH, so = axis == 1 ? WH : W;
-      const i64 n_other = axis == 1 ? D : H;
-      hipLaunchKernelGGL((k_soft_argminmax_walk<10>), dim3((unsigned)(xblocks(W) * n_other)),
-                         dim3(NT), 0, s, vmn, imn, vmx, imx, dst, (uint32_t*)(dst + N), dst + 2 * N,
-                         (uint32_t*)(dst + 3 * N), W, L, sa, so, xblocks(W));
-    } else if (axis == 0 && rad[0] <= kXR) {  // x, the first pass: indices are positions
+    if (axis == 0 && rad[0] <= kXR) {  // x, the first pass: indices are positions
       hipLaunchKernelGGL(k_soft_argminmax_x, dim3(grid_rows(W, H, D)), dim3(NT), 0, s, v, dst,
                          (uint32_t*)(dst + N), dst + 2 * N, (uint32_t*)(dst + 3 * N), W, rad[0],
                          xblocks(W));
@@ -744,7 +1129,6 @@ hipError_t launch_soft_normalize(const float* v, float* norm, float2* ed, uint32
   float2* p1 = ed;
   hipLaunchKernelGGL(k_pack_pair, dim3(g), dim3(NT), 0, s, res, res + 2 * N, p0, N);
   float2* bufs[2] = {p0, p1};
-  const i64 WH = (i64)W * H;
   for (int axis = 0; axis < 3; ++axis) {
     // x: p0 -> ed, y: ed -> p0, z: p0 -> ed; y and z by the normalization's box passes
     if (axis == 0 && rad[0] <= kXR) {

@@ -284,3 +284,65 @@ def test_soft_sigma_gradients_of_any_radii(hd, s1, s2):
     want = torch.cat([a2.grad, b2.grad])
     assert int(mask.sum()) > 100
     assert float((got - want).abs().max()) <= 2e-3 * float(want.abs().max())
+
+
+def soft_normalize_by_hand(v, m, rxy, rz):
+    """Windows of (value, lowest linear index) extremes, NaN skipped (none: +-inf, all ones),
+    FP32 box sums in window order; x, then y, then z."""
+    shape, N = v.shape, v.size
+    mn, mx = (np.where(np.isnan(v), np.float32(f), v) for f in (np.inf, -np.inf))
+    own = np.where(np.isnan(v), 0xFFFFFFFF, np.arange(N).reshape(shape)).astype(np.uint32)
+    jn, jx = own.copy(), own.copy()
+    for axis, r in ((2, rxy), (1, rxy), (0, rz)):
+        taps = [np.clip(np.arange(shape[axis]) + t, 0, shape[axis] - 1) for t in range(-r, r + 1)]
+        for f, j, best in ((mn, jn, np.less), (mx, jx, np.greater)):
+            g, h = f.copy(), j.copy()
+            for t in taps:
+                a, k = np.take(f, t, axis), np.take(j, t, axis)
+                take = best(a, g) | ((a == g) & (k < h))
+                g, h = np.where(take, a, g), np.where(take, k, h)
+            f[...], j[...] = g, h
+    e, d = mn.copy(), mx.copy()
+    for axis, r in ((2, rxy), (1, rxy), (0, rz)):
+        k = np.float32(1) / np.float32(2 * r + 1)
+        for f in (e, d):
+            s = np.zeros_like(f)
+            for t in range(-r, r + 1):
+                s += np.take(f, np.clip(np.arange(shape[axis]) + t, 0, shape[axis] - 1), axis)
+            f[...] = s * k
+    n = np.where(v >= np.float32(m), (v - e) / (d - e), np.float32(0))
+    return n, np.stack([e, d], -1), np.stack([jn, jx])
+
+
+# soft normalization forward: windows shorter than a group of outputs, longer, the longest with
+# a walk, beyond; lines shorter than the window, strips and segments with remainders; ties,
+# signed zeros, infinities and windows of NaN only
+@pytest.mark.parametrize("rxy,rz", [(1, 1), (2, 3), (3, 2), (4, 5), (10, 10), (23, 23), (24, 2),
+                                    (5, 24)])
+@pytest.mark.parametrize("kind", ["noise", "ties", "special"])
+def test_soft_normalization_bitexact(hd, rxy, rz, kind):
+    import torch
+    from hdog import _capi as C
+    shape = (37, 43, 133) if kind != "special" else (5, 9, 70)
+    rng = np.random.default_rng(rxy)
+    v = rng.standard_normal(shape).astype(np.float32)
+    if kind == "ties":
+        v = np.round(v)  # -0 and +0 among them
+    if kind == "special":
+        v[:, :, 0:30] = np.nan
+        v[:, 3:, 40:60] = np.inf
+        v[2:, :, 65:] = -np.inf
+    D, H, W = shape
+    vd = torch.from_numpy(v).to(hd.device)
+    n = torch.empty_like(vd)
+    ed = torch.empty(shape + (2,), dtype=torch.float32, device=hd.device)
+    arg = torch.empty((2,) + shape, dtype=torch.int32, device=hd.device)
+    p = C.ctypes.c_void_p
+    hd._check(C.hdog_soft_normalize_forward(hd._h, hd._stream(), p(vd.data_ptr()), p(n.data_ptr()),
+                                            p(ed.data_ptr()), p(arg.data_ptr()), -0.25, W, H, D,
+                                            rxy, rz))
+    with np.errstate(all="ignore"):
+        wn, wed, warg = soft_normalize_by_hand(v, -0.25, rxy, rz)
+    np.testing.assert_array_equal(arg.cpu().numpy().view(np.uint32), warg)
+    np.testing.assert_array_equal(ed.cpu().numpy(), wed)
+    np.testing.assert_array_equal(n.cpu().numpy(), wn)
