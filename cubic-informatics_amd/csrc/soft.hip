@@ -392,7 +392,21 @@ constexpr int arg_line_pitch(int r) { return (64 + 2 * r + 7) / 8 * 8 + 1; }
 constexpr size_t arg_xy_lds(int r) {
   return (size_t)4 * OK * arg_line_pitch(r) * 4 + (size_t)(2 * r + kStep) * (65 * 8 + 66 * 2);
 }
-static_assert(arg_xy_lds(kArgRadius) <= 64 * 1024, "LDS of a launch");
+static_assert(arg_xy_lds(kArgRadius) <= 64 * 1024, "LDS of a launch");  // the largest
+constexpr size_t box_xy_lds(int r) {
+  return ((size_t)4 * OK * arg_line_pitch(r) + 2 * (size_t)(2 * r + kStep) * 65) * 4;
+}
+struct XyRun {  // grid of a walk over the rows of 64-column strips
+  int nxs, nys, rows;
+  unsigned blocks;
+};
+XyRun xy_run(int W, int H, int D, int r) {
+  XyRun x;
+  x.nxs = (W + 63) / 64;
+  walk_segments(H, WalkShape{(i64)x.nxs * D * 4, kStep, 2 * r}, &x.nys, &x.rows);
+  x.blocks = (unsigned)((i64)x.nxs * D * x.nys);
+  return x;
+}
 
 // First and second pass (x, y) of the window extremes: four waves walk the rows of one plane
 // for a strip of 64 columns, eight rows per wave and step.
@@ -878,6 +892,298 @@ __global__ __launch_bounds__(NT) void k_soft_box_adj_x(const float2* __restrict_
   out[base + p] = make_float2(se * k, sd * k);
 }
 
+// Transpose of the clamped box mean over eight positions c .. c + 7 of a line of L (radius r):
+// acc holds the window sums over the line (zero outside it); the border positions also
+// receive the taps that clamp onto them.  B: position `first` of the line, `pitch` apart.
+__device__ __forceinline__ void add_clamped(const float* B, int pitch, int first, int c, int L,
+                                            int r, float (&acc)[OK]) {
+  if (c == 0)  // taps c - r + j < 0 of the windows of c < r
+    for (int i = 0; i <= min(L - 1, r - 1); ++i) acc[0] += B[(i - first) * pitch] * (float)(r - i);
+  if (c <= L - 1 && L - 1 < c + OK) {  // taps beyond L - 1 of the windows of c > L - 1 - r
+    float t = 0.0f;
+    for (int i = max(0, L - r); i <= L - 1; ++i)
+      t += B[(i - first) * pitch] * (float)(i + r - L + 1);
+#pragma unroll
+    for (int o = 0; o < OK; ++o)
+      if (c + o == L - 1) acc[o] += t;
+  }
+}
+
+// Adjoint of the normalization and, transposed, of its z boxes: the direct term into gv, (dL/dE,
+// dL/dD) summed along z into dst.  Bound by its 28 bytes per voxel: 184 us at 128 x 512 x 512,
+// radius 10 (in two passes, 152 + 112).
+template <int R>
+__global__ __launch_bounds__(256) void k_soft_adj_z(const float* __restrict__ v,
+                                                    const float2* __restrict__ ed,
+                                                    const float* __restrict__ gn,
+                                                    float* __restrict__ gv,
+                                                    float2* __restrict__ dst, float min_int, int W,
+                                                    int D, i64 sa, int r, unsigned nxb,
+                                                    unsigned no, int len, float k) {
+  extern __shared__ float sm_adjz[];
+  const int hist = 2 * r;
+  float* B1 = sm_adjz;
+  float* B2 = B1 + (hist + kStep) * 64;
+  const RunAt a = run_at(D, W, nxb, no, len);
+  const bool out = a.x0 + a.l < W;
+  const int xc = min(a.x0 + a.l, W - 1);
+  float qv[OK], qg[OK];
+  float2 qe[OK];
+  auto fetch = [&](int p) {
+#pragma unroll
+    for (int j = 0; j < OK; ++j) {
+      const i64 at = a.base + (i64)clampi(p + j, 0, D - 1) * sa + xc;
+      qv[j] = v[at];
+      qe[j] = ed[at];
+      qg[j] = gn[at];
+    }
+  };
+  auto put = [&](int row, int p) {  // the fetched positions p .. p + 7
+#pragma unroll
+    for (int j = 0; j < OK; ++j) {
+      const bool in = p + j >= 0 && p + j < D;
+      const float I = qv[j], g = I >= min_int ? qg[j] : 0.0f;
+      const float inv = 1.0f / (qe[j].y - qe[j].x);
+      B1[(row + j) * 64 + a.l] = in ? g * (I - qe[j].y) * inv * inv : 0.0f;
+      B2[(row + j) * 64 + a.l] = in ? -g * (I - qe[j].x) * inv * inv : 0.0f;
+      if (out && p + j >= a.s0 && p + j < a.s1)
+        gv[a.base + (i64)(p + j) * sa + a.x0 + a.l] = g * inv;
+    }
+  };
+  for (int g = a.wave; OK * g < hist; g += 4) {  // (the last may reach into the step's rows)
+    fetch(a.s0 - r + OK * g);
+    put(OK * g, a.s0 - r + OK * g);
+  }
+  fetch(a.s0 + r + OK * a.wave);
+  __syncthreads();
+  for (int c0 = a.s0; c0 < a.s1; c0 += kStep) {
+    const int c = c0 + OK * a.wave;
+    put(hist + OK * a.wave, c + r);
+    fetch(c + kStep + r);
+    __syncthreads();
+    if (c < a.s1) {
+      float e[OK], d[OK];
+      const float* p = B1 + OK * a.wave * 64 + a.l;
+      sum8<R>([&] { const float u = *p; p += 64; return u; }, r, e);
+      p = B2 + OK * a.wave * 64 + a.l;
+      sum8<R>([&] { const float u = *p; p += 64; return u; }, r, d);
+      add_clamped(B1 + a.l, 64, c0 - r, c, D, r, e);
+      add_clamped(B2 + a.l, 64, c0 - r, c, D, r, d);
+      if (out) {
+#pragma unroll
+        for (int j = 0; j < OK; ++j)
+          if (c + j < a.s1)
+            st_nt(dst + a.base + (i64)(c + j) * sa + a.x0 + a.l, make_float2(e[j] * k, d[j] * k));
+      }
+    }
+    if (c0 + kStep >= a.s1) break;  // uniform
+    __syncthreads();
+    shift_rows<256, kStep, 64>(B1, hist);
+    shift_rows<256, kStep, 64>(B2, hist);
+    __syncthreads();
+  }
+}
+
+// Sum of v over the run of equal consecutive keys (lanes of one wave) that starts at each
+// run's first lane, where *head is set; every lane of the wave must be active.  A segmented
+// suffix sum by lane shifts: after the step of offset o each lane holds the sum over
+// [lane, lane + 2o) within its run.
+__device__ __forceinline__ float run_sum(uint32_t key, float v, bool* head) {
+  const int lane = (int)(threadIdx.x & 63);
+  const uint32_t prev = __shfl_up(key, 1, 64);
+  *head = lane == 0 || prev != key;
+  const unsigned long long heads = __ballot(*head);
+  const unsigned long long after = lane == 63 ? 0ull : heads & (~0ull << (lane + 1));
+  const int tail = after ? __builtin_ctzll(after) - 1 : 63;  // last lane of the run
+  for (int o = 1; o < 64; o <<= 1) {
+    const float w = __shfl_down(v, o, 64);
+    if (lane + o <= tail) v += w;
+  }
+  return v;
+}
+
+// Sums per target of the values that a work-group routes in a step, in LDS: windows of a patch
+// share a few dozen extremes.  A target that finds no slot in kProbes (plateaus, where every
+// window has its own extreme) goes to memory, where it is then not contended.
+constexpr uint32_t kNone = 0xFFFFFFFFu;
+constexpr int kRouteSlots = 512, kProbes = 4;
+struct RouteTable {
+  uint32_t* key;
+  float* sum;
+  __device__ __forceinline__ void add(uint32_t k, float s, float* gv) const {
+    uint32_t slot = k * 2654435761u >> 23;
+    static_assert(kRouteSlots == 1 << 9, "hash bits");
+    for (int p = 0; p < kProbes; ++p, slot = (slot + 1) & (kRouteSlots - 1)) {
+      uint32_t cur = key[slot];
+      if (cur == kNone) {
+        cur = atomicCAS(&key[slot], kNone, k);
+        if (cur == kNone) cur = k;
+      }
+      if (cur == k) {
+        __hip_atomic_fetch_add(&sum[slot], s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        return;
+      }
+    }
+    atomicAdd(gv + k, s);
+  }
+  // whole work-group, between barriers: the sums leave (to memory, unless clearing only)
+  __device__ __forceinline__ void flush(float* gv) const {
+    for (int i = (int)threadIdx.x; i < kRouteSlots; i += 256) {
+      const uint32_t k = key[i];
+      if (gv && k != kNone) atomicAdd(gv + k, sum[i]);
+      key[i] = kNone;
+      sum[i] = 0.0f;
+    }
+  }
+};
+// A lane's eight rows of one column: mostly one or two targets, summed before they go to the
+// table, and once more over runs of equal targets in neighbouring columns (LDS adds to one
+// address take turns: 392 us for the whole pass below without, 208 with no routing at all).
+// Rows without a target have key kNone and value 0.
+__device__ __forceinline__ void route8(const uint32_t (&key)[OK], const float (&val)[OK],
+                                       const RouteTable& t, float* gv) {
+  uint32_t k1 = key[0], k2 = kNone;
+  float s1 = val[0], s2 = 0.0f;
+#pragma unroll
+  for (int o = 1; o < OK; ++o) {
+    const uint32_t k = key[o];
+    const bool m1 = k == k1, m2 = !m1 && (k == k2 || k2 == kNone);
+    s1 += m1 ? val[o] : 0.0f;
+    s2 += m2 ? val[o] : 0.0f;
+    k2 = m2 ? k : k2;
+    if (!m1 && !m2 && k != kNone) t.add(k, val[o], gv);
+  }
+  bool h1, h2;
+  s1 = run_sum(k1, s1, &h1);
+  s2 = run_sum(k2, s2, &h2);
+  if (h1 && k1 != kNone) t.add(k1, s1, gv);
+  if (h2 && k2 != kNone) t.add(k2, s2, gv);
+}
+
+// The transposed x and y boxes (walked as k_soft_box_xy, zero outside the plane), and the
+// routing of their sums by subgradient: gv[argmin(i)] += dL/dmin(i), gv[argmax(i)] +=
+// dL/dmax(i).  The sums never leave the chip.  355 us at 128 x 512 x 512, radius 10 (the two
+// boxes and a routing pass with one atomic per run of equal targets in a row of 64: 308 + 183 +
+// 490), of which the routing takes 147: short runs in the maximum's plateaus.
+template <int R>
+__global__ __launch_bounds__(256) void k_soft_adj_xy(const float2* __restrict__ src,
+                                                     const uint32_t* __restrict__ amn,
+                                                     const uint32_t* __restrict__ amx,
+                                                     float* __restrict__ gv, int W, int H, int r,
+                                                     int nxs, int nys, int rows, float k) {
+  extern __shared__ float sm_axy[];
+  constexpr int BP = 65;
+  const int hist = 2 * r, span = 64 + 2 * r, AP = arg_line_pitch(r);
+  const int l = (int)(threadIdx.x & 63);
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  float* A = sm_axy + wave * (OK * AP);
+  float* B1 = sm_axy + 4 * (OK * AP);
+  float* B2 = B1 + (hist + kStep) * BP;
+  const RouteTable table = {reinterpret_cast<uint32_t*>(B2 + (hist + kStep) * BP),
+                            B2 + (hist + kStep) * BP + kRouteSlots};
+  table.flush(nullptr);  // (cleared; barriers follow)
+  const unsigned t = xcd_tile(blockIdx.x, gridDim.x);
+  const int y0 = (int)(t % (unsigned)nys) * rows, y1 = min(H, y0 + rows);
+  const unsigned tile = t / (unsigned)nys;
+  const int x0 = (int)(tile % (unsigned)nxs) * 64;
+  const i64 pbase = (i64)(tile / (unsigned)nxs) * H * W;
+  int xl[2];
+  bool xin[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int x = x0 - r + 64 * j + l;
+    xl[j] = clampi(x, 0, W - 1);
+    xin[j] = x >= 0 && x < W;
+  }
+  float2 q[OK][2];
+  auto fetch = [&](int y) {
+#pragma unroll
+    for (int i = 0; i < OK; ++i) {
+      const float2* row = src + pbase + (i64)clampi(y + i, 0, H - 1) * W;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) q[i][j] = row[xl[j]];
+    }
+  };
+  const int xr = l % OK, xg = l / OK;
+  auto xsum = [&](float* b) {
+    wave_lds_sync();
+    const float* line = A + xr * AP;
+    const float* p = line + OK * xg;
+    float o[OK];
+    sum8<R>([&] { return *p++; }, r, o);
+    add_clamped(line, 1, x0 - r, x0 + OK * xg, W, r, o);
+#pragma unroll
+    for (int i = 0; i < OK; ++i) b[i] = o[i] * k;
+    wave_lds_sync();
+  };
+  auto xpass = [&](int row, int y, int ahead) {  // the fetched rows y .. y + 7
+    const int b = (row + xr) * BP + OK * xg;
+#pragma unroll
+    for (int i = 0; i < OK; ++i) {
+      const bool in = y + i >= 0 && y + i < H;
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        if (64 * j + l < span) A[i * AP + 64 * j + l] = in && xin[j] ? q[i][j].x : 0.0f;
+    }
+    xsum(B1 + b);
+#pragma unroll
+    for (int i = 0; i < OK; ++i) {
+      const bool in = y + i >= 0 && y + i < H;
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        if (64 * j + l < span) A[i * AP + 64 * j + l] = in && xin[j] ? q[i][j].y : 0.0f;
+    }
+    fetch(ahead);
+    xsum(B2 + b);
+  };
+  const int main0 = y0 + r + OK * wave;
+  if (OK * wave < hist) {
+    fetch(y0 - r + OK * wave);
+    for (int g = wave; OK * g < hist; g += 4)
+      xpass(OK * g, y0 - r + OK * g, OK * (g + 4) < hist ? y0 - r + OK * (g + 4) : main0);
+  } else {
+    fetch(main0);
+  }
+  __syncthreads();
+  const int xc = min(x0 + l, W - 1);
+  const bool out = x0 + l < W;
+  for (int c0 = y0; c0 < y1; c0 += kStep) {
+    const int c = c0 + OK * wave;
+    xpass(hist + OK * wave, c + r, c + kStep + r);
+    uint32_t kn[OK], kx[OK];
+#pragma unroll
+    for (int o = 0; o < OK; ++o) {
+      const i64 at = pbase + (i64)min(c + o, H - 1) * W + xc;
+      kn[o] = amn[at];
+      kx[o] = amx[at];
+    }
+    __syncthreads();
+    if (c < y1) {
+      auto channel = [&](const float* B, uint32_t (&key)[OK]) {
+        float acc[OK];
+        const float* p = B + OK * wave * BP + l;
+        sum8<R>([&] { const float u = *p; p += BP; return u; }, r, acc);
+        add_clamped(B + l, BP, c0 - r, c, H, r, acc);
+#pragma unroll
+        for (int o = 0; o < OK; ++o) {
+          acc[o] *= k;
+          if (!out || c + o >= y1 || acc[o] == 0.0f) key[o] = kNone;
+          if (key[o] == kNone) acc[o] = 0.0f;
+        }
+        route8(key, acc, table, gv);
+      };
+      channel(B1, kn);
+      channel(B2, kx);
+    }
+    __syncthreads();
+    table.flush(gv);
+    if (c0 + kStep >= y1) break;  // uniform
+    shift_rows<256, kStep, BP>(B1, hist);
+    shift_rows<256, kStep, BP>(B2, hist);
+    __syncthreads();
+  }
+}
+
 // ---- any radius ------------------------------------------------------------------------
 // clamped box mean of the (E, D) pair along one axis (FP32 sums in window order)
 __global__ __launch_bounds__(NT) void k_soft_box(const float2* __restrict__ in,
@@ -933,53 +1239,6 @@ __global__ __launch_bounds__(NT) void k_soft_box_adj(const float2* __restrict__ 
   }
 }
 
-// The transpose along y or z for radius R as a column walker: a register ring of the
-// 2R+1 inputs around each position (zero outside the line), unrolled by the ring period;
-// the two border positions add the taps that clamp onto them from direct loads.
-template <int R>
-__global__ __launch_bounds__(NT) void k_soft_box_adj_walk(const float2* __restrict__ in,
-                                                          float2* __restrict__ out, int W, int L,
-                                                          i64 sa, i64 so, unsigned nxb) {
-  constexpr int WB = 2 * R + 1;
-  const float k = 1.0f / (float)WB;
-  const int x = (int)(blockIdx.x % nxb) * NT + (int)threadIdx.x;
-  if (x >= W) return;
-  const i64 base = (i64)(blockIdx.x / nxb) * so + x;
-  auto at = [&](int c) -> float2 {
-    return (c >= 0 && c < L) ? in[base + (i64)c * sa] : make_float2(0.0f, 0.0f);
-  };
-  float2 ring[WB];  // position p lives in ring[(p + R) % WB]
-#pragma unroll
-  for (int q = 0; q < WB; ++q) ring[q] = at(q - R);
-  for (int c0 = 0;; c0 += WB) {
-#pragma unroll
-    for (int q = 0; q < WB; ++q) {
-      const int c = c0 + q;
-      if (c >= L) return;
-      float se = 0.0f, sd = 0.0f;
-#pragma unroll
-      for (int j = 0; j < WB; ++j) {  // positions c - R .. c + R
-        se += ring[(q + j) % WB].x;
-        sd += ring[(q + j) % WB].y;
-      }
-      if (c == 0)  // taps t - R + j < 0 of the windows of t < R clamp onto 0
-        for (int t = 0; t <= min(L - 1, R - 1); ++t) {
-          const float2 v = in[base + (i64)t * sa];
-          se += v.x * (float)(R - t);
-          sd += v.y * (float)(R - t);
-        }
-      if (c == L - 1)  // taps beyond L - 1 of the windows of t > L - 1 - R clamp onto L - 1
-        for (int t = max(0, L - R); t <= L - 1; ++t) {
-          const float2 v = in[base + (i64)t * sa];
-          se += v.x * (float)(t + R - L + 1);
-          sd += v.y * (float)(t + R - L + 1);
-        }
-      out[base + (i64)c * sa] = make_float2(se * k, sd * k);
-      ring[q] = at(c + R + 1);  // replaces position c - R
-    }
-  }
-}
-
 __global__ __launch_bounds__(NT) void k_soft_norm(const float* __restrict__ v,
                                                   const float2* __restrict__ ed,
                                                   float* __restrict__ norm, float min_int, i64 N) {
@@ -1007,24 +1266,6 @@ __global__ __launch_bounds__(NT) void k_soft_norm_adj(const float* __restrict__ 
   }
 }
 
-// Sum of v over the run of equal consecutive keys (lanes of one wave) that starts at each
-// run's first lane, where *head is set; every lane of the wave must be active.  A segmented
-// suffix sum by lane shifts: after the step of offset o each lane holds the sum over
-// [lane, lane + 2o) within its run.
-__device__ __forceinline__ float run_sum(uint32_t key, float v, bool* head) {
-  const int lane = (int)(threadIdx.x & 63);
-  const uint32_t prev = __shfl_up(key, 1, 64);
-  *head = lane == 0 || prev != key;
-  const unsigned long long heads = __ballot(*head);
-  const unsigned long long after = lane == 63 ? 0ull : heads & (~0ull << (lane + 1));
-  const int tail = after ? __builtin_ctzll(after) - 1 : 63;  // last lane of the run
-  for (int o = 1; o < 64; o <<= 1) {
-    const float w = __shfl_down(v, o, 64);
-    if (lane + o <= tail) v += w;
-  }
-  return v;
-}
-
 // subgradient routing: gv[argmin(i)] += dL/dmin(i), gv[argmax(i)] += dL/dmax(i).  Windows
 // of neighbouring voxels mostly share their extreme, so a wave first sums its lanes' values
 // per run of equal targets and adds each run with one atomic (one atomic per voxel made the
@@ -1033,7 +1274,6 @@ __global__ __launch_bounds__(NT) void k_soft_route(const float2* __restrict__ g,
                                                    const uint32_t* __restrict__ amn,
                                                    const uint32_t* __restrict__ amx,
                                                    float* __restrict__ gv, i64 N) {
-  constexpr uint32_t kNone = 0xFFFFFFFFu;  // lanes past the volume (N < 2^32 - 1)
   const int lane = (int)(threadIdx.x & 63);
   for (i64 b = (i64)blockIdx.x * NT + (threadIdx.x - lane); b < N; b += (i64)gridDim.x * NT) {
     const i64 i = b + lane;  // the whole wave iterates together
@@ -1060,17 +1300,14 @@ hipError_t launch_soft_normalize(const float* v, float* norm, float2* ed, uint32
     uint32_t* pk = (uint32_t*)scratch;       // keys and taps, 3 N words
     float2* pair = (float2*)(pk + 3 * N);    // 2 N words
     float2* exy = (float2*)scratch;          // in the place of the keys
-    const int nxs = (W + 63) / 64;
-    int nys, rows;
-    walk_segments(H, WalkShape{(i64)nxs * D * 4, kStep, 2 * rxy}, &nys, &rows);
-    const dim3 grid((unsigned)((i64)nxs * D * nys));
+    const XyRun x = xy_run(W, H, D, rxy);
     const LineGrid g = run_grid(W, D, H, 2 * rz);
     const float kxy = 1.0f / (float)(2 * rxy + 1), kz = 1.0f / (float)(2 * rz + 1);
     const size_t zrows = (size_t)(2 * rz + kStep) * 64 * 4;
     hipError_t e = dispatch_short(rxy, [&](auto rs) {
       constexpr int R = decltype(rs)::value;
-      hipLaunchKernelGGL((k_soft_arg_xy<R>), grid, dim3(256), arg_xy_lds(rxy), s, v, pk, pk + N,
-                         pk + 2 * N, W, H, rxy, nxs, nys, rows);
+      hipLaunchKernelGGL((k_soft_arg_xy<R>), dim3(x.blocks), dim3(256), arg_xy_lds(rxy), s, v, pk, pk + N,
+                         pk + 2 * N, W, H, rxy, x.nxs, x.nys, x.rows);
       return hipGetLastError();
     });
     if (e != hipSuccess) return e;
@@ -1083,10 +1320,8 @@ hipError_t launch_soft_normalize(const float* v, float* norm, float2* ed, uint32
     if (e != hipSuccess) return e;
     e = dispatch_short(rxy, [&](auto rs) {
       constexpr int R = decltype(rs)::value;
-      const size_t lds =
-          ((size_t)4 * OK * arg_line_pitch(rxy) + 2 * (size_t)(2 * rxy + kStep) * 65) * 4;
-      hipLaunchKernelGGL((k_soft_box_xy<R>), grid, dim3(256), lds, s, pair, exy, W, H, rxy, nxs,
-                         nys, rows, kxy);
+      hipLaunchKernelGGL((k_soft_box_xy<R>), dim3(x.blocks), dim3(256), box_xy_lds(rxy), s, pair,
+                         exy, W, H, rxy, x.nxs, x.nys, x.rows, kxy);
       return hipGetLastError();
     });
     if (e != hipSuccess) return e;
@@ -1151,29 +1386,41 @@ hipError_t launch_soft_normalize_adjoint(const float* v, const float2* ed, const
                                          const float* gn, float* gv, void* scratch,
                                          float min_int, int W, int H, int D, int rxy, int rz,
                                          hipStream_t s) {
-  const i64 N = (i64)W * H * D;
+  const i64 N = (i64)W * H * D, WH = (i64)W * H;
   float2* q0 = (float2*)scratch;
+  if (rxy <= kArgRadius && rz <= kArgRadius) {
+    const LineGrid g = run_grid(W, D, H, 2 * rz);
+    hipError_t e = dispatch_short(rz, [&](auto rs) {
+      constexpr int R = decltype(rs)::value;
+      hipLaunchKernelGGL((k_soft_adj_z<R>), dim3(g.blocks), dim3(256),
+                         2 * (size_t)(2 * rz + kStep) * 64 * 4, s, v, ed, gn, gv, q0, min_int, W, D,
+                         WH, rz, g.nxb, g.no, g.len, 1.0f / (float)(2 * rz + 1));
+      return hipGetLastError();
+    });
+    if (e != hipSuccess) return e;
+    const XyRun x = xy_run(W, H, D, rxy);
+    return dispatch_short(rxy, [&](auto rs) {
+      constexpr int R = decltype(rs)::value;
+      hipLaunchKernelGGL((k_soft_adj_xy<R>), dim3(x.blocks), dim3(256),
+                         box_xy_lds(rxy) + kRouteSlots * 8, s, q0, arg, arg + N, gv, W, H, rxy,
+                         x.nxs, x.nys, x.rows, 1.0f / (float)(2 * rxy + 1));
+      return hipGetLastError();
+    });
+  }
   float2* q1 = q0 + N;
   const unsigned g = grid_for(N);
   const int rad[3] = {rxy, rxy, rz};
   hipLaunchKernelGGL(k_soft_norm_adj, dim3(g), dim3(NT), 0, s, v, ed, gn, gv, q0, min_int, N);
   // the box was applied x, y, z: its transpose runs z, y, x
   float2* bufs[2] = {q0, q1};
-  const i64 WH = (i64)W * H;
   for (int k = 0; k < 3; ++k) {
     const int axis = 2 - k;
-    if (axis > 0 && rad[axis] == 10) {  // z, y: column walker
-      const i64 n_other = axis == 1 ? D : H;
-      hipLaunchKernelGGL((k_soft_box_adj_walk<10>), dim3((unsigned)(xblocks(W) * n_other)),
-                         dim3(NT), 0, s, bufs[k & 1], bufs[(k + 1) & 1], W, axis == 1 ? H : D,
-                         axis == 1 ? (i64)W : WH, axis == 1 ? WH : (i64)W, xblocks(W));
-    } else if (axis == 0 && rad[0] <= kXR) {
+    if (axis == 0 && rad[0] <= kXR)
       hipLaunchKernelGGL(k_soft_box_adj_x, dim3(grid_rows(W, H, D)), dim3(NT), 0, s,
                          bufs[k & 1], bufs[(k + 1) & 1], W, rad[0], xblocks(W));
-    } else {
+    else
       hipLaunchKernelGGL(k_soft_box_adj, dim3(grid_rows(W, H, D)), dim3(NT), 0, s, bufs[k & 1],
                          bufs[(k + 1) & 1], W, H, D, axis, rad[axis], xblocks(W));
-    }
   }
   hipLaunchKernelGGL(k_soft_route, dim3(g), dim3(NT), 0, s, bufs[1], arg, arg + N, gv, N);
   return hipGetLastError();

@@ -346,3 +346,49 @@ def test_soft_normalization_bitexact(hd, rxy, rz, kind):
     np.testing.assert_array_equal(arg.cpu().numpy().view(np.uint32), warg)
     np.testing.assert_array_equal(ed.cpu().numpy(), wed)
     np.testing.assert_array_equal(n.cpu().numpy(), wn)
+
+
+# its adjoint at the same radii, against FP64 sums over the same indices: few extremes per
+# patch, plateaus where every window has its own, NaN windows without one.  Bound: three FP32
+# window sums of up to 47 terms and some hundred terms per target, of 6e-8 each, on the sum of
+# the terms' magnitudes
+@pytest.mark.parametrize("rxy,rz", [(1, 1), (2, 3), (3, 2), (4, 5), (10, 10), (23, 23), (24, 2)])
+@pytest.mark.parametrize("shape,kind", [((37, 43, 133), "noise"), ((5, 70, 64), "plateau"),
+                                        ((2, 3, 65), "noise"), ((9, 8, 70), "nan")])
+def test_soft_normalization_adjoint(hd, rxy, rz, shape, kind):
+    import torch
+    from hdog import _capi as C
+    rng = np.random.default_rng(rz)
+    v = rng.standard_normal(shape).astype(np.float32)
+    if kind == "plateau":
+        v = np.maximum(v - 2.5, 0).astype(np.float32)
+    D, H, W = shape
+    N = v.size
+    gn = rng.standard_normal(shape).astype(np.float32)
+    e = rng.standard_normal(shape).astype(np.float32)
+    ed = np.stack([e, e + 1 + rng.random(shape).astype(np.float32)], -1)
+    vin = v.copy()
+    if kind == "nan":
+        vin[:, :, :50] = np.nan
+    with np.errstate(all="ignore"):
+        arg = soft_normalize_by_hand(vin, 0.0, rxy, rz)[2]
+    dev = [torch.from_numpy(np.ascontiguousarray(a)).to(hd.device)
+           for a in (v, ed, arg.view(np.int32), gn)]
+    gv = torch.empty_like(dev[0])
+    p = [C.ctypes.c_void_p(a.data_ptr()) for a in dev + [gv]]
+    hd._check(C.hdog_soft_normalize_backward(hd._h, hd._stream(), *p, -0.25, W, H, D, rxy, rz))
+    E, Dl, v64 = ed[..., 0].astype(np.float64), ed[..., 1].astype(np.float64), v.astype(np.float64)
+    g = np.where(v >= np.float32(-0.25), gn, 0).astype(np.float64)
+    want = g / (Dl - E)
+    size = np.abs(want)
+    for part, j in ((g * (v64 - Dl) / (Dl - E) ** 2, arg[0]), (-g * (v64 - E) / (Dl - E) ** 2, arg[1])):
+        for out, x in ((want, part), (size, np.abs(part))):
+            for axis, r in ((0, rz), (1, rxy), (2, rxy)):
+                L = shape[axis]
+                M = np.zeros((L, L))  # M[p, c]: taps of the window of c that land on p
+                for t in range(-r, r + 1):
+                    np.add.at(M, (np.clip(np.arange(L) + t, 0, L - 1), np.arange(L)), 1.0 / (2 * r + 1))
+                x = np.moveaxis(np.tensordot(M, x, (1, axis)), 0, axis)
+            ok = j.ravel() != 0xFFFFFFFF
+            out += np.bincount(j.ravel()[ok].astype(np.int64), x.ravel()[ok], N).reshape(shape)
+    assert np.all(np.abs(gv.cpu().numpy() - want) <= 4e-5 * size)
