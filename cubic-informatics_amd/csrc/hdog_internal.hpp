@@ -38,7 +38,7 @@ constexpr int kBufferWord3 = 0x00020000;
 // store is compiled on gfx950
 constexpr int kCachePolicyNT = 2;
 // Hessian tiles: 64 x 8 outputs per work-group over 16 slices.  Candidate records are kept
-// per tile in a block of kCandTile slots x 7 words (voxel index, then the six elements).
+// per tile in a block of kCandTile slots x 7 words: the positions, then per slot six elements.
 // The tile height and the region pass's tile group are build-time choices (-DHDOG_HESS_TY,
 // -DHDOG_ACC_GY / GZ; static_asserts guard the limits); 8 and 2 x 2 measured fastest.
 #ifndef HDOG_HESS_TY
@@ -46,6 +46,30 @@ constexpr int kCachePolicyNT = 2;
 #endif
 constexpr int kHessTX = 64, kHessTY = HDOG_HESS_TY, kHessTZ = 16;
 constexpr int kCandTile = kHessTX * kHessTY * kHessTZ;
+// Element words of slot i: kCandTile + 6 i, in this order (two groups of three: one 12-byte
+// access each; the adjoint's halo rows need only the first).  As six planes, a row with a few
+// candidates took seven stores of a few lanes each instead of three: 393 us instead of
+// 366 for the Hessian pass of 32 x 2160 x 2560.
+enum RecWord { kRecXY, kRecYY, kRecYZ, kRecXX, kRecXZ, kRecZZ };
+struct RecHalf {
+  float a, b, c;
+};
+__device__ __forceinline__ RecHalf rec_load(const float* rec, uint32_t slot, int half) {
+  return *reinterpret_cast<const RecHalf*>(rec + kCandTile + 6 * (size_t)slot + 3 * half);
+}
+__device__ __forceinline__ void rec_store(float* rec, uint32_t slot, int half, RecHalf v) {
+  *reinterpret_cast<RecHalf*>(rec + kCandTile + 6 * (size_t)slot + 3 * half) = v;
+}
+// xx, xy, xz, yy, yz, zz of a slot
+__device__ __forceinline__ void rec_elements(const float* rec, uint32_t slot, float (&h)[6]) {
+  const RecHalf u = rec_load(rec, slot, 0), v = rec_load(rec, slot, 1);
+  h[0] = v.a;
+  h[1] = u.a;
+  h[2] = v.b;
+  h[3] = u.b;
+  h[4] = u.c;
+  h[5] = v.c;
+}
 // reduced-precision forms: default FP64 re-evaluation band of the leading minors (relative
 // to the sum of the magnitudes of their terms)
 constexpr float kDefaultMinorBand = 1e-5f;
@@ -367,7 +391,7 @@ template <typename TD, typename TH>
 // hess and pd may be NULL (not written).  cand / cand_cnt (optional): per Hessian tile
 // (kHessTX x kHessTY x kHessTZ, tiles x-fastest), the number of candidate voxels and their
 // records: the voxel's position in the tile, lx + kHessTX (ly + kHessTY lz), then the six
-// elements rounded to TH, as 7 SoA words of kCandTile slots; cand holds hessian_tiles() *
+// elements rounded to TH, as described at kCandTile; cand holds hessian_tiles() *
 // kCandTile * 7 words.  Voxel 0 never has a record (its label is 0 whatever its mask).
 // band: the FP64 re-evaluation band of the leading minors when TD or TH is a 2-byte type.
 hipError_t launch_hessian(const TD* dog, TH* hess, uint8_t* pd, int W, int H, int D,

@@ -306,8 +306,8 @@ __global__ __launch_bounds__(NT, 5) void k_hessian(const TD* __restrict__ dog, T
           if (is_cand) {
             const uint32_t slot = base + (uint32_t)__popcll(bal & ((1ull << lane) - 1ull));
             rec[slot] = __uint_as_float(cidx);
-#pragma unroll
-            for (int q = 0; q < 6; ++q) rec[(size_t)kCandTile * (1 + q) + slot] = h6[q];
+            rec_store(rec, slot, 0, {h6[1], h6[3], h6[4]});
+            rec_store(rec, slot, 1, {h6[0], h6[2], h6[5]});
           }
         }
       }
@@ -384,6 +384,7 @@ __device__ __forceinline__ float swap_pairs(float v) {
 // the mask volume holds, whatever their minors, and each tile row's bits and first record:
 // the records of a row are consecutive, in lane order).
 constexpr int kDetect = 0, kWriteMask = 1, kGivenMask = 2;
+typedef uint32_t U3 __attribute__((ext_vector_type(3)));
 template <typename TD, typename TS, bool BAND, int MODE>
 __global__ __launch_bounds__(64 * kRecWaves) void k_hessian_rec(
     const TD* __restrict__ dog, int W, int H, int D, int nbx, int nby, int nbyg, int nz,
@@ -497,14 +498,13 @@ __global__ __launch_bounds__(64 * kRecWaves) void k_hessian_rec(
                                            (uint32_t)(act >> 32),
                                            __builtin_amdgcn_mbcnt_lo((uint32_t)act, 0u));
           const uint32_t cidx = (uint32_t)lane + 64u * ((uint32_t)(ty0 + r) + kHessTY * lz);
-          const int vb = (int)(slot * 4u);
-          const float h6[6] = {round_to<TS>(xx), round_to<TS>(xy), round_to<TS>(xz),
-                               round_to<TS>(yy), round_to<TS>(yz), round_to<TS>(zz)};
-          __builtin_amdgcn_raw_buffer_store_b32(cidx, rr, vb, 0, 0);
-#pragma unroll
-          for (int q = 0; q < 6; ++q)
-            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(h6[q]), rr, vb,
-                                                  (1 + q) * kCandTile * 4, 0);
+          const U3 u = {__float_as_uint(round_to<TS>(xy)), __float_as_uint(round_to<TS>(yy)),
+                        __float_as_uint(round_to<TS>(yz))};
+          const U3 v = {__float_as_uint(round_to<TS>(xx)), __float_as_uint(round_to<TS>(xz)),
+                        __float_as_uint(round_to<TS>(zz))};
+          __builtin_amdgcn_raw_buffer_store_b32(cidx, rr, (int)(slot * 4u), 0, 0);
+          __builtin_amdgcn_raw_buffer_store_b96(u, rr, (int)(slot * 24u), kCandTile * 4, 0);
+          __builtin_amdgcn_raw_buffer_store_b96(v, rr, (int)(slot * 24u) + 12, kCandTile * 4, 0);
         }
       }
     }

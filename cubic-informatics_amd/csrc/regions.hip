@@ -487,7 +487,7 @@ __global__ __launch_bounds__(NT) void k_accum(const uint32_t* __restrict__ L,
 }
 
 // Region sums from the candidate records of the Hessian kernel: one work-group per
-// kAccGY x kAccGZ Hessian tiles folds their records (voxel index + six elements, SoA) into
+// kAccGY x kAccGZ Hessian tiles folds their records (voxel position + six elements) into
 // the table, gathering the label, normalized and raw intensity of each candidate voxel; no
 // pass over the non-candidate voxels.
 static_assert(kAccGY * kAccGZ * kCandTile < (1 << 16) && kHessTX <= 256 &&
@@ -549,8 +549,7 @@ __global__ __launch_bounds__(NT) void k_accum_cand(const float* __restrict__ can
         y = ty0 + (v / kHessTX) % kHessTY;
         z = tz0 + v / (kHessTX * kHessTY);
         const uint32_t idx = z * WH + y * W + x;
-#pragma unroll
-        for (int k = 0; k < 6; ++k) hv[k] = t[(size_t)kCandTile * (1 + k) + i];
+        rec_elements(t, i, hv);
         const uint32_t root = rl[i];
         r = rid[root];
         // the labeling marks every region that reaches beyond one work-group's tiles

@@ -74,8 +74,7 @@ __global__ __launch_bounds__(NT) void k_soft_loss(const float* __restrict__ cand
       const size_t at = ((size_t)(T.z0 + (int)(v / (kHessTX * kHessTY))) * H +
                          (T.y0 + (int)(v / kHessTX % kHessTY))) * W + T.x0 + (int)(v % kHessTX);
       float e[6];
-#pragma unroll
-      for (int k = 0; k < 6; ++k) e[k] = rec[(size_t)kCandTile * (1 + k) + i];
+      rec_elements(rec, i, e);
       const double u = -det3(e[0], e[1], e[2], e[3], e[4], e[5]) * inv_tau;
       ls += softplus(u) - (target[at] ? u : 0.0);
       cnt += 1.0;
@@ -101,21 +100,19 @@ __global__ __launch_bounds__(NT) void k_soft_grad_h(float* __restrict__ cand,
       const uint32_t v = __float_as_uint(rec[i]);
       const size_t at = ((size_t)(T.z0 + (int)(v / (kHessTX * kHessTY))) * H +
                          (T.y0 + (int)(v / kHessTX % kHessTY))) * W + T.x0 + (int)(v % kHessTX);
-      float* h = rec + kCandTile + i;
-      const double xx = h[0], xy = h[kCandTile], xz = h[2 * kCandTile], yy = h[3 * kCandTile],
-                   yz = h[4 * kCandTile], zz = h[5 * kCandTile];
+      float h[6];
+      rec_elements(rec, i, h);
+      const double xx = h[0], xy = h[1], xz = h[2], yy = h[3], yz = h[4], zz = h[5];
       const double d = det3(xx, xy, xz, yy, yz, zz);
       const double u = -d * inv_tau;
       const double p = 1.0 / (1.0 + exp(-u));
       const double gu = (p - (target[at] ? 1.0 : 0.0)) * inv_count;  // dL/du
       gt += gu * d * inv_tau * inv_tau;                               // du/dtau = det / tau^2
       const double gd = -gu * inv_tau;                                // dL/ddet
-      h[0] = (float)(gd * (yy * zz - yz * yz));
-      h[kCandTile] = (float)(gd * 2.0 * (xz * yz - zz * xy));
-      h[2 * kCandTile] = (float)(gd * 2.0 * (xy * yz - yy * xz));
-      h[3 * kCandTile] = (float)(gd * (xx * zz - xz * xz));
-      h[4 * kCandTile] = (float)(gd * 2.0 * (xy * xz - xx * yz));
-      h[5 * kCandTile] = (float)(gd * (xx * yy - xy * xy));
+      rec_store(rec, i, 0, {(float)(gd * 2.0 * (xz * yz - zz * xy)), (float)(gd * (xx * zz - xz * xz)),
+                            (float)(gd * 2.0 * (xy * xz - xx * yz))});
+      rec_store(rec, i, 1, {(float)(gd * (yy * zz - yz * yz)),
+                            (float)(gd * 2.0 * (xy * yz - yy * xz)), (float)(gd * (xx * yy - xy * xy))});
     }
   }
   double a[1] = {gt};
@@ -132,12 +129,13 @@ __global__ __launch_bounds__(NT) void k_soft_grad_h(float* __restrict__ cand,
 // from the records: its bits (from the two tiles that the 64 lanes touch) say which lanes hold
 // one and which one; a lane without one reads past the end of the buffer, which gives 0 without
 // touching memory.  Nothing dense but the result leaves the chip.  Bound by instruction issue
-// (two row lookups and eight loads per output row).  As dense volumes dL/dH went out and back
+// (two row lookups and three loads per output row).  As dense volumes dL/dH went out and back
 // in two passes: 262 + 132 us at 128 x 512 x 512 with 7 % masked, and 76 for the dot product
-// (229 here; with tiles of 64 x 8 x 8 in LDS, one element at a time, 820).
+// (221 here; with tiles of 64 x 8 x 8 in LDS, one element at a time, 820).
 constexpr int AR = 4;       // rows of outputs of a wave
 constexpr int kAdjX = 60;   // columns of outputs: lanes 2 .. 61
 constexpr int AI = AR + 4;  // rows of inputs, two beyond either side
+typedef float F3 __attribute__((ext_vector_type(3)));
 __device__ __forceinline__ float lane_up(float v) {  // the value of lane - 1
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, false));
 }
@@ -205,28 +203,29 @@ __global__ __launch_bounds__(NT, 4) void k_hessian_adjoint(const float* __restri
           const unsigned long long ml = mhi << 32 | mlo;
           const unsigned long long m = ml | (unsigned long long)read_lane(ohi, AI + j) << 32 |
                                        read_lane(olo, AI + j);
-          const uint32_t fl = read_lane(first, j);
-          const uint32_t fr = read_lane(first, AI + j) - (uint32_t)__popcll(ml) + kTileWords;
+          const uint32_t fl = read_lane(first, j) * 24u;
+          const uint32_t fr =
+              (read_lane(first, AI + j) - (uint32_t)__popcll(ml)) * 24u + kTileWords * 4u;
           // two tiles' records, never used beyond the last tile's (no bits there)
           const __amdgpu_buffer_rsrc_t r = buf_rsrc(
               cand + ((i64)tz * nby * nbx + (i64)ty * nbx + tl) * (i64)kTileWords, kTileWords * 8u);
           const uint32_t rank = __builtin_amdgcn_mbcnt_hi(
               (uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-          const uint32_t slot = rank + (right ? fr : fl);
-          const int off = (int)((m >> lane) & 1ull ? slot * 4u : 0xF0000000u);
-          auto get = [&](int k) {
-            return __uint_as_float(
-                __builtin_amdgcn_raw_buffer_load_b32(r, off, kCandTile * (1 + k) * 4, 0));
-          };
-          gyy[j] = get(3);
+          const uint32_t slot = rank * 24u + (right ? fr : fl);  // in bytes
+          const int off = (int)((m >> lane) & 1ull ? slot : 0xF0000000u);
+          const F3 u = __builtin_bit_cast(
+              F3, __builtin_amdgcn_raw_buffer_load_b96(r, off, kCandTile * 4, 0));
+          gyy[j] = u[kRecYY];
           if (j >= 1 && j <= AR + 2) {
-            gxy[j - 1] = get(1);
-            nyz[j - 1] = get(4);
+            gxy[j - 1] = u[kRecXY];
+            nyz[j - 1] = u[kRecYZ];
           }
           if (j >= 2 && j <= AR + 1) {
-            gxx[j - 2] = get(0);
-            nxz[j - 2] = get(2);
-            nzz[j - 2] = get(5);
+            const F3 v = __builtin_bit_cast(
+                F3, __builtin_amdgcn_raw_buffer_load_b96(r, off + 12, kCandTile * 4, 0));
+            gxx[j - 2] = v[kRecXX - 3];
+            nxz[j - 2] = v[kRecXZ - 3];
+            nzz[j - 2] = v[kRecZZ - 3];
           }
         }
       }
