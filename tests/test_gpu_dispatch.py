@@ -392,3 +392,12 @@ def test_soft_normalization_adjoint(hd, rxy, rz, shape, kind):
             ok = j.ravel() != 0xFFFFFFFF
             out += np.bincount(j.ravel()[ok].astype(np.int64), x.ravel()[ok], N).reshape(shape)
     assert np.all(np.abs(gv.cpu().numpy() - want) <= 4e-5 * size)
+
+
+# fused y / z min/max: windows longer than the volume, just as long, ending and starting blocks
+# of 21 slices on either side of the volume's end, several z segments with short ones
+@pytest.mark.parametrize("depth", [2, 10, 11, 12, 21, 22, 31, 32, 33, 43, 74])
+def test_minmax_zy_of_any_depth(hd, depth):
+    img = noise((depth, 37, 70), depth)
+    got = hd.Normalize3DFilter(img, 100, 10, 10)
+    np.testing.assert_array_equal(got.cpu().numpy(), oracle.normalize3d(img, 100, 10, 10))
