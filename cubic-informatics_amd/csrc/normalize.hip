@@ -886,6 +886,96 @@ __global__ __launch_bounds__(256) void k_minmax_run(const void* __restrict__ src
   }
 }
 
+// out[o] = packed minimum of v[o] .. v[o + 2 R], in registers
+template <int R, int N>
+__device__ __forceinline__ void min8_regs(const uint32_t (&v)[N], uint32_t (&out)[OK]) {
+  static_assert(2 * R >= OK && 2 * R + OK <= N, "inputs that all eight share");
+  uint32_t m[4] = {v[OK - 1], v[OK - 1], v[OK - 1], v[OK - 1]};
+#pragma unroll
+  for (int i = OK; i <= 2 * R; ++i) m[i & 3] = pkmin(m[i & 3], v[i]);
+  uint32_t t = pkmin(pkmin(m[0], m[1]), pkmin(m[2], m[3]));
+  out[OK - 1] = t;
+#pragma unroll
+  for (int o = OK - 2; o >= 0; --o) out[o] = t = pkmin(t, v[o]);
+  t = v[2 * R + 1];
+#pragma unroll
+  for (int o = 1; o < OK; ++o) {
+    if (o > 1) t = pkmin(t, v[2 * R + o]);
+    out[o] = pkmin(out[o], t);
+  }
+}
+
+// Packed min / max along y and z in one pass (k_minmax_zy_walk for other radii, at least 4): a
+// work-group of eight waves walks z for a tile of 64 columns x 8 rows, eight slices per step.
+//   1. wave w holds the 8 + 2 ry rows of slice w, loaded a step ahead (clamped; a lane a
+//      column), and forms the eight y windows in registers, whose number NQ fits four radii,
+//      told apart by a uniform switch; they enter an LDS block of the last 2 rz + 8 slices;
+//   2. wave w forms the eight z windows of row w.
+// The halo rows come from L2 (three rows read per row written at ry = 8).  70 x 1080 x 1280 at
+// radii 8 / 4: 171 us, in two passes 137 + 181.
+constexpr int kZyRadiusZ = 12;  // 64 KB of LDS
+// Above, a wave holds too many rows in flight (70 x 1080 x 1280, in two passes in brackets:
+// 171 us (318) at 8 / 4, 198 (317) at 4 / 12, 287 (327) at 16 / 12, 348 (317) at 20 / 4).
+constexpr int kZyRadiusY = 16;
+template <int NQ>
+__global__ __launch_bounds__(512) void k_minmax_zy_run(const uint16_t* __restrict__ img,
+                                                       uint32_t* __restrict__ dst, int W, int H,
+                                                       int D, int ry, int rz, unsigned nyt,
+                                                       unsigned nxt, int len) {
+  extern __shared__ uint32_t sm_zy[];
+  constexpr int TY = OK, PL = TY * 64, RM = (NQ - OK) / 2;  // the largest radius
+  const unsigned t = xcd_tile(blockIdx.x, gridDim.x);
+  const int y0 = (int)(t % nyt) * TY, x0 = (int)(t / nyt % nxt) * 64;
+  const int s0 = (int)(t / nyt / nxt) * len, s1 = min(D, s0 + len);
+  const int l = (int)(threadIdx.x & 63);
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int xc = min(x0 + l, W - 1), hist = 2 * rz;
+  uint32_t q[NQ];
+  auto fetch = [&](int s) {
+    const uint16_t* slice = img + (i64)clampi(s, 0, D - 1) * H * W;
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) q[i] = slice[(i64)clampi(y0 - ry + i, 0, H - 1) * W + xc];
+  };
+  auto ymin = [&](int plane, int ahead) {
+    uint32_t v[NQ], o[OK];
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) v[i] = pack(q[i]);
+    if (ry == RM) min8_regs<RM>(v, o);
+    if constexpr (RM > 4) {
+      if (ry == RM - 1) min8_regs<RM - 1>(v, o);
+      if (ry == RM - 2) min8_regs<RM - 2>(v, o);
+      if (ry == RM - 3) min8_regs<RM - 3>(v, o);
+    }
+    fetch(ahead);
+#pragma unroll
+    for (int i = 0; i < OK; ++i) sm_zy[plane * PL + i * 64 + l] = o[i];
+  };
+  fetch(s0 - rz + wave);
+  for (int g = wave; g < hist; g += 8)
+    ymin(g, g + 8 < hist ? s0 - rz + g + 8 : s0 + rz + wave);
+  if (wave >= hist) fetch(s0 + rz + wave);
+  const int y = y0 + wave;
+  const bool out = x0 + l < W && y < H;
+  const i64 WH = (i64)W * H;
+  uint32_t* d = dst + (i64)y * W + x0 + l;
+  for (int c = s0; c < s1; c += OK) {
+    ymin(hist + wave, c + OK + rz + wave);
+    __syncthreads();
+    const uint32_t* p = sm_zy + wave * 64 + l;
+    uint32_t o[OK];
+    min8<0>([&] { const uint32_t v = *p; p += PL; return v; }, rz, o);
+    if (out) {
+#pragma unroll
+      for (int k = 0; k < OK; ++k)
+        if (c + k < s1) st_nt(d + (i64)(c + k) * WH, o[k]);
+    }
+    if (c + OK >= s1) break;  // uniform
+    __syncthreads();
+    shift_rows<512, OK, PL>(sm_zy, hist);
+    __syncthreads();
+  }
+}
+
 // Clamped box mean of (E, D) pairs along y or z, with NORM fused with the normalization; ero
 // and dil (optional) receive E and D.  Bound by its 14 (16) bytes per voxel: 275 us for
 // 70 x 1080 x 1280 at radius 4 (4.9 TB/s), 568 with an LDS tile per 64 outputs.
@@ -1259,6 +1349,21 @@ hipError_t launch_normalize(const uint16_t* img, TS* norm, void* tmp1, void* tmp
     hipLaunchKernelGGL((k_minmax_zy_walk<10, 10, HDOG_ZY_PF>),
                        dim3((unsigned)((i64)nxt * nyt * nzs)), dim3(1024), 0, s, img, p2, W, H, D,
                        nyt, nxt, zlen);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    mark("normalize/minmax_zy", s);
+  } else if (rxy >= 4 && rxy <= kZyRadiusY && rz >= 4 && rz <= kZyRadiusZ) {
+    const unsigned nxt = (W + 63) / 64, nyt = (H + OK - 1) / OK;
+    int nzs, zlen;
+    line_segments(D, (i64)nxt * nyt * 8, 1024.0, 2.0, false, 2 * rz, &nzs, &zlen);
+    const dim3 grid((unsigned)((i64)nxt * nyt * nzs));
+    const size_t lds = (size_t)(2 * rz + OK) * OK * 64 * 4;
+#define X(NQ)                                                                                   \
+  if (2 * rxy + OK <= NQ && 2 * rxy > NQ - 2 * OK)                                                 \
+    hipLaunchKernelGGL((k_minmax_zy_run<NQ>), grid, dim3(512), lds, s, img, p2, W, H, D, rxy, rz, \
+                       nyt, nxt, zlen);
+    X(16) X(24) X(32) X(40)
+#undef X
+    static_assert(2 * kZyRadiusY + OK == 40, "the largest");
     if ((e = hipGetLastError()) != hipSuccess) return e;
     mark("normalize/minmax_zy", s);
   } else {

@@ -401,3 +401,14 @@ def test_minmax_zy_of_any_depth(hd, depth):
     img = noise((depth, 37, 70), depth)
     got = hd.Normalize3DFilter(img, 100, 10, 10)
     np.testing.assert_array_equal(got.cpu().numpy(), oracle.normalize3d(img, 100, 10, 10))
+
+
+# one-pass y / z min/max of other radii: every group of four radii along y and each within
+# one, both ends along z, just beyond them (two passes); tiles and segments with remainders
+@pytest.mark.parametrize("shape", [(2, 5, 65), (43, 37, 70)])
+@pytest.mark.parametrize("rxy,rz", [(4, 4), (4, 12), (5, 5), (6, 7), (7, 4), (8, 12), (9, 8), (13, 6),
+                                    (14, 4), (15, 9), (16, 12), (17, 4), (8, 13), (3, 4), (4, 3)])
+def test_minmax_zy_of_other_radii(hd, shape, rxy, rz):
+    img = noise(shape, rxy + rz)
+    got = hd.Normalize3DFilter(img, 100, rxy, rz)
+    np.testing.assert_array_equal(got.cpu().numpy(), oracle.normalize3d(img, 100, rxy, rz))
