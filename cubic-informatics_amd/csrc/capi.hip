@@ -689,7 +689,7 @@ int autotune_t(hdog_ctx* ctx, hipStream_t s, const hdog_params* p, const uint16_
     float* ms;
     bool dog;
   } stages[2] = {{norm_walk_shape(p->radius_xy, W, D), best_norm, ms_norm, false},
-                 {gauss_walk_shape(ctx->r[0], ctx->r[2], W, D), best_gauss, ms_gauss, true}};
+                 {gauss_walk_shape(ctx->r[0], ctx->r[2], W, H, D), best_gauss, ms_gauss, true}};
   for (const Stage& st : stages) {
     // the built-in shape (choice 2) stays unless another one is faster by more than 3 %: a
     // choice within the timing noise would change nothing but the launch shape

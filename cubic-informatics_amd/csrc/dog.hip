@@ -607,16 +607,29 @@ hipError_t gauss_xy_run(const TS* src, float2* dst, const float* wx1, const floa
   return hipGetLastError();
 }
 
+// The compile-time walkers take a wave per strip of 64 columns.  On the smallest stacks, where
+// a wave would walk hardly more rows than its window, the walk of any radii with four waves on
+// a strip is the faster one (radii 8 / 13, rows of all strips: its us / the walker's):
+// 24 x 96 x 112, 4608: 13 / 20; 40 x 160 x 160, 19200: 18 / 23; 48 x 192 x 192, 27648: 22 / 24;
+// 20 x 256 x 400, 35840: 26 / 25; 64 x 200 x 200, 51200: 35 / 27.  Windows of radius 6 and less
+// gain nothing (radii 4 / 6 at 40 x 160 x 160: 13 / 12).
+bool gauss_row_walker(int r1, int r2, int W, int H, int D) {
+  return has_pair(r1, r2) &&
+         (std::max(r1, r2) < 8 || (i64)((W + 63) / 64) * D * H > 28 * 1024);
+}
+
 // Fused x + y passes of radii r1, r2 on both axes; AXES: with their own weights along y
 template <bool AXES, typename TS>
 hipError_t gauss_xy(const TS* src, float2* dst, const float* w1, const float* w2, const float* wy1,
                     const float* wy2, int r1, int r2, int W, int H, int D, hipStream_t s,
                     int segments) {
+  if (!gauss_row_walker(r1, r2, W, H, D))
+    return gauss_xy_run<TS>(src, dst, w1, w2, wy1, wy2, r1, r2, r1, r2, W, H, D, s, segments);
 #define X(A, B)                                                                              \
   if (r1 == A && r2 == B) {                                                                  \
     const int nxs = (W + 63) / 64;                                                           \
     int nys, rows;                                                                           \
-    walk_segments(H, gauss_walk_shape(A, B, W, D), &nys, &rows, segments);                   \
+    walk_segments(H, gauss_walk_shape(A, B, W, H, D), &nys, &rows, segments);                   \
     const i64 nblk = (i64)nxs * D * nys;                                                     \
     hipLaunchKernelGGL((k_gauss_xy_walk<A, B, AXES, TS>), dim3((unsigned)nblk), dim3(64), 0, \
                        s, src, dst, w1, w2, wy1, wy2, W, H, nxs, nys, rows);                 \
@@ -624,7 +637,7 @@ hipError_t gauss_xy(const TS* src, float2* dst, const float* w1, const float* w2
   }
   HDOG_GAUSS_PAIRS(X)
 #undef X
-  return gauss_xy_run<TS>(src, dst, w1, w2, wy1, wy2, r1, r2, r1, r2, W, H, D, s, segments);
+  return hipErrorInvalidValue;
 }
 
 // z pass: the difference (dog), or with DOT the sums of both with a
@@ -658,9 +671,9 @@ hipError_t gauss_z(const float2* src, TS* dog, const float* a, double* dots, con
 
 }  // namespace
 
-WalkShape gauss_walk_shape(int r1, int r2, int W, int D) {
+WalkShape gauss_walk_shape(int r1, int r2, int W, int H, int D) {
   const int R = std::max(r1, r2);
-  if (!has_pair(r1, r2)) return xy_run_shape(R, R, W, D);
+  if (!gauss_row_walker(r1, r2, W, H, D)) return xy_run_shape(R, R, W, D);
   return {(i64)((W + 63) / 64) * D, 2 * R + 1, 2 * R};
 }
 

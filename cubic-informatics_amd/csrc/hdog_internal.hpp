@@ -377,9 +377,9 @@ hipError_t launch_box_pair(const float2* src, float2* dst, int W, int L, i64 sa,
 template <typename TN, typename TD>
 hipError_t launch_dog(const TN* norm, TD* dog, void* tmp1, const float* weights, const int r[4], float normalizer, int W, int H, int D, hipStream_t s,
                       int segments = 0);
-// how the xy walkers of the two stages split planes of W columns, D of them
+// how the xy walkers of the two stages split planes of W columns (and H rows), D of them
 WalkShape norm_walk_shape(int rxy, int W, int D);
-WalkShape gauss_walk_shape(int r1, int r2, int W, int D);
+WalkShape gauss_walk_shape(int r1, int r2, int W, int H, int D);
 // Differentiable form: separable pair of Gaussians, weights w[0..2] = x, y, z of the first and
 // w[3..5] of the second, each symmetric, radii r[6]; tmp1 >= 8*N bytes.  launch_gauss_dog:
 // dog = (G1 - G2) * nz; launch_gauss_dots: out[0] += <a, G1>, out[1] += <a, G2>.

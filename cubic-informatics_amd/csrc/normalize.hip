@@ -1318,8 +1318,18 @@ hipError_t launch_box_pair(const float2* src, float2* dst, int W, int L, i64 sa,
   return box_line<false, float>(src, dst, nullptr, nullptr, 0.0f, W, L, sa, so, n_other, r, s);
 }
 
+// The row walker with its window in registers (radius 10) takes a wave per strip of 128
+// columns.  Too few strips leave the chip idle or are cut into segments that each walk 20 rows
+// more; the walk of any radius puts four waves on a strip of 64 (x min/max and x/y boxes,
+// strips: its us / the walker's): 24 x 96 x 112, 24: 12 / 28; 128 x 256 x 256, 256: 51 / 67;
+// 64 x 512 x 512, 256: 83 / 99; 96 x 512 x 512, 384: 120 / 121; 128 x 512 x 512, 512: 149 / 140;
+// 300 x 200 x 200, 600: 85 / 68; 32 x 2160 x 2560, 640: 655 / 558.
+static bool norm_row_walker(int rxy, int W, int D) {
+  return rxy == 10 && (i64)((W + 127) / 128) * D > 384;
+}
+
 WalkShape norm_walk_shape(int rxy, int W, int D) {
-  if (rxy == 10) return {(i64)((W + 127) / 128) * D, 21, 20};
+  if (norm_row_walker(rxy, W, D)) return {(i64)((W + 127) / 128) * D, 21, 20};
   return {(i64)((W + 63) / 64) * D * 4, 32, 2 * rxy};
 }
 
@@ -1376,7 +1386,7 @@ hipError_t launch_normalize(const uint16_t* img, TS* norm, void* tmp1, void* tmp
   // min/max along x, box along x and box along y in one row walker -> (E, D) in tmp1
   const float2* exy = (const float2*)tmp1;
   const float k = 1.0f / (float)(2 * rxy + 1);
-  if (rxy == 10) {
+  if (norm_row_walker(rxy, W, D)) {
     constexpr int CW = 128;
     const int nxs = (W + CW - 1) / CW;
     int nys, rows;

@@ -412,3 +412,16 @@ def test_minmax_zy_of_other_radii(hd, shape, rxy, rz):
     img = noise(shape, rxy + rz)
     got = hd.Normalize3DFilter(img, 100, rxy, rz)
     np.testing.assert_array_equal(got.cpu().numpy(), oracle.normalize3d(img, 100, rxy, rz))
+
+
+# either side of the sizes where the row walkers take over from the walks of any radius
+@pytest.mark.parametrize("shape", [(384, 24, 20), (385, 24, 20), (64, 448, 20), (64, 449, 20)])
+def test_row_walkers_by_size(hd, shape):
+    img = noise(shape, 2)
+    got = hd.Normalize3DFilter(img, 100, 10, 10)
+    np.testing.assert_array_equal(got.cpu().numpy(), oracle.normalize3d(img, 100, 10, 10))
+    s = (2.0, 1.6, 3.2, 2.56)
+    hd.initGaussian3DKernel(*s, truncate=4.0)
+    dog = hd.DoG3DFilter(got)
+    ref, _ = oracle.dog3d(got.cpu().numpy(), *s, truncate=4.0, gamma=1.0)
+    np.testing.assert_array_equal(dog.cpu().numpy(), ref)
