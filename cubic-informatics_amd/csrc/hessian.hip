@@ -336,10 +336,10 @@ __global__ __launch_bounds__(NT, 5) void k_hessian(const TD* __restrict__ dog, T
 // taken as (hi - lo) * 0.5f, without the leading 0 + of the per-stage form, which only
 // turns a -0 into +0; every non-zero value is the same, bit for bit.
 //
-// Layout: a wave owns 64 x-adjacent columns (one lane each) and kRecTY consecutive output
-// rows; a work-group is the kHessTY / kRecTY waves of one Hessian tile row block, walking
+// Layout: a wave owns 64 x-adjacent columns (one lane each) and TY consecutive output
+// rows; a work-group is the kHessTY / TY waves of a Hessian tile row block each, walking
 // kRecNZ Hessian tiles in z.  Everything a lane needs in y and z stays in its registers:
-// dog rows y-2 .. y+kRecTY+1 of each slice arrive from global memory (one row descriptor
+// dog rows y-2 .. y+TY+1 of each slice arrive from global memory (one row descriptor
 // each, so that rows and slices outside the volume, and columns outside the plane, read
 // zero), Hy and the y second differences are register arithmetic, and the z differences
 // walk three-slice register rings.  The x neighbours come from the adjacent lanes by DPP
@@ -358,11 +358,10 @@ __global__ __launch_bounds__(NT, 5) void k_hessian(const TD* __restrict__ dog, T
 #ifndef HDOG_REC_TILES_Y
 #define HDOG_REC_TILES_Y 2
 #endif
-constexpr int kRecTY = 4;                     // output rows per lane
 constexpr int kRecTilesY = HDOG_REC_TILES_Y;  // Hessian tiles per work-group, along y
-constexpr int kRecWaves = kRecTilesY * kHessTY / kRecTY;  // waves per work-group
+constexpr int rec_waves(int ty) { return kRecTilesY * kHessTY / ty; }  // waves per work-group
 constexpr int kRecNZ = 4;  // most Hessian tiles per work-group along z (records_walk_tiles)
-static_assert(kHessTX == 64 && kHessTY % kRecTY == 0, "one wave spans a tile row");
+static_assert(kHessTX == 64 && kHessTY % 4 == 0, "one wave spans a tile row");
 
 // v of lane i - 1 (lane 0 keeps old) and of lane i + 1 (lane 63 keeps old); one DPP move
 // each, written over old.  The whole wave must be active.
@@ -385,12 +384,12 @@ __device__ __forceinline__ float swap_pairs(float v) {
 // the records of a row are consecutive, in lane order).
 constexpr int kDetect = 0, kWriteMask = 1, kGivenMask = 2;
 typedef uint32_t U3 __attribute__((ext_vector_type(3)));
-template <typename TD, typename TS, bool BAND, int MODE>
-__global__ __launch_bounds__(64 * kRecWaves) void k_hessian_rec(
+template <typename TD, typename TS, bool BAND, int MODE, int TY>
+__global__ __launch_bounds__(64 * rec_waves(TY)) void k_hessian_rec(
     const TD* __restrict__ dog, int W, int H, int D, int nbx, int nby, int nbyg, int nz,
     float* __restrict__ cand, uint32_t* __restrict__ cand_cnt, float band,
     uint8_t* __restrict__ mask, TileRow* __restrict__ rows) {
-  constexpr int TY = kRecTY, NR = TY + 4, NH = TY + 2;  // dog rows, first-difference rows
+  constexpr int NR = TY + 4, NH = TY + 2;  // dog rows, first-difference rows
   __shared__ uint32_t s_cnt[kRecTilesY][kRecNZ];
   if (threadIdx.x < kRecTilesY * kRecNZ) s_cnt[threadIdx.x / kRecNZ][threadIdx.x % kRecNZ] = 0u;
   const unsigned g = xcd_tile(blockIdx.x, gridDim.x);
@@ -610,6 +609,30 @@ int records_walk_tiles(i64 columns, int nbz) {
   return best;
 }
 
+// Four rows per wave, or two on stacks that leave the chip with two waves per SIMD or fewer,
+// where a walk's steps wait for their loads and their own chain of instructions
+// (24 x 96 x 112, 24 work-groups: 28 us at four rows, 22 at two, 23 at one; 128 x 256 x 256,
+// 512: 36, 33, 47; 64 x 512 x 512, 1024: 51, 55, 88): a wave of two rows forms a third more
+// first differences per row.
+template <typename TD, typename TS, bool BAND, int MODE>
+void launch_rec(const TD* dog, int W, int H, int D, float* cand, uint32_t* cand_cnt, float band,
+                uint8_t* mask, TileRow* rows, hipStream_t s) {
+  const int nbx = (W + TX - 1) / TX, nby = (H + TY - 1) / TY, nbz = (D + ZC - 1) / ZC;
+  const int nbyg = (nby + kRecTilesY - 1) / kRecTilesY;
+  const int nz = records_walk_tiles((i64)nbx * nbyg, nbz);
+  const i64 groups = (i64)nbx * nbyg * ((nbz + nz - 1) / nz);
+  auto launch = [&](auto rows_c) {
+    constexpr int R = decltype(rows_c)::value;
+    hipLaunchKernelGGL((k_hessian_rec<TD, TS, BAND, MODE, R>), dim3((unsigned)groups),
+                       dim3(64 * rec_waves(R)), 0, s, dog, W, H, D, nbx, nby, nbyg, nz, cand,
+                       cand_cnt, band, mask, rows);
+  };
+  if (groups <= 512)
+    launch(std::integral_constant<int, 2>());
+  else
+    launch(std::integral_constant<int, 4>());
+}
+
 }  // namespace
 
 template <typename TD, typename TH>
@@ -622,12 +645,7 @@ hipError_t launch_hessian(const TD* dog, TH* hess, uint8_t* pd, int W, int H, in
   // reduced-precision storage anywhere on the path: FP64 re-evaluation band for the minors
   constexpr bool reduced = !std::is_same<TD, float>::value || !std::is_same<TH, float>::value;
   if (!hess && !pd && cand && cand_cnt) {  // records only
-    const int nbyg = (nby + kRecTilesY - 1) / kRecTilesY;
-    const int nz = records_walk_tiles((i64)nbx * nbyg, nbz);
-    const i64 ngroups = (i64)nbx * nbyg * ((nbz + nz - 1) / nz);
-    hipLaunchKernelGGL((k_hessian_rec<TD, TH, reduced, kDetect>), dim3((unsigned)ngroups),
-                       dim3(64 * kRecWaves), 0, s, dog, W, H, D, nbx, nby, nbyg, nz, cand,
-                       cand_cnt, band, (uint8_t*)nullptr, (TileRow*)nullptr);
+    launch_rec<TD, TH, reduced, kDetect>(dog, W, H, D, cand, cand_cnt, band, nullptr, nullptr, s);
   } else {
     hipLaunchKernelGGL((k_hessian<TD, TH, reduced>), dim3((unsigned)nblk), dim3(NT), 0, s, dog,
                        hess, pd, W, H, D, nbx, nby, cand, cand_cnt, band);
@@ -640,17 +658,11 @@ hipError_t launch_hessian(const TD* dog, TH* hess, uint8_t* pd, int W, int H, in
 // with rows, decides.
 hipError_t launch_hessian_records(const float* dog, uint8_t* mask, TileRow* rows, int W, int H,
                                   int D, float* cand, uint32_t* cand_cnt, hipStream_t s) {
-  const int nbx = (W + TX - 1) / TX, nby = (H + TY - 1) / TY, nbz = (D + ZC - 1) / ZC;
   if ((i64)W * H * (i64)sizeof(float) >= 0xFFFFFFF0ll) return hipErrorInvalidValue;
-  const int nbyg = (nby + kRecTilesY - 1) / kRecTilesY;
-  const int nz = records_walk_tiles((i64)nbx * nbyg, nbz);
-  const dim3 grid((unsigned)((i64)nbx * nbyg * ((nbz + nz - 1) / nz)));
   if (rows)
-    hipLaunchKernelGGL((k_hessian_rec<float, float, false, kGivenMask>), grid, dim3(64 * kRecWaves),
-                       0, s, dog, W, H, D, nbx, nby, nbyg, nz, cand, cand_cnt, 0.0f, mask, rows);
+    launch_rec<float, float, false, kGivenMask>(dog, W, H, D, cand, cand_cnt, 0.0f, mask, rows, s);
   else
-    hipLaunchKernelGGL((k_hessian_rec<float, float, false, kWriteMask>), grid, dim3(64 * kRecWaves),
-                       0, s, dog, W, H, D, nbx, nby, nbyg, nz, cand, cand_cnt, 0.0f, mask, rows);
+    launch_rec<float, float, false, kWriteMask>(dog, W, H, D, cand, cand_cnt, 0.0f, mask, rows, s);
   return hipGetLastError();
 }
 
