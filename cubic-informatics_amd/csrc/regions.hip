@@ -504,9 +504,10 @@ __global__ __launch_bounds__(NT) void k_accum(const uint32_t* __restrict__ L,
 static_assert(kAccGY * kAccGZ * kCandTile < (1 << 16) && kHessTX <= 256 &&
                   kAccGY * kHessTY <= 256 && kAccGZ * kHessTZ <= 256,
               "packed table sums: count below 2^16, offsets below 256");
-// S: table slots.
-template <typename TN, bool AVE, int S>
-__global__ __launch_bounds__(NT) void k_accum_cand(const float* __restrict__ cand,
+// S: table slots.  G: groups of four waves; a tile's records are folded by one group, so with
+// G = 4 the tiles of a work-group go side by side.
+template <typename TN, bool AVE, int S, int G>
+__global__ __launch_bounds__(NT * G) void k_accum_cand(const float* __restrict__ cand,
                                                    const uint32_t* __restrict__ cand_cnt,
                                                    const uint32_t* __restrict__ rlab,
                                                    const unsigned long long* __restrict__ multi,
@@ -540,15 +541,17 @@ __global__ __launch_bounds__(NT) void k_accum_cand(const float* __restrict__ can
   tab.init(bx * kHessTX, gy * kAccGY * kHessTY, gz * kAccGZ * kHessTZ);
   const bool has_img = img != nullptr;
   __syncthreads();
+  const int group = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / NT));
 #pragma unroll
   for (int q = 0; q < TPW; ++q) {
+    if (G > 1 && q % G != group) continue;  // uniform over the wave
     const float* t = cand + (size_t)tiles[q] * kCandTile * 7;
     const uint32_t* rl = rlab + (size_t)tiles[q] * kCandTile;  // each record's root label
     // tile origin: records hold the voxel's position in the tile
     const uint32_t tx0 = bx * kHessTX, ty0 = tby[q] * kHessTY, tz0 = tbz[q] * kHessTZ;
     // the whole wave walks the records together (the group sums below move values across
     // lanes); lanes past the tile's records load nothing and add nothing
-    for (uint32_t b = threadIdx.x - lane; b < n[q]; b += NT) {
+    for (uint32_t b = threadIdx.x % NT - lane; b < n[q]; b += NT) {
       const uint32_t i = b + lane;
       const bool ok = i < n[q];
       uint32_t r = 0u, x = 0u, y = 0u, z = 0u, iv = 0u;
@@ -783,11 +786,21 @@ hipError_t launch_region_accum_cand(const float* cand, const uint32_t* cand_cnt,
   // 150 they fill up and regions pay global atomics per voxel: 61 x 900 x 1111 at 270 regions
   // takes 362 us with 256 slots, 222 with 512.
   const bool many = blob < 3.2f;
+  // One group of four waves per work-group, or, where the work-groups leave the chip idle, one
+  // per tile (24 x 96 x 112, 12 work-groups: 21 us with one, 16 with four;
+  // 128 x 256 x 256, 256: 31, 24; 128 x 512 x 512, 1024: 65, 62; 32 x 2160 x 2560, 5400: 227, 243).
   auto go = [&](auto ave, auto slots) {
-    hipLaunchKernelGGL((k_accum_cand<TN, decltype(ave)::value, decltype(slots)::value>),
-                       dim3((unsigned)ngroups), dim3(NT), 0, s, cand, cand_cnt, rlab, multi, rid,
-                       norm, img, acc, (uint32_t)std::min<i64>(cap, 0xFFFFFFFFll), (uint32_t)W,
-                       (uint32_t)((i64)W * H), nbx, nby, nbz);
+    auto launch = [&](auto groups) {
+      constexpr int G = decltype(groups)::value;
+      hipLaunchKernelGGL((k_accum_cand<TN, decltype(ave)::value, decltype(slots)::value, G>),
+                         dim3((unsigned)ngroups), dim3(NT * G), 0, s, cand, cand_cnt, rlab, multi,
+                         rid, norm, img, acc, (uint32_t)std::min<i64>(cap, 0xFFFFFFFFll),
+                         (uint32_t)W, (uint32_t)((i64)W * H), nbx, nby, nbz);
+    };
+    if (ngroups <= 1024)
+      launch(std::integral_constant<int, kAccGY * kAccGZ>{});
+    else
+      launch(std::integral_constant<int, 1>{});
   };
   using S256 = std::integral_constant<int, 256>;
   using S512 = std::integral_constant<int, 512>;
