@@ -575,17 +575,26 @@ __global__ __launch_bounds__(NTR) void k_label_rows(const float* __restrict__ ca
   uint32_t* base = P + (size_t)T.z0 * WH + (size_t)T.y0 * Wu + T.x0;
   if (vec) {  // width and volume aligned: a quad lies in the row or outside it
     typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+    const bool nt = whole_lines((i64)W * 4);
     for (int e = (int)threadIdx.x; e < RTV / 4; e += NTR) {
       const int lx = e % (RTX / 4) * 4, row = e / (RTX / 4), ly = row % RTY, lz = row / RTY;
-      if (lx < T.ex && ly < T.ey && lz < T.ez)
-        __builtin_nontemporal_store(*reinterpret_cast<const u4*>(lv + 4 * e),
-                                    reinterpret_cast<u4*>(base + (size_t)lz * WH + (size_t)ly * Wu + lx));
+      if (lx < T.ex && ly < T.ey && lz < T.ez) {
+        u4* p = reinterpret_cast<u4*>(base + (size_t)lz * WH + (size_t)ly * Wu + lx);
+        const u4 v = *reinterpret_cast<const u4*>(lv + 4 * e);
+        if (nt) {
+          __builtin_nontemporal_store(v, p);
+        } else {
+          asm volatile("");  // (as in st_if)
+          *p = v;
+          asm volatile("");
+        }
+      }
     }
   } else {
     for (int e = (int)threadIdx.x; e < RTV; e += NTR) {
       const int lx = e % RTX, row = e / RTX, ly = row % RTY, lz = row / RTY;
       if (lx < T.ex && ly < T.ey && lz < T.ez)
-        __builtin_nontemporal_store(lv[e], base + (size_t)lz * WH + (size_t)ly * Wu + lx);
+        base[(size_t)lz * WH + (size_t)ly * Wu + lx] = lv[e];
     }
   }
 }

@@ -318,7 +318,7 @@ __global__ __launch_bounds__(256) void k_gauss_line_run(const float2* __restrict
             d[0] += v * a1[o];
             d[1] += v * a2[o];
           } else {
-            st_nt(dog + idx, (a1[o] - a2[o]) * nz);
+            dog[idx] = cvt<TS>((a1[o] - a2[o]) * nz);
           }
         }
       }
@@ -418,7 +418,7 @@ __global__ __launch_bounds__(NT) void k_gauss_walk(const float2* __restrict__ sr
           d[1] += v * s2;
           pa[q % PF] = next_a();
         } else {
-          st_nt(dog + idx, (s1 - s2) * nz);
+          dog[idx] = cvt<TS>((s1 - s2) * nz);
           idx += sa;
         }
         ring[q] = pf[q % PF];  // position c + R + 1 replaces position c - R
@@ -640,32 +640,37 @@ hipError_t gauss_xy(const TS* src, float2* dst, const float* w1, const float* w2
   return hipErrorInvalidValue;
 }
 
-// z pass: the difference (dog), or with DOT the sums of both with a
+// z pass: the difference (dog), or with DOT the sums of both with a.  (The difference leaves by
+// plain stores: streaming ones are slower where the planes do not start on whole lines, 217 us
+// for 93 x 777 x 1001 and 166 plain, and no faster where they do: 195 and 194 for
+// 64 x 1080 x 1280.)
 template <bool DOT, typename TS>
 hipError_t gauss_z(const float2* src, TS* dog, const float* a, double* dots, const float* w1,
                    const float* w2, int r1, int r2, float nz, int W, int H, int D, hipStream_t s) {
   const i64 WH = (i64)W * H;
+  const ZColumns z = z_columns(W, H);
+  const int n = z.n, m = z.rows;
 #define X(A, B)                                                                              \
   if (r1 == A && r2 == B) {                                                                  \
-    const LineGrid g = line_grid(W, D, H, 2 * (A > B ? A : B));                              \
+    const LineGrid g = line_grid(n, D, m, 2 * (A > B ? A : B));                              \
     hipLaunchKernelGGL((k_gauss_walk<A, B, DOT, TS>), dim3(g.blocks), dim3(NT), 0, s, src,   \
-                       dog, a, dots, w1, w2, nz, W, D, WH, (i64)W, g.nxb, g.no, g.len);      \
+                       dog, a, dots, w1, w2, nz, n, D, WH, (i64)W, g.nxb, g.no, g.len);      \
     return hipGetLastError();                                                                \
   }
   HDOG_GAUSS_PAIRS(X)
 #undef X
   const int R = std::max(r1, r2);
-  const i64 nxb = (W + 63) / 64;
+  const i64 nxb = (n + 63) / 64;
   int nseg, len;
-  line_segments(D, nxb * H * 4, 1024.0, 2.0, false, 2 * R, &nseg, &len);
-  const dim3 grid((unsigned)(nxb * H * nseg));
+  line_segments(D, nxb * m * 4, 1024.0, 2.0, false, 2 * R, &nseg, &len);
+  const dim3 grid((unsigned)(nxb * m * nseg));
   const size_t lds = 2 * (size_t)(2 * R + 4 * GK) * 64 * 4;
   if (R <= kLaneRadius)
     hipLaunchKernelGGL((k_gauss_line_run<DOT, false, TS>), grid, dim3(256), lds, s, src, dog, a,
-                       dots, w1, w2, r1, r2, nz, W, D, WH, (i64)W, (unsigned)nxb, (unsigned)H, len);
+                       dots, w1, w2, r1, r2, nz, n, D, WH, (i64)W, (unsigned)nxb, (unsigned)m, len);
   else
     hipLaunchKernelGGL((k_gauss_line_run<DOT, true, TS>), grid, dim3(256), lds, s, src, dog, a,
-                       dots, w1, w2, r1, r2, nz, W, D, WH, (i64)W, (unsigned)nxb, (unsigned)H, len);
+                       dots, w1, w2, r1, r2, nz, n, D, WH, (i64)W, (unsigned)nxb, (unsigned)m, len);
   return hipGetLastError();
 }
 

@@ -100,6 +100,7 @@ __global__ __launch_bounds__(NT, 5) void k_hessian(const TD* __restrict__ dog, T
   const int x0 = bx * TX, y0 = by * TY;
   const int z0 = (int)b * ZC, z1 = min(z0 + ZC, D);
   const uint32_t Wu = (uint32_t)W, WH = Wu * (uint32_t)H;
+  const bool nt = whole_lines((i64)W * sizeof(TS));
   auto inplane = [&](int gx, int gy) { return gx >= 0 && gx < W && gy >= 0 && gy < H; };
 
   // slice-invariant addressing of this thread: the byte offset in the slice; positions
@@ -278,12 +279,12 @@ __global__ __launch_bounds__(NT, 5) void k_hessian(const TD* __restrict__ dog, T
           const uint32_t idx = zb + po[k];
           if (hess) {  // NULL: mask only (the region pass reads the candidate records)
             const i64 N = (i64)WH * D;
-            hess[idx] = cvt<TS>(xx);
-            hess[N + idx] = cvt<TS>(xy);
-            hess[2 * N + idx] = cvt<TS>(xz);
-            hess[3 * N + idx] = cvt<TS>(yy);
-            hess[4 * N + idx] = cvt<TS>(yz);
-            hess[5 * N + idx] = cvt<TS>(zz);
+            st_if(nt, hess + idx, xx);
+            st_if(nt, hess + N + idx, xy);
+            st_if(nt, hess + 2 * N + idx, xz);
+            st_if(nt, hess + 3 * N + idx, yy);
+            st_if(nt, hess + 4 * N + idx, yz);
+            st_if(nt, hess + 5 * N + idx, zz);
           }
           const uint8_t m =
               BAND ? negdef_band(xx, xy, xz, yy, yz, zz, band) : negdef32(xx, xy, xz, yy, yz, zz);

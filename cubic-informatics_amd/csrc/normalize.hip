@@ -1346,6 +1346,7 @@ hipError_t launch_normalize(const uint16_t* img, TS* norm, void* tmp1, void* tmp
     return hipGetLastError();
   }
   hipError_t e;
+  const ZColumns zc = z_columns(W, H);
   uint32_t* p1 = (uint32_t*)tmp1;
   uint32_t* p2 = (uint32_t*)tmp2;
   if (rxy == 10 && rz == 10 && WH * 4 < 0xFFFFFFF0ll) {
@@ -1378,7 +1379,7 @@ hipError_t launch_normalize(const uint16_t* img, TS* norm, void* tmp1, void* tmp
     mark("normalize/minmax_zy", s);
   } else {
     // min/max along z (lines over x, y fixed per work-group), then along y
-    if ((e = minmax_line(img, true, p1, W, D, WH, W, H, rz, s)) != hipSuccess) return e;
+    if ((e = minmax_line(img, true, p1, zc.n, D, WH, W, zc.rows, rz, s)) != hipSuccess) return e;
     mark("normalize/minmax_z", s);
     if ((e = minmax_line(p1, false, p2, W, H, W, WH, D, rxy, s)) != hipSuccess) return e;
     mark("normalize/minmax_y", s);
@@ -1435,7 +1436,7 @@ hipError_t launch_normalize(const uint16_t* img, TS* norm, void* tmp1, void* tmp
   // box along z fused with the normalization
   if (ero && dil && rz > kRunRadius) {  // E and D by a z pass of their own, then split
     float2* ed = exy == (const float2*)tmp1 ? (float2*)tmp2 : (float2*)tmp1;
-    if ((e = box_line<false, TS>(exy, ed, nullptr, nullptr, 0.0f, W, D, WH, W, H, rz, s)) !=
+    if ((e = box_line<false, TS>(exy, ed, nullptr, nullptr, 0.0f, zc.n, D, WH, W, zc.rows, rz, s)) !=
         hipSuccess)
       return e;
     const i64 nb = std::min<i64>((N + NT - 1) / NT, 1 << 20);
@@ -1443,7 +1444,7 @@ hipError_t launch_normalize(const uint16_t* img, TS* norm, void* tmp1, void* tmp
                        N);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
-  e = box_line<true, TS>(exy, nullptr, norm, img, min_intensity, W, D, WH, W, H, rz, s,
+  e = box_line<true, TS>(exy, nullptr, norm, img, min_intensity, zc.n, D, WH, W, zc.rows, rz, s,
                          rz <= kRunRadius ? ero : nullptr, dil);
   mark("normalize/box_z_norm", s);
   return e;

@@ -530,8 +530,8 @@ __global__ __launch_bounds__(256) void k_soft_arg_z(const uint32_t* __restrict__
                                                     const uint32_t* __restrict__ ptap,
                                                     float2* __restrict__ pair,
                                                     uint32_t* __restrict__ amn,
-                                                    uint32_t* __restrict__ amx, int W, int H,
-                                                    int D, int rxy, int r, unsigned nxb,
+                                                    uint32_t* __restrict__ amx, int n, int W,
+                                                    int H, int D, int rxy, int r, unsigned nxb,
                                                     unsigned no, int len) {
   extern __shared__ uint32_t sm_argz[];
   const int hist = 2 * r;
@@ -540,7 +540,8 @@ __global__ __launch_bounds__(256) void k_soft_arg_z(const uint32_t* __restrict__
   uint32_t* Bx = Bn + (hist + kStep) * 64;
   uint32_t* Bt = Bx + (hist + kStep) * 64;
   const RunAt a = run_at(D, W, nxb, no, len);
-  const int x = a.x0 + a.l, y = (int)(a.base / W), xc = min(x, W - 1);
+  const int xn = a.x0 + a.l, xc = min(xn, n - 1);  // column of the plane, or of the row
+  const int x = xn % W, y = (int)(a.base / W) + xn / W;
   uint32_t qn[OK], qx[OK], qt[OK];
   auto fetch = [&](int p) {
 #pragma unroll
@@ -581,7 +582,7 @@ __global__ __launch_bounds__(256) void k_soft_arg_z(const uint32_t* __restrict__
         p += 64;
         return b;
       }, r, o);
-      if (x < W) {
+      if (xn < n) {
 #pragma unroll
         for (int k = 0; k < OK; ++k) {
           const int z = c + k;
@@ -592,7 +593,7 @@ __global__ __launch_bounds__(256) void k_soft_arg_z(const uint32_t* __restrict__
                       jz = clampi(z - r + (int)(tap >> 16) - k, 0, D - 1);
             return ((uint32_t)jz * (uint32_t)H + (uint32_t)jy) * (uint32_t)W + (uint32_t)jx;
           };
-          const i64 at = a.base + (i64)z * sa + x;
+          const i64 at = a.base + (i64)z * sa + xn;
           const bool none = o[k].kn == 0xFFFFFFFFu;  // NaN only: then kx is 0
           st_nt(pair + at, make_float2(none ? INFINITY : key_value(o[k].kn),
                                        none ? -INFINITY : key_value(o[k].kx - 1u)));
@@ -1300,7 +1301,8 @@ hipError_t launch_soft_normalize(const float* v, float* norm, float2* ed, uint32
     float2* pair = (float2*)(pk + 3 * N);    // 2 N words
     float2* exy = (float2*)scratch;          // in the place of the keys
     const XyRun x = xy_run(W, H, D, rxy);
-    const LineGrid g = run_grid(W, D, H, 2 * rz);
+    const ZColumns c = z_columns(W, H);
+    const LineGrid g = run_grid(c.n, D, c.rows, 2 * rz);
     const float kxy = 1.0f / (float)(2 * rxy + 1), kz = 1.0f / (float)(2 * rz + 1);
     const size_t zrows = (size_t)(2 * rz + kStep) * 64 * 4;
     hipError_t e = dispatch_short(rxy, [&](auto rs) {
@@ -1313,7 +1315,7 @@ hipError_t launch_soft_normalize(const float* v, float* norm, float2* ed, uint32
     e = dispatch_short(rz, [&](auto rs) {
       constexpr int R = decltype(rs)::value;
       hipLaunchKernelGGL((k_soft_arg_z<R>), dim3(g.blocks), dim3(256), 3 * zrows, s, pk, pk + N,
-                         pk + 2 * N, pair, arg, arg + N, W, H, D, rxy, rz, g.nxb, g.no, g.len);
+                         pk + 2 * N, pair, arg, arg + N, c.n, W, H, D, rxy, rz, g.nxb, g.no, g.len);
       return hipGetLastError();
     });
     if (e != hipSuccess) return e;
@@ -1327,7 +1329,7 @@ hipError_t launch_soft_normalize(const float* v, float* norm, float2* ed, uint32
     return dispatch_short(rz, [&](auto rs) {
       constexpr int R = decltype(rs)::value;
       hipLaunchKernelGGL((k_soft_box_norm<R>), dim3(g.blocks), dim3(256), 2 * zrows, s, exy, v, ed,
-                         norm, min_int, W, D, WH, rz, g.nxb, g.no, g.len, kz);
+                         norm, min_int, c.n, D, WH, rz, g.nxb, g.no, g.len, kz);
       return hipGetLastError();
     });
   }
@@ -1388,12 +1390,13 @@ hipError_t launch_soft_normalize_adjoint(const float* v, const float2* ed, const
   const i64 N = (i64)W * H * D, WH = (i64)W * H;
   float2* q0 = (float2*)scratch;
   if (rxy <= kArgRadius && rz <= kArgRadius) {
-    const LineGrid g = run_grid(W, D, H, 2 * rz);
+    const ZColumns c = z_columns(W, H);
+    const LineGrid g = run_grid(c.n, D, c.rows, 2 * rz);
     hipError_t e = dispatch_short(rz, [&](auto rs) {
       constexpr int R = decltype(rs)::value;
       hipLaunchKernelGGL((k_soft_adj_z<R>), dim3(g.blocks), dim3(256),
-                         2 * (size_t)(2 * rz + kStep) * 64 * 4, s, v, ed, gn, gv, q0, min_int, W, D,
-                         WH, rz, g.nxb, g.no, g.len, 1.0f / (float)(2 * rz + 1));
+                         2 * (size_t)(2 * rz + kStep) * 64 * 4, s, v, ed, gn, gv, q0, min_int,
+                         c.n, D, WH, rz, g.nxb, g.no, g.len, 1.0f / (float)(2 * rz + 1));
       return hipGetLastError();
     });
     if (e != hipSuccess) return e;

@@ -425,3 +425,18 @@ def test_row_walkers_by_size(hd, shape):
     dog = hd.DoG3DFilter(got)
     ref, _ = oracle.dog3d(got.cpu().numpy(), *s, truncate=4.0, gamma=1.0)
     np.testing.assert_array_equal(dog.cpu().numpy(), ref)
+
+
+# widths whose rows and planes start anywhere in a cache line, on lines, and beyond one group of
+# lanes; lines along z run over a whole plane's columns
+@pytest.mark.parametrize("shape", [(5, 3, 21), (26, 11, 61), (23, 16, 80), (22, 30, 132)])
+@pytest.mark.parametrize("rxy,rz", [(10, 10), (8, 4), (3, 2), (4, 25)])
+def test_lines_along_z_of_any_width(hd, shape, rxy, rz):
+    img = noise(shape, rz)
+    got = hd.Normalize3DFilter(img, 100, rxy, rz)
+    np.testing.assert_array_equal(got.cpu().numpy(), oracle.normalize3d(img, 100, rxy, rz))
+    s = (2.0, 1.6, 3.2, 2.56) if rxy == 10 else (1.3, 2.3, 2.1, 3.7)
+    hd.initGaussian3DKernel(*s, truncate=4.0)
+    dog = hd.DoG3DFilter(got)
+    ref, _ = oracle.dog3d(got.cpu().numpy(), *s, truncate=4.0, gamma=1.0)
+    np.testing.assert_array_equal(dog.cpu().numpy(), ref)
