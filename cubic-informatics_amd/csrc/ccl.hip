@@ -584,7 +584,7 @@ __global__ __launch_bounds__(NTR) void k_label_rows(const float* __restrict__ ca
         if (nt) {
           __builtin_nontemporal_store(v, p);
         } else {
-          asm volatile("");  // (as in st_if)
+          asm volatile("");  // keeps the two stores apart: merged into one, both would be plain
           *p = v;
           asm volatile("");
         }

@@ -157,23 +157,8 @@ __device__ __forceinline__ void st_nt(float4* p, float4 v) {
 }
 template <typename T> __device__ __forceinline__ void st_nt(T* p, float v) { *p = cvt<T>(v); }
 
-// Streaming stores or plain ones, for rows that may start anywhere: a streaming store of a
-// piece of a cache line does not wait for the rest of it (the Hessian volumes of
-// 64 x 1080 x 1279: 1118 us, plain 848; of 1280 columns 626, plain 683).
-template <typename T, typename V>
-__device__ __forceinline__ void st_if(bool nt, T* p, V v) {
-  if (nt) {  // uniform
-    st_nt(p, v);
-  } else {
-    asm volatile("");  // keep the two stores apart: merged into one, both would be plain
-    if constexpr (std::is_same<T, V>::value)
-      *p = v;
-    else
-      *p = cvt<T>(v);
-    asm volatile("");
-  }
-}
-__host__ __device__ inline bool whole_lines(i64 bytes) { return bytes % 64 == 0; }  // (rows apart)
+// rows `bytes` apart start on whole lines (half of them)
+__host__ __device__ inline bool whole_lines(i64 bytes) { return bytes % 64 == 0; }
 
 // The lines along z as rows of n columns: a plane's columns as one row where they can be
 // counted, so that no lanes idle at the rows' ends and odd rows do not shift each row's lines.

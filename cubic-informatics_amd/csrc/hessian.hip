@@ -74,7 +74,10 @@ __device__ __forceinline__ uint8_t negdef_band(float xx, float xy, float xz, flo
 // slots rotate instead of being recomputed; global indices are 32-bit (N < 2^32).
 // (the second bound keeps the register allocation within five waves per SIMD, the most
 // that the LDS rings allow)
-template <typename TD, typename TS, bool BAND>
+// STREAM: streaming stores of the element volumes, where their rows start on whole lines
+// (64 x 1080 x 1280: 626 us, plain 683); elsewhere a streaming store of a piece of a line does
+// not wait for the rest of it (1279 columns: 1118, plain 848).
+template <typename TD, typename TS, bool BAND, bool STREAM>
 __global__ __launch_bounds__(NT, 5) void k_hessian(const TD* __restrict__ dog, TS* __restrict__ hess,
                                                 uint8_t* __restrict__ pd, int W, int H, int D,
                                                 int nbx, int nby, float* __restrict__ cand,
@@ -100,7 +103,12 @@ __global__ __launch_bounds__(NT, 5) void k_hessian(const TD* __restrict__ dog, T
   const int x0 = bx * TX, y0 = by * TY;
   const int z0 = (int)b * ZC, z1 = min(z0 + ZC, D);
   const uint32_t Wu = (uint32_t)W, WH = Wu * (uint32_t)H;
-  const bool nt = whole_lines((i64)W * sizeof(TS));
+  auto put_element = [](TS* p, float v) {
+    if (STREAM)
+      st_nt(p, v);
+    else
+      *p = cvt<TS>(v);
+  };
   auto inplane = [&](int gx, int gy) { return gx >= 0 && gx < W && gy >= 0 && gy < H; };
 
   // slice-invariant addressing of this thread: the byte offset in the slice; positions
@@ -279,12 +287,12 @@ __global__ __launch_bounds__(NT, 5) void k_hessian(const TD* __restrict__ dog, T
           const uint32_t idx = zb + po[k];
           if (hess) {  // NULL: mask only (the region pass reads the candidate records)
             const i64 N = (i64)WH * D;
-            st_if(nt, hess + idx, xx);
-            st_if(nt, hess + N + idx, xy);
-            st_if(nt, hess + 2 * N + idx, xz);
-            st_if(nt, hess + 3 * N + idx, yy);
-            st_if(nt, hess + 4 * N + idx, yz);
-            st_if(nt, hess + 5 * N + idx, zz);
+            put_element(hess + idx, xx);
+            put_element(hess + N + idx, xy);
+            put_element(hess + 2 * N + idx, xz);
+            put_element(hess + 3 * N + idx, yy);
+            put_element(hess + 4 * N + idx, yz);
+            put_element(hess + 5 * N + idx, zz);
           }
           const uint8_t m =
               BAND ? negdef_band(xx, xy, xz, yy, yz, zz, band) : negdef32(xx, xy, xz, yy, yz, zz);
@@ -648,8 +656,14 @@ hipError_t launch_hessian(const TD* dog, TH* hess, uint8_t* pd, int W, int H, in
   if (!hess && !pd && cand && cand_cnt) {  // records only
     launch_rec<TD, TH, reduced, kDetect>(dog, W, H, D, cand, cand_cnt, band, nullptr, nullptr, s);
   } else {
-    hipLaunchKernelGGL((k_hessian<TD, TH, reduced>), dim3((unsigned)nblk), dim3(NT), 0, s, dog,
-                       hess, pd, W, H, D, nbx, nby, cand, cand_cnt, band);
+    auto launch = [&](auto stream) {
+      hipLaunchKernelGGL((k_hessian<TD, TH, reduced, decltype(stream)::value>), dim3((unsigned)nblk),
+                         dim3(NT), 0, s, dog, hess, pd, W, H, D, nbx, nby, cand, cand_cnt, band);
+    };
+    if (whole_lines((i64)W * (i64)sizeof(TH)))
+      launch(std::true_type());
+    else
+      launch(std::false_type());
   }
   mark("hessian/hessian_pd", s);
   return hipGetLastError();
