@@ -11,9 +11,9 @@
 // stay FP32 whatever the storage type of norm / dog.
 //
 // Radius pairs (r1, r2) that occur in practice have compile-time kernels: the x and y passes
-// fused in a row walker, the z pass (and the differentiable form's separate passes) as column
-// walkers (one thread per line, a register ring, every input read once, no LDS).  Other radii
-// have walkers with LDS rings that form eight outputs at a time.
+// fused in a row walker, the z pass as a column walker (one thread per line, a register ring,
+// every input read once, no LDS).  Other radii, and the smallest stacks along x and y, have
+// walks with their history in LDS that form eight outputs at a time.
 #include "hdog_internal.hpp"
 
 namespace hdog {

@@ -28,8 +28,8 @@
 // the weight of every window tap that clamps onto them); the min filter is taken by its
 // subgradient: each output's gradient goes to the voxel that attains the window minimum
 // (the lowest linear index among equal minima), likewise for the max.  The argmin / argmax
-// of the 3-D window are found by three separable passes over (value, index) pairs, which
-// is exact because the order "smaller value, then smaller index" is total.
+// of the 3-D window are found by separable passes over (value, index) pairs, which is exact
+// because the order "smaller value, then smaller index" is total.
 #include "run8.hpp"
 
 namespace hdog {
