@@ -1350,10 +1350,15 @@ hipError_t launch_normalize(const uint16_t* img, TS* norm, void* tmp1, void* tmp
   const ZColumns zc = z_columns(W, H);
   uint32_t* p1 = (uint32_t*)tmp1;
   uint32_t* p2 = (uint32_t*)tmp2;
-  if (rxy == 10 && rz == 10 && WH * 4 < 0xFFFFFFF0ll) {
+  // The z walk of radius 10 keeps its window in registers and goes slice by slice, a barrier
+  // each; the walk of other radii goes eight slices at a time, which is sooner done where there
+  // are few (slices of 64 x 32 tiles: its us / the walk's): 24 x 96 x 112, 144: 10 / 18;
+  // 40 x 160 x 160, 600: 13 / 23; 64 x 200 x 200, 1792: 22 / 24; 128 x 256 x 256, 4096: 32 / 30;
+  // 20 x 1080 x 1280, 13600: 92 / 59.
+  const unsigned nxt = (W + 63) / 64, nyt = (H + 31) / 32;
+  if (rxy == 10 && rz == 10 && (i64)nxt * nyt * D > 2048 && WH * 4 < 0xFFFFFFF0ll) {
     // min/max along y and z in one z walk over 64 x 32 tiles (slices addressed by buffer
     // descriptors with 32-bit byte offsets)
-    const unsigned nxt = (W + 63) / 64, nyt = (H + 31) / 32;
     int nzs, zlen;
     // one 1024-thread work-group per CU: whole rounds of 256 (128 x 256 x 256, 32 work-groups
     // per segment: 93 us whole, 28 in eight segments, 43 in twelve)
@@ -1364,15 +1369,15 @@ hipError_t launch_normalize(const uint16_t* img, TS* norm, void* tmp1, void* tmp
     if ((e = hipGetLastError()) != hipSuccess) return e;
     mark("normalize/minmax_zy", s);
   } else if (rxy >= 4 && rxy <= kZyRadiusY && rz >= 4 && rz <= kZyRadiusZ) {
-    const unsigned nxt = (W + 63) / 64, nyt = (H + OK - 1) / OK;
+    const unsigned nyg = (H + OK - 1) / OK;
     int nzs, zlen;
-    line_segments(D, (i64)nxt * nyt * 8, 1024.0, 2.0, false, 2 * rz, &nzs, &zlen);
-    const dim3 grid((unsigned)((i64)nxt * nyt * nzs));
+    line_segments(D, (i64)nxt * nyg * 8, 1024.0, 2.0, false, 2 * rz, &nzs, &zlen);
+    const dim3 grid((unsigned)((i64)nxt * nyg * nzs));
     const size_t lds = (size_t)(2 * rz + OK) * OK * 64 * 4;
 #define X(NQ)                                                                                   \
   if (2 * rxy + OK <= NQ && 2 * rxy > NQ - 2 * OK)                                                 \
     hipLaunchKernelGGL((k_minmax_zy_run<NQ>), grid, dim3(512), lds, s, img, p2, W, H, D, rxy, rz, \
-                       nyt, nxt, zlen);
+                       nyg, nxt, zlen);
     X(16) X(24) X(32) X(40)
 #undef X
     static_assert(2 * kZyRadiusY + OK == 40, "the largest");

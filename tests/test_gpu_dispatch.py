@@ -440,3 +440,21 @@ def test_lines_along_z_of_any_width(hd, shape, rxy, rz):
     dog = hd.DoG3DFilter(got)
     ref, _ = oracle.dog3d(got.cpu().numpy(), *s, truncate=4.0, gamma=1.0)
     np.testing.assert_array_equal(dog.cpu().numpy(), ref)
+
+
+# either side of the size where the z walk of radius 10 takes over: 2048 slices of 64 x 32 tiles
+# and one more, and a plane of more tiles than that
+@pytest.mark.parametrize("shape", [(1024, 33, 20), (683, 65, 20), (2, 33, 65), (3, 2160, 700)])
+def test_minmax_zy_by_size(hd, shape):
+    img = noise(shape, 4)
+    got = hd.Normalize3DFilter(img, 100, 10, 10)
+    np.testing.assert_array_equal(got.cpu().numpy(), oracle.normalize3d(img, 100, 10, 10))
+
+
+# the z walk of radius 10 itself at the depths of test_minmax_zy_of_any_depth (1100 tiles: from
+# two slices on)
+@pytest.mark.parametrize("depth", [2, 10, 11, 12, 21, 22, 31, 32, 33, 43, 74])
+def test_minmax_zy_walk_of_any_depth(hd, depth):
+    img = noise((depth, 35200, 3), depth)
+    got = hd.Normalize3DFilter(img, 100, 10, 10)
+    np.testing.assert_array_equal(got.cpu().numpy(), oracle.normalize3d(img, 100, 10, 10))
