@@ -458,3 +458,42 @@ def test_minmax_zy_walk_of_any_depth(hd, depth):
     img = noise((depth, 35200, 3), depth)
     got = hd.Normalize3DFilter(img, 100, 10, 10)
     np.testing.assert_array_equal(got.cpu().numpy(), oracle.normalize3d(img, 100, 10, 10))
+
+
+# the row walkers and the z walk themselves, beyond the sizes that the walks of any radius take:
+# odd columns, one and several segments with short last ones
+@pytest.mark.parametrize("shape", [(400, 83, 130), (389, 201, 61), (130, 301, 401), (770, 43, 65)])
+@pytest.mark.parametrize("sigmas,truncate", [((2.0, 1.6, 3.2, 2.56), 4.0), ((4.0, 1.8, 6.0, 2.7), 2.0)])
+def test_row_walkers_bitexact(hd, shape, sigmas, truncate):
+    img = noise(shape, 8)
+    got = hd.Normalize3DFilter(img, 100, 10, 10)
+    np.testing.assert_array_equal(got.cpu().numpy(), oracle.normalize3d(img, 100, 10, 10))
+    hd.initGaussian3DKernel(*sigmas, truncate=truncate)
+    dog = hd.DoG3DFilter(got)
+    ref, _ = oracle.dog3d(got.cpu().numpy(), *sigmas, truncate=truncate, gamma=1.0)
+    np.testing.assert_array_equal(dog.cpu().numpy(), ref)
+
+
+# soft response with the row walker's weights of their own along y (more than 28 k rows)
+def test_soft_sigma_gradients_by_the_row_walker(hd):
+    import soft_reference as ref
+    import torch
+    from hdog import soft
+    shape, s1, s2 = (40, 241, 190), [1.6, 2.0, 2.0], [2.56, 3.2, 3.2]
+    rad1, rad2 = soft.radii(s1), soft.radii(s2)
+    rng = np.random.default_rng(6)
+    v = torch.from_numpy(rng.standard_normal(shape).astype(np.float32))
+    t = torch.from_numpy((rng.random(shape) < 0.1).astype(np.uint8))
+    a, b = (torch.tensor(s, dtype=torch.float64, requires_grad=True) for s in (s1, s2))
+    tau = torch.tensor(0.05, dtype=torch.float64)
+    vd, td = v.to(hd.device).requires_grad_(), t.to(hd.device)
+    # (the loss's own mask: sigmas given as lists would be rounded to FP32 on the way)
+    mask = soft.run_forward(hd, vd.detach(), td, a, b, 0.05, rad1, rad2)[3].cpu()
+    soft.soft_loss(hd, vd, td, a, b, tau, rad1, rad2).backward()
+    v64 = v.double().requires_grad_()
+    a2, b2 = (torch.tensor(s, dtype=torch.float64, requires_grad=True) for s in (s1, s2))
+    ref.forward(v64, a2, b2, tau, t, rad1, rad2, mask=mask.bool())[0].backward()
+    got, want = torch.cat([a.grad, b.grad]), torch.cat([a2.grad, b2.grad])
+    assert float((got - want).abs().max()) <= 2e-3 * float(want.abs().max())
+    err = (vd.grad.cpu().double() - v64.grad).abs().max()
+    assert float(err) <= 2e-3 * float(v64.grad.abs().max())
