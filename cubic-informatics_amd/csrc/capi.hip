@@ -67,7 +67,7 @@ struct hdog_ctx {
   float sigma[4] = {0, 0, 0, 0};
   double truncate = 0.0;
   int r[4] = {0, 0, 0, 0};
-  i64 R = 0;
+  i64 R = 0;  // regions of the list in the o_ arrays; kNoList: the call that fills it has not finished
   uint32_t* h_R = nullptr;         // page-locked: the region count, written by the device
   hipEvent_t counted = nullptr;   // recorded after the kernel that writes it
   void* stage = nullptr;          // page-locked, kStageBytes: short region lists on their way
@@ -88,6 +88,7 @@ struct hdog_ctx {
   };
   std::vector<Tuned> tuned;
 };
+constexpr i64 kNoList = -1;
 
 thread_local hdog::Prof* hdog::tl_prof = nullptr;
 
@@ -295,6 +296,8 @@ int copy_out(hdog_ctx* ctx, const CopyList& want, hipStream_t s) {
   size_t total = 0;
   int locked = 0, pageable = 0;
   for (int k = 0; k < want.n; ++k) {
+    // the runtime's copies refuse it, a kernel would read address 0
+    if (!want.src[k]) return fail(ctx, HDOG_ERR_STATE, "the region list has no memory");
     total += (want.bytes[k] + 15) / 16 * 16;
     void* d = nullptr;
     const HostMem m = host_memory(want.dst[k], want.bytes[k], &d);
@@ -347,6 +350,9 @@ int regional_features_t(hdog_ctx* ctx, hipStream_t s, uint32_t* labels, const TH
   // The rest is launched for as many regions as the arrays hold, and the count, which the
   // first of its kernels writes, read meanwhile; only when they hold too few (the first call,
   // a stack with more regions) are they grown and the rest run again.
+  // Until the end there is no list: the kernels write over the last call's, and an allocation
+  // that fails leaves some of its arrays without memory.
+  ctx->R = kNoList;
   i64 R = 0, cap = region_capacity(ctx);
   for (;;) {
     RegionAcc* acc = (RegionAcc*)ctx->acc.p;
@@ -988,7 +994,9 @@ int hdog_regional_features(hdog_ctx* ctx, void* stream, const uint32_t* d_labels
 int hdog_regions_download(hdog_ctx* ctx, void* stream, hdog_regions* out) {
   if (!ctx || !out) return HDOG_ERR_ARG;
   const i64 R = ctx->R;
-  out->count = R;
+  out->count = std::max<i64>(R, 0);
+  if (R == kNoList)
+    return fail(ctx, HDOG_ERR_STATE, "the last call that forms regions did not finish");
   if (R > out->capacity)
     return fail(ctx, HDOG_ERR_CAPACITY, "%lld regions exceed the caller capacity %lld",
                 (long long)R, (long long)out->capacity);

@@ -159,8 +159,10 @@ int hdog_regional_features(hdog_ctx* ctx, void* stream, const uint32_t* d_labels
                            int is_ave_mode, int64_t* num_regions);
 
 /* Copies the last hdog_regional_features result into caller host arrays (regions
- * 0..count-1; entry 0 zero) and synchronizes `stream`.  Replaces the D2H copies of
- * src/3D/HDoG3D_main.cpp:216-227. */
+ * 0..count-1; entry 0 zero) and synchronizes `stream`.  A call refused for its arguments
+ * leaves the last list as it was; after one that failed while it formed the regions (e.g. out
+ * of memory) there is none, and this returns HDOG_ERR_STATE with count 0.  Replaces the D2H
+ * copies of src/3D/HDoG3D_main.cpp:216-227. */
 int hdog_regions_download(hdog_ctx* ctx, void* stream, hdog_regions* out);
 
 /* ---- fused substack ------------------------------------------------------- */

@@ -1,0 +1,111 @@
+"""Host code of libhdog.so where a GPU cannot or must not be brought to the case: allocations
+that fail, scratch sizes, saved files.  The library runs in a process of its own on a stand-in
+for the HIP runtime (host_runtime/), which launches nothing and notes what would be launched."""
+import ctypes
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "host_runtime")
+
+
+@pytest.fixture(scope="module")
+def runtime(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("host_runtime") / "host_runtime.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-D__HIP_PLATFORM_AMD__",
+                    "-I/opt/rocm/include", "-shared", "-fPIC", "-o", so,
+                    os.path.join(HERE, "host_runtime.cpp")], check=True)
+    return so
+
+
+def session(runtime, name, *args):
+    r = subprocess.run([sys.executable, os.path.join(HERE, "session.py"), runtime, name,
+                        *map(str, args)], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+# ---- region lists ----------------------------------------------------------------------
+ARRAYS = (("label", 4), ("size", 2), ("voxels", 8), ("centroid_x", 4), ("centroid_y", 4),
+          ("centroid_z", 4), ("structureness", 4), ("blobness", 4), ("max_normalized", 4),
+          ("hessian", 24), ("intensity_sum", 8), ("intensity_max", 2))
+
+
+class CopyList(ctypes.Structure):
+    _fields_ = [("src", ctypes.c_uint64 * 18), ("dst", ctypes.c_uint64 * 18),
+                ("bytes", ctypes.c_uint64 * 18), ("n", ctypes.c_int)]
+
+
+def region_arrays(C, h, cap, locked):
+    reg, keep = C.Regions(), []
+    reg.capacity = cap
+    for name, size in ARRAYS:
+        if locked:
+            p = ctypes.c_void_p()
+            assert C.hdog_host_alloc(h, cap * size, ctypes.byref(p)) == C.HDOG_OK
+            setattr(reg, name, p.value)
+        else:
+            keep.append(ctypes.create_string_buffer(cap * size))
+            setattr(reg, name, ctypes.addressof(keep[-1]))
+    return reg, keep
+
+
+def copies(rt):
+    """The copy lists launched since the last clear."""
+    return [CopyList.from_address(rt.host_launch_arg0(i)) for i in range(rt.host_launches())
+            if b"k_copy_list" in rt.host_launch_name(i)]
+
+
+def features(C, h, labels=4096):
+    n = ctypes.c_int64(-1)
+    rc = C.hdog_regional_features(h, None, labels, 8192, 12288, 16384, 64, 16, 16, 0,
+                                  ctypes.byref(n))
+    return rc, n.value
+
+
+def download_after_failure(rt, C, h, locked, failing):
+    reg, keep = region_arrays(C, h, 4000, locked == "1")
+    rt.host_set_regions(100)
+    assert features(C, h) == (C.HDOG_OK, 100)
+    rt.host_clear()
+    assert C.hdog_regions_download(h, None, ctypes.byref(reg)) == C.HDOG_OK and reg.count == 100
+    assert [l.n for l in copies(rt)] == [17] and all(l.src[k] for l in copies(rt) for k in range(17))
+    # a call refused for its arguments leaves the list as it was
+    assert features(C, h, None)[0] == C.HDOG_ERR_ARG
+    assert C.hdog_regions_download(h, None, ctypes.byref(reg)) == C.HDOG_OK and reg.count == 100
+    # one that fails while its arrays grow leaves none: no copy is launched
+    rt.host_set_regions(3000)
+    rt.host_fail_allocation(int(failing))
+    assert features(C, h)[0] == C.HDOG_ERR_HIP
+    rt.host_clear()
+    assert C.hdog_regions_download(h, None, ctypes.byref(reg)) == C.HDOG_ERR_STATE
+    assert rt.host_launches() == 0 and reg.count == 0
+    # the next call that finishes brings one again
+    rt.host_fail_allocation(-1)
+    assert features(C, h) == (C.HDOG_OK, 3000)
+    rt.host_clear()
+    assert C.hdog_regions_download(h, None, ctypes.byref(reg)) == C.HDOG_OK and reg.count == 3000
+    assert all(l.src[k] for l in copies(rt) for k in range(l.n))
+
+
+# every array of the list in turn, and the accumulators after them
+@pytest.mark.parametrize("failing", range(10))
+@pytest.mark.parametrize("locked", [0, 1])
+def test_download_after_a_call_that_ran_out_of_memory(runtime, locked, failing):
+    session(runtime, "download_after_failure", locked, failing)
+
+
+def no_list_yet(rt, C, h):
+    reg, keep = region_arrays(C, h, 16, False)
+    assert C.hdog_regions_download(h, None, ctypes.byref(reg)) == C.HDOG_OK and reg.count == 0
+    rt.host_set_regions(5)
+    assert features(C, h) == (C.HDOG_OK, 5)
+    assert C.hdog_release_scratch(h) == C.HDOG_OK
+    rt.host_clear()
+    assert C.hdog_regions_download(h, None, ctypes.byref(reg)) == C.HDOG_OK and reg.count == 0
+    assert rt.host_launches() == 0
+
+
+def test_download_without_a_list_is_empty(runtime):
+    session(runtime, "no_list_yet")
