@@ -52,13 +52,19 @@ __device__ __forceinline__ uint8_t negdef_band(float xx, float xy, float xz, flo
   const float m3 = t1 + t2 - t3 - t4 - t5;
   const float s2 = fabsf(p1) + fabsf(p2);
   const float s3 = fabsf(t1) + fabsf(t2) + fabsf(t3) + fabsf(t4) + fabsf(t5);
-  if (fabsf(m2) < band * s2 || fabsf(m3) < band * s3) {
-    const double a = xx, b = xy, c = xz, d = yy, e = yz, f = zz;
-    const double n2 = a * d - b * b;
+  bool in = (xx < 0) & (m2 > 0) & (m3 < 0);
+  // (the FP32 answer and each FP64 minor are settled before the next one's terms are formed:
+  // with all of them live the records-only kernel of FP32 DoG and 16-bit elements took 129
+  // vector registers, one too many for four waves per SIMD; 127 so)
+  const bool near2 = fabsf(m2) < band * s2, near3 = fabsf(m3) < band * s3;
+  if (near2 | near3) {
+    const double a = xx, b = xy, d = yy;
+    const bool in2 = (a < 0) & (a * d - b * b > 0);
+    const double c = xz, e = yz, f = zz;
     const double n3 = a * d * f + 2 * b * e * c - a * e * e - d * c * c - f * b * b;
-    return (a < 0 && n2 > 0 && n3 < 0) ? 1 : 0;
+    in = in2 & (n3 < 0);
   }
-  return (xx < 0 && m2 > 0 && m3 < 0) ? 1 : 0;
+  return in ? 1 : 0;
 }
 
 // z-streaming form.  A work-group owns a TX x TY column of outputs over ZC consecutive
