@@ -1196,7 +1196,7 @@ int hdog_soft_forward(hdog_ctx* ctx, void* stream, const float* d_v, const uint8
   const i64 N = (i64)width * height * depth;
   HIPCHK(ensure(ctx->tmp1, (size_t)N * 8));
   const i64 ntiles = hessian_tiles(width, height, depth);
-  HIPCHK(ensure(ctx->cand, (size_t)ntiles * kCandTile * 7 * 4));
+  HIPCHK(ensure(ctx->cand, (size_t)N * 7 * 4));
   HIPCHK(ensure(ctx->cand_cnt, (size_t)ntiles * 4));
   HIPCHK(ensure(ctx->sums, 64 * 8));
   HIPCHK(launch_gauss_dog(d_v, ctx->tmp1.p, S.w, S.r, (float)S.s, d_dog, width, height, depth, s));
@@ -1230,7 +1230,7 @@ int hdog_soft_backward(hdog_ctx* ctx, void* stream, const float* d_v, const floa
   const i64 N = (i64)width * height * depth;
   HIPCHK(ensure(ctx->tmp1, (size_t)N * 8));
   const i64 ntiles = hessian_tiles(width, height, depth);
-  HIPCHK(ensure(ctx->cand, (size_t)ntiles * kCandTile * 7 * 4));
+  HIPCHK(ensure(ctx->cand, (size_t)N * 7 * 4));
   HIPCHK(ensure(ctx->cand_cnt, (size_t)ntiles * 4));
   HIPCHK(ensure(ctx->ddog, (size_t)N * 4));
   HIPCHK(ensure(ctx->sums, 64 * 8));
@@ -1238,7 +1238,7 @@ int hdog_soft_backward(hdog_ctx* ctx, void* stream, const float* d_v, const floa
   float* cand = (float*)ctx->cand.p;
   uint32_t* cnt = (uint32_t*)ctx->cand_cnt.p;
   float* ddog = (float*)ctx->ddog.p;
-  HIPCHK(ensure(ctx->rows, (size_t)fg_words(width, height, depth) * sizeof(TileRow)));
+  HIPCHK(ensure(ctx->rows, (size_t)height * depth * row_pieces(width) * sizeof(TileRow)));
   TileRow* rows = (TileRow*)ctx->rows.p;
   HIPCHK(launch_zero_f64(sums, 8, s));
   // H is recomputed from the checkpointed DoG; the mask from the forward pass is used

@@ -46,23 +46,24 @@ constexpr int kCachePolicyNT = 2;
 #endif
 constexpr int kHessTX = 64, kHessTY = HDOG_HESS_TY, kHessTZ = 16;
 constexpr int kCandTile = kHessTX * kHessTY * kHessTZ;
-// Element words of slot i: kCandTile + 6 i, in this order (two groups of three: one 12-byte
-// access each; the adjoint's halo rows need only the first).  As six planes, a row with a few
+// Element words of slot i: kCandTile + 6 i (the functions below take the address of slot 0's), in
+// this order (two groups of three: one 12-byte access each; the adjoint's halo rows need only
+// the first).  As six planes, a row with a few
 // candidates took seven stores of a few lanes each instead of three: 393 us instead of
 // 366 for the Hessian pass of 32 x 2160 x 2560.
 enum RecWord { kRecXY, kRecYY, kRecYZ, kRecXX, kRecXZ, kRecZZ };
 struct RecHalf {
   float a, b, c;
 };
-__device__ __forceinline__ RecHalf rec_load(const float* rec, uint32_t slot, int half) {
-  return *reinterpret_cast<const RecHalf*>(rec + kCandTile + 6 * (size_t)slot + 3 * half);
+__device__ __forceinline__ RecHalf rec_load(const float* el, uint32_t slot, int half) {
+  return *reinterpret_cast<const RecHalf*>(el + 6 * (size_t)slot + 3 * half);
 }
-__device__ __forceinline__ void rec_store(float* rec, uint32_t slot, int half, RecHalf v) {
-  *reinterpret_cast<RecHalf*>(rec + kCandTile + 6 * (size_t)slot + 3 * half) = v;
+__device__ __forceinline__ void rec_store(float* el, uint32_t slot, int half, RecHalf v) {
+  *reinterpret_cast<RecHalf*>(el + 6 * (size_t)slot + 3 * half) = v;
 }
 // xx, xy, xz, yy, yz, zz of a slot
-__device__ __forceinline__ void rec_elements(const float* rec, uint32_t slot, float (&h)[6]) {
-  const RecHalf u = rec_load(rec, slot, 0), v = rec_load(rec, slot, 1);
+__device__ __forceinline__ void rec_elements(const float* el, uint32_t slot, float (&h)[6]) {
+  const RecHalf u = rec_load(el, slot, 0), v = rec_load(el, slot, 1);
   h[0] = v.a;
   h[1] = u.a;
   h[2] = v.b;
@@ -79,6 +80,19 @@ inline i64 hessian_tiles(int W, int H, int D) {
 }
 // words of the candidate bit mask: one per (z, y) row of each Hessian tile, tile-major
 inline i64 fg_words(int W, int H, int D) { return hessian_tiles(W, H, D) * kHessTY * kHessTZ; }
+// The differentiable form keeps no blocks of kCandTile slots: the block of the tile at
+// (x0, y0, z0) has a slot per voxel that the tile holds of the volume, and the blocks follow one
+// another, 28 bytes per voxel for any shape.  (Whole tiles would be 16 times that for a
+// single plane, more than the card has for 30000 x 30000.)
+struct RecBlock {
+  i64 first;  // slots before the block; its words start at 7 first
+  int slots;
+};
+__host__ __device__ inline RecBlock rec_block(int x0, int y0, int z0, int W, int H, int D) {
+  const int ex = W - x0 < kHessTX ? W - x0 : kHessTX, ey = H - y0 < kHessTY ? H - y0 : kHessTY,
+            ez = D - z0 < kHessTZ ? D - z0 : kHessTZ;
+  return {(i64)z0 * W * H + ez * ((i64)y0 * W + ey * (i64)x0), ex * ey * ez};
+}
 // Region sums from candidate records: one work-group folds kAccGY x kAccGZ Hessian tiles
 // (y, z); a region inside one such group is summed by that work-group alone.
 #ifndef HDOG_ACC_GY
@@ -498,14 +512,17 @@ hipError_t launch_ccl_candidates(const float* cand, const uint32_t* cand_cnt, i6
 hipError_t launch_mask_records(const uint8_t* pd, float* pos, uint32_t* cand_cnt, int W, int H,
                                int D, hipStream_t s);
 // differentiable blob response (soft.hip)
-// One 64-voxel row of a Hessian tile (ly + kHessTY lz): its masked voxels, and where in the
-// tile's records theirs start (consecutive, in x order).
+// 64 voxels of a row, x0 .. x0 + 63 for x0 a multiple of 64: the masked ones, and where in the
+// tile's records theirs start (consecutive, in x order).  Row y of slice z has its pieces at
+// ((z H + y) + 0, 1, ...) * row_pieces(W).
 struct TileRow {
   unsigned long long bits;
   unsigned long long first;
 };
-// The records of the masked voxels of a DoG volume, voxel 0 included, in the Hessian pass's
-// layout; the mask volume is written, or, with `rows` (one per tile row, written), decides.
+inline int row_pieces(int W) { return (W + kHessTX - 1) / kHessTX; }
+// The records of the masked voxels of a DoG volume, voxel 0 included, in blocks as rec_block
+// says (7 words per voxel); the mask volume is written, or, with `rows` (one per piece of a row,
+// written), decides.
 hipError_t launch_hessian_records(const float* dog, uint8_t* mask, TileRow* rows, int W, int H,
                                   int D, float* cand, uint32_t* cand_cnt, hipStream_t s);
 // sums[0] = loss sum, sums[1] = |M| over the records

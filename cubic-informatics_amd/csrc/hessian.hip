@@ -321,8 +321,8 @@ __global__ __launch_bounds__(NT, 5) void k_hessian(const TD* __restrict__ dog, T
           if (is_cand) {
             const uint32_t slot = base + (uint32_t)__popcll(bal & ((1ull << lane) - 1ull));
             rec[slot] = __uint_as_float(cidx);
-            rec_store(rec, slot, 0, {h6[1], h6[3], h6[4]});
-            rec_store(rec, slot, 1, {h6[0], h6[2], h6[5]});
+            rec_store(rec + kCandTile, slot, 0, {h6[1], h6[3], h6[4]});
+            rec_store(rec + kCandTile, slot, 1, {h6[0], h6[2], h6[5]});
           }
         }
       }
@@ -395,8 +395,8 @@ __device__ __forceinline__ float swap_pairs(float v) {
 
 // MODE: kDetect, or for the differentiable form, which keeps voxel 0 as any other,
 // kWriteMask (the mask volume is written too) or kGivenMask (the records of the voxels that
-// the mask volume holds, whatever their minors, and each tile row's bits and first record:
-// the records of a row are consecutive, in lane order).
+// the mask volume holds, whatever their minors, and the bits and first record of each piece of a
+// row: its records are consecutive, in lane order).
 constexpr int kDetect = 0, kWriteMask = 1, kGivenMask = 2;
 typedef uint32_t U3 __attribute__((ext_vector_type(3)));
 template <typename TD, typename TS, bool BAND, int MODE, int TY>
@@ -470,8 +470,14 @@ __global__ __launch_bounds__(64 * rec_waves(TY)) void k_hessian_rec(
       const int tz = (z - z0) / kHessTZ;  // Hessian tile of the slice within the walk
       const unsigned tile = (unsigned)(((gz * nz + tz) * nby + by) * nbx + bx);
       const uint32_t lz = (uint32_t)(z - (z0 + tz * kHessTZ));
-      const __amdgpu_buffer_rsrc_t rr =
-          buf_rsrc(cand + (size_t)tile * kCandTile * 7, (uint32_t)kCandTile * 7u * 4u);
+      i64 first = (i64)tile * kCandTile;  // the tile's block of records
+      int slots = kCandTile;
+      if (MODE != kDetect) {
+        const RecBlock b = rec_block(x0, by * kHessTY, z0 + tz * kHessTZ, W, H, D);
+        first = b.first;
+        slots = b.slots;
+      }
+      const __amdgpu_buffer_rsrc_t rr = buf_rsrc(cand + first * 7, (uint32_t)slots * 28u);
 #pragma unroll
       for (int r = 0; r < TY; ++r) {
         const float xx = Hxx[C][r];
@@ -505,8 +511,8 @@ __global__ __launch_bounds__(64 * rec_waves(TY)) void k_hessian_rec(
         uint32_t base = 0;
         if (act && lane == 0) base = atomicAdd(&s_cnt[tt][tz], (uint32_t)__popcll(act));
         base = __builtin_amdgcn_readfirstlane(base);
-        if (MODE == kGivenMask && lane == 0 && by < nby)
-          rows[(size_t)tile * (kHessTY * kHessTZ) + (uint32_t)(ty0 + r) + kHessTY * lz] = {act, base};
+        if (MODE == kGivenMask && lane == 0 && (!CLIP || y + r < H))
+          rows[((size_t)z * (size_t)H + (size_t)(y + r)) * (size_t)nbx + (size_t)bx] = {act, base};
         if (is_c) {
           const uint32_t slot = base + __builtin_amdgcn_mbcnt_hi(
                                            (uint32_t)(act >> 32),
@@ -517,8 +523,8 @@ __global__ __launch_bounds__(64 * rec_waves(TY)) void k_hessian_rec(
           const U3 v = {__float_as_uint(round_to<TS>(xx)), __float_as_uint(round_to<TS>(xz)),
                         __float_as_uint(round_to<TS>(zz))};
           __builtin_amdgcn_raw_buffer_store_b32(cidx, rr, (int)(slot * 4u), 0, 0);
-          __builtin_amdgcn_raw_buffer_store_b96(u, rr, (int)(slot * 24u), kCandTile * 4, 0);
-          __builtin_amdgcn_raw_buffer_store_b96(v, rr, (int)(slot * 24u) + 12, kCandTile * 4, 0);
+          __builtin_amdgcn_raw_buffer_store_b96(u, rr, (int)(slot * 24u), slots * 4, 0);
+          __builtin_amdgcn_raw_buffer_store_b96(v, rr, (int)(slot * 24u) + 12, slots * 4, 0);
         }
       }
     }

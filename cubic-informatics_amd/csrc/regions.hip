@@ -563,7 +563,7 @@ __global__ __launch_bounds__(NT * G) void k_accum_cand(const float* __restrict__
         y = ty0 + (v / kHessTX) % kHessTY;
         z = tz0 + v / (kHessTX * kHessTY);
         const uint32_t idx = z * WH + y * W + x;
-        rec_elements(t, i, hv);
+        rec_elements(t + kCandTile, i, hv);
         const uint32_t root = rl[i];
         r = rid[root];
         // the labeling marks every region that reaches beyond one work-group's tiles

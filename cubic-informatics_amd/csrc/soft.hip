@@ -63,18 +63,21 @@ __global__ __launch_bounds__(NT) void k_soft_loss(const float* __restrict__ cand
                                                   const uint32_t* __restrict__ cand_cnt,
                                                   const uint8_t* __restrict__ target,
                                                   unsigned ntiles, unsigned nbx, unsigned nby,
-                                                  int W, int H, double inv_tau, double* sums) {
+                                                  int W, int H, int D, double inv_tau,
+                                                  double* sums) {
   double ls = 0.0, cnt = 0.0;
   for (unsigned tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
     const uint32_t n = cand_cnt[tile];
-    const float* rec = cand + (size_t)tile * kCandTile * 7;
     const TileOf T = tile_of(tile, nbx, nby);
+    const RecBlock b = rec_block(T.x0, T.y0, T.z0, W, H, D);
+    const float* rec = cand + b.first * 7;
+    const float* el = rec + b.slots;
     for (uint32_t i = threadIdx.x; i < n; i += NT) {
       const uint32_t v = __float_as_uint(rec[i]);
       const size_t at = ((size_t)(T.z0 + (int)(v / (kHessTX * kHessTY))) * H +
                          (T.y0 + (int)(v / kHessTX % kHessTY))) * W + T.x0 + (int)(v % kHessTX);
       float e[6];
-      rec_elements(rec, i, e);
+      rec_elements(el, i, e);
       const double u = -det3(e[0], e[1], e[2], e[3], e[4], e[5]) * inv_tau;
       ls += softplus(u) - (target[at] ? u : 0.0);
       cnt += 1.0;
@@ -89,19 +92,21 @@ __global__ __launch_bounds__(NT) void k_soft_grad_h(float* __restrict__ cand,
                                                     const uint32_t* __restrict__ cand_cnt,
                                                     const uint8_t* __restrict__ target,
                                                     unsigned ntiles, unsigned nbx, unsigned nby,
-                                                    int W, int H, double inv_tau,
+                                                    int W, int H, int D, double inv_tau,
                                                     double inv_count, double* sums) {
   double gt = 0.0;
   for (unsigned tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
     const uint32_t n = cand_cnt[tile];
-    float* rec = cand + (size_t)tile * kCandTile * 7;
     const TileOf T = tile_of(tile, nbx, nby);
+    const RecBlock b = rec_block(T.x0, T.y0, T.z0, W, H, D);
+    float* rec = cand + b.first * 7;
+    float* el = rec + b.slots;
     for (uint32_t i = threadIdx.x; i < n; i += NT) {
       const uint32_t v = __float_as_uint(rec[i]);
       const size_t at = ((size_t)(T.z0 + (int)(v / (kHessTX * kHessTY))) * H +
                          (T.y0 + (int)(v / kHessTX % kHessTY))) * W + T.x0 + (int)(v % kHessTX);
       float h[6];
-      rec_elements(rec, i, h);
+      rec_elements(el, i, h);
       const double xx = h[0], xy = h[1], xz = h[2], yy = h[3], yz = h[4], zz = h[5];
       const double d = det3(xx, xy, xz, yy, yz, zz);
       const double u = -d * inv_tau;
@@ -109,10 +114,10 @@ __global__ __launch_bounds__(NT) void k_soft_grad_h(float* __restrict__ cand,
       const double gu = (p - (target[at] ? 1.0 : 0.0)) * inv_count;  // dL/du
       gt += gu * d * inv_tau * inv_tau;                               // du/dtau = det / tau^2
       const double gd = -gu * inv_tau;                                // dL/ddet
-      rec_store(rec, i, 0, {(float)(gd * 2.0 * (xz * yz - zz * xy)), (float)(gd * (xx * zz - xz * xz)),
-                            (float)(gd * 2.0 * (xy * xz - xx * yz))});
-      rec_store(rec, i, 1, {(float)(gd * (yy * zz - yz * yz)),
-                            (float)(gd * 2.0 * (xy * yz - yy * xz)), (float)(gd * (xx * yy - xy * xy))});
+      rec_store(el, i, 0, {(float)(gd * 2.0 * (xz * yz - zz * xy)), (float)(gd * (xx * zz - xz * xz)),
+                           (float)(gd * 2.0 * (xy * xz - xx * yz))});
+      rec_store(el, i, 1, {(float)(gd * (yy * zz - yz * yz)),
+                           (float)(gd * 2.0 * (xy * yz - yy * xz)), (float)(gd * (xx * yy - xy * xy))});
     }
   }
   double a[1] = {gt};
@@ -151,9 +156,8 @@ __global__ __launch_bounds__(NT, 4) void k_hessian_adjoint(const float* __restri
                                                            const TileRow* __restrict__ rows,
                                                            const float* __restrict__ dog,
                                                            float* __restrict__ out, int nsx,
-                                                           int nsy, int nbx, int nby, int len,
-                                                           int W, int H, int D, double* dot) {
-  constexpr uint32_t kTileWords = (uint32_t)kCandTile * 7u;
+                                                           int nsy, int nbx, int len, int W, int H,
+                                                           int D, double* dot) {
   const int lane = (int)(threadIdx.x & 63);
   const int strip = __builtin_amdgcn_readfirstlane(
       (int)blockIdx.x * (NT / 64) + (int)(threadIdx.x >> 6));  // x fastest, then y, then z
@@ -169,15 +173,23 @@ __global__ __launch_bounds__(NT, 4) void k_hessian_adjoint(const float* __restri
     // lane j < AI looks up row y0 - 2 + j, of the left tile, lane AI + j of the right one
     const int lt = lane >= AI ? tl + 1 : tl, ly = y0 - 2 + (lane >= AI ? lane - AI : lane);
     const bool look = lane < 2 * AI && lt >= 0 && lt < nbx && ly >= 0 && ly < H;
-    const i64 rowbase = ((i64)(look ? ly / kHessTY : 0) * nbx + (look ? lt : 0)) *
-                            (kHessTY * kHessTZ) + (look ? ly % kHessTY : 0);
+    const i64 rowbase = look ? (i64)ly * nbx + lt : 0;
     auto find = [&](int z) -> TileRow {
       TileRow r = {0ull, 0ull};
-      if (look && z >= 0 && z < D)
-        r = rows[rowbase + (i64)(z / kHessTZ) * nby * nbx * (kHessTY * kHessTZ) +
-                 z % kHessTZ * kHessTY];
+      if (look && z >= 0 && z < D) r = rows[rowbase + (i64)z * H * nbx];
       return r;
     };
+    // bytes from the left tile's block to the elements of the lane's tile, per slice of theirs
+    const int exl = min(kHessTX, W - tl * kHessTX), exr = min(kHessTX, W - (tl + 1) * kHessTX);
+    const uint32_t head =
+        look ? (uint32_t)((lane < AI ? exl * 4 : exl * 28 + exr * 4) *
+                          min(kHessTY, H - ly / kHessTY * kHessTY)) : 0u;
+    // the rows lie in two tile rows at most, the second from row yt on; where the left block of
+    // each starts in its layer of tiles, per slice of theirs
+    const int yu = max(y0 - 2, 0) / kHessTY * kHessTY, yt = yu + kHessTY;
+    const i64 upper = (i64)yu * W + (i64)min(kHessTY, H - yu) * (tl * kHessTX),
+              lower = (i64)yt * W + (i64)min(kHessTY, H - yt) * (tl * kHessTX);
+    static_assert(AI <= kHessTY + 1, "rows y0 - 2 .. y0 + AR + 1 in two tile rows");
     auto half = [](float hi, float lo) { return (hi - lo) * 0.5f; };
     // [z & 1]: the values of two slices ago until this one's replace them
     float xz[2][AR] = {}, yz[2][AR + 2] = {}, zz[2][AR] = {}, pz[2][AR] = {};
@@ -193,30 +205,31 @@ __global__ __launch_bounds__(NT, 4) void k_hessian_adjoint(const float* __restri
       float gxx[AR] = {}, gxy[AR + 2] = {}, gyy[AI] = {}, nxz[AR] = {}, nyz[AR + 2] = {}, nzz[AR] = {};
       // bits of the lanes' columns and, per side, the slot of the first record among them
       const unsigned long long own = lane < AI ? cur.bits >> sh : sh ? cur.bits << split : 0ull;
-      const uint32_t first = (uint32_t)cur.first +
-          (lane < AI && sh ? (uint32_t)__popcll(cur.bits << split) : 0u);
+      const int zt = max(z, 0) / kHessTZ * kHessTZ, ez = min(kHessTZ, D - zt);
+      const uint32_t first = ((uint32_t)cur.first +
+          (lane < AI && sh ? (uint32_t)__popcll(cur.bits << split) : 0u)) * 24u +
+          head * (uint32_t)ez;  // in bytes
       if (__ballot(own != 0ull)) {
         const uint32_t olo = (uint32_t)own, ohi = (uint32_t)(own >> 32);
+        const float* layer = cand + (i64)zt * W * H * 7;
+        const float *ru = layer + upper * ez * 7, *rl = layer + lower * ez * 7;
 #pragma unroll
         for (int j = 0; j < AI; ++j) {
-          const int y = y0 - 2 + j;
-          const int ty = max(y, 0) / kHessTY, tz = max(z, 0) / kHessTZ;
           const unsigned long long mlo = read_lane(olo, j), mhi = read_lane(ohi, j);
           const unsigned long long ml = mhi << 32 | mlo;
           const unsigned long long m = ml | (unsigned long long)read_lane(ohi, AI + j) << 32 |
                                        read_lane(olo, AI + j);
-          const uint32_t fl = read_lane(first, j) * 24u;
-          const uint32_t fr =
-              (read_lane(first, AI + j) - (uint32_t)__popcll(ml)) * 24u + kTileWords * 4u;
+          const uint32_t fl = read_lane(first, j);
+          const uint32_t fr = read_lane(first, AI + j) - (uint32_t)__popcll(ml) * 24u;
           // two tiles' records, never used beyond the last tile's (no bits there)
-          const __amdgpu_buffer_rsrc_t r = buf_rsrc(
-              cand + ((i64)tz * nby * nbx + (i64)ty * nbx + tl) * (i64)kTileWords, kTileWords * 8u);
+          const __amdgpu_buffer_rsrc_t r =
+              buf_rsrc(y0 - 2 + j < yt ? ru : rl, (uint32_t)kCandTile * 7u * 8u);
           const uint32_t rank = __builtin_amdgcn_mbcnt_hi(
               (uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
           const uint32_t slot = rank * 24u + (right ? fr : fl);  // in bytes
           const int off = (int)((m >> lane) & 1ull ? slot : 0xF0000000u);
           const F3 u = __builtin_bit_cast(
-              F3, __builtin_amdgcn_raw_buffer_load_b96(r, off, kCandTile * 4, 0));
+              F3, __builtin_amdgcn_raw_buffer_load_b96(r, off, 0, 0));
           gyy[j] = u[kRecYY];
           if (j >= 1 && j <= AR + 2) {
             gxy[j - 1] = u[kRecXY];
@@ -224,7 +237,7 @@ __global__ __launch_bounds__(NT, 4) void k_hessian_adjoint(const float* __restri
           }
           if (j >= 2 && j <= AR + 1) {
             const F3 v = __builtin_bit_cast(
-                F3, __builtin_amdgcn_raw_buffer_load_b96(r, off + 12, kCandTile * 4, 0));
+                F3, __builtin_amdgcn_raw_buffer_load_b96(r, off + 12, 0, 0));
             gxx[j - 2] = v[kRecXX - 3];
             nxz[j - 2] = v[kRecXZ - 3];
             nzz[j - 2] = v[kRecZZ - 3];
@@ -1440,7 +1453,7 @@ hipError_t launch_soft_loss(const float* cand, const uint32_t* cand_cnt, const u
                  nby = (unsigned)((H + kHessTY - 1) / kHessTY);
   hipLaunchKernelGGL(k_zero_f64, dim3(1), dim3(64), 0, s, sums, 2);
   hipLaunchKernelGGL(k_soft_loss, dim3(grid_tiles(nt)), dim3(NT), 0, s, cand, cand_cnt, target,
-                     (unsigned)nt, nbx, nby, W, H, inv_tau, sums);
+                     (unsigned)nt, nbx, nby, W, H, D, inv_tau, sums);
   return hipGetLastError();
 }
 
@@ -1451,7 +1464,7 @@ hipError_t launch_soft_grad_h(float* cand, const uint32_t* cand_cnt, const uint8
   const unsigned nbx = (unsigned)((W + kHessTX - 1) / kHessTX),
                  nby = (unsigned)((H + kHessTY - 1) / kHessTY);
   hipLaunchKernelGGL(k_soft_grad_h, dim3(grid_tiles(nt)), dim3(NT), 0, s, cand, cand_cnt, target,
-                     (unsigned)nt, nbx, nby, W, H, inv_tau, inv_count, sums);
+                     (unsigned)nt, nbx, nby, W, H, D, inv_tau, inv_count, sums);
   return hipGetLastError();
 }
 
@@ -1463,8 +1476,8 @@ hipError_t launch_hessian_adjoint(const float* cand, const TileRow* rows, const 
   line_segments(D, groups, 1024.0, 1.0, false, 4, &nseg, &len);
   const i64 waves = (i64)nsx * nsy * nseg;
   hipLaunchKernelGGL(k_hessian_adjoint, dim3((unsigned)((waves + NT / 64 - 1) / (NT / 64))),
-                     dim3(NT), 0, s, cand, rows, dog, out, nsx, nsy, (W + kHessTX - 1) / kHessTX,
-                     (H + kHessTY - 1) / kHessTY, len, W, H, D, dot);
+                     dim3(NT), 0, s, cand, rows, dog, out, nsx, nsy, row_pieces(W), len, W, H, D,
+                     dot);
   return hipGetLastError();
 }
 

@@ -283,7 +283,9 @@ int hdog_stage_times(hdog_ctx* ctx, double* ms, const char** names, int max_entr
  *   H   = Hessian of dog by the detector's central differences, M = its candidate mask
  *   loss = mean over M of BCE(sigmoid(-det(H) / tau), target)   (target: uint8 0/1)
  * hdog_soft_forward writes the DoG (checkpoint for the backward pass) and M, and
- * returns the loss and |M|; it synchronizes `stream`.  hdog_soft_backward recomputes H
+ * returns the loss and |M|; it synchronizes `stream`.  The context keeps 36 bytes of scratch
+ * per voxel for it, whatever the volume's shape, and for the backward pass 4 more per voxel and
+ * 16 per 64 columns of a row.  hdog_soft_backward recomputes H
  * from the DoG, holds M fixed and returns grad_out * d loss / d (v, sigma1, sigma2, tau)
  * through hand-written adjoints; it synchronizes `stream`. */
 int hdog_soft_forward(hdog_ctx* ctx, void* stream, const float* d_v, const uint8_t* d_target,

@@ -497,3 +497,61 @@ def test_soft_sigma_gradients_by_the_row_walker(hd):
     assert float((got - want).abs().max()) <= 2e-3 * float(want.abs().max())
     err = (vd.grad.cpu().double() - v64.grad).abs().max()
     assert float(err) <= 2e-3 * float(v64.grad.abs().max())
+
+
+# records of the differentiable form, a slot per voxel: planes, rows, few columns, tiles cut
+# along every axis (whose upper and lower neighbours' blocks then differ in size), and enough
+# work-groups for four rows per wave.  FP32 volumes of unit size and chains of some fifty
+# roundings (6e-8 each) on either side of a product of three elements: 1e-4 of the largest
+# gradient
+@pytest.mark.parametrize("shape", [(1, 200, 500), (2, 200, 500), (3, 2, 700), (35, 61, 3),
+                                   (18, 43, 131), (3, 1030, 1100)])
+def test_soft_gradient_by_blocks_of_any_shape(hd, shape):
+    import types
+
+    import soft_reference as ref
+    import torch
+    from hdog import soft
+    s1, s2, tau = [1.6, 2.0, 2.0], [2.56, 3.2, 3.2], 0.05
+    rad1, rad2 = soft.radii(s1), soft.radii(s2)
+    g = torch.Generator().manual_seed(shape[2])
+    v = torch.randn(shape, generator=g)
+    t = (torch.rand(shape, generator=g) < 0.1).to(torch.uint8)
+    m = (torch.rand(shape, generator=g) < 0.2).to(torch.uint8)
+    vd, td = v.to(hd.device), t.to(hd.device)
+    dog = soft.run_forward(hd, vd, td, s1, s2, tau, rad1, rad2)[2]
+    ctx = types.SimpleNamespace(saved_tensors=(vd, dog, m.to(hd.device), td), hd=hd, s1=s1[::-1],
+                                s2=s2[::-1], r1=list(rad1)[::-1], r2=list(rad2)[::-1], gamma=1.0,
+                                tau=tau, count=int(m.sum()), dev_sigma=torch.device("cpu"))
+    gv, _, _, gtau = soft._SoftFn.backward(ctx, 1.0)[:4]
+    v64 = v.double().requires_grad_()
+    t64 = torch.tensor(tau, dtype=torch.float64, requires_grad=True)
+    ref.forward(v64, torch.tensor(s1, dtype=torch.float64), torch.tensor(s2, dtype=torch.float64),
+                t64, t, rad1, rad2, mask=m.bool())[0].backward()
+    err = float((gv.cpu().double() - v64.grad).abs().max())
+    most = float(v64.grad.abs().max())  # 0 for a plane, whose differences along z are
+    print(shape, "error", err, "largest gradient", most, flush=True)
+    assert err <= 1e-4 * most
+    assert abs(float(gtau) - float(t64.grad)) <= 1e-4 * abs(float(t64.grad)) + 1e-6
+
+
+def test_soft_mask_and_loss_by_blocks_of_any_shape(hd):
+    # the forward pass: the mask is the Hessian stage's of the same DoG volume, the count its
+    # number of voxels, and the loss the FP64 one of its elements
+    import torch
+    from hdog import soft
+    s1, s2, tau = [1.6, 2.0, 2.0], [2.56, 3.2, 3.2], 1e-3
+    for shape in [(2, 200, 500), (3, 2, 700), (35, 61, 3), (18, 43, 131), (3, 1030, 1100)]:
+        g = torch.Generator().manual_seed(shape[1])
+        v = torch.randn(shape, generator=g).to(hd.device)
+        t = (torch.rand(shape, generator=g) < 0.1).to(torch.uint8).to(hd.device)
+        loss, count, dog, mask = soft.run_forward(hd, v, t, s1, s2, tau, soft.radii(s1),
+                                                  soft.radii(s2))
+        hess, pd = hd.HessianPositiveDefiniteWithElement(dog)
+        assert torch.equal(mask.view(torch.uint8), pd.view(torch.uint8)), shape
+        on = pd.view(torch.uint8).bool()
+        assert count == int(on.sum()) > 0
+        xx, xy, xz, yy, yz, zz = (hess[k][on].double() for k in range(6))
+        u = -(xx * yy * zz + 2 * xy * yz * xz - xx * yz * yz - yy * xz * xz - zz * xy * xy) / tau
+        want = float((torch.nn.functional.softplus(u) - t[on].bool() * u).sum() / count)
+        assert abs(float(loss) - want) <= 1e-9 * abs(want), shape

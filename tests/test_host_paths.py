@@ -109,3 +109,27 @@ def no_list_yet(rt, C, h):
 
 def test_download_without_a_list_is_empty(runtime):
     session(runtime, "no_list_yet")
+
+
+# ---- scratch of the differentiable form -------------------------------------------------
+def soft_scratch(rt, C, h, *shape):
+    D, H, W = map(int, shape)
+    n = D * H * W
+    d3, i3 = ctypes.c_double * 3, ctypes.c_int * 3
+    s1, s2, r1, r2 = d3(2.0, 2.0, 1.6), d3(3.2, 3.2, 2.56), i3(8, 8, 6), i3(13, 13, 10)
+    loss, count, tau = ctypes.c_double(), ctypes.c_int64(), ctypes.c_double()
+    fixed = 1 << 20  # weights, sums, the library's other allocations of a size of their own
+    # 40 and 49 bytes per voxel hold the passes' pair volumes and the Hessian as dense volumes
+    assert C.hdog_soft_forward(h, None, 4096, 8192, W, H, D, s1, s2, r1, r2, 1.0, 1e-3, 12288,
+                               16384, ctypes.byref(loss), ctypes.byref(count)) == C.HDOG_OK
+    assert rt.host_device_peak() <= 40 * n + fixed, rt.host_device_peak() / n
+    assert C.hdog_soft_backward(h, None, 4096, 12288, 16384, 8192, W, H, D, s1, s2, r1, r2, 1.0,
+                                1e-3, 10, 1.0, 20480, d3(), d3(), ctypes.byref(tau)) == C.HDOG_OK
+    assert rt.host_device_peak() <= 49 * n + fixed, rt.host_device_peak() / n
+
+
+# a single plane, tiles cut along every axis, a few columns or rows, whole tiles
+@pytest.mark.parametrize("shape", [(1, 30000, 30000), (17, 4097, 4097), (3001, 1001, 2),
+                                   (2000, 1, 3000), (128, 512, 512)])
+def test_soft_scratch_goes_with_the_volume(runtime, shape):
+    session(runtime, "soft_scratch", *shape)
