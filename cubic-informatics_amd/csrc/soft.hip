@@ -1306,14 +1306,14 @@ __global__ __launch_bounds__(NT) void k_soft_route(const float2* __restrict__ g,
 }  // namespace
 
 // norm, and for the backward pass ed (E, D pairs) and arg (argmin N, then argmax N);
-// scratch: 8 N words (radii up to kArgRadius: 5 N)
+// scratch: 8 N words (radii up to kArgRadius: 5 N, one more for an odd N)
 hipError_t launch_soft_normalize(const float* v, float* norm, float2* ed, uint32_t* arg,
                                  void* scratch, float min_int, int W, int H, int D, int rxy,
                                  int rz, hipStream_t s) {
   const i64 N = (i64)W * H * D, WH = (i64)W * H;
   if (rxy <= kArgRadius && rz <= kArgRadius) {
     uint32_t* pk = (uint32_t*)scratch;       // keys and taps, 3 N words
-    float2* pair = (float2*)(pk + 3 * N);    // 2 N words
+    float2* pair = (float2*)(pk + (3 * N + 1) / 2 * 2);  // 2 N words, on whole pairs
     float2* exy = (float2*)scratch;          // in the place of the keys
     const XyRun x = xy_run(W, H, D, rxy);
     const ZColumns c = z_columns(W, H);

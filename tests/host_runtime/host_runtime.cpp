@@ -15,7 +15,7 @@ struct Launch {
   std::string name;
   dim3 grid, block;
   size_t lds;
-  std::vector<unsigned char> arg0;
+  std::vector<unsigned char> args;
 };
 std::map<const void*, std::string>& names() {
   static std::map<const void*, std::string> m;
@@ -56,8 +56,13 @@ size_t host_device_peak() { return device_peak; }
 int host_launches() { return (int)launches.size(); }
 const char* host_launch_name(int i) { return launches[i].name.c_str(); }
 unsigned host_launch_blocks(int i) { return launches[i].grid.x; }
-// the first argument of launch i (bytes of it as far as they were kept)
-const void* host_launch_arg0(int i) { return launches[i].arg0.data(); }
+// what was kept of the arguments of launch i
+const void* host_launch_args(int i) { return launches[i].args.data(); }
+// where the device allocation that holds p ends (0: none does)
+uintptr_t host_allocation_end(uintptr_t p) {
+  const auto* a = within(device, p);
+  return a ? a->first + a->second : 0;
+}
 
 // ---- the runtime
 void** __hipRegisterFatBinary(const void*) { return (void**)&handle; }
@@ -85,8 +90,14 @@ hipError_t hipLaunchKernel(const void* f, dim3 g, dim3 b, void** args, size_t ld
   // k_copy_list(CopyList): 18 sources, 18 destinations, 18 sizes, their number
   if (l.name.find("k_copy_list") != std::string::npos) {
     const unsigned char* a = (const unsigned char*)args[0];
-    l.arg0.assign(a, a + 3 * 18 * 8 + 4);
+    l.args.assign(a, a + 3 * 18 * 8 + 4);
   }
+  // k_soft_arg_z(keys, keys, taps, pairs, ...), k_soft_box_xy(pairs, ...): the pairs
+  for (const auto& k : {std::make_pair("k_soft_arg_z", 3), std::make_pair("k_soft_box_xy", 0)})
+    if (l.name.find(k.first) != std::string::npos) {
+      const unsigned char* a = (const unsigned char*)args[k.second];
+      l.args.assign(a, a + 8);
+    }
   // k_assign_ids(..., d_R, h_R)
   if (l.name.find("k_assign_ids") != std::string::npos)
     if (uint32_t* h = *(uint32_t**)args[10]) *h = regions;

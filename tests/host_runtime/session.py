@@ -17,7 +17,9 @@ def load(runtime):
     rt = ctypes.CDLL(runtime, ctypes.RTLD_GLOBAL)
     rt.host_device_peak.restype = ctypes.c_size_t
     rt.host_launch_name.restype = ctypes.c_char_p
-    rt.host_launch_arg0.restype = ctypes.c_void_p
+    rt.host_launch_args.restype = ctypes.c_void_p
+    rt.host_allocation_end.argtypes = [ctypes.c_size_t]
+    rt.host_allocation_end.restype = ctypes.c_size_t
     rt.host_fail_allocation.argtypes = [ctypes.c_long]
     sys.modules["torch"] = types.ModuleType("torch")
     spec = importlib.util.spec_from_file_location("hdog_capi", os.path.join(PKG, "_capi.py"))

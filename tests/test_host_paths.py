@@ -53,7 +53,7 @@ def region_arrays(C, h, cap, locked):
 
 def copies(rt):
     """The copy lists launched since the last clear."""
-    return [CopyList.from_address(rt.host_launch_arg0(i)) for i in range(rt.host_launches())
+    return [CopyList.from_address(rt.host_launch_args(i)) for i in range(rt.host_launches())
             if b"k_copy_list" in rt.host_launch_name(i)]
 
 
@@ -133,3 +133,21 @@ def soft_scratch(rt, C, h, *shape):
                                    (2000, 1, 3000), (128, 512, 512)])
 def test_soft_scratch_goes_with_the_volume(runtime, shape):
     session(runtime, "soft_scratch", *shape)
+
+
+# the (min, max) pairs of the normalization lie behind three words per voxel
+def soft_pairs(rt, C, h, *shape):
+    D, H, W = map(int, shape)
+    rt.host_clear()
+    assert C.hdog_soft_normalize_forward(h, None, 4096, 8192, 12288, 16384, 0.0, W, H, D, 10,
+                                         10) == C.HDOG_OK
+    at = [ctypes.c_uint64.from_address(rt.host_launch_args(i)).value
+          for i in range(rt.host_launches())
+          if b"k_soft_arg_z" in rt.host_launch_name(i) or b"k_soft_box_xy" in rt.host_launch_name(i)]
+    assert len(at) == 2 and at[0] == at[1]
+    assert at[0] % 8 == 0 and at[0] + 8 * D * H * W <= rt.host_allocation_end(at[0])
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1), (3, 5, 7), (4, 5, 7), (65, 127, 33)])
+def test_soft_pairs_are_aligned_and_fit(runtime, shape):
+    session(runtime, "soft_pairs", *shape)
