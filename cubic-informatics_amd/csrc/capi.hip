@@ -82,7 +82,7 @@ struct hdog_ctx {
   hipEvent_t run_done[2] = {nullptr, nullptr};  // last run reading the slot complete
   int up_shape[2][3] = {{0, 0, 0}, {0, 0, 0}};  // (W, H, D) of each slot's upload
   int up_valid[2] = {0, 0};                      // slices before the zero fill
-  // launch shapes chosen by hdog_autotune per stack shape and storage form
+  // launch shapes chosen by hdog_autotune per stack shape and storage form (walk_segments)
   struct Tuned {
     int W, H, D, precision, norm_segments, gauss_segments;
   };
@@ -1083,16 +1083,25 @@ int hdog_autotune(hdog_ctx* ctx, void* stream, const hdog_params* p, const uint1
   const int W = p->width, H = p->height, D = p->depth, prec = p->precision;
   int ns = 0, gs = 0;
   bool found = false;
-  if (cache_path && *cache_path) {  // lines "width height depth precision norm gauss"
+  // lines "width height depth precision norm gauss"
+  if (cache_path && *cache_path) {
     if (FILE* f = std::fopen(cache_path, "r")) {
-      int w, h, d, pr, a, b;
-      while (std::fscanf(f, "%d %d %d %d %d %d", &w, &h, &d, &pr, &a, &b) == 6)
-        if (w == W && h == H && d == D && pr == prec && a >= 1 && a <= kMaxSegments && b >= 1 &&
-            b <= kMaxSegments) {
-          ns = a;
-          gs = b;
-          found = true;
-        }
+      char line[256];
+      while (std::fgets(line, sizeof line, f)) {
+        int w, h, d, pr, a, b;
+        if (std::sscanf(line, "%d %d %d %d %d %d", &w, &h, &d, &pr, &a, &b) != 6) continue;
+        if (w != W || h != H || d != D || pr != prec || a < 1 || a > kMaxSegments || b < 1 ||
+            b > kMaxSegments)
+          continue;
+        // separated by tabs: choices of this tuner.  By blanks: of one that counted segments,
+        // for walkers that have changed since; better timed again, where there is a stack to
+        // time, else taken as what they say
+        const bool counts = !std::strchr(line, '\t');
+        if (counts && (d_img || (found && ns > 0))) continue;
+        ns = counts ? -a : a;
+        gs = counts ? -b : b;
+        found = true;
+      }
       std::fclose(f);
     }
   }
@@ -1114,7 +1123,7 @@ int hdog_autotune(hdog_ctx* ctx, void* stream, const hdog_params* p, const uint1
     if (rc) return rc;
     if (cache_path && *cache_path) {
       if (FILE* f = std::fopen(cache_path, "a")) {
-        std::fprintf(f, "%d %d %d %d %d %d\n", W, H, D, prec, ns, gs);
+        std::fprintf(f, "%d\t%d\t%d\t%d\t%d\t%d\n", W, H, D, prec, ns, gs);
         std::fclose(f);
       } else {
         return fail(ctx, HDOG_ERR_ARG, "cannot append to the tuning cache %s", cache_path);
@@ -1129,8 +1138,8 @@ int hdog_autotune(hdog_ctx* ctx, void* stream, const hdog_params* p, const uint1
       have = true;
     }
   if (!have) ctx->tuned.push_back({W, H, D, prec, ns, gs});
-  if (norm_segments) *norm_segments = ns;
-  if (gauss_segments) *gauss_segments = gs;
+  if (norm_segments) *norm_segments = std::abs(ns);
+  if (gauss_segments) *gauss_segments = std::abs(gs);
   return HDOG_OK;
 }
 

@@ -258,7 +258,7 @@ inline void mark(const char* name, hipStream_t s) {
 // segments, 543 with eight, 528 with sixteen; 128 x 256 x 256: 165 us with one, 54 with seven,
 // 60 with thirteen; gauss_xy there 102, 46 and 51 us with one, five and ten; on a full tile
 // 2 to 4 segments are within 2 %.  A tuned launch shape `want` (1 .. 4) takes want / 2 of the
-// built-in count.
+// built-in count; a negative one is a number of segments.
 struct WalkShape {
   i64 strips;        // waves per segment, all planes
   int period, halo;  // segment length: a multiple of period; rows of context
@@ -282,8 +282,8 @@ inline void walk_segments(int H, const WalkShape& w, int* nys, int* rows, int wa
       best = n;
     }
   }
-  const int n = want > 0 ? std::max(1, std::min(most, (best * want + 1) / 2)) : best;
-  shape(n, nys, rows);
+  const int n = want > 0 ? (best * want + 1) / 2 : want < 0 ? -want : best;
+  shape(std::max(1, std::min(most, n)), nys, rows);
 }
 
 // Segments of a line of L positions, each reading `halo` positions more than it writes.

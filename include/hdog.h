@@ -223,9 +223,11 @@ int hdog_run_device(hdog_ctx* ctx, void* stream, const hdog_params* p, const uin
  * src/3D/NormalizeFilter.cu:13-47, src/3D/DoG3DFilter.cu:29-58): the number of row
  * segments each of the normalization's and the DoG's row walkers splits a plane into, in
  * halves of the built-in count, chosen by timing every candidate (1..4) on d_img with HIP
- * events (median of 3).  With
- * cache_path, a line "width height depth precision norm gauss" for the shape is read from
- * that file when present (d_img may then be NULL), and a new measurement is appended.  The
+ * events (median of 3).  With cache_path, a line "width height depth precision norm gauss"
+ * (separated by tabs) for the shape is read from that file when present (d_img may then be
+ * NULL), and a new measurement is appended.  In a line separated by blanks, as an earlier
+ * tuner wrote them, the last two numbers are counts of segments: it is used only when there
+ * is no d_img to time.  The
  * choice is kept in the context and used by hdog_run_device and hdog_batch_plan for stacks
  * of that shape; it changes launch shapes only, never results. */
 int hdog_autotune(hdog_ctx* ctx, void* stream, const hdog_params* p, const uint16_t* d_img,

@@ -151,3 +151,53 @@ def soft_pairs(rt, C, h, *shape):
 @pytest.mark.parametrize("shape", [(1, 1, 1), (3, 5, 7), (4, 5, 7), (65, 127, 33)])
 def test_soft_pairs_are_aligned_and_fit(runtime, shape):
     session(runtime, "soft_pairs", *shape)
+
+
+# ---- the tuner's file -------------------------------------------------------------------
+def tuning_file(rt, C, h, path):
+    D, H, W = 24, 700, 260
+    p = C.Params(width=W, height=H, depth=D, radius_xy=10, radius_z=10, min_intensity=0.0,
+                 sigma_xy1=2.0, sigma_z1=2.0, sigma_xy2=3.2, sigma_z2=3.2, truncate=4.0, gamma=1.0)
+    ns, gs = ctypes.c_int(), ctypes.c_int()
+
+    def tune(img):
+        rt.host_clear()
+        rc = C.hdog_autotune(h, None, ctypes.byref(p), img, path.encode(), ctypes.byref(ns),
+                             ctypes.byref(gs))
+        assert rc == C.HDOG_OK
+        return ns.value, gs.value, rt.host_launches()
+
+    def segments():  # of the normalization's walker over strips of 64 columns
+        rt.host_clear()
+        n = ctypes.c_int64()
+        assert C.hdog_run_device(h, None, ctypes.byref(p), 4096, None, None, None, None, None,
+                                 ctypes.byref(n)) == C.HDOG_OK
+        blocks = [rt.host_launch_blocks(i) for i in range(rt.host_launches())
+                  if b"k_norm_xy_run" in rt.host_launch_name(i)]
+        return blocks[0] // (D * ((W + 63) // 64))
+
+    def write(*lines):
+        with open(path, "w") as f:
+            f.writelines(lines)
+
+    builtin = segments()
+    assert builtin > 4
+    old, key = "260 700 24 0 %d %d\n", "260\t700\t24\t0\t"
+    # counts of segments: as they stand, if there is no stack to time ...
+    for count in (1, 2, 3, 4):
+        write(old % (count, count))
+        assert tune(None) == (count, count, 0) and segments() == count
+    # ... else timed again, and the new line goes before the old one from then on
+    write(old % (1, 4), "261 700 24 0 3 3\n")
+    ns1, gs1, launches = tune(4096)
+    assert launches > 0 and segments() == builtin  # (all candidates take the same time here)
+    assert open(path).read().endswith(key + f"{ns1}\t{gs1}\n")
+    assert tune(None) == (ns1, gs1, 0) and segments() == builtin
+    # halves of the built-in count, whatever lines of the other kind stand around them
+    write(old % (1, 1), key + "4\t1\n", old % (3, 3))
+    assert tune(None) == (4, 1, 0) and segments() > builtin
+    assert tune(4096) == (4, 1, 0)
+
+
+def test_tuning_files_keep_their_meaning(runtime, tmp_path):
+    session(runtime, "tuning_file", tmp_path / "tune.txt")
