@@ -263,10 +263,11 @@ __global__ __launch_bounds__(NTR) void k_cand_local(const float* __restrict__ ca
   // this work-group's share of the root and region-spanning bitmaps, cleared for kernel C
   // (a tile's voxels have RTV / 64 words; the tiles' voxels cover the volume's)
   if (roots) {
-    static_assert(NTR >= 2 * (RTV / 64), "one word per thread, both bitmaps");
-    const i64 w = (i64)tile * (RTV / 64) + (threadIdx.x & (RTV / 64 - 1));
-    if (threadIdx.x < 2 * (RTV / 64) && w < root_words)
-      (threadIdx.x < RTV / 64 ? roots : multi)[w] = 0ull;
+    constexpr int WORDS = RTV / 64;
+    for (int i = (int)threadIdx.x; i < 2 * WORDS; i += NTR) {
+      const i64 w = (i64)tile * WORDS + i % WORDS;
+      if (w < root_words) (i < WORDS ? roots : multi)[w] = 0ull;
+    }
   }
   if (tile == 0)  // and the region numbering's chunk counts
     for (int i = (int)threadIdx.x; i < chunks; i += NTR) chunk_counts[i] = 0u;

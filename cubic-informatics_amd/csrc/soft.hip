@@ -184,12 +184,16 @@ __global__ __launch_bounds__(NT, 4) void k_hessian_adjoint(const float* __restri
     const uint32_t head =
         look ? (uint32_t)((lane < AI ? exl * 4 : exl * 28 + exr * 4) *
                           min(kHessTY, H - ly / kHessTY * kHessTY)) : 0u;
-    // the rows lie in two tile rows at most, the second from row yt on; where the left block of
+    // the rows lie in KT tile rows at most, the first from row yu on; where the left block of
     // each starts in its layer of tiles, per slice of theirs
-    const int yu = max(y0 - 2, 0) / kHessTY * kHessTY, yt = yu + kHessTY;
-    const i64 upper = (i64)yu * W + (i64)min(kHessTY, H - yu) * (tl * kHessTX),
-              lower = (i64)yt * W + (i64)min(kHessTY, H - yt) * (tl * kHessTX);
-    static_assert(AI <= kHessTY + 1, "rows y0 - 2 .. y0 + AR + 1 in two tile rows");
+    constexpr int KT = (AI + kHessTY - 2) / kHessTY + 1;
+    const int yu = max(y0 - 2, 0) / kHessTY * kHessTY;
+    i64 start[KT];
+#pragma unroll
+    for (int k = 0; k < KT; ++k) {
+      const int yk = yu + k * kHessTY;
+      start[k] = (i64)yk * W + (i64)min(kHessTY, H - yk) * (tl * kHessTX);
+    }
     auto half = [](float hi, float lo) { return (hi - lo) * 0.5f; };
     // [z & 1]: the values of two slices ago until this one's replace them
     float xz[2][AR] = {}, yz[2][AR + 2] = {}, zz[2][AR] = {}, pz[2][AR] = {};
@@ -212,7 +216,9 @@ __global__ __launch_bounds__(NT, 4) void k_hessian_adjoint(const float* __restri
       if (__ballot(own != 0ull)) {
         const uint32_t olo = (uint32_t)own, ohi = (uint32_t)(own >> 32);
         const float* layer = cand + (i64)zt * W * H * 7;
-        const float *ru = layer + upper * ez * 7, *rl = layer + lower * ez * 7;
+        const float* block[KT];
+#pragma unroll
+        for (int k = 0; k < KT; ++k) block[k] = layer + start[k] * ez * 7;
 #pragma unroll
         for (int j = 0; j < AI; ++j) {
           const unsigned long long mlo = read_lane(olo, j), mhi = read_lane(ohi, j);
@@ -222,8 +228,11 @@ __global__ __launch_bounds__(NT, 4) void k_hessian_adjoint(const float* __restri
           const uint32_t fl = read_lane(first, j);
           const uint32_t fr = read_lane(first, AI + j) - (uint32_t)__popcll(ml) * 24u;
           // two tiles' records, never used beyond the last tile's (no bits there)
-          const __amdgpu_buffer_rsrc_t r =
-              buf_rsrc(y0 - 2 + j < yt ? ru : rl, (uint32_t)kCandTile * 7u * 8u);
+          const float* at_block = block[0];
+#pragma unroll
+          for (int k = 1; k < KT; ++k)
+            if (y0 - 2 + j >= yu + k * kHessTY) at_block = block[k];  // uniform
+          const __amdgpu_buffer_rsrc_t r = buf_rsrc(at_block, (uint32_t)kCandTile * 7u * 8u);
           const uint32_t rank = __builtin_amdgcn_mbcnt_hi(
               (uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
           const uint32_t slot = rank * 24u + (right ? fr : fl);  // in bytes
