@@ -505,7 +505,9 @@ static_assert(kAccGY * kAccGZ * kCandTile < (1 << 16) && kHessTX <= 256 &&
                   kAccGY * kHessTY <= 256 && kAccGZ * kHessTZ <= 256,
               "packed table sums: count below 2^16, offsets below 256");
 // S: table slots.  G: groups of four waves; a tile's records are folded by one group, so with
-// G = 4 the tiles of a work-group go side by side.
+// G = 4 four tiles of a work-group go side by side.
+constexpr int kTileGroups = kAccGY * kAccGZ < 4 ? kAccGY * kAccGZ : 4;
+static_assert(NT * kTileGroups <= 1024, "threads of a work-group");
 template <typename TN, bool AVE, int S, int G>
 __global__ __launch_bounds__(NT * G) void k_accum_cand(const float* __restrict__ cand,
                                                    const uint32_t* __restrict__ cand_cnt,
@@ -798,7 +800,7 @@ hipError_t launch_region_accum_cand(const float* cand, const uint32_t* cand_cnt,
                          (uint32_t)W, (uint32_t)((i64)W * H), nbx, nby, nbz);
     };
     if (ngroups <= 1024)
-      launch(std::integral_constant<int, kAccGY * kAccGZ>{});
+      launch(std::integral_constant<int, kTileGroups>{});
     else
       launch(std::integral_constant<int, 1>{});
   };
