@@ -34,6 +34,7 @@ struct Config {
 };
 std::vector<Config> configs;
 int handle;
+hipError_t last_error = hipSuccess;
 
 const std::pair<const uintptr_t, size_t>* within(const std::map<uintptr_t, size_t>& m, uintptr_t p) {
   auto it = m.upper_bound(p);
@@ -86,6 +87,7 @@ hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* lds, hipStream_t*
   return hipSuccess;
 }
 hipError_t hipLaunchKernel(const void* f, dim3 g, dim3 b, void** args, size_t lds, hipStream_t) {
+  if ((size_t)b.x * b.y * b.z > 1024) return last_error = hipErrorInvalidConfiguration;
   Launch l{names()[f], g, b, lds, {}};
   // k_copy_list(CopyList): 18 sources, 18 destinations, 18 sizes, their number
   if (l.name.find("k_copy_list") != std::string::npos) {
@@ -164,7 +166,11 @@ hipError_t hipGetDeviceCount(int* n) {
   return hipSuccess;
 }
 hipError_t hipSetDevice(int) { return hipSuccess; }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() {
+  const hipError_t e = last_error;
+  last_error = hipSuccess;
+  return e;
+}
 const char* hipGetErrorString(hipError_t e) { return e == hipErrorOutOfMemory ? "out of memory" : "error"; }
 hipError_t hipEventCreate(hipEvent_t* e) {
   *e = (hipEvent_t)&handle;

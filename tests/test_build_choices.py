@@ -1,7 +1,6 @@
 """The build-time choices of csrc/hdog_internal.hpp (tile height, the region pass's tile group)
 within the limits that its comments and static_asserts name.  Compiler only, no GPU."""
 import os
-import re
 import shutil
 import subprocess
 
@@ -28,11 +27,3 @@ def compile_with(unit, choices, *args):
 def test_tile_heights_compile(unit, choices):
     r = compile_with(unit, choices, "-fsyntax-only")
     assert r.returncode == 0, r.stderr[-2000:]
-
-
-# 3 x 2 tiles per work-group: no kernel asks for more threads than a work-group may have
-def test_work_groups_of_six_tiles_launch():
-    r = compile_with("regions", ["-DHDOG_ACC_GY=3", "-DHDOG_ACC_GZ=2"], "-O1", "-S", "-o", "-")
-    assert r.returncode == 0, r.stderr[-2000:]
-    threads = [int(n) for n in re.findall(r"\.max_flat_workgroup_size: (\d+)", r.stdout)]
-    assert threads and max(threads) <= 1024, sorted(set(threads))

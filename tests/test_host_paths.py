@@ -20,9 +20,10 @@ def runtime(tmp_path_factory):
     return so
 
 
-def session(runtime, name, *args):
+def session(runtime, name, *args, library=""):
     r = subprocess.run([sys.executable, os.path.join(HERE, "session.py"), runtime, name,
-                        *map(str, args)], capture_output=True, text=True, timeout=120)
+                        *map(str, args)], capture_output=True, text=True, timeout=120,
+                       env=dict(os.environ, HDOG_LIBRARY=library))
     assert r.returncode == 0, r.stdout + r.stderr
 
 
@@ -201,3 +202,31 @@ def tuning_file(rt, C, h, path):
 
 def test_tuning_files_keep_their_meaning(runtime, tmp_path):
     session(runtime, "tuning_file", tmp_path / "tune.txt")
+
+
+# ---- build-time choices -----------------------------------------------------------------
+def region_sums_launch(rt, C, h):
+    # few and many work-groups, in both modes of the intensity feature
+    for D, H, W in ((24, 96, 112), (64, 2160, 2560)):
+        for ave in (0, 1):
+            p = C.Params(width=W, height=H, depth=D, radius_xy=10, radius_z=10, min_intensity=0.0,
+                         sigma_xy1=2.0, sigma_z1=2.0, sigma_xy2=3.2, sigma_z2=3.2, truncate=4.0,
+                         gamma=1.0, is_ave_mode=ave)
+            rt.host_set_regions(100)
+            n = ctypes.c_int64()
+            rc = C.hdog_run_device(h, None, ctypes.byref(p), 4096, None, None, None, None, None,
+                                   ctypes.byref(n))
+            assert rc == C.HDOG_OK, C.hdog_last_error(h)
+
+
+def test_region_sums_of_six_tiles_launch(runtime, tmp_path):
+    # a library with 3 x 2 tiles to a work-group of the region pass: no launch of more threads
+    # than a work-group may have (unoptimized: its kernels never run)
+    if not os.path.exists("/opt/rocm/bin/hipcc"):
+        pytest.skip("no HIP compiler")
+    pkg = os.path.join(os.path.dirname(os.path.dirname(HERE)), "cubic-informatics_amd")
+    lib = str(tmp_path / "libhdog.so")
+    subprocess.run(["make", "-s", f"-j{min(16, os.cpu_count() or 1)}", "-C", pkg, f"BUILD={tmp_path}",
+                    f"LIB={lib}", "EXTRA_HIPFLAGS=-O0 -Xarch_device -O0 -DHDOG_ACC_GY=3", lib],
+                   check=True, capture_output=True, timeout=600)
+    session(runtime, "region_sums_launch", library=lib)
