@@ -1038,7 +1038,8 @@ struct RouteTable {
     uint32_t slot = k * 2654435761u >> 23;
     static_assert(kRouteSlots == 1 << 9, "hash bits");
     for (int p = 0; p < kProbes; ++p, slot = (slot + 1) & (kRouteSlots - 1)) {
-      uint32_t cur = key[slot];
+      // (a key, once set, stays until the flush; other lanes may be setting it)
+      uint32_t cur = __atomic_load_n(&key[slot], __ATOMIC_RELAXED);
       if (cur == kNone) {
         cur = atomicCAS(&key[slot], kNone, k);
         if (cur == kNone) cur = k;
