@@ -555,3 +555,74 @@ def test_soft_mask_and_loss_by_blocks_of_any_shape(hd):
         u = -(xx * yy * zz + 2 * xy * yz * xz - xx * yz * yz - yy * xz * xz - zz * xy * xy) / tau
         want = float((torch.nn.functional.softplus(u) - t[on].bool() * u).sum() / count)
         assert abs(float(loss) - want) <= 1e-9 * abs(want), shape
+
+
+def records_equal_given_labels(hd, img, p, bufs, ave):
+    """The regions of the records-only pass, against those of the materialized volumes' labels
+    (a fold of its own).  Sums: FP64 in another order, rounded once to FP32."""
+    want = hd.RegionalFeatures(bufs["labels"], bufs["hess"], bufs["norm"], img, ave)
+    hd.run_device(img, p)
+    got = hd.download_regions()
+    assert len(want["label"]) > 1000
+    for k in ("label", "count", "isum", "imax", "centroid"):
+        np.testing.assert_array_equal(got[k], want[k], err_msg=k)
+    n = want["count"][:, None].astype(np.float64)
+    big = max(float(bufs["hess"].abs().max()), float(bufs["norm"].abs().max()))
+    for k in ("hsum", "norm"):
+        a, b = (x[k].astype(np.float64).reshape(len(n), -1) for x in (got, want))
+        assert np.all(np.abs(a - b) <= 1.2e-7 * np.abs(b) + 1e-12 * n * big), k
+
+
+# one group of waves for a work-group's tiles (above 1024 work-groups) and four, with either
+# table size
+@pytest.mark.parametrize("shape", [(3, 1040, 1040), (3, 1040, 960)])
+@pytest.mark.parametrize("sigmas", [(0.9, 0.7, 1.5, 1.2), (1.6, 1.25, 2.6, 2.0)])
+@pytest.mark.parametrize("ave", [False, True])
+def test_region_sums_by_work_groups(hd, shape, sigmas, ave):
+    img = hd._dev(noise(shape, 12), __import__("torch").uint16)
+    p = hd.make_params(shape, 3, 3, 0, *sigmas, truncate=3.0, is_ave_mode=ave)
+    bufs = hd.alloc_intermediates(shape)
+    hd.run_device(img, p, bufs)
+    records_equal_given_labels(hd, img, p, bufs, ave)
+
+
+# records of walks over one to four Hessian tiles, two rows per wave and four: all six elements
+@pytest.mark.parametrize("shape", [(70, 40, 70), (33, 640, 700), (49, 1500, 1600)])
+def test_records_walks_give_the_elements(hd, shape):
+    blobs = synth.blob_table(shape, shape[0] * shape[1] * shape[2] // 20000, 11)
+    img = hd.synth_volume(shape, blobs, 11, 200.0, 200.0, 20.0)
+    p = hd.make_params(shape, 10, 10, 0, 1.2, 1.0, 2.0, 1.6, 3.0)
+    bufs = hd.alloc_intermediates(shape)
+    hd.run_device(img, p, bufs)
+    records_equal_given_labels(hd, img, p, bufs, False)
+
+
+# 16-bit storage at radii without kernels of their own: the normalized stack is the FP32 one
+# rounded; the DoG of that stack, formed in FP32, equals the oracle's where it stays FP32, and
+# is at most a unit in the last place from it where it is rounded to 16 bits (the product with
+# the scale may be rounded on the way or not)
+@pytest.mark.parametrize("form,dtype,digits", [("fp16", "float16", 10), ("bf16", "bfloat16", 7),
+                                               ("fp16_dog32", "float16", 0),
+                                               ("bf16_dog32", "bfloat16", 0)])
+@pytest.mark.parametrize("rxy,rz,s", [(8, 4, (2.2, 1.1, 3.6, 1.8)), (3, 2, (0.3, 0.2, 0.6, 0.5)),
+                                      (9, 25, (8.1, 1.3, 9.6, 2.1))])
+def test_16_bit_storage_at_any_radii(hd, form, dtype, digits, rxy, rz, s):
+    import torch
+    dtype = getattr(torch, dtype)
+    for shape in ((34, 41, 70), (9, 75, 193)):
+        img = hd._dev(noise(shape, 5), torch.uint16)
+        norm = hd.Normalize3DFilter(img, 100, rxy, rz)
+        p = hd.make_params(shape, rxy, rz, 100, *s, truncate=4.0, precision=form)
+        bufs = hd.alloc_intermediates(shape, form)
+        hd.run_device(img, p, bufs)
+        assert torch.equal(bufs["norm"], norm.to(dtype))
+        want = torch.from_numpy(oracle.dog3d(bufs["norm"].float().cpu().numpy(), *s, truncate=4.0,
+                                             gamma=1.0)[0])
+        got = bufs["dog"].cpu()
+        if not digits:
+            assert got.dtype == torch.float32 and torch.equal(got, want)
+        else:
+            assert got.dtype == dtype
+            want = want.to(dtype).double()
+            least = 2.0 ** -24 if dtype == torch.float16 else 0.0
+            assert bool(((got.double() - want).abs() <= want.abs() * 2.0 ** -digits + least).all())
