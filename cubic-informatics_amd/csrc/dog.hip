@@ -293,15 +293,15 @@ __global__ __launch_bounds__(256) void k_gauss_line_run(const float2* __restrict
     fetch(s0 - R + GK * g);
     put(GK * g);
   }
-  fetch(s0 + R + GK * wave);
+  if (s0 + GK * wave < s1) fetch(s0 + R + GK * wave);
   __syncthreads();
   const bool out = x0 + l < W;
   double d[2] = {0.0, 0.0};
   for (int c0 = s0; c0 < s1; c0 += STEP) {
-    put(hist + GK * wave);
-    fetch(c0 + STEP + R + GK * wave);
-    __syncthreads();
     const int c = c0 + GK * wave;
+    if (c < s1) put(hist + GK * wave);
+    if (c + STEP < s1) fetch(c + STEP + R);
+    __syncthreads();
     if (c < s1) {
       float a1[GK], a2[GK];
       const float* p = B1 + (GK * wave + R - r1) * 64 + l;

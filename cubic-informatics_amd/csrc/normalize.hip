@@ -863,13 +863,13 @@ __global__ __launch_bounds__(256) void k_minmax_run(const void* __restrict__ src
     fetch(a.s0 - r + OK * g);
     put(OK * g);
   }
-  fetch(a.s0 + r + OK * a.wave);
+  if (a.s0 + OK * a.wave < a.s1) fetch(a.s0 + r + OK * a.wave);
   __syncthreads();
   for (int c0 = a.s0; c0 < a.s1; c0 += STEP) {
-    put(hist + OK * a.wave);
-    fetch(c0 + STEP + r + OK * a.wave);
-    __syncthreads();
     const int c = c0 + OK * a.wave;
+    if (c < a.s1) put(hist + OK * a.wave);
+    if (c + STEP < a.s1) fetch(c + STEP + r);
+    __syncthreads();
     if (c < a.s1) {
       const uint32_t* p = sm_mm + OK * a.wave * 64 + a.l;
       uint32_t o[OK];
@@ -937,7 +937,7 @@ __global__ __launch_bounds__(512) void k_minmax_zy_run(const uint16_t* __restric
 #pragma unroll
     for (int i = 0; i < NQ; ++i) q[i] = slice[(i64)clampi(y0 - ry + i, 0, H - 1) * W + xc];
   };
-  auto ymin = [&](int plane, int ahead) {
+  auto ymin = [&](int plane, int ahead, bool more) {
     uint32_t v[NQ], o[OK];
 #pragma unroll
     for (int i = 0; i < NQ; ++i) v[i] = pack(q[i]);
@@ -947,20 +947,19 @@ __global__ __launch_bounds__(512) void k_minmax_zy_run(const uint16_t* __restric
       if (ry == RM - 2) min8_regs<RM - 2>(v, o);
       if (ry == RM - 3) min8_regs<RM - 3>(v, o);
     }
-    fetch(ahead);
+    if (more) fetch(ahead);
 #pragma unroll
     for (int i = 0; i < OK; ++i) sm_zy[plane * PL + i * 64 + l] = o[i];
   };
   fetch(s0 - rz + wave);
   for (int g = wave; g < hist; g += 8)
-    ymin(g, g + 8 < hist ? s0 - rz + g + 8 : s0 + rz + wave);
-  if (wave >= hist) fetch(s0 + rz + wave);
+    ymin(g, g + 8 < hist ? s0 - rz + g + 8 : s0 + rz + wave, g + 8 < hist || s0 + wave < s1);
   const int y = y0 + wave;
   const bool out = x0 + l < W && y < H;
   const i64 WH = (i64)W * H;
   uint32_t* d = dst + (i64)y * W + x0 + l;
   for (int c = s0; c < s1; c += OK) {
-    ymin(hist + wave, c + OK + rz + wave);
+    if (c + wave < s1) ymin(hist + wave, c + OK + rz + wave, c + OK + wave < s1);
     __syncthreads();
     const uint32_t* p = sm_zy + wave * 64 + l;
     uint32_t o[OK];
@@ -1012,16 +1011,18 @@ __global__ __launch_bounds__(256) void k_box_run(const float2* __restrict__ src,
     fetch(a.s0 - r + OK * g);
     put(OK * g);
   }
-  fetch(a.s0 + r + OK * a.wave);
+  if (a.s0 + OK * a.wave < a.s1) fetch(a.s0 + r + OK * a.wave);
   __syncthreads();
   for (int c0 = a.s0; c0 < a.s1; c0 += STEP) {
     const int c = c0 + OK * a.wave;
-    put(hist + OK * a.wave);
-    if (NORM) {
+    if (c < a.s1) {
+      put(hist + OK * a.wave);
+      if (NORM) {
 #pragma unroll
-      for (int j = 0; j < OK; ++j) iq[j] = img[a.base + (i64)min(c + j, L - 1) * sa + xc];
+        for (int j = 0; j < OK; ++j) iq[j] = img[a.base + (i64)min(c + j, L - 1) * sa + xc];
+      }
     }
-    fetch(c0 + STEP + r + OK * a.wave);
+    if (c + STEP < a.s1) fetch(c + STEP + r);
     __syncthreads();
     if (c < a.s1) {
       float e[OK], d[OK];

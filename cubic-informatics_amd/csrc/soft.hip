@@ -588,13 +588,13 @@ __global__ __launch_bounds__(256) void k_soft_arg_z(const uint32_t* __restrict__
     fetch(a.s0 - r + OK * g);
     put(OK * g);
   }
-  fetch(a.s0 + r + OK * a.wave);
+  if (a.s0 + OK * a.wave < a.s1) fetch(a.s0 + r + OK * a.wave);
   __syncthreads();
   for (int c0 = a.s0; c0 < a.s1; c0 += kStep) {
-    put(hist + OK * a.wave);
-    fetch(c0 + kStep + r + OK * a.wave);
-    __syncthreads();
     const int c = c0 + OK * a.wave;
+    if (c < a.s1) put(hist + OK * a.wave);
+    if (c + kStep < a.s1) fetch(c + kStep + r);
+    __syncthreads();
     if (c < a.s1) {
       const uint32_t* p = Bn + OK * a.wave * 64 + a.l;
       const int plane = (hist + kStep) * 64;
@@ -760,14 +760,16 @@ __global__ __launch_bounds__(256) void k_soft_box_norm(const float2* __restrict_
     fetch(a.s0 - r + OK * g);
     put(OK * g);
   }
-  fetch(a.s0 + r + OK * a.wave);
+  if (a.s0 + OK * a.wave < a.s1) fetch(a.s0 + r + OK * a.wave);
   __syncthreads();
   for (int c0 = a.s0; c0 < a.s1; c0 += kStep) {
     const int c = c0 + OK * a.wave;
-    put(hist + OK * a.wave);
+    if (c < a.s1) {
+      put(hist + OK * a.wave);
 #pragma unroll
-    for (int j = 0; j < OK; ++j) vq[j] = v[a.base + (i64)min(c + j, D - 1) * sa + xc];
-    fetch(c0 + kStep + r + OK * a.wave);
+      for (int j = 0; j < OK; ++j) vq[j] = v[a.base + (i64)min(c + j, D - 1) * sa + xc];
+    }
+    if (c + kStep < a.s1) fetch(c + kStep + r);
     __syncthreads();
     if (c < a.s1) {
       float e[OK], d[OK];
@@ -978,12 +980,12 @@ __global__ __launch_bounds__(256) void k_soft_adj_z(const float* __restrict__ v,
     fetch(a.s0 - r + OK * g);
     put(OK * g, a.s0 - r + OK * g);
   }
-  fetch(a.s0 + r + OK * a.wave);
+  if (a.s0 + OK * a.wave < a.s1) fetch(a.s0 + r + OK * a.wave);
   __syncthreads();
   for (int c0 = a.s0; c0 < a.s1; c0 += kStep) {
     const int c = c0 + OK * a.wave;
-    put(hist + OK * a.wave, c + r);
-    fetch(c + kStep + r);
+    if (c < a.s1) put(hist + OK * a.wave, c + r);
+    if (c + kStep < a.s1) fetch(c + kStep + r);
     __syncthreads();
     if (c < a.s1) {
       float e[OK], d[OK];
