@@ -332,6 +332,49 @@ __global__ __launch_bounds__(256) void k_gauss_line_run(const float2* __restrict
   if (DOT) group_add<256>(d, dots);
 }
 
+// The z pass for lines of at most kShallow positions.  Taps past the line meet zeros and change
+// nothing but the sign of a sum that rounded to -0: one of them stands for all.
+template <bool DOT, typename TS>
+__global__ __launch_bounds__(NT) void k_gauss_shallow(const float2* __restrict__ src,
+                                                      TS* __restrict__ dog,
+                                                      const float* __restrict__ a,
+                                                      double* __restrict__ dots,
+                                                      const float* __restrict__ w1,
+                                                      const float* __restrict__ w2, int r1, int r2,
+                                                      float nz, int W, int L, i64 sa, i64 so,
+                                                      unsigned nxb, unsigned no) {
+  const LineAt la = line_at_block(nxb, no, L, L);
+  double sum[2] = {0.0, 0.0};
+  if (la.x < W) {
+    const i64 base = (i64)la.other * so + la.x;
+    float2 v[kShallow];
+#pragma unroll
+    for (int i = 0; i < kShallow; ++i)
+      if (i < L) v[i] = src[base + i * sa];  // uniform, as all that follow
+#pragma unroll
+    for (int c = 0; c < kShallow; ++c) {
+      if (c >= L) break;
+      float s1 = 0.0f, s2 = 0.0f;
+#pragma unroll
+      for (int i = 0; i < kShallow; ++i) {
+        if (i < L && i - c <= r1 && c - i <= r1) s1 = fmaf(w1[r1 + c - i], v[i].x, s1);
+        if (i < L && i - c <= r2 && c - i <= r2) s2 = fmaf(w2[r2 + c - i], v[i].y, s2);
+      }
+      if (c + r1 >= L) s1 = fmaf(w1[r1 + c - L], 0.0f, s1);
+      if (c + r2 >= L) s2 = fmaf(w2[r2 + c - L], 0.0f, s2);
+      const i64 idx = base + c * sa;
+      if (DOT) {
+        const double u = a[idx];
+        sum[0] += u * s1;
+        sum[1] += u * s2;
+      } else {
+        dog[idx] = cvt<TS>((s1 - s2) * nz);
+      }
+    }
+  }
+  if (DOT) group_add<NT>(sum, dots);
+}
+
 // ------------------------------------------------------------- compile-time radii
 // z pass as a column walker: one thread per line, a register ring of the last 2R+1
 // (G1, G2) pairs (zero outside the line), unrolled by the ring period so every index is
@@ -659,6 +702,12 @@ hipError_t gauss_z(const float2* src, TS* dog, const float* a, double* dots, con
   }
   HDOG_GAUSS_PAIRS(X)
 #undef X
+  if (D <= kShallow) {
+    const unsigned nxs = (unsigned)((n + NT - 1) / NT);
+    hipLaunchKernelGGL((k_gauss_shallow<DOT, TS>), dim3((unsigned)((i64)nxs * m)), dim3(NT), 0, s,
+                       src, dog, a, dots, w1, w2, r1, r2, nz, n, D, WH, (i64)W, nxs, (unsigned)m);
+    return hipGetLastError();
+  }
   const int R = std::max(r1, r2);
   const i64 nxb = (n + 63) / 64;
   int nseg, len;

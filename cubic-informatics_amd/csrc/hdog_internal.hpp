@@ -186,6 +186,15 @@ inline ZColumns z_columns(int W, int H) {
   return WH < (1ll << 31) - 256 ? ZColumns{(int)WH, 1} : ZColumns{W, H};
 }
 
+// Lines of at most this many positions have passes with a thread per line that holds it in
+// registers (k_minmax_shallow, k_box_shallow, k_gauss_shallow): a walk's work-group, its history
+// and its barriers would serve a step of which a line fills a part.  Along z, 4000 x 5000 columns
+// of one slice / 3000 x 3001 of eight, the walk and this: minima of radius 3, 344 and 61 us / 205
+// and 134; box of radius 5 with the normalization, 546 and 85 / 350 and 205; Gaussians of radius 1,
+// 482 and 110 / 258 and 181.  (The Gaussians' compiled walks stay: 190 us at radii 6 / 10 and
+// 8 x 1500 x 2001, 220 so.)
+constexpr int kShallow = 8;
+
 // ---- tile staging -----------------------------------------------------------------
 // Copies n elements global -> LDS with B independent loads in flight per lane before the
 // first LDS store (a plain strided loop waits for each load in turn).

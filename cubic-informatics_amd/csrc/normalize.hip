@@ -887,6 +887,31 @@ __global__ __launch_bounds__(256) void k_minmax_run(const void* __restrict__ src
   }
 }
 
+// The same for lines of at most kShallow positions.
+template <bool FROM_U16>
+__global__ __launch_bounds__(NT) void k_minmax_shallow(const void* __restrict__ src,
+                                                       uint32_t* __restrict__ dst, int W, int L,
+                                                       i64 sa, i64 so, int r, unsigned nxb,
+                                                       unsigned no) {
+  const LineAt la = line_at_block(nxb, no, L, L);
+  if (la.x >= W) return;
+  const i64 base = (i64)la.other * so + la.x;
+  uint32_t v[kShallow];
+#pragma unroll
+  for (int i = 0; i < kShallow; ++i)
+    if (i < L)  // uniform, as all that follow
+      v[i] = FROM_U16 ? pack(((const uint16_t*)src)[base + i * sa]) : ((const uint32_t*)src)[base + i * sa];
+#pragma unroll
+  for (int c = 0; c < kShallow; ++c) {
+    if (c >= L) break;
+    uint32_t m = v[c];
+#pragma unroll
+    for (int i = 0; i < kShallow; ++i)
+      if (i != c && i < L && i - c <= r && c - i <= r) m = pkmin(m, v[i]);
+    st_nt(dst + base + c * sa, m);
+  }
+}
+
 // out[o] = packed minimum of v[o] .. v[o + 2 R], in registers
 template <int R, int N>
 __device__ __forceinline__ void min8_regs(const uint32_t (&v)[N], uint32_t (&out)[OK]) {
@@ -1054,6 +1079,64 @@ __global__ __launch_bounds__(256) void k_box_run(const float2* __restrict__ src,
     shift_rows<256, STEP, 64>(B1, hist);
     shift_rows<256, STEP, 64>(B2, hist);
     __syncthreads();
+  }
+}
+
+// The same for lines of at most kShallow positions: the positions that repeat at the line's ends
+// are added as often as the window holds them, in its order.
+template <bool NORM, typename TS>
+__global__ __launch_bounds__(NT) void k_box_shallow(const float2* __restrict__ src,
+                                                    float2* __restrict__ dst,
+                                                    TS* __restrict__ norm,
+                                                    const uint16_t* __restrict__ img,
+                                                    float* __restrict__ ero,
+                                                    float* __restrict__ dil, float min_int, int W,
+                                                    int L, i64 sa, i64 so, int r, unsigned nxb,
+                                                    unsigned no, float k) {
+  const LineAt la = line_at_block(nxb, no, L, L);
+  if (la.x >= W) return;
+  const i64 base = (i64)la.other * so + la.x;
+  float2 v[kShallow], last = make_float2(0.0f, 0.0f);
+  uint16_t iv[kShallow];
+#pragma unroll
+  for (int i = 0; i < kShallow; ++i)
+    if (i < L) {  // uniform, as all that follow
+      v[i] = src[base + i * sa];
+      if (NORM) iv[i] = img[base + i * sa];
+      last = v[i];
+    }
+#pragma unroll
+  for (int c = 0; c < kShallow; ++c) {
+    if (c >= L) break;
+    float e = 0.0f, d = 0.0f;
+    // taps at or before the first position (all of them on a line of one), and after the last
+    const int first = L == 1 ? 2 * r + 1 : r - c + 1, beyond = L == 1 ? 0 : c + r - (L - 2);
+    for (int t = 0; t < first; ++t) {
+      e += v[0].x;
+      d += v[0].y;
+    }
+#pragma unroll
+    for (int i = 1; i < kShallow - 1; ++i)
+      if (i < L - 1 && i - c <= r && c - i <= r) {
+        e += v[i].x;
+        d += v[i].y;
+      }
+    for (int t = 0; t < beyond; ++t) {
+      e += last.x;
+      d += last.y;
+    }
+    const i64 idx = base + c * sa;
+    const float ve = e * k, vd = d * k;
+    if (NORM) {
+      const float I = (float)iv[c];
+      st_nt(norm + idx, (I >= min_int) ? (I - ve) / (vd - ve) : 0.0f);
+      if (ero) {
+        st_nt(ero + idx, ve);
+        st_nt(dil + idx, vd);
+      }
+    } else {
+      st_nt(dst + idx, make_float2(ve, vd));
+    }
   }
 }
 
@@ -1227,6 +1310,17 @@ hipError_t minmax_walk(const void* src, bool from_u16, uint32_t* dst, int W, int
 
 hipError_t minmax_line(const void* src, bool from_u16, uint32_t* dst, int W, int L, i64 sa,
                        i64 so, i64 n_other, int r, hipStream_t s) {
+  if (L <= kShallow) {
+    const unsigned nxb = (unsigned)((W + NT - 1) / NT);
+    const dim3 grid((unsigned)(nxb * n_other));
+    if (from_u16)
+      hipLaunchKernelGGL((k_minmax_shallow<true>), grid, dim3(NT), 0, s, src, dst, W, L, sa, so, r,
+                         nxb, (unsigned)n_other);
+    else
+      hipLaunchKernelGGL((k_minmax_shallow<false>), grid, dim3(NT), 0, s, src, dst, W, L, sa, so, r,
+                         nxb, (unsigned)n_other);
+    return hipGetLastError();
+  }
   // the configured radius has a walk with its window in registers (70 x 1080 x 1280 along y:
   // 166 us; the walk of any radius 180 at 8, 182 at 12; at 3 and 5 the two take the same)
   if (r == 10) return minmax_walk<10>(src, from_u16, dst, W, L, sa, so, n_other, s);
@@ -1275,7 +1369,14 @@ hipError_t box_line(const float2* src, float2* dst, TS* norm, const uint16_t* im
                     int W, int L, i64 sa, i64 so, i64 n_other, int r, hipStream_t s,
                     float* ero = nullptr, float* dil = nullptr) {
   const float k = 1.0f / (float)(2 * r + 1);
-  const bool ed = NORM && ero && dil;  // only the walk of any radius writes them
+  const bool ed = NORM && ero && dil;  // the walks of any radius write them
+  if (L <= kShallow) {
+    const unsigned nxb = (unsigned)((W + NT - 1) / NT);
+    hipLaunchKernelGGL((k_box_shallow<NORM, TS>), dim3((unsigned)(nxb * n_other)), dim3(NT), 0, s,
+                       src, dst, norm, img, ed ? ero : nullptr, ed ? dil : nullptr, min_int, W, L,
+                       sa, so, r, nxb, (unsigned)n_other, k);
+    return hipGetLastError();
+  }
   // (70 x 1080 x 1280, fused with the normalization: 267 us; the walk of any radius 275 at 4,
   // 277 at 6)
   if (r == 10 && !ed)
@@ -1369,7 +1470,7 @@ hipError_t launch_normalize(const uint16_t* img, TS* norm, void* tmp1, void* tmp
                        nyt, nxt, zlen);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     mark("normalize/minmax_zy", s);
-  } else if (rxy >= 4 && rxy <= kZyRadiusY && rz >= 4 && rz <= kZyRadiusZ) {
+    } else if (rxy >= 4 && rxy <= kZyRadiusY && rz >= 4 && rz <= kZyRadiusZ) {
     const unsigned nyg = (H + OK - 1) / OK;
     int nzs, zlen;
     line_segments(D, (i64)nxt * nyg * 8, 1024.0, 2.0, false, 2 * rz, &nzs, &zlen);

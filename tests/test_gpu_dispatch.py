@@ -626,3 +626,34 @@ def test_16_bit_storage_at_any_radii(hd, form, dtype, digits, rxy, rz, s):
             want = want.to(dtype).double()
             least = 2.0 ** -24 if dtype == torch.float16 else 0.0
             assert bool(((got.double() - want).abs() <= want.abs() * 2.0 ** -digits + least).all())
+
+
+# lines of at most eight slices, held in registers, and one more; windows within the line, at its
+# ends, past both, longer than a walk takes; E and D; values that a tap outside the line, or one
+# too many at its end, would change
+@pytest.mark.parametrize("depth", [1, 2, 3, 7, 8, 9])
+@pytest.mark.parametrize("rxy,rz", [(3, 1), (8, 5), (10, 10), (16, 2), (4, 24), (25, 3), (2, 30)])
+def test_normalize_of_few_slices(hd, depth, rxy, rz):
+    for shape in ((depth, 9, 257), (depth, 37, 6)):
+        img = noise(shape, 100 * depth + rz)
+        img[:, 2:4, 3:5] = 65535
+        want, e, d = oracle.normalize3d(img, 300, rxy, rz, return_ed=True)
+        got, ge, gd = hd.Normalize3DFilterWithBounds(img, 300, rxy, rz)
+        for a, b, name in ((got, want, "norm"), (ge, e, "E"), (gd, d, "D")):
+            np.testing.assert_array_equal(a.cpu().numpy(), b, err_msg=name)
+
+
+@pytest.mark.parametrize("depth", [1, 2, 5, 8, 9])
+@pytest.mark.parametrize("s,trunc", [((1.3, 0.3, 2.1, 0.5), 2.0), ((2.2, 1.1, 3.6, 1.8), 4.0),
+                                     ((1.0, 7.9, 1.5, 9.9), 4.0)])
+@pytest.mark.parametrize("finite", [True, False])
+def test_dog_of_few_slices(hd, depth, s, trunc, finite):
+    for shape in ((depth, 9, 257), (depth, 37, 6)):
+        rng = np.random.default_rng(depth)
+        norm = (rng.standard_normal(shape) * 0.3).astype(np.float32)
+        if not finite:
+            for v in (np.nan, np.inf, -np.inf):
+                norm[tuple(int(rng.integers(n)) for n in shape)] = v
+        hd.initGaussian3DKernel(*s, truncate=trunc)
+        ref, _ = oracle.dog3d(norm, *s, truncate=trunc, gamma=1.0)
+        np.testing.assert_array_equal(hd.DoG3DFilter(norm).cpu().numpy(), ref)

@@ -230,3 +230,24 @@ def test_region_sums_of_six_tiles_launch(runtime, tmp_path):
                     f"LIB={lib}", "EXTRA_HIPFLAGS=-O0 -Xarch_device -O0 -DHDOG_ACC_GY=3", lib],
                    check=True, capture_output=True, timeout=600)
     session(runtime, "region_sums_launch", library=lib)
+
+
+# ---- stacks of a few slices --------------------------------------------------------------
+def passes_along_z(rt, C, h):
+    # up to eight slices the passes along z of radii without kernels of their own are those of a
+    # thread per line: a walk's work-group per 64 lines takes up to four times as long
+    for depth in (1, 8, 9):
+        p = C.Params(width=300, height=200, depth=depth, radius_xy=16, radius_z=3,
+                     min_intensity=0.0, sigma_xy1=2.2, sigma_z1=1.1, sigma_xy2=3.6, sigma_z2=1.8,
+                     truncate=4.0, gamma=1.0)
+        n = ctypes.c_int64()
+        rt.host_clear()
+        assert C.hdog_run_device(h, None, ctypes.byref(p), 4096, None, None, None, None, None,
+                                 ctypes.byref(n)) == C.HDOG_OK
+        names = b" ".join(rt.host_launch_name(i) for i in range(rt.host_launches()))
+        for kernel in (b"k_minmax", b"k_box", b"k_gauss"):
+            assert (kernel + b"_shallow" in names) == (depth <= 8), (depth, kernel)
+
+
+def test_passes_along_few_slices(runtime):
+    session(runtime, "passes_along_z")
