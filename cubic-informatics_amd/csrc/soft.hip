@@ -937,14 +937,15 @@ __device__ __forceinline__ void add_clamped(const float* B, int pitch, int first
 
 // Adjoint of the normalization and, transposed, of its z boxes: the direct term into gv, (dL/dE,
 // dL/dD) summed along z into dst.  Bound by its 28 bytes per voxel: 184 us at 128 x 512 x 512,
-// radius 10 (in two passes, 152 + 112).
+// radius 10 (in two passes, 152 + 112).  rbox: the boxes' radius; r: that of the sums, which
+// need no more than the line's length, being zero past its ends.
 template <int R>
 __global__ __launch_bounds__(256) void k_soft_adj_z(const float* __restrict__ v,
                                                     const float2* __restrict__ ed,
                                                     const float* __restrict__ gn,
                                                     float* __restrict__ gv,
                                                     float2* __restrict__ dst, float min_int, int W,
-                                                    int D, i64 sa, int r, unsigned nxb,
+                                                    int D, i64 sa, int r, int rbox, unsigned nxb,
                                                     unsigned no, int len, float k) {
   extern __shared__ float sm_adjz[];
   const int hist = 2 * r;
@@ -993,8 +994,8 @@ __global__ __launch_bounds__(256) void k_soft_adj_z(const float* __restrict__ v,
       sum8<R>([&] { const float u = *p; p += 64; return u; }, r, e);
       p = B2 + OK * a.wave * 64 + a.l;
       sum8<R>([&] { const float u = *p; p += 64; return u; }, r, d);
-      add_clamped(B1 + a.l, 64, c0 - r, c, D, r, e);
-      add_clamped(B2 + a.l, 64, c0 - r, c, D, r, d);
+      add_clamped(B1 + a.l, 64, c0 - r, c, D, rbox, e);
+      add_clamped(B2 + a.l, 64, c0 - r, c, D, rbox, d);
       if (out) {
 #pragma unroll
         for (int j = 0; j < OK; ++j)
@@ -1331,7 +1332,10 @@ hipError_t launch_soft_normalize(const float* v, float* norm, float2* ed, uint32
     const ZColumns c = z_columns(W, H);
     const LineGrid g = run_grid(c.n, D, c.rows, 2 * rz);
     const float kxy = 1.0f / (float)(2 * rxy + 1), kz = 1.0f / (float)(2 * rz + 1);
-    const size_t zrows = (size_t)(2 * rz + kStep) * 64 * 4;
+    // the extremes of a window past both ends of its line are those of one that reaches them
+    const int mz = std::min(rz, std::max(1, D - 1));
+    const LineGrid m = run_grid(c.n, D, c.rows, 2 * mz);
+    const size_t zrows = (size_t)(2 * rz + kStep) * 64 * 4, mrows = (size_t)(2 * mz + kStep) * 64 * 4;
     hipError_t e = dispatch_short(rxy, [&](auto rs) {
       constexpr int R = decltype(rs)::value;
       hipLaunchKernelGGL((k_soft_arg_xy<R>), dim3(x.blocks), dim3(256), arg_xy_lds(rxy), s, v, pk, pk + N,
@@ -1339,10 +1343,10 @@ hipError_t launch_soft_normalize(const float* v, float* norm, float2* ed, uint32
       return hipGetLastError();
     });
     if (e != hipSuccess) return e;
-    e = dispatch_short(rz, [&](auto rs) {
+    e = dispatch_short(mz, [&](auto rs) {
       constexpr int R = decltype(rs)::value;
-      hipLaunchKernelGGL((k_soft_arg_z<R>), dim3(g.blocks), dim3(256), 3 * zrows, s, pk, pk + N,
-                         pk + 2 * N, pair, arg, arg + N, c.n, W, H, D, rxy, rz, g.nxb, g.no, g.len);
+      hipLaunchKernelGGL((k_soft_arg_z<R>), dim3(m.blocks), dim3(256), 3 * mrows, s, pk, pk + N,
+                         pk + 2 * N, pair, arg, arg + N, c.n, W, H, D, rxy, mz, m.nxb, m.no, m.len);
       return hipGetLastError();
     });
     if (e != hipSuccess) return e;
@@ -1353,6 +1357,12 @@ hipError_t launch_soft_normalize(const float* v, float* norm, float2* ed, uint32
       return hipGetLastError();
     });
     if (e != hipSuccess) return e;
+    if (D <= kShallow) {
+      e = launch_box_pair(exy, ed, c.n, D, WH, W, c.rows, rz, s);
+      if (e != hipSuccess) return e;
+      hipLaunchKernelGGL(k_soft_norm, dim3(grid_for(N)), dim3(NT), 0, s, v, ed, norm, min_int, N);
+      return hipGetLastError();
+    }
     return dispatch_short(rz, [&](auto rs) {
       constexpr int R = decltype(rs)::value;
       hipLaunchKernelGGL((k_soft_box_norm<R>), dim3(g.blocks), dim3(256), 2 * zrows, s, exy, v, ed,
@@ -1418,12 +1428,13 @@ hipError_t launch_soft_normalize_adjoint(const float* v, const float2* ed, const
   float2* q0 = (float2*)scratch;
   if (rxy <= kArgRadius && rz <= kArgRadius) {
     const ZColumns c = z_columns(W, H);
-    const LineGrid g = run_grid(c.n, D, c.rows, 2 * rz);
-    hipError_t e = dispatch_short(rz, [&](auto rs) {
+    const int sz = std::min(rz, D);
+    const LineGrid g = run_grid(c.n, D, c.rows, 2 * sz);
+    hipError_t e = dispatch_short(sz, [&](auto rs) {
       constexpr int R = decltype(rs)::value;
       hipLaunchKernelGGL((k_soft_adj_z<R>), dim3(g.blocks), dim3(256),
-                         2 * (size_t)(2 * rz + kStep) * 64 * 4, s, v, ed, gn, gv, q0, min_int,
-                         c.n, D, WH, rz, g.nxb, g.no, g.len, 1.0f / (float)(2 * rz + 1));
+                         2 * (size_t)(2 * sz + kStep) * 64 * 4, s, v, ed, gn, gv, q0, min_int,
+                         c.n, D, WH, sz, rz, g.nxb, g.no, g.len, 1.0f / (float)(2 * rz + 1));
       return hipGetLastError();
     });
     if (e != hipSuccess) return e;

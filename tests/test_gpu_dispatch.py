@@ -657,3 +657,28 @@ def test_dog_of_few_slices(hd, depth, s, trunc, finite):
         hd.initGaussian3DKernel(*s, truncate=trunc)
         ref, _ = oracle.dog3d(norm, *s, truncate=trunc, gamma=1.0)
         np.testing.assert_array_equal(hd.DoG3DFilter(norm).cpu().numpy(), ref)
+
+
+# soft normalization of a few slices: windows past both ends of a line, ties among the voxels that
+# they repeat; either side of the depth that has passes of its own
+@pytest.mark.parametrize("depth", [1, 2, 8, 9])
+@pytest.mark.parametrize("rxy,rz", [(3, 2), (8, 5), (4, 23)])
+def test_soft_normalization_of_few_slices(hd, depth, rxy, rz):
+    import torch
+    from hdog import _capi as C
+    for shape in ((depth, 13, 133), (depth, 37, 6)):
+        v = np.round(np.random.default_rng(rz).standard_normal(shape) * 2).astype(np.float32)
+        D, H, W = shape
+        vd = torch.from_numpy(v).to(hd.device)
+        n = torch.empty_like(vd)
+        ed = torch.empty(shape + (2,), dtype=torch.float32, device=hd.device)
+        arg = torch.empty((2,) + shape, dtype=torch.int32, device=hd.device)
+        p = C.ctypes.c_void_p
+        hd._check(C.hdog_soft_normalize_forward(hd._h, hd._stream(), p(vd.data_ptr()),
+                                                p(n.data_ptr()), p(ed.data_ptr()),
+                                                p(arg.data_ptr()), -0.25, W, H, D, rxy, rz))
+        with np.errstate(all="ignore"):
+            wn, wed, warg = soft_normalize_by_hand(v, -0.25, rxy, rz)
+        np.testing.assert_array_equal(arg.cpu().numpy().view(np.uint32), warg)
+        np.testing.assert_array_equal(ed.cpu().numpy(), wed)
+        np.testing.assert_array_equal(n.cpu().numpy(), wn)

@@ -251,3 +251,17 @@ def passes_along_z(rt, C, h):
 
 def test_passes_along_few_slices(runtime):
     session(runtime, "passes_along_z")
+
+
+def soft_passes_along_z(rt, C, h):
+    for depth in (1, 8, 9):
+        rt.host_clear()
+        assert C.hdog_soft_normalize_forward(h, None, 4096, 8192, 12288, 16384, 0.0, 300, 200,
+                                             depth, 8, 5) == C.HDOG_OK
+        names = b" ".join(rt.host_launch_name(i) for i in range(rt.host_launches()))
+        assert (b"k_box_shallow" in names) == (depth <= 8), depth
+        assert (b"k_soft_box_norm" in names) == (depth > 8), depth
+
+
+def test_soft_passes_along_few_slices(runtime):
+    session(runtime, "soft_passes_along_z")
