@@ -634,6 +634,11 @@ template <typename TS>
 hipError_t gauss_xy_run(const TS* src, float2* dst, const float* wx1, const float* wx2,
                         const float* wy1, const float* wy2, int rx1, int rx2, int ry1, int ry2,
                         int W, int H, int D, hipStream_t s, int segments) {
+  // taps past a plane of few rows meet zeros: one of them stands for all (k_gauss_shallow)
+  wy1 += ry1 - std::min(ry1, H);
+  wy2 += ry2 - std::min(ry2, H);
+  ry1 = std::min(ry1, H);
+  ry2 = std::min(ry2, H);
   const int RX = std::max(rx1, rx2), RY = std::max(ry1, ry2);
   const int nxs = (W + 63) / 64;
   const int nw = xy_run_waves(RX, RY);
@@ -727,7 +732,7 @@ hipError_t gauss_z(const float2* src, TS* dog, const float* a, double* dots, con
 
 WalkShape gauss_walk_shape(int r1, int r2, int W, int H, int D) {
   const int R = std::max(r1, r2);
-  if (!gauss_row_walker(r1, r2, W, H, D)) return xy_run_shape(R, R, W, D);
+  if (!gauss_row_walker(r1, r2, W, H, D)) return xy_run_shape(R, std::min(R, H), W, D);
   return {(i64)((W + 63) / 64) * D, 2 * R + 1, 2 * R};
 }
 

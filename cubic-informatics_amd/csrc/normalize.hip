@@ -1505,7 +1505,11 @@ hipError_t launch_normalize(const uint16_t* img, TS* norm, void* tmp1, void* tmp
                        (float4*)tmp1, W, H, nxs, nys, rows, k);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     mark("normalize/minmax_x_box_xy", s);
-  } else if (rxy <= kRunRadius) {
+  } else if (rxy <= kRunRadius && 2 * H >= 3 * rxy) {
+    // (a walk forms the x windows of 2 rxy rows above and below a plane's own; on planes of fewer
+    // rows than half of those, the two passes below are sooner done: 300 x 5 x 2000 at radius 8
+    // 75 us, the walk 104; x 8 at 16: 98, 161; x 33 at 23: 351, 557.  300 x 15 x 300 at 8: 38, 35;
+    // 100 x 30 x 300 at 16: 38, 32)
     const int nxs = (W + 63) / 64;
     int nys, rows;
     walk_segments(H, norm_walk_shape(rxy, W, D), &nys, &rows, segments);

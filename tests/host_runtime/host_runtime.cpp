@@ -57,6 +57,7 @@ size_t host_device_peak() { return device_peak; }
 int host_launches() { return (int)launches.size(); }
 const char* host_launch_name(int i) { return launches[i].name.c_str(); }
 unsigned host_launch_blocks(int i) { return launches[i].grid.x; }
+size_t host_launch_lds(int i) { return launches[i].lds; }
 // what was kept of the arguments of launch i
 const void* host_launch_args(int i) { return launches[i].args.data(); }
 // where the device allocation that holds p ends (0: none does)

@@ -16,6 +16,7 @@ def load(runtime):
     runtime, and torch, which the binding imports for its runtime alone, is left out."""
     rt = ctypes.CDLL(runtime, ctypes.RTLD_GLOBAL)
     rt.host_device_peak.restype = ctypes.c_size_t
+    rt.host_launch_lds.restype = ctypes.c_size_t
     rt.host_launch_name.restype = ctypes.c_char_p
     rt.host_launch_args.restype = ctypes.c_void_p
     rt.host_allocation_end.argtypes = [ctypes.c_size_t]

@@ -682,3 +682,29 @@ def test_soft_normalization_of_few_slices(hd, depth, rxy, rz):
         np.testing.assert_array_equal(arg.cpu().numpy().view(np.uint32), warg)
         np.testing.assert_array_equal(ed.cpu().numpy(), wed)
         np.testing.assert_array_equal(n.cpu().numpy(), wn)
+
+
+# planes of few rows: either side of the row count where the walk along x and y begins (2 H = 3 r)
+@pytest.mark.parametrize("shape,r", [((6, 11, 200), 8), ((6, 12, 200), 8), ((5, 35, 130), 24),
+                                     ((5, 36, 130), 24), ((400, 1, 70), 3), ((7, 4, 300), 3)])
+def test_normalize_of_few_rows(hd, shape, r):
+    img = noise(shape, r)
+    got, ge, gd = hd.Normalize3DFilterWithBounds(img, 300, r, 4)
+    want, e, d = oracle.normalize3d(img, 300, r, 4, return_ed=True)
+    for a, b, name in ((got, want, "norm"), (ge, e, "E"), (gd, d, "D")):
+        np.testing.assert_array_equal(a.cpu().numpy(), b, err_msg=name)
+
+
+# Gaussians longer than the plane has rows, whose taps past it are left out but for one
+@pytest.mark.parametrize("rows", [1, 3, 8, 31, 32, 33])
+@pytest.mark.parametrize("finite", [True, False])
+def test_dog_of_few_rows(hd, rows, finite):
+    rng = np.random.default_rng(rows)
+    norm = (rng.standard_normal((11, rows, 130)) * 0.3).astype(np.float32)
+    if not finite:
+        for v in (np.nan, np.inf, -np.inf):
+            norm[tuple(int(rng.integers(n)) for n in norm.shape)] = v
+    for s in ((7.9, 1.1, 9.9, 1.8), (2.0, 2.0, 3.2, 3.2)):
+        hd.initGaussian3DKernel(*s, truncate=4.0)
+        ref, _ = oracle.dog3d(norm, *s, truncate=4.0, gamma=1.0)
+        np.testing.assert_array_equal(hd.DoG3DFilter(norm).cpu().numpy(), ref)

@@ -265,3 +265,25 @@ def soft_passes_along_z(rt, C, h):
 
 def test_soft_passes_along_few_slices(runtime):
     session(runtime, "soft_passes_along_z")
+
+
+def passes_over_few_rows(rt, C, h):
+    # the walk along x and y forms a window's rows above and below the plane: not on planes of
+    # fewer; a Gaussian's history is no longer than the plane
+    for rows, walks in ((8, False), (300, True)):
+        p = C.Params(width=2000, height=rows, depth=100, radius_xy=16, radius_z=3,
+                     min_intensity=0.0, sigma_xy1=7.9, sigma_z1=1.1, sigma_xy2=9.9, sigma_z2=1.8,
+                     truncate=4.0, gamma=1.0)
+        n = ctypes.c_int64()
+        rt.host_clear()
+        assert C.hdog_run_device(h, None, ctypes.byref(p), 4096, None, None, None, None, None,
+                                 ctypes.byref(n)) == C.HDOG_OK
+        at = {rt.host_launch_name(i): rt.host_launch_lds(i) for i in range(rt.host_launches())}
+        assert any(b"k_norm_xy_run" in k for k in at) == walks, rows
+        gauss = [v for k, v in at.items() if b"k_gauss_xy_run" in k]
+        # two planes of the rows that windows of radius 40 reach, 65 words each
+        assert len(gauss) == 1 and (gauss[0] > 2 * 80 * 65 * 4) == walks, gauss
+
+
+def test_passes_over_planes_of_few_rows(runtime):
+    session(runtime, "passes_over_few_rows")
