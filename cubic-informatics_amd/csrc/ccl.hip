@@ -264,9 +264,14 @@ __global__ __launch_bounds__(NTR) void k_cand_local(const float* __restrict__ ca
   // (a tile's voxels have RTV / 64 words; the tiles' voxels cover the volume's)
   if (roots) {
     constexpr int WORDS = RTV / 64;
-    for (int i = (int)threadIdx.x; i < 2 * WORDS; i += NTR) {
-      const i64 w = (i64)tile * WORDS + i % WORDS;
-      if (w < root_words) (i < WORDS ? roots : multi)[w] = 0ull;
+    if constexpr (2 * WORDS <= NTR) {  // four rows, or eight: a word per thread, both bitmaps
+      const i64 w = (i64)tile * WORDS + (threadIdx.x & (WORDS - 1));
+      if (threadIdx.x < 2 * WORDS && w < root_words) (threadIdx.x < WORDS ? roots : multi)[w] = 0ull;
+    } else {
+      for (int i = (int)threadIdx.x; i < 2 * WORDS; i += NTR) {
+        const i64 w = (i64)tile * WORDS + i % WORDS;
+        if (w < root_words) (i < WORDS ? roots : multi)[w] = 0ull;
+      }
     }
   }
   if (tile == 0)  // and the region numbering's chunk counts
