@@ -570,8 +570,9 @@ __global__ __launch_bounds__(NTR) void k_label_rows(const float* __restrict__ ca
   const CandTile T = cand_tile(tile, W, H, D, nbx, nby);
   const uint32_t Wu = (uint32_t)W, WH = Wu * (uint32_t)H;
   __shared__ __align__(16) uint32_t lv[RTV];
-#pragma unroll
-  for (int k = 0; k < RTV / (4 * NTR); ++k)
+  // (the tile's slices within the volume only: of a plane, a sixteenth of the tile)
+  const int nv = T.ez * (RTX * RTY);
+  for (int k = 0; 4 * k * NTR < nv; ++k)
     *reinterpret_cast<uint4*>(lv + 4 * (threadIdx.x + k * NTR)) = make_uint4(0u, 0u, 0u, 0u);
   __syncthreads();
   const float* rec = cand + (size_t)tile * kCandTile * rec_words;
@@ -582,7 +583,10 @@ __global__ __launch_bounds__(NTR) void k_label_rows(const float* __restrict__ ca
   if (vec) {  // width and volume aligned: a quad lies in the row or outside it
     typedef uint32_t u4 __attribute__((ext_vector_type(4)));
     const bool nt = whole_lines((i64)W * 4);
-    for (int e = (int)threadIdx.x; e < RTV / 4; e += NTR) {
+#pragma unroll
+    for (int k = 0; k < RTV / 4 / NTR; ++k) {
+      if (4 * k * NTR >= nv) break;
+      const int e = (int)threadIdx.x + k * NTR;
       const int lx = e % (RTX / 4) * 4, row = e / (RTX / 4), ly = row % RTY, lz = row / RTY;
       if (lx < T.ex && ly < T.ey && lz < T.ez) {
         u4* p = reinterpret_cast<u4*>(base + (size_t)lz * WH + (size_t)ly * Wu + lx);
@@ -597,7 +601,7 @@ __global__ __launch_bounds__(NTR) void k_label_rows(const float* __restrict__ ca
       }
     }
   } else {
-    for (int e = (int)threadIdx.x; e < RTV; e += NTR) {
+    for (int e = (int)threadIdx.x; e < nv; e += NTR) {
       const int lx = e % RTX, row = e / RTX, ly = row % RTY, lz = row / RTY;
       if (lx < T.ex && ly < T.ey && lz < T.ez)
         base[(size_t)lz * WH + (size_t)ly * Wu + lx] = lv[e];
