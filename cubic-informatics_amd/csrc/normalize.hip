@@ -45,17 +45,11 @@ __device__ __forceinline__ uint32_t pkmin(uint32_t a, uint32_t b) {
 // gfx950, interleaved chains do not (min is exact, so the order is free)
 template <int R>
 __device__ __forceinline__ uint32_t mid_min(const uint32_t* w) {
-  if constexpr (2 * R - 2 < 4) {  // w[3 .. 2R]: a short chain
-    uint32_t m = w[3];
+  static_assert(2 * R >= 6, "four chains");
+  uint32_t m[4] = {w[3], w[4], w[5], w[6]};
 #pragma unroll
-    for (int t = 4; t <= 2 * R; ++t) m = pkmin(m, w[t]);
-    return m;
-  } else {
-    uint32_t m[4] = {w[3], w[4], w[5], w[6]};
-#pragma unroll
-    for (int t = 7; t <= 2 * R; ++t) m[(t - 3) & 3] = pkmin(m[(t - 3) & 3], w[t]);
-    return pkmin(pkmin(m[0], m[1]), pkmin(m[2], m[3]));
-  }
+  for (int t = 7; t <= 2 * R; ++t) m[(t - 3) & 3] = pkmin(m[(t - 3) & 3], w[t]);
+  return pkmin(pkmin(m[0], m[1]), pkmin(m[2], m[3]));
 }
 __device__ __forceinline__ uint32_t pack(uint32_t v) { return v | ((65535u - v) << 16); }
 
@@ -1539,7 +1533,7 @@ hipError_t launch_normalize(const uint16_t* img, TS* norm, void* tmp1, void* tmp
                        (float2*)tmp1, W, nrows, rxy, nct, k);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     mark("normalize/minmax_x_box_x", s);
-    if ((e = box_line<false, TS>((const float2*)tmp1, (float2*)tmp2, nullptr, nullptr, 0.0f, W, H,
+    if ((e = box_line<false, float>((const float2*)tmp1, (float2*)tmp2, nullptr, nullptr, 0.0f, W, H,
                                  W, WH, D, rxy, s)) != hipSuccess)
       return e;
     mark("normalize/box_y", s);
@@ -1548,7 +1542,7 @@ hipError_t launch_normalize(const uint16_t* img, TS* norm, void* tmp1, void* tmp
   // box along z fused with the normalization
   if (ero && dil && rz > kRunRadius) {  // E and D by a z pass of their own, then split
     float2* ed = exy == (const float2*)tmp1 ? (float2*)tmp2 : (float2*)tmp1;
-    if ((e = box_line<false, TS>(exy, ed, nullptr, nullptr, 0.0f, zc.n, D, WH, W, zc.rows, rz, s)) !=
+    if ((e = box_line<false, float>(exy, ed, nullptr, nullptr, 0.0f, zc.n, D, WH, W, zc.rows, rz, s)) !=
         hipSuccess)
       return e;
     const i64 nb = std::min<i64>((N + NT - 1) / NT, 1 << 20);
