@@ -260,10 +260,6 @@ struct CandRecords {
   i64 ntiles = 0;
 };
 
-// With cand.rec the components come from launch_ccl_candidates (their root bits already
-// in ctx->rmask, each record's label in cand.rlab) and the region sums from the records
-// (labels and hess unused); else from the label volume (final labels, only read) and the
-// materialized Hessian.
 // What the caller's array [p, p + bytes) is: page-locked host memory that the device can write
 // (*view is the device's address of p), pageable memory, or something only the runtime's copies
 // handle.
@@ -329,6 +325,10 @@ int copy_out(hdog_ctx* ctx, const CopyList& want, hipStream_t s) {
   return HDOG_OK;
 }
 
+// With cand.rec the components come from launch_ccl_candidates (their root bits already
+// in ctx->rmask, each record's label in cand.rlab) and the region sums from the records
+// (labels and hess unused); else from the label volume (final labels, only read) and the
+// materialized Hessian.
 template <typename TH, typename TN>
 int regional_features_t(hdog_ctx* ctx, hipStream_t s, uint32_t* labels, const TH* hess,
                         const TN* norm, const uint16_t* img, int W, int H, int D, int is_ave,
@@ -379,7 +379,8 @@ int regional_features_t(hdog_ctx* ctx, hipStream_t s, uint32_t* labels, const TH
       o.hess = (float*)ctx->o_hess.p;
       o.isum = (u64*)ctx->o_isum.p;
       o.imax = (uint16_t*)ctx->o_imax.p;
-      // (a 26-connected labeling has at most N / 8 regions)
+      // (N / 8, about the most regions that many slices hold, only sizes the grid, which strides:
+      // a few slices or rows may hold more)
       HIPCHK(launch_region_finalize(acc, dR, cap, std::min(cap, N / 8 + 2), is_ave, o, pitch,
                                     s));
     }

@@ -4,16 +4,16 @@
 // weights) -> z (z weights) with zero padding; every output is the FMA chain
 // sum = fmaf(w[r-j], s[c+j], sum), j = -r..r, from 0.  dog = (G1 - G2) * normalizer.
 //
-// MI355X design: both Gaussians are evaluated from one read of each tile.  The x pass
-// reads `norm` once and writes (G1_x, G2_x) as float2, the y pass works on the pair, and
-// the z pass forms the difference directly, so `norm` is read once and the two
-// intermediate volumes of the reference become one interleaved stream.  Intermediates
-// stay FP32 whatever the storage type of norm / dog.
+// MI355X design: both Gaussians are evaluated from one read of `norm`.  The x and y passes are
+// one walk over the rows of a plane, which writes the pair (G1, G2) as float2, and the z pass
+// forms the difference of the pair directly, so the reference's intermediate volumes become
+// one interleaved stream.  Intermediates stay FP32 whatever the storage type of norm / dog.
 //
-// Radius pairs (r1, r2) that occur in practice have compile-time kernels: the x and y passes
-// fused in a row walker, the z pass as a column walker (one thread per line, a register ring,
-// every input read once, no LDS).  Other radii, and the smallest stacks along x and y, have
-// walks with their history in LDS that form eight outputs at a time.
+// Radius pairs (r1, r2) that occur in practice have compile-time kernels: a row walker along x
+// and y, and along z a column walker (one thread per line, a register ring, every input read
+// once, no LDS).  Other radii, and the smallest stacks along x and y, have walks with their
+// history in LDS that form eight outputs at a time; along z up to eight slices of those radii
+// are a thread's registers.
 #include "hdog_internal.hpp"
 
 namespace hdog {
@@ -243,7 +243,7 @@ __global__ __launch_bounds__(64 * NW) void k_gauss_xy_run(
   }
 }
 
-// One pass along y (sa = W) or z (sa = W H) for any radii: a work-group of four waves walks a
+// The z pass (sa = W H) for any radii: a work-group of four waves walks a
 // segment of 64 x-adjacent lines, eight positions per wave and step, through two LDS planes of
 // the last 2R + 32 positions (zero outside the line).  Bound by its 12 or 16 bytes per voxel
 // for short windows (61 x 900 x 1111 along z at radii 4 / 7: 377 us with one output per thread

@@ -9,19 +9,18 @@
 //   * Erosion and dilation run together: each voxel is packed into one 32-bit word
 //     (v, 65535 - v) so a single v_pk_min_u16 advances both filters (max(v) =
 //     65535 - min(65535 - v)).
-//   * Each 1-D min/max pass is van Herk / Gil-Werman (3 packed mins per output for any
-//     radius) on an LDS tile; tiles are x-contiguous so every HBM access coalesces.
 //   * Min/max over a clamped box is separable and exact in any order, so the y and z
 //     passes run first (in one z walk for radius 10, k_minmax_zy_walk, and for most others,
-//     k_minmax_zy_run; else z then y) and the x pass is fused with the x pass of the box filter (sums of integers,
-//     exact in any order, so a sliding sum is used).  The y and z box passes sum FP32
-//     values and keep the reference's sequential order (c-r .. c+r); the z pass is fused
-//     with the normalization.
-//   * For the radii in use, the z box pass (and the separate y / z min/max passes) are
-//     column walkers: one thread per line keeps a compile-time-sized register ring, reads
-//     every input once and needs no LDS.  Other radii up to kRunRadius, and stacks too small
-//     for the row walker, have walks with the radius at run time and their history in LDS,
-//     larger radii the LDS-tile kernels.
+//     k_minmax_zy_run; else z then y) and the x pass is fused with the box filter along x (sums
+//     of integers, exact in any order, so a sliding sum is used) and y.  The y and z box passes
+//     sum FP32 values and keep the reference's sequential order (c-r .. c+r); the z pass is
+//     fused with the normalization.
+//   * Radius 10 has column walkers along z (one thread per line, a compile-time-sized register
+//     ring, every input read once, no LDS) and a row walker along x and y.  Other radii up to
+//     kRunRadius, and stacks too small for the row walker, have walks with the radius at run time
+//     and their history in LDS; lines of a few positions are a thread's registers, and planes
+//     of a few rows have their x and y passes apart.  Larger radii take LDS tiles, min/max by
+//     van Herk / Gil-Werman (3 packed mins per output).
 #include "run8.hpp"
 
 namespace hdog {
