@@ -555,16 +555,19 @@ __global__ __launch_bounds__(NTR) void k_cand_flatten(const float* __restrict__ 
 }
 
 // The full label volume, in place of the parent array: the tile's labels are laid out in LDS
-// and leave as whole rows, zeros included, 16 bytes per lane where the rows are aligned
-// (vec), so the volume is written once.  A kernel of its own, since the flatten still reads
-// other tiles' entries.  Bound by its 4 bytes per voxel: 102 us for 96 x 1080 x 1280 (5.2
+// and leave as whole rows, zeros included, 16 bytes per lane where the rows are aligned, so the
+// volume is written once; by streaming stores where the rows start on whole lines
+// (96 x 1080 x 1280, the whole call: 428 us, 481 plain; elsewhere they are the slower ones).  A
+// kernel of its own, since the flatten still reads other tiles' entries.  Bound by its 4 bytes per voxel: 102 us for 96 x 1080 x 1280 (5.2
 // TB/s), the flatten 41; clearing the volume first (74 us) and storing each label where it
 // belongs from the flatten (132 us) took 206.
+constexpr int kWords = 0, kQuads = 1, kQuadsStreamed = 2;
+template <int STORE>
 __global__ __launch_bounds__(NTR) void k_label_rows(const float* __restrict__ cand,
                                                    const uint32_t* __restrict__ cand_cnt,
                                                    const uint32_t* __restrict__ rlab,
                                                    uint32_t* __restrict__ P, int W, int H, int D,
-                                                   int nbx, int nby, int rec_words, int vec) {
+                                                   int nbx, int nby, int rec_words) {
   const unsigned tile = xcd_tile(blockIdx.x, gridDim.x);
   const uint32_t n = cand_cnt[tile];
   const CandTile T = cand_tile(tile, W, H, D, nbx, nby);
@@ -580,9 +583,8 @@ __global__ __launch_bounds__(NTR) void k_label_rows(const float* __restrict__ ca
   for (uint32_t i = threadIdx.x; i < n; i += NTR) lv[__float_as_uint(rec[i])] = rl[i];
   __syncthreads();
   uint32_t* base = P + (size_t)T.z0 * WH + (size_t)T.y0 * Wu + T.x0;
-  if (vec) {  // width and volume aligned: a quad lies in the row or outside it
+  if (STORE != kWords) {  // width and volume aligned: a quad lies in the row or outside it
     typedef uint32_t u4 __attribute__((ext_vector_type(4)));
-    const bool nt = whole_lines((i64)W * 4);
 #pragma unroll
     for (int k = 0; k < RTV / 4 / NTR; ++k) {
       if (4 * k * NTR >= nv) break;
@@ -591,13 +593,10 @@ __global__ __launch_bounds__(NTR) void k_label_rows(const float* __restrict__ ca
       if (lx < T.ex && ly < T.ey && lz < T.ez) {
         u4* p = reinterpret_cast<u4*>(base + (size_t)lz * WH + (size_t)ly * Wu + lx);
         const u4 v = *reinterpret_cast<const u4*>(lv + 4 * e);
-        if (nt) {
+        if (STORE == kQuadsStreamed)
           __builtin_nontemporal_store(v, p);
-        } else {
-          asm volatile("");  // keeps the two stores apart: merged into one, both would be plain
+        else
           *p = v;
-          asm volatile("");
-        }
       }
     }
   } else {
@@ -739,9 +738,16 @@ hipError_t launch_ccl_candidates(const float* cand, const uint32_t* cand_cnt, i6
   if ((e = hipGetLastError()) != hipSuccess) return e;
   mark("ccl/cand_flatten", s);
   if (dense) {
-    const int vec = W % 4 == 0 && (uintptr_t)P % 16 == 0;
-    hipLaunchKernelGGL(k_label_rows, dim3((unsigned)ntiles), dim3(NTR), 0, s, cand, cand_cnt,
-                       (const uint32_t*)rlab, P, W, H, D, nbx, nby, rec_words, vec);
+    auto rows = [&](auto store) {
+      hipLaunchKernelGGL((k_label_rows<decltype(store)::value>), dim3((unsigned)ntiles), dim3(NTR), 0,
+                         s, cand, cand_cnt, (const uint32_t*)rlab, P, W, H, D, nbx, nby, rec_words);
+    };
+    if (W % 4 != 0 || (uintptr_t)P % 16 != 0)
+      rows(std::integral_constant<int, kWords>());
+    else if (whole_lines((i64)W * 4))
+      rows(std::integral_constant<int, kQuadsStreamed>());
+    else
+      rows(std::integral_constant<int, kQuads>());
     mark("ccl/label_rows", s);
   }
   return hipGetLastError();
