@@ -136,9 +136,10 @@ __global__ __launch_bounds__(NT) void k_soft_grad_h(float* __restrict__ cand,
 // touching memory.  Nothing dense but the result leaves the chip.  Bound by instruction issue
 // (seven row lookups and ten loads for three output rows).  As dense volumes dL/dH went out and back
 // in two passes: 262 + 132 us at 128 x 512 x 512 with 7 % masked, and 76 for the dot product
-// (172 here; with tiles of 64 x 8 x 8 in LDS, one element at a time, 820).
+// (154 here; with tiles of 64 x 8 x 8 in LDS, one element at a time, 820).
 // Rows of outputs of a wave: with more the registers leave fewer waves, with fewer more rows
-// are laid out twice (us at 128 x 512 x 512: 2: 199, 3: 172, 4: 221, 6: 215, 8: 290).
+// are laid out twice (us at 128 x 512 x 512, each row's block looked up for itself: 2: 199, 3: 172,
+// 4: 221, 6: 215, 8: 290; looked up once per slice and side, 3: 154).
 constexpr int AR = 3;
 constexpr int kAdjX = 60;   // columns of outputs: lanes 2 .. 61
 constexpr int AI = AR + 4;  // rows of inputs, two beyond either side
